@@ -122,6 +122,7 @@ void parallel_copy(std::initializer_list<CopyJob> jobs)
         w.join();
     }
 }
+constexpr int64_t kPqTrainBytes = (int64_t)4 << 30;   // sub-vectors, codes and member lists of the sub-quantizers trained together
 constexpr int64_t kCoarseExactMaxMacs = (int64_t)1 << 27;   // queries x centroids x dims up to which a search selects its lists exactly
 
 // ---- arena kernels ------------------------------------------------------------------------------
@@ -418,12 +419,22 @@ __global__ __launch_bounds__(256) void sort_segments_kernel(int64_t *__restrict_
 }
 
 // Re-seeds empty clusters by splitting the most populated one (symmetric perturbation), in ascending order of the
-// empty clusters, each split seeing the counts the earlier ones left.  One workgroup.
+// empty clusters, each split seeing the counts the earlier ones left.  One workgroup per quantizer of k clusters
+// (the coarse one, or every sub-quantizer).
 __global__ __launch_bounds__(1024) void split_empty_kernel(float *__restrict__ cent, unsigned long long *__restrict__ cnt,
                                                            int64_t k, int dim)
 {
     __shared__ long long s_val[1024], s_idx[1024];
     const int tid = threadIdx.x;
+    cent += (int64_t)blockIdx.x * k * dim;
+    cnt += (int64_t)blockIdx.x * k;
+    bool some = false;   // the usual case, no empty cluster, costs one pass over the counts
+    for (int64_t c = tid; c < k; c += 1024) {
+        some |= cnt[c] == 0;
+    }
+    if (!__syncthreads_or(some)) {
+        return;
+    }
     long long last = -1;
     while (true) {
         long long mine = INT64_MAX;
@@ -501,80 +512,6 @@ __global__ __launch_bounds__(256) void normalise_rows_kernel(float *__restrict__
         for (int t = 0; t < dim; t++) {
             cent[c * dim + t] = (float)(cent[c * dim + t] / nn);
         }
-    }
-}
-
-// Sub-quantizer update of PQ training: acc[m][k][t] = sum in float64, IN SAMPLE ORDER, of x[i][m*dsub + t]
-// over the samples i whose code for sub-quantizer m is k; cnt[m][k] = their number.  One workgroup
-// per sub-quantizer, thread k owns codeword k: tiles of 256 samples (their sub-vectors and codes) are
-// staged in LDS and every thread walks the tile in order, so each sum is built in the order of the
-// host loop this replaces, whatever the hardware's scheduling.
-template <int DSUB>
-__global__ __launch_bounds__(256) void pq_update_kernel(const float *__restrict__ x, const uint8_t *__restrict__ codes,
-                                                        int64_t ns, int d, int M, double *__restrict__ acc,
-                                                        long long *__restrict__ cnt)
-{
-    __shared__ float tile[256][DSUB + 1];
-    __shared__ uint8_t tcode[256];
-    const int m = blockIdx.x, k = threadIdx.x;
-    double sum[DSUB];
-#pragma unroll
-    for (int t = 0; t < DSUB; t++) {
-        sum[t] = 0.0;
-    }
-    long long mine = 0;
-    for (int64_t i0 = 0; i0 < ns; i0 += 256) {
-        const int64_t i = i0 + k;
-        if (i < ns) {
-            const float *src = x + i * d + m * DSUB;
-#pragma unroll
-            for (int t = 0; t < DSUB; t++) {
-                tile[k][t] = src[t];
-            }
-            tcode[k] = codes[i * M + m];
-        }
-        __syncthreads();
-        const int lim = (int)(ns - i0 < 256 ? ns - i0 : 256);
-        for (int j = 0; j < lim; j++) {
-            if (tcode[j] == k) {
-                mine++;
-#pragma unroll
-                for (int t = 0; t < DSUB; t++) {
-                    sum[t] += (double)tile[j][t];
-                }
-            }
-        }
-        __syncthreads();
-    }
-#pragma unroll
-    for (int t = 0; t < DSUB; t++) {
-        acc[((int64_t)m * 256 + k) * DSUB + t] = sum[t];
-    }
-    cnt[m * 256 + k] = mine;
-}
-
-template <int DSUB>
-void launch_pq_update_t(const float *x, const uint8_t *codes, int64_t ns, int d, int M, double *acc, long long *cnt,
-                        hipStream_t s)
-{
-    hipLaunchKernelGGL(pq_update_kernel<DSUB>, dim3((unsigned)M), dim3(256), 0, s, x, codes, ns, d, M, acc, cnt);
-}
-
-// false: sub-vector length not served (the caller keeps its host loop)
-bool launch_pq_update(const float *x, const uint8_t *codes, int64_t ns, int d, int M, int dsub, double *acc,
-                      long long *cnt, hipStream_t s)
-{
-    switch (dsub) {
-    case 1: launch_pq_update_t<1>(x, codes, ns, d, M, acc, cnt, s); return true;
-    case 2: launch_pq_update_t<2>(x, codes, ns, d, M, acc, cnt, s); return true;
-    case 3: launch_pq_update_t<3>(x, codes, ns, d, M, acc, cnt, s); return true;
-    case 4: launch_pq_update_t<4>(x, codes, ns, d, M, acc, cnt, s); return true;
-    case 5: launch_pq_update_t<5>(x, codes, ns, d, M, acc, cnt, s); return true;
-    case 6: launch_pq_update_t<6>(x, codes, ns, d, M, acc, cnt, s); return true;
-    case 8: launch_pq_update_t<8>(x, codes, ns, d, M, acc, cnt, s); return true;
-    case 12: launch_pq_update_t<12>(x, codes, ns, d, M, acc, cnt, s); return true;
-    case 16: launch_pq_update_t<16>(x, codes, ns, d, M, acc, cnt, s); return true;
-    default: return false;
     }
 }
 
@@ -1866,9 +1803,9 @@ const SearchStats &IvfpqIndex::stats()
 // -------------------------------------------------------------------------------------------------
 // Training.  The reference delegates to faiss::Clustering (CPU mode) or runs device assignment with
 // a host centroid update (NPU mode: FR/ascendhost/src/impl/AscendClusteringImpl.cpp:686-762); this
-// build does the latter: assignment on the GPU (stage-1 kernels, PQ encode kernel); the coarse centroid
-// update also runs on the GPU (float64 sums in sample order, so the result does not depend on the
-// hardware's scheduling), the sub-quantizer update on the host in float64.  Sampling follows
+// build keeps both halves on the device: assignment (stage-1 kernels, PQ encode kernel) and both centroid
+// updates (float64 sums in sample order, so the result does not depend on the hardware's scheduling).
+// Sampling follows
 // computeTrainTotalSize / sampleTrainData (FR/ascend/impl/AscendIndexIVFPQImpl.cpp:51-112).  Plain Lloyd
 // unless cfg.spherical.
 
@@ -1913,45 +1850,6 @@ void IvfpqIndex::train(int64_t n, const float *x, bool on_device)
     kmeans_pq(sample_dev.data(), ns);
     trained_ = true;
 }
-
-namespace {
-
-// Re-seeds empty clusters by splitting the most populated one (symmetric perturbation).
-void split_empty(std::vector<float> &cent, std::vector<int64_t> &cnt, int64_t k, int dim)
-{
-    for (int64_t c = 0; c < k; c++) {
-        if (cnt[(size_t)c] != 0) {
-            continue;
-        }
-        const int64_t big = std::max_element(cnt.begin(), cnt.begin() + k) - cnt.begin();
-        for (int t = 0; t < dim; t++) {
-            const float v = cent[(size_t)(big * dim + t)];
-            const float eps = (t & 1) ? 1.0f / 1024 : -1.0f / 1024;
-            cent[(size_t)(c * dim + t)] = v * (1.0f + eps);
-            cent[(size_t)(big * dim + t)] = v * (1.0f - eps);
-        }
-        cnt[(size_t)c] = cnt[(size_t)big] / 2;
-        cnt[(size_t)big] -= cnt[(size_t)c];
-    }
-}
-
-void normalise_rows(std::vector<float> &cent, int64_t k, int dim)
-{
-    for (int64_t c = 0; c < k; c++) {
-        double nn = 0;
-        for (int t = 0; t < dim; t++) {
-            nn += (double)cent[(size_t)(c * dim + t)] * cent[(size_t)(c * dim + t)];
-        }
-        nn = std::sqrt(nn);
-        if (nn > 0) {
-            for (int t = 0; t < dim; t++) {
-                cent[(size_t)(c * dim + t)] = (float)(cent[(size_t)(c * dim + t)] / nn);
-            }
-        }
-    }
-}
-
-}  // namespace
 
 void IvfpqIndex::kmeans_coarse(const float *sample_dev, int64_t ns)
 {
@@ -2030,68 +1928,38 @@ void IvfpqIndex::kmeans_pq(const float *sample_dev, int64_t ns)
             }
         }
     }
-    struct {
-        const float *p;
-        const float *data() const { return p; }
-    } xs{sample_dev};
-    std::vector<float> sample;   // host copy of the sample: only the host update of long sub-vectors needs it
-    DeviceBuffer<uint8_t> codes((size_t)ns * M_);
-    std::vector<uint8_t> h_codes((size_t)ns * M_);
-    std::vector<double> acc((size_t)M_ * 256 * dsub_);
-    std::vector<int64_t> cnt((size_t)M_ * 256);
-    DeviceBuffer<double> acc_dev(acc.size());
-    DeviceBuffer<long long> cnt_dev(cnt.size());
-    static_assert(sizeof(long long) == sizeof(int64_t), "count buffers are copied as they are");
-    for (int it = 0; it < niter; it++) {
-        upload_trained(nullptr, cb.data());
-        launch_pq_encode(xs.data(), ns, d_, M_, codebook_.data(), codes.data(), stream_);
-        // sums per codeword in float64, in sample order: on the device for the usual sub-vector
-        // lengths, else by the host loop the kernel restates (same order, same results)
-        if (launch_pq_update(xs.data(), codes.data(), ns, d_, M_, dsub_, acc_dev.data(), cnt_dev.data(), stream_)) {
-            acc_dev.download(acc.data(), acc.size(), stream_);
-            cnt_dev.download(reinterpret_cast<long long *>(cnt.data()), cnt.size(), stream_);
-        } else {
-            if (sample.empty()) {
-                sample.resize((size_t)ns * d_);
-                IXA_HIP(hipMemcpyAsync(sample.data(), sample_dev, sample.size() * sizeof(float), hipMemcpyDeviceToHost,
-                                       stream_));
-                sync_stream(stream_);
-            }
-            codes.download(h_codes.data(), h_codes.size(), stream_);
-            std::fill(acc.begin(), acc.end(), 0.0);
-            std::fill(cnt.begin(), cnt.end(), 0);
-            for (int64_t i = 0; i < ns; i++) {
-                for (int m = 0; m < M_; m++) {
-                    const size_t slot = (size_t)m * 256 + h_codes[(size_t)i * M_ + m];
-                    cnt[slot]++;
-                    for (int t = 0; t < dsub_; t++) {
-                        acc[slot * dsub_ + t] += sample[(size_t)i * d_ + m * dsub_ + t];
-                    }
-                }
-            }
-        }
-        for (int m = 0; m < M_; m++) {
-            std::vector<float> sub(cb.begin() + (size_t)m * 256 * dsub_, cb.begin() + (size_t)(m + 1) * 256 * dsub_);
-            std::vector<int64_t> sc(cnt.begin() + (size_t)m * 256, cnt.begin() + (size_t)(m + 1) * 256);
-            for (int k = 0; k < 256; k++) {
-                if (sc[(size_t)k] > 0) {
-                    for (int t = 0; t < dsub_; t++) {
-                        sub[(size_t)k * dsub_ + t] =
-                            (float)(acc[((size_t)m * 256 + k) * dsub_ + t] / (double)sc[(size_t)k]);
-                    }
-                }
-            }
-            split_empty(sub, sc, 256, dsub_);
+    codebook_.upload(cb.data(), cb.size(), stream_);
+    // From here on an iteration is queued without a wait: codes of the sample (sub-quantizer-major, as the update reads
+    // them), the members of every codeword in sample order, their means (float64 sums in that order), empty codewords
+    // re-seeded, all in device memory.  The sub-quantizers do not depend on each other: they are trained in groups whose
+    // sub-vectors, codes and member lists stay within kPqTrainBytes.
+    const int64_t per_m = ns * (4 * dsub_ + 1 + 4);
+    const int group = (int)std::max<int64_t>(1, std::min<int64_t>(M_, kPqTrainBytes / per_m));
+    DeviceBuffer<float> subs((size_t)ns * group * dsub_);
+    DeviceBuffer<uint8_t> codes((size_t)ns * group);
+    DeviceBuffer<unsigned long long> cnt((size_t)group * 256);
+    PqUpdateWorkspace ws;
+    for (int m0 = 0; m0 < M_; m0 += group) {
+        const int mg = std::min(group, M_ - m0);
+        float *book = codebook_.data() + (int64_t)m0 * 256 * dsub_;
+        launch_pq_subvectors(sample_dev, ns, d_, m0, mg, dsub_, subs.data(), stream_);
+        for (int it = 0; it < niter; it++) {
+            launch_pq_encode_subvectors(subs.data(), ns, mg, dsub_, book, codes.data(), stream_);
+            launch_pq_update(subs.data(), codes.data(), ns, mg, dsub_, book, cnt.data(), ws, stream_);
+            hipLaunchKernelGGL(split_empty_kernel, dim3((unsigned)mg), dim3(1024), 0, stream_, book, cnt.data(),
+                               (int64_t)256, dsub_);
             // cfg_.spherical (the coarse quantizer's flag) is not applied here; the reference's HOST training
             // normalises the sub-quantizers as well (AscendIndexIVFPQImpl.cpp:1064-1067), its device training does
             // not: pq_spherical asks for the former
             if (cfg_.pq_spherical) {
-                normalise_rows(sub, 256, dsub_);
+                hipLaunchKernelGGL(normalise_rows_kernel, dim3(blocks_for((int64_t)mg * 256)), dim3(256), 0, stream_,
+                                   book, (int64_t)mg * 256, dsub_);
             }
-            std::copy(sub.begin(), sub.end(), cb.begin() + (size_t)m * 256 * dsub_);
         }
     }
-    upload_trained(nullptr, cb.data());
+    cbnorm_.resize((size_t)M_ * 256);
+    launch_sqnorm_rows(codebook_.data(), (int64_t)M_ * 256, dsub_, cbnorm_.data(), stream_);
+    sync_stream(stream_);   // the temporaries above are freed on return
 }
 
 }  // namespace ixa

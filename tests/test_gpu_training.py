@@ -1,0 +1,51 @@
+"""Training kernels at the sizes where they can go wrong: remainders of their tiles, one-component and very long
+sub-vectors, codewords without members."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _ix():
+    import indexsdk_amd as ix
+    return ix
+
+
+def lloyd_step(x, codes, book):
+    """One update of a codebook [256][dsub]: float64 sums in sample order, then empty codewords in ascending order
+    split the most populated one (symmetric perturbation)."""
+    out, cnt = book.copy(), np.bincount(codes, minlength=256).astype(np.int64)
+    for k in range(256):
+        if cnt[k]:
+            out[k] = (np.cumsum(x[codes == k].astype(np.float64), axis=0)[-1] / cnt[k]).astype(np.float32)
+    eps = np.where(np.arange(x.shape[1]) % 2, np.float32(1.0 / 1024), np.float32(-1.0 / 1024)).astype(np.float32)
+    for k in range(256):
+        if cnt[k] == 0:
+            big = int(np.argmax(cnt))
+            v = out[big].copy()
+            out[k] = v * (np.float32(1) + eps)
+            out[big] = v * (np.float32(1) - eps)
+            cnt[k] = cnt[big] // 2
+            cnt[big] -= cnt[k]
+    return out
+
+
+# sub-vectors of 1, 5, 20, 64 and 96 components; samples of less than one piece of the counting sort, of a piece and a
+# remainder, of many pieces; `distinct` rows only, so that most codewords have no member and one has many
+@pytest.mark.parametrize("d,M,n,distinct", [(3, 3, 257, 257), (40, 8, 1025, 1025), (40, 2, 5000, 5000), (128, 2, 1900, 1900),
+                                            (96, 1, 700, 700), (32, 8, 70001, 70001), (16, 4, 3000, 40)])
+def test_sub_quantizer_update_with_remainders_and_empty_codewords(oracle, d, M, n, distinct):
+    ix = _ix()
+    rng = np.random.default_rng(d + n)
+    x = rng.standard_normal((distinct, d)).astype(np.float32)[rng.integers(0, distinct, n)]
+    books = []
+    for niter in (1, 2):
+        cfg = ix.AscendIndexIVFPQConfig(niter=1, pq_niter=niter, train_samples_per_list=1 << 20)
+        gpu = ix.AscendIndexIVFPQ(d, ix.METRIC_L2, 4, M, 8, cfg)
+        gpu.train(x)
+        books.append(gpu.get_trained()[1])
+    codes = oracle.pq_encode(x, books[0])
+    dsub = d // M
+    for m in range(M):
+        want = lloyd_step(x[:, m * dsub:(m + 1) * dsub], codes[:, m], books[0][m])
+        assert np.array_equal(want.view(np.uint32), books[1][m].view(np.uint32)), m
