@@ -114,8 +114,13 @@ __device__ __forceinline__ uint32_t byte_times_pow2(uint32_t w, int j)
     return r;
 }
 
+// Short codes with the shared pool leave LDS room for four workgroups per CU and are bound by latency, not by registers'
+// worth of prefetch: those kernels are held to 64 registers (8 waves per SIMD).  Left alone the allocator takes a few more,
+// which halves the resident workgroups (64 queries x 128 lists of 16000 four-byte codes: 512 of 1024 workgroups at a time).
 template <int MT, typename LutT, int LAYOUT, int W, bool SHARED>
-__global__ __launch_bounds__(W * 64, (LAYOUT == 1 && sizeof(LutT) == 2 && !SHARED) ? 4 : 1) void ivfpq_scan_kernel(
+__global__ __launch_bounds__(W * 64, (LAYOUT == 1 && sizeof(LutT) == 2 && !SHARED) ? 4
+                                     : (SHARED && W == 8 && MT > 0 && MT <= 8)    ? 8
+                                                                                   : 1) void ivfpq_scan_kernel(
     ScanParams p)
 {
     extern __shared__ __align__(16) unsigned char smem_raw[];
@@ -408,10 +413,41 @@ __global__ __launch_bounds__(W * 64, (LAYOUT == 1 && sizeof(LutT) == 2 && !SHARE
     }
     auto adc = [&](uint32_t slot, const uint32_t (&w)[NW]) -> float {
         if (MT == 0) {
+            // run-time M: up to 32 code bytes are requested before the first is used, as words where the codes allow it
             const uint8_t *cp = p.codes + (int64_t)slot * M;
             float s = 0.f;
-            for (int m = 0; m < M; m++) {
-                s = __fadd_rn(s, from_lut(lut[m * 256 + cp[m]]));
+            if ((M & 3) == 0) {
+                for (int m0 = 0; m0 < M; m0 += 32) {
+                    uint32_t u[8];
+#pragma unroll
+                    for (int i = 0; i < 8; i++) {
+                        u[i] = m0 + 4 * i < M ? reinterpret_cast<const uint32_t *>(cp + m0)[i] : 0u;
+                    }
+#pragma unroll
+                    for (int i = 0; i < 8; i++) {
+                        if (m0 + 4 * i < M) {
+                            const LutT *row = lut + (m0 + 4 * i) * 256;
+#pragma unroll
+                            for (int j = 0; j < 4; j++) {
+                                s = __fadd_rn(s, from_lut(row[j * 256 + ((u[i] >> (8 * j)) & 0xffu)]));
+                            }
+                        }
+                    }
+                }
+                return s;
+            }
+            for (int m0 = 0; m0 < M; m0 += 8) {
+                uint8_t c[8];
+#pragma unroll
+                for (int i = 0; i < 8; i++) {
+                    c[i] = m0 + i < M ? cp[m0 + i] : (uint8_t)0;
+                }
+#pragma unroll
+                for (int i = 0; i < 8; i++) {
+                    if (m0 + i < M) {
+                        s = __fadd_rn(s, from_lut(lut[(m0 + i) * 256 + c[i]]));
+                    }
+                }
             }
             return s;
         }
@@ -521,7 +557,7 @@ __global__ __launch_bounds__(W * 64, (LAYOUT == 1 && sizeof(LutT) == 2 && !SHARE
             adopt_shared();                                                                           \
         }                                                                                             \
     } while (0)
-    // The same step for the shared pool: poll for a pending prune, evaluate, reserve-and-append;
+    // The same step for the shared pool of sixteen wavefronts: poll for a pending prune, evaluate, reserve-and-append;
     // a failed reservation is retried after the workgroup has pruned the pool.
 #define IXA_SCAN_STEP_SHARED(G, CUR, WCUR, NXT, WNXT, PF)                                             \
     do {                                                                                              \
@@ -540,39 +576,81 @@ __global__ __launch_bounds__(W * 64, (LAYOUT == 1 && sizeof(LutT) == 2 && !SHARE
         }                                                                                             \
     } while (0)
     int total_keys;
-    if constexpr (SHARED) {
+    if constexpr (SHARED && W == 16) {
+        // sixteen wavefronts hide the latency by themselves, and their registers admit no second workgroup anyway: the
+        // plain loop, which leaves the last group without a request (100M x 96, nprobe 256, k 1024: 2.5 % faster than
+        // unconditional requests; 20M x 96, 1024 queries: 3.38 ms against 3.63 with the loop around one rendezvous below)
         if (wave < total) {
             uint32_t wa[NW] = {}, wb[NW] = {};
             GroupRef ga = locate(wave), gb = ga;
             if (!kSkipPadding || ga.valid) {
                 load_codes(ga.slot, wa);
             }
-            if constexpr (W == 16) {
-                // sixteen wavefronts hide the latency by themselves, and the plain loop measured 2.5 % faster
-                // there (100M x 96, nprobe 256, k 1024: scan 4.34 against 4.44 ms)
-                for (int G = wave; G < total; G += 2 * W) {
-                    IXA_SCAN_STEP_SHARED(G, ga, wa, gb, wb, G + W < total);
-                    if (G + W < total) {
-                        IXA_SCAN_STEP_SHARED(G + W, gb, wb, ga, wa, G + 2 * W < total);
-                    }
-                }
-            } else {
-                int G = wave;
-                for (; G + 2 * W < total; G += 2 * W) {   // the groups G, G + W and G + 2 W exist
-                    IXA_SCAN_STEP_SHARED(G, ga, wa, gb, wb, 1);
-                    IXA_SCAN_STEP_SHARED(G + W, gb, wb, ga, wa, 1);
-                }
-                if (G + W < total) {   // two groups left (the first is in set a), or one
-                    IXA_SCAN_STEP_SHARED(G, ga, wa, gb, wb, 1);
-                    IXA_SCAN_STEP_SHARED(G + W, gb, wb, ga, wa, 0);
-                } else {
-                    IXA_SCAN_STEP_SHARED(G, ga, wa, gb, wb, 0);
+            for (int G = wave; G < total; G += 2 * W) {
+                IXA_SCAN_STEP_SHARED(G, ga, wa, gb, wb, G + W < total);
+                if (G + W < total) {
+                    IXA_SCAN_STEP_SHARED(G + W, gb, wb, ga, wa, G + 2 * W < total);
                 }
             }
         }
         bpool.finish_wave(lane);
         while (!bpool.rendezvous(tid)) {
         }
+        total_keys = bpool.sort_all(tid);
+    } else if constexpr (SHARED) {
+        // One loop around ONE rendezvous: a wavefront scans until a prune is pending, its reservation fails or its groups
+        // are done, and then meets the others.  With the rendezvous inside every step of the scan its code (histograms,
+        // a sort) stood in the kernel six times, was fetched cold at each, and its registers were the kernel's (106 at
+        // M = 4: two resident workgroups per CU).  A group whose push failed is evaluated again afterwards.
+        // The next group's codes are requested unconditionally (behind the last group: the last group again), so that
+        // the compiler's wait counts exactly the loads of the group in flight.
+        int G = wave;
+        uint32_t wa[NW] = {}, wb[NW] = {};
+        GroupRef ga{}, gb{};
+        if (G < total) {
+            ga = locate(G);
+            if (!kSkipPadding || ga.valid) {
+                load_codes(ga.slot, wa);
+            }
+        }
+        auto step = [&](GroupRef &cur, uint32_t(&wcur)[NW], GroupRef &nxt, uint32_t(&wnxt)[NW]) -> bool {
+            nxt = locate(G + W < total ? G + W : G);
+            if (!kSkipPadding || nxt.valid) {   // lanes past the list's end fetch nothing
+                load_codes(nxt.slot, wnxt);     // in flight while the current group is evaluated
+            }
+            if (bpool.poll()) {
+                return false;
+            }
+            const float s_ = adc(cur.slot, wcur);
+            if (!bpool.try_push(cur.valid && s_ <= bpool.bound, s_, cur.slot, lane)) {
+                return false;
+            }
+            G += W;
+            return true;
+        };
+        bool finished = false;
+        do {
+            while (G < total) {
+                if (!step(ga, wa, gb, wb)) {
+                    break;
+                }
+                if (G >= total) {
+                    break;
+                }
+                if (!step(gb, wb, ga, wa)) {
+                    ga = gb;
+#pragma unroll
+                    for (int v = 0; v < NW; v++) {
+                        wa[v] = wb[v];
+                    }
+                    break;
+                }
+            }
+            if (G >= total && !finished) {
+                bpool.finish_wave(lane);
+                finished = true;
+            }
+        } while (!bpool.rendezvous(tid));
         total_keys = bpool.sort_all(tid);
     } else {
         if (wave < total) {
@@ -909,14 +987,7 @@ __global__ __launch_bounds__(kMergeSelectThreads) void ivfpq_merge_kernel(
         }
         return;
     }
-    int n2 = 512;
-    while (n2 < kept) {
-        n2 <<= 1;
-    }
-    for (int i = kept + tid; i < n2; i += NT) {
-        surv[i] = kEmptyKey;
-    }
-    block_bitonic_sort(surv, n2, tid, NT);
+    block_sort_keys<NT>(surv, kept, tid);
     for (int i = tid; i < k; i += NT) {
         const key_t kk = i < kept ? surv[i] : kEmptyKey;
         const bool ok = kk != kEmptyKey;
@@ -1149,6 +1220,13 @@ static void dispatch_m(const ScanParams &p, int64_t nq, size_t smem, hipStream_t
         case 8: return launch_one<8, LutT, 0>(p, nq, smem, s);
         case 16: return launch_one<16, LutT, 0>(p, nq, smem, s);
         case 32: return launch_one<32, LutT, 0>(p, nq, smem, s);
+        // ... as have the multiples of 4 up to 24 and of 8 up to 64: the kernel with run-time M keeps no codes in flight
+        // across groups
+        case 12: return launch_one<12, LutT, 0>(p, nq, smem, s);
+        case 20: return launch_one<20, LutT, 0>(p, nq, smem, s);
+        case 24: return launch_one<24, LutT, 0>(p, nq, smem, s);
+        case 40: return launch_one<40, LutT, 0>(p, nq, smem, s);
+        case 56: return launch_one<56, LutT, 0>(p, nq, smem, s);
         case 48: return launch_one<48, LutT, 0>(p, nq, smem, s);
         case 64: return launch_one<64, LutT, 0>(p, nq, smem, s);
         case 96: return launch_one<96, LutT, 0>(p, nq, smem, s);

@@ -135,6 +135,143 @@ __device__ inline void block_bitonic_sort(key_t *buf, int n, int tid, int nthrea
     __syncthreads();
 }
 
+// One bitonic network over KPT keys per thread held in registers: thread t owns positions t * KPT .. + KPT.  Strides inside
+// a thread cost no communication, strides inside a wavefront are lane shuffles, and only strides across wavefronts go
+// through LDS with barriers: 6 of the 66 stages of 2048 keys on 512 threads (the LDS network above pays two LDS round trips
+// and a barrier in every stage: 11.3 us for those keys).
+template <int KPT, int NT>
+__device__ inline void block_sort_regs(key_t *buf, int tid)
+{
+    constexpr int N = KPT * NT;
+    key_t e[KPT];
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < KPT; j++) {
+        e[j] = buf[tid * KPT + j];
+    }
+    for (int size = 2; size <= N; size <<= 1) {
+        int stride = size >> 1;
+        for (; stride >= KPT * kWave; stride >>= 1) {
+            __syncthreads();   // everyone has read the positions that are overwritten now
+#pragma unroll
+            for (int j = 0; j < KPT; j++) {
+                buf[tid * KPT + j] = e[j];
+            }
+            __syncthreads();
+            const bool low = ((tid * KPT) & stride) == 0, up = ((tid * KPT) & size) == 0;
+#pragma unroll
+            for (int j = 0; j < KPT; j++) {
+                const key_t o = buf[(tid * KPT + j) ^ stride];
+                e[j] = ((o < e[j]) == (low == up)) ? o : e[j];
+            }
+        }
+        for (; stride >= KPT; stride >>= 1) {
+            const bool low = ((tid * KPT) & stride) == 0, up = ((tid * KPT) & size) == 0;
+#pragma unroll
+            for (int j = 0; j < KPT; j++) {
+                const key_t o = __shfl_xor(e[j], stride / KPT);
+                e[j] = ((o < e[j]) == (low == up)) ? o : e[j];
+            }
+        }
+        if constexpr (KPT > 1) {
+#pragma unroll
+            for (int st = KPT / 2; st > 0; st >>= 1) {
+                if (st < size) {
+#pragma unroll
+                    for (int j = 0; j < KPT; j++) {
+                        if ((j & st) == 0) {
+                            const bool up = ((tid * KPT + j) & size) == 0;
+                            const key_t a = e[j], b = e[j | st];
+                            const bool swap = (a > b) == up;
+                            e[j] = swap ? b : a;
+                            e[j | st] = swap ? a : b;
+                        }
+                    }
+                }
+            }
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < KPT; j++) {
+        buf[tid * KPT + j] = e[j];
+    }
+    __syncthreads();
+}
+
+// Ascending order of n <= NT keys by counting ranks: 2^p neighbouring lanes share a key and count over every 2^p-th pair
+// of the array (few distinct LDS addresses per read: broadcasts).  Equal keys keep their order, so every key has a rank of
+// its own.  buf holds n + 1 keys, 16-byte aligned.
+template <int NT>
+__device__ inline void block_rank_sort(key_t *buf, int n, int tid)
+{
+    int shift = 0;
+    while (shift < 4 && (n << (shift + 1)) <= NT) {
+        shift++;
+    }
+    const int e = tid >> shift, part = tid & ((1 << shift) - 1);
+    __syncthreads();
+    if (tid == 0 && (n & 1)) {
+        buf[n] = kEmptyKey;
+    }
+    const key_t mine = e < n ? buf[e] : kEmptyKey;
+    __syncthreads();
+    const ulonglong2 *pairs = reinterpret_cast<const ulonglong2 *>(buf);
+    const int npairs = (n + 1) >> 1, step = 1 << shift;
+    // before this wavefront's own keys an equal key counts, behind them it does not, among them it depends on the lane
+    const int own0 = __builtin_amdgcn_readfirstlane(((tid & ~63) >> shift) >> 1);
+    const int own1 = __builtin_amdgcn_readfirstlane(((tid | 63) >> shift) >> 1);
+    int rank = 0, f = part;
+    for (; f < own0 && f < npairs; f += step) {
+        const ulonglong2 v = pairs[f];
+        rank += (v.x <= mine) + (v.y <= mine);
+    }
+    for (; f <= own1 && f < npairs; f += step) {
+        const ulonglong2 v = pairs[f];
+        rank += (v.x < mine || (v.x == mine && 2 * f < e)) + (v.y < mine || (v.y == mine && 2 * f + 1 < e));
+    }
+    for (; f < npairs; f += step) {
+        const ulonglong2 v = pairs[f];
+        rank += (v.x < mine) + (v.y < mine);
+    }
+    for (int o = 1; o < step; o <<= 1) {
+        rank += __shfl_xor(rank, o);
+    }
+    __syncthreads();
+    if (part == 0 && e < n) {
+        buf[rank] = mine;
+    }
+    __syncthreads();
+}
+
+// Sorts buf[0 .. n) ascending; buf has room for the next power of two (at least two keys).  All NT threads of the workgroup
+// call it, barriers inside.  Up to 256 keys are ranked by counting; beyond, the squared number of comparisons costs more
+// issue slots than the network's stages (400 keys at the end of every query of 10M x 32 bytes, nprobe 64: +1.5 %).
+template <int NT>
+__device__ inline void block_sort_keys(key_t *buf, int n, int tid)
+{
+    if (n <= 256) {
+        block_rank_sort<NT>(buf, n, tid);
+        return;
+    }
+    int n2 = NT < 512 ? 512 : NT;
+    while (n2 < n) {
+        n2 <<= 1;
+    }
+    for (int i = n + tid; i < n2; i += NT) {
+        buf[i] = kEmptyKey;
+    }
+    if (n2 == NT) {
+        block_sort_regs<1, NT>(buf, tid);
+    } else if (n2 == 2 * NT) {
+        block_sort_regs<2, NT>(buf, tid);
+    } else if (n2 == 4 * NT) {
+        block_sort_regs<4, NT>(buf, tid);
+    } else {
+        block_bitonic_sort(buf, n2, tid, NT);
+    }
+}
+
 template <typename S = float>
 struct WavePool {
     key_t *buf;   // LDS, cap entries, private to this wave, unsorted
@@ -334,14 +471,7 @@ __device__ inline int block_merge_pools(key_t *pools, int cap, const int *counts
         pools[total + i] = extra[i];
     }
     total += extra_n;
-    int n = 2;
-    while (n < total) {
-        n <<= 1;
-    }
-    for (int i = total + tid; i < n; i += NT) {
-        pools[i] = kEmptyKey;
-    }
-    block_bitonic_sort(pools, n, tid, NT);
+    block_sort_keys<NT>(pools, total, tid);
     return total;
 }
 
@@ -410,6 +540,23 @@ struct BlockPool {
             c->done = 0;
             c->kept = 0;
             c->bound = __builtin_inff();
+        }
+    }
+
+    // Counts one key per lane.  Tied scores put most keys of a wavefront into one bin: the lanes that share the first
+    // counted lane's bin add once for all of them.
+    __device__ __forceinline__ void count_bins(bool counted, uint32_t bin, int lane)
+    {
+        const unsigned long long any = __ballot(counted);
+        if (any) {
+            const int leader = __builtin_ctzll(any);
+            const uint32_t leader_bin = (uint32_t)__builtin_amdgcn_readlane((int)bin, leader);
+            const unsigned long long same = __ballot(counted && bin == leader_bin);
+            if (lane == leader) {
+                lds_add(&hist[leader_bin], __popcll(same));
+            } else if (counted && bin != leader_bin) {
+                lds_add(&hist[bin], 1);
+            }
         }
     }
 
@@ -518,9 +665,7 @@ struct BlockPool {
             __syncthreads();
 #pragma unroll
             for (int j = 0; j < kMaxPerThread; j++) {
-                if (e[j] != kEmptyKey) {
-                    lds_add(&hist[(uint32_t)(e[j] >> (32 + SH + 10))], 1);
-                }
+                count_bins(e[j] != kEmptyKey, (uint32_t)(e[j] >> (32 + SH + 10)), lane);
             }
             __syncthreads();
             find_bin(k, tid);
@@ -535,9 +680,7 @@ struct BlockPool {
 #pragma unroll
             for (int j = 0; j < kMaxPerThread; j++) {
                 const uint32_t pre = (uint32_t)(e[j] >> (32 + SH));
-                if (e[j] != kEmptyKey && (pre >> 10) == b1) {
-                    lds_add(&hist[pre & 1023u], 1);
-                }
+                count_bins(e[j] != kEmptyKey && (pre >> 10) == b1, pre & 1023u, lane);
             }
             __syncthreads();
             find_bin(rank2, tid);
@@ -570,10 +713,7 @@ struct BlockPool {
         float top = ScoreOps<float>::bucket_top((P << SH) | ((1u << SH) - 1u));
         if (kept > cap - NT) {
             // one bucket holds almost everything: exact selection by sorting
-            for (int i = kept + tid; i < cap; i += NT) {
-                buf[i] = kEmptyKey;
-            }
-            block_bitonic_sort((key_t *)buf, cap, tid, NT);
+            block_sort_keys<NT>((key_t *)buf, kept, tid);
             kept = k;
             top = key_score(buf[k - 1]);
             if (tid == 0) {
@@ -605,20 +745,12 @@ struct BlockPool {
         return d == W;
     }
 
-    // After the last rendezvous: sorts the pool ascending in place, returns the number of keys.  Only the
-    // smallest power of two that holds them is sorted (a pool pruned to little more than k is far from full).
+    // After the last rendezvous: sorts the pool ascending in place, returns the number of keys.
     __device__ inline int sort_all(int tid)
     {
         const int n = size();
-        int n2 = 2;
-        while (n2 < n) {
-            n2 <<= 1;
-        }
         __syncthreads();
-        for (int i = n + tid; i < n2; i += NT) {
-            buf[i] = kEmptyKey;
-        }
-        block_bitonic_sort((key_t *)buf, n2, tid, NT);
+        block_sort_keys<NT>((key_t *)buf, n, tid);
         return n;
     }
 };

@@ -971,3 +971,29 @@ def test_host_batch_beyond_the_staging_buffer_equals_its_pieces(ix, oracle):
     ref = oracle.CsrIndex.build(d, M, ix.METRIC_L2, cent, cb, x, np.arange(n, dtype=np.int64))
     Dr, Ir = ref.search(q[:500], k, 8)
     assert_topk_parity(oracle, ref, q[:500], D[:500], I[:500], Dr, Ir, TOL_FP32)
+
+
+@pytest.mark.parametrize("M", [12, 20, 24, 40, 56, 36, 9])
+def test_sub_quantizer_counts_off_the_powers_of_two(ix, oracle, M):
+    """Compile-time M (multiples of 4 up to 24, of 8 up to 64), run-time M by words (36) and by bytes (9); a batch that is
+    split over workgroups and one that is not, private pools and the shared pool."""
+    gpu, ref, x, q, ids = build_pair(ix, oracle, 300 + M, 9001, 70, 4 * M, 24, M, ix.METRIC_L2)
+    gpu.setNumProbes(5)
+    for k in (10, 300):
+        for nq in (70, 1):
+            D, I = gpu.search(q[:nq], k)
+            Dr, Ir = ref.search(q[:nq], k, 5)
+            assert_topk_parity(oracle, ref, q[:nq], D, I, Dr, Ir, TOL_FP32)
+
+
+@pytest.mark.parametrize("k", [1, 2, 255, 256, 257, 511, 512, 513, 1023, 1024, 1025, 2047, 2048])
+def test_key_counts_at_the_edges_of_the_sorts(ix, oracle, k):
+    """k at both sides of every boundary of the workgroup sorts (ranks by counting, networks of one, two and four keys per
+    thread): the same answer from one workgroup per query and from several whose slices are merged."""
+    gpu, ref, x, q, ids = build_pair(ix, oracle, 77, 12000, 500, 32, 16, 8, ix.METRIC_L2)
+    gpu.setNumProbes(8)
+    D, I = gpu.search(q, k)
+    Dr, Ir = ref.search(q[:40], k, 8)
+    assert_topk_parity(oracle, ref, q[:40], D[:40], I[:40], Dr, Ir, TOL_FP32)
+    D1, I1 = gpu.search(q[:2], k)
+    assert np.array_equal(I1, I[:2]) and np.array_equal(D1.view(np.uint32), D[:2].view(np.uint32))
