@@ -126,15 +126,18 @@ void launch_fold_refine_boundary(const float *Q, int64_t nq, const float *C, int
 // out[row] = [hi | hi | lo] (query side) or [hi | lo | hi] (base side) of x[row], each segment
 // zero-padded from d to dp elements of bf16 (stored as uint16_t); out has n * 3 * dp elements.
 void launch_split_bf16x3(const float *x, int64_t n, int d, int dp, bool base_side, uint16_t *out, hipStream_t s);
+// the same, eight elements per thread, for rows in bulk (out 16-byte aligned); a NaN stays a NaN
+void launch_split_bf16x3_rows(const float *x, int64_t n, int d, int dp, bool base_side, uint16_t *out, hipStream_t s);
 // launch_sqnorm_rows(x -> norms) and the query-side launch_split_bf16x3(x -> split) in one launch
 void launch_sqnorm_and_split_bf16x3(const float *x, int64_t n, int d, int dp, float *norms, uint16_t *split, hipStream_t s);
 
 // Sets *flag = 1 if some query's approximate candidate list (running[nq][ncand], ascending keys) is
-// not provably a superset of its best nout centroids; see score_ring.hip.
+// not provably a superset of its best nout centroids; see score_ring.hip.  finite_only: a query whose norm is not
+// finite counts as unproven.
 void launch_verify_superset(const unsigned long long *running, int ncand, const float *exact_dist, int nout,
                             const float *qn, float cmax, float err_scale, float round_scale, int metric, int64_t nq,
                             int *flag,
-                            hipStream_t s);
+                            hipStream_t s, bool finite_only = false);
 
 // Largest selection size of launch_select_rows*: the private pools of its wavefronts hold 4096 keys.
 constexpr int kSelectMaxK = 3072;

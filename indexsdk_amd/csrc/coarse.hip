@@ -12,6 +12,8 @@
 
 #include "topk.h"
 
+#include <type_traits>
+
 namespace ixa {
 
 typedef float floatx16 __attribute__((ext_vector_type(16)));
@@ -147,6 +149,54 @@ __global__ __launch_bounds__(256) void split_bf16x3_kernel(const float *__restri
     split_bf16x3_block(x, n, d, dp, base_side, out, blockIdx.x);
 }
 
+// The same split for rows in bulk (Flat search: every base row of every call): a thread takes eight elements with two 128-bit
+// loads and three 128-bit stores.  A NaN stays one in both parts.
+__device__ __forceinline__ uint32_t bf16_rne_nan(float v) { return v != v ? 0x7fc0u : (uint32_t)bf16_rne(v); }
+
+template <bool VEC>
+__global__ __launch_bounds__(256) void split_bf16x3_rows_kernel(const float *__restrict__ x, int64_t n, int d, int dp,
+                                                                int base_side, uint16_t *__restrict__ out)
+{
+    const int per = dp >> 3;
+    const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (e >= n * per) {
+        return;
+    }
+    const int64_t row = e / per;
+    const int j = (int)(e - row * per) * 8;
+    const float *src = x + row * d + j;
+    float v[8];
+#pragma unroll
+    for (int h = 0; h < 8; h += 4) {
+        if (VEC) {   // d % 4 == 0: four elements lie inside the row or behind it together
+            const float4 f = j + h < d ? *reinterpret_cast<const float4 *>(src + h) : make_float4(0.f, 0.f, 0.f, 0.f);
+            v[h] = f.x;
+            v[h + 1] = f.y;
+            v[h + 2] = f.z;
+            v[h + 3] = f.w;
+        } else {
+#pragma unroll
+            for (int t = 0; t < 4; t++) {
+                v[h + t] = j + h + t < d ? src[h + t] : 0.f;
+            }
+        }
+    }
+    uint32_t hi[4], lo[4];
+#pragma unroll
+    for (int t = 0; t < 4; t++) {
+        const uint32_t h0 = bf16_rne_nan(v[2 * t]), h1 = bf16_rne_nan(v[2 * t + 1]);
+        const uint32_t l0 = bf16_rne_nan(v[2 * t] - __uint_as_float(h0 << 16));
+        const uint32_t l1 = bf16_rne_nan(v[2 * t + 1] - __uint_as_float(h1 << 16));
+        hi[t] = h0 | (h1 << 16);
+        lo[t] = l0 | (l1 << 16);
+    }
+    const uint4 h4 = make_uint4(hi[0], hi[1], hi[2], hi[3]), l4 = make_uint4(lo[0], lo[1], lo[2], lo[3]);
+    uint16_t *o = out + row * 3 * dp + j;
+    *reinterpret_cast<uint4 *>(o) = h4;
+    *reinterpret_cast<uint4 *>(o + dp) = base_side ? l4 : h4;
+    *reinterpret_cast<uint4 *>(o + 2 * dp) = base_side ? h4 : l4;
+}
+
 // Both of the above in one launch (the first blocks add up the norms, the others split): what a search does to its
 // queries before the coarse stage's first score launch.
 __global__ __launch_bounds__(256) void sqnorm_and_split_kernel(const float *__restrict__ x, int64_t n, int d, int dp,
@@ -172,6 +222,15 @@ void launch_sqnorm_and_split_bf16x3(const float *x, int64_t n, int d, int dp, fl
     } else {
         launch_sqnorm_rows(x, n, d, norms, s);
         launch_split_bf16x3(x, n, d, dp, false, split, s);
+    }
+}
+
+void launch_split_bf16x3_rows(const float *x, int64_t n, int d, int dp, bool base_side, uint16_t *out, hipStream_t s)
+{
+    if (n > 0) {
+        const bool vec = d % 4 == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0;
+        hipLaunchKernelGGL(vec ? split_bf16x3_rows_kernel<true> : split_bf16x3_rows_kernel<false>,
+                           dim3((unsigned)((n * (dp / 8) + 255) / 256)), dim3(256), 0, s, x, n, d, dp, base_side ? 1 : 0, out);
     }
 }
 
@@ -1056,6 +1115,103 @@ void launch_tau_from_minima(const float *gm, int G, int rank, int64_t nq, float 
     }
 }
 
+// Few keys from short float rows (assignment during training and adding, small coarse stages): one wavefront per row, the row
+// in registers, and one extraction of the smallest key per result.  The pools above pay a workgroup, a merge and a sort per
+// row for the same few keys: 9 of 1024 columns 121 us per 12000 rows, 17 of the 40 ms of GPU time of building a 1M index.
+// Beyond kSelWaveMaxK extractions their serial chain is longer than the pools' work.
+constexpr int kSelWaveMaxK = 24, kSelWaveMaxCols = 2048;
+
+template <int V>
+__global__ __launch_bounds__(256) void select_rows_wave_kernel(const float *__restrict__ scores, int64_t nrows, int64_t ld,
+                                                               int nc, int ksel, int32_t *__restrict__ out_idx,
+                                                               int64_t col_base, key_t *__restrict__ running, bool fresh)
+{
+    const int lane = threadIdx.x & 63;
+    const int64_t r = (int64_t)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (r >= nrows) {
+        return;
+    }
+    constexpr uint32_t kNone = 0xffffffffu;   // above the ordered bits of every number
+    const float *row = scores + r * ld;
+    uint32_t o[V];
+#pragma unroll
+    for (int i = 0; i < V; i++) {
+        const int c = i * 64 + lane;
+        const float v = c < nc ? row[c] : __builtin_nanf("");
+        o[i] = v == v ? ordered_bits(v) : kNone;   // a NaN is never selected
+    }
+    // the running keys (ascending, empty ones last): lane j holds the j-th, `used` of them are taken
+    const key_t old = (running && !fresh && lane < ksel) ? running[r * ksel + lane] : kEmptyKey;
+    int used = 0;
+    key_t head = wave_uniform_key(old);
+    uint32_t best;
+    int at;   // the lane's smallest value and its index, the first of equal ones
+    auto find_best = [&]() {
+        best = o[0];
+        at = 0;
+#pragma unroll
+        for (int i = 1; i < V; i++) {
+            if (o[i] < best) {
+                best = o[i];
+                at = i;
+            }
+        }
+    };
+    find_best();
+    key_t mine = kEmptyKey;   // lane j: the j-th result
+    for (int j = 0; j < ksel; j++) {
+        uint32_t m = best;
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) {
+            const uint32_t x = (uint32_t)__shfl_xor((int)m, off);
+            m = x < m ? x : m;
+        }
+        m = (uint32_t)__builtin_amdgcn_readfirstlane((int)m);
+        int col = at * 64 + lane, owner = -1;
+        key_t k = kEmptyKey;
+        if (m != kNone) {
+            const unsigned long long tied = __ballot(best == m);
+            owner = __builtin_ctzll(tied);
+            if (tied & (tied - 1)) {   // equal scores: the smallest column
+                int low = best == m ? col : 0x7fffffff;
+#pragma unroll
+                for (int off = 32; off > 0; off >>= 1) {
+                    const int x = __shfl_xor(low, off);
+                    low = x < low ? x : low;
+                }
+                owner = __builtin_amdgcn_readfirstlane(low) & 63;
+            }
+            k = ((key_t)m << 32) | (uint32_t)(__builtin_amdgcn_readlane(col, owner) + col_base);
+        }
+        if (head < k) {
+            k = head;
+            used++;
+            head = used < ksel ? wave_uniform_key(__shfl(old, used)) : kEmptyKey;
+        } else if (owner < 0) {
+            break;   // nothing left on either side
+        } else if (lane == owner) {
+#pragma unroll
+            for (int i = 0; i < V; i++) {
+                if (i == at) {
+                    o[i] = kNone;
+                }
+            }
+            find_best();
+        }
+        if (lane == j) {
+            mine = k;
+        }
+    }
+    if (lane < ksel) {
+        if (out_idx) {
+            out_idx[r * ksel + lane] = mine == kEmptyKey ? -1 : (int32_t)key_index(mine);
+        }
+        if (running) {
+            running[r * ksel + lane] = mine;
+        }
+    }
+}
+
 template <typename S>
 static void launch_select_rows_t(const S *scores, int64_t nrows, int64_t ld, int64_t nc, int ksel, int32_t *out_idx,
                                  int64_t col_base, unsigned long long *running, bool fresh, hipStream_t s)
@@ -1065,6 +1221,16 @@ static void launch_select_rows_t(const S *scores, int64_t nrows, int64_t ld, int
     }
     IXA_REQUIRE(ksel >= 1 && ksel <= kSelectMaxK, kErrInvalidParam, "selection size %d out of range [1, %d]", ksel,
                 kSelectMaxK);
+    if constexpr (std::is_same<S, float>::value) {
+        if (ksel <= kSelWaveMaxK && nc <= kSelWaveMaxCols) {
+            auto kern = nc <= 256 ? select_rows_wave_kernel<4>
+                                  : (nc <= 512 ? select_rows_wave_kernel<8>
+                                               : (nc <= 1024 ? select_rows_wave_kernel<16> : select_rows_wave_kernel<32>));
+            hipLaunchKernelGGL(kern, dim3((unsigned)((nrows + 3) / 4)), dim3(256), 0, s, scores, nrows, ld, (int)nc, ksel,
+                               out_idx, col_base, running, fresh);
+            return;
+        }
+    }
     const int cap = wave_pool_capacity(ksel);
     // four scanning wavefronts when their pools and the merge fit LDS, else two, else one
     int active = 4;

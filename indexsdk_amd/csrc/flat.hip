@@ -495,6 +495,7 @@ void FlatIndex::add(int64_t n, const float *x, const int64_t *ids, bool on_devic
     float sq;
     std::memcpy(&sq, &bits, 4);
     bmax_ = std::max(bmax_, std::sqrt(sq));
+    finite_ = finite_ && std::isfinite(sq);
     norms_ = std::move(nn);
 }
 
@@ -591,6 +592,11 @@ void FlatIndex::search_with_masks(int64_t n, const float *x, int64_t k, const ui
     }
 }
 
+namespace {
+constexpr int64_t kSplitBytes = (int64_t)256 << 20;   // split base rows in flight: what the memory-side cache holds
+constexpr int64_t kSplitMinQueries = 256, kSplitMinBase = 32768;
+}  // namespace
+
 void FlatIndex::search_masked(int64_t n, const float *x, int64_t k, float *dist, int64_t *labels, bool on_device,
                               const uint8_t *mask_dev, int64_t mask_stride)
 {
@@ -610,16 +616,35 @@ void FlatIndex::search_masked(int64_t n, const float *x, int64_t k, float *dist,
         dd = ws_dist_.data();
         ld = ws_labels_.data();
     }
-    const int ncand = (int)std::min<int64_t>(std::max<int64_t>(ntotal_, 1), k + 8 + k / 8);
+    // Large batches form their candidate scores from bf16 x 3 splits on the bf16 matrix cores (three products at about ten
+    // times the fp32 rate), everything else on the fp32 ones.  Splitting the base costs 10 bytes of traffic per element and
+    // search: about what 140 queries save.  Short bases stay with one launch, and vectors so small that products of their
+    // parts leave the normal range stay with fp32.
+    const int dp = (int)round_up(d_, 32);
+    int64_t split_rows = std::min<int64_t>(scratch_bytes_ / 2, kSplitBytes) / (6 * dp) / 2048 * 2048;
+    split_rows = std::min<int64_t>(split_rows, round_up(ntotal_, 2048));
+    const bool split = !mask_dev && n >= kSplitMinQueries && ntotal_ >= kSplitMinBase && split_rows >= 16384 && bmax_ >= 1e-6f &&
+                       finite_;
+    const int ncand = (int)std::min<int64_t>(std::max<int64_t>(ntotal_, 1), k + (split ? 16 : 8) + k / 8);
     ws_qn_.resize((size_t)n);
     ws_running_.resize((size_t)n * ncand);
     ws_cand_.resize((size_t)n * ncand);
     ws_idx_.resize((size_t)n * k);
     IXA_HIP(hipEventRecord(ev_[0], stream_));
-    launch_sqnorm_rows(xd, n, d_, ws_qn_.data(), stream_);
-    const int launches = stream_select_f32(xd, n, base_.data(), ntotal_, d_, ws_qn_.data(), norms_.data(), metric_,
-                                           ncand, ws_running_.data(), ws_sel_, scratch_bytes_, stream_, mask_dev,
-                                           mask_stride);
+    int launches;
+    if (split) {
+        ws_qsplit_.resize((size_t)n * 3 * dp);
+        ws_bsplit_.resize((size_t)(split_rows + kSplitMinRows) * 3 * dp);
+        launch_sqnorm_rows(xd, n, d_, ws_qn_.data(), stream_);
+        launch_split_bf16x3_rows(xd, n, d_, dp, false, ws_qsplit_.data(), stream_);
+        launches = stream_select_f32_split(xd, n, base_.data(), ntotal_, d_, ws_qn_.data(), norms_.data(), metric_, ncand,
+                                           ws_running_.data(), ws_sel_, scratch_bytes_ - scratch_bytes_ / 2, stream_,
+                                           SplitBase{ws_qsplit_.data(), ws_bsplit_.data(), split_rows, dp});
+    } else {
+        launch_sqnorm_rows(xd, n, d_, ws_qn_.data(), stream_);
+        launches = stream_select_f32(xd, n, base_.data(), ntotal_, d_, ws_qn_.data(), norms_.data(), metric_, ncand,
+                                     ws_running_.data(), ws_sel_, scratch_bytes_, stream_, mask_dev, mask_stride);
+    }
     if (mask_dev) {
         launch_drop_worst_keys_f32(ws_running_.data(), n * ncand, stream_);   // vectors the query leaves out
     }
@@ -637,12 +662,15 @@ void FlatIndex::search_masked(int64_t n, const float *x, int64_t k, float *dist,
     stats_.exact_reruns = 0;
     if (ncand < ntotal_) {
         const float u = 5.9604645e-8f;
-        const float err_scale = (metric_ == kMetricL2 ? 2.0f : 1.0f) * (float)(2 * d_ + 8) * u;
+        // (bf16 x 3: hi + lo misses at most 2^-18 of a value, so the three products kept miss at most 3 x 2^-18 sum |x_i y_i|;
+        // their 3 dp terms are exact and summed in some order)
+        const float dots = metric_ == kMetricL2 ? 2.0f : 1.0f;
+        const float err_scale = split ? dots * (3.0f / 262144.0f + (float)(3 * dp + d_ + 8) * u) : dots * (float)(2 * d_ + 8) * u;
         const float round_scale = metric_ == kMetricL2 ? 4.0f * u : 0.0f;
         ws_flag_.resize((size_t)n + 1);
         IXA_HIP(hipMemsetAsync(ws_flag_.data(), 0, sizeof(int32_t), stream_));
         launch_verify_superset(ws_running_.data(), ncand, dd, (int)k, ws_qn_.data(), bmax_, err_scale, round_scale, metric_,
-                               n, ws_flag_.data(), stream_);
+                               n, ws_flag_.data(), stream_, split);
         int32_t nfail = 0;
         ws_flag_.download(&nfail, 1, stream_);
         if (nfail > 0) {

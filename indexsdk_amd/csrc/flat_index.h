@@ -92,6 +92,7 @@ public:
         borrow_base(owner);
         norms_.borrow(owner.norms_);
         bmax_ = owner.bmax_;
+        finite_ = owner.finite_;
     }
 
 private:
@@ -101,10 +102,12 @@ private:
     void search_masked(int64_t n, const float *x, int64_t k, float *dist, int64_t *labels, bool on_device,
                        const uint8_t *mask_dev, int64_t mask_stride);
     DeviceBuffer<float> norms_, ws_qn_, ws_dist_;
+    DeviceBuffer<uint16_t> ws_qsplit_, ws_bsplit_;   // bf16 x 3 splits of a search's queries and of a stretch of the base
     StreamSelectWorkspace<float> ws_sel_;
     DeviceBuffer<int32_t> ws_cand_, ws_idx_, ws_flag_;
     DeviceBuffer<int64_t> ws_labels_;
     float bmax_ = 0.f;   // largest base vector norm
+    bool finite_ = true; // no vector with an infinite or undefined norm was added
 };
 
 class FlatI8Index : public FlatBase<int8_t> {

@@ -721,13 +721,17 @@ __global__ __launch_bounds__(256) void verify_superset_kernel(const key_t *__res
                                                               const float *__restrict__ exact_dist, int nout,
                                                               const float *__restrict__ qn, float cmax, float err_scale,
                                                               float round_scale, int metric, int64_t nq,
-                                                              int *__restrict__ flag)
+                                                              int *__restrict__ flag, bool finite_only)
 {
     const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (i >= nq) {
         return;
     }
     const key_t last = running[i * ncand + (ncand - 1)];
+    if (finite_only && !(qn[i] < __builtin_inff())) {
+        flag[1 + atomicAdd(flag, 1)] = (int)i;   // products of split parts say nothing about such a query
+        return;
+    }
     if (last == kEmptyKey) {
         return;
     }
@@ -743,11 +747,11 @@ __global__ __launch_bounds__(256) void verify_superset_kernel(const key_t *__res
 
 void launch_verify_superset(const unsigned long long *running, int ncand, const float *exact_dist, int nout,
                             const float *qn, float cmax, float err_scale, float round_scale, int metric, int64_t nq,
-                            int *flag, hipStream_t s)
+                            int *flag, hipStream_t s, bool finite_only)
 {
     if (nq > 0) {
         hipLaunchKernelGGL(verify_superset_kernel, dim3((unsigned)((nq + 255) / 256)), dim3(256), 0, s, running, ncand,
-                           exact_dist, nout, qn, cmax, err_scale, round_scale, metric, nq, flag);
+                           exact_dist, nout, qn, cmax, err_scale, round_scale, metric, nq, flag, finite_only);
     }
 }
 

@@ -29,6 +29,19 @@ struct StreamSelectWorkspace {
 int stream_select_f32(const float *Q, int64_t nq, const float *B, int64_t nb, int d, const float *qn, const float *bn,
                       int metric, int ncand, unsigned long long *running, StreamSelectWorkspace<float> &ws,
                       int64_t scratch_bytes, hipStream_t s, const uint8_t *mask = nullptr, int64_t mask_stride = 0);
+// The same selection with the scores of fp32 operands formed from their bf16 x 3 splits (approximate: the caller refines and
+// proves).  query: the split queries (rows of 3 dp elements); base: room for rows + kSplitMinRows split base rows, which are
+// written stretch by stretch on the stream.  No mask.
+constexpr int64_t kSplitMinRows = 2048;   // shorter stretches take the fp32 kernels
+struct SplitBase {
+    const uint16_t *query;
+    uint16_t *base;
+    int64_t rows;
+    int dp;
+};
+int stream_select_f32_split(const float *Q, int64_t nq, const float *B, int64_t nb, int d, const float *qn, const float *bn,
+                            int metric, int ncand, unsigned long long *running, StreamSelectWorkspace<float> &ws,
+                            int64_t scratch_bytes, hipStream_t s, const SplitBase &split);
 // Same selection with approximate scores: Qs / Bs are the bf16 x 3 splits of the operands (rows of d3
 // bf16 elements, see launch_split_bf16x3), qn / bn the exact fp32 norms.  Returns -1 without doing
 // anything when the shape does not qualify for the bf16 matrix-core kernel.

@@ -127,6 +127,62 @@ struct F32Ops {
     }
 };
 
+// fp32 operands whose products run on the bf16 matrix cores: queries split once per call ([hi | hi | lo], by the caller),
+// base rows split ([hi | lo | hi]) stretch by stretch into a buffer small enough to stay in the memory-side cache until the
+// score launch reads it.  Three bf16 products per element run about 3.5 x as fast as one fp32 product; splitting a row costs
+// 10 bytes of traffic per element, whatever the number of queries, so large batches take this path (flat.hip has the line).
+//
+// At this rate an admitted key (an atomic each) costs as much as thousands of scores, so the bound is tightened early, as for
+// int8: a longer seed and chunks of twice what has been seen.  1M x 128, 1000 queries, k 100: fp32 scores 3.19 ms; splits with
+// the fp32 plan's seed of 2048 and chunks of 4 x 2.30 ms (the first 50000 rows alone 0.45 ms).
+struct F32SplitOps : F32Ops {
+    static constexpr int64_t kSeedRows = 16384, kMaxGrowth = 2;
+    SplitBase sp;
+    F32SplitOps(const float *qn_, const float *bn_, int metric_, const SplitBase &sp_) : F32Ops{qn_, bn_, metric_}, sp(sp_) {}
+    // calls fn(first row, rows) for the stretches of [b0, b0 + nb), none shorter than the ring kernel takes
+    template <typename Fn>
+    void stretches(int64_t nb, Fn &&fn) const
+    {
+        for (int64_t o = 0; o < nb;) {
+            const int64_t rows = nb - o < sp.rows + kSplitMinRows ? nb - o : sp.rows;
+            fn(o, rows);
+            o += rows;
+        }
+    }
+    void scores(const T *Q, int64_t nq, int64_t q0, const T *B, int64_t nb, int64_t b0, int d, S *out, int64_t ldo,
+                hipStream_t s) const
+    {
+        if (nb < kSplitMinRows) {
+            F32Ops::scores(Q, nq, q0, B, nb, b0, d, out, ldo, s);
+            return;
+        }
+        stretches(nb, [&](int64_t o, int64_t rows) {
+            launch_split_bf16x3_rows(B + (b0 + o) * d, rows, d, sp.dp, true, sp.base, s);
+            if (!launch_score_ring_bf16(sp.query + q0 * 3 * sp.dp, nq, sp.base, rows, 3 * sp.dp, qn + q0, bn + b0 + o,
+                                        metric, out + o, ldo, false, ScoreFilter<float>{}, s)) {
+                F32Ops::scores(Q, nq, q0, B, rows, b0 + o, d, out + o, ldo, s);
+            }
+        });
+    }
+    void filtered(const T *Q, int64_t nq, int64_t q0, const T *B, int64_t nb, int64_t b0, int d, ScoreFilter<S> flt,
+                  hipStream_t s) const
+    {
+        if (nb < kSplitMinRows) {
+            F32Ops::filtered(Q, nq, q0, B, nb, b0, d, flt, s);
+            return;
+        }
+        const int64_t col_base = flt.col_base;
+        stretches(nb, [&](int64_t o, int64_t rows) {
+            flt.col_base = col_base + o;
+            launch_split_bf16x3_rows(B + (b0 + o) * d, rows, d, sp.dp, true, sp.base, s);
+            if (!launch_score_ring_bf16(sp.query + q0 * 3 * sp.dp, nq, sp.base, rows, 3 * sp.dp, qn + q0, bn + b0 + o,
+                                        metric, nullptr, 0, true, flt, s)) {
+                F32Ops::filtered(Q, nq, q0, B, rows, b0 + o, d, flt, s);
+            }
+        });
+    }
+};
+
 struct Bf16Ops {
     using T = uint16_t;
     using S = float;
@@ -342,6 +398,13 @@ int stream_select_f32(const float *Q, int64_t nq, const float *B, int64_t nb, in
 {
     return stream_select(F32Ops{qn, bn, metric}, Q, nq, B, nb, d, ncand, running, ws, scratch_bytes, s, mask,
                          mask_stride);
+}
+
+int stream_select_f32_split(const float *Q, int64_t nq, const float *B, int64_t nb, int d, const float *qn, const float *bn,
+                            int metric, int ncand, unsigned long long *running, StreamSelectWorkspace<float> &ws,
+                            int64_t scratch_bytes, hipStream_t s, const SplitBase &split)
+{
+    return stream_select(F32SplitOps(qn, bn, metric, split), Q, nq, B, nb, d, ncand, running, ws, scratch_bytes, s);
 }
 
 void launch_apply_mask(float *scores, int64_t nq, int64_t ld, int64_t nc, const uint8_t *mask, int64_t mask_stride,

@@ -441,3 +441,47 @@ def test_flat_int8_mask_precision_recipe(ix, oracle):
         Dr, Ir = oracle.flat_i8(base[sel], q, k, ids=sel.astype(np.int64))
         assert np.array_equal(Im, Ir) and np.array_equal(Dm, Dr)
         assert passes[Im].all()
+
+
+# Batches of 256 queries and more over bases of 32768 rows and more form their candidate scores from bf16 x 3 splits; the
+# results are canonical scores all the same, so they equal the fp32 plan's bit for bit.
+@pytest.mark.parametrize("metric_name", ["L2", "IP"])
+@pytest.mark.parametrize("d,n,k,scratch", [(64, 32768, 1, 0), (100, 34817, 100, 0), (33, 70001, 20, 24 << 20),
+                                           (200, 50001, 300, 64 << 20)])
+def test_flat_f32_large_batches_equal_small_ones(ix, oracle, metric_name, d, n, k, scratch):
+    metric = ix.METRIC_L2 if metric_name == "L2" else ix.METRIC_INNER_PRODUCT
+    rng = np.random.default_rng(n + d)
+    centres = rng.standard_normal((200, d)).astype(np.float32)
+    base = (centres[rng.integers(0, 200, n)] + 0.4 * rng.standard_normal((n, d))).astype(np.float32)
+    base[n - 3] = base[100]
+    base[5] *= 50.0
+    q = (centres[rng.integers(0, 200, 259)] + 0.4 * rng.standard_normal((259, d))).astype(np.float32)
+    q[0] = base[100]
+    q[3] *= 1e-3
+    q[7, 1] = np.nan
+    q[8, 2] = np.inf
+    q[9, 0] = -np.inf
+    index = ix.AscendIndexFlat(d, metric, scratch_bytes=scratch)
+    index.add(base)
+    D, I = index.search(q, k)
+    for s in range(0, 259, 130):
+        Ds, Is = index.search(q[s:s + 130], k)
+        assert np.array_equal(I[s:s + 130], Is)
+        assert np.array_equal(D[s:s + 130].view(np.uint32), Ds.view(np.uint32))
+    Dr, Ir = oracle.flat_f32(base, q[10:40], k, metric)
+    assert np.array_equal(I[10:40], Ir) and np.array_equal(D[10:40].view(np.uint32), Dr.view(np.uint32))
+
+
+def test_flat_f32_base_with_values_out_of_range_keeps_the_fp32_plan(ix):
+    rng = np.random.default_rng(5)
+    d, n, k = 32, 40000, 10
+    base = rng.standard_normal((n, d)).astype(np.float32)
+    base[17, 3] = np.inf
+    base[18, 3] = np.nan
+    q = rng.standard_normal((300, d)).astype(np.float32)
+    for metric in (ix.METRIC_L2, ix.METRIC_INNER_PRODUCT):
+        index = ix.AscendIndexFlat(d, metric)
+        index.add(base)
+        D, I = index.search(q, k)
+        Ds, Is = index.search(q[:100], k)
+        assert np.array_equal(I[:100], Is) and np.array_equal(D[:100].view(np.uint32), Ds.view(np.uint32))
