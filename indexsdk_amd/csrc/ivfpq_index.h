@@ -157,7 +157,7 @@ private:
     void relayout(const std::vector<int32_t> &cap, int64_t min_slots);
     void sync_list_tables();
     void kmeans_coarse(const float *sample_dev, int64_t ns);
-    void kmeans_pq(const float *sample_dev, int64_t ns);
+    void kmeans_pq(const float *sample_dev, int64_t ns, const std::vector<int64_t> &rows_of);
 
     int d_, M_, dsub_, metric_;
     int64_t nlist_;

@@ -5,10 +5,12 @@
 #include <cmath>
 #include <cstdlib>
 #include <cstring>
+#include <future>
 #include <initializer_list>
 #include <mutex>
 #include <numeric>
 #include <random>
+#include <system_error>
 #include <thread>
 #include <unordered_set>
 
@@ -1809,6 +1811,22 @@ const SearchStats &IvfpqIndex::stats()
 // computeTrainTotalSize / sampleTrainData (FR/ascend/impl/AscendIndexIVFPQImpl.cpp:51-112).  Plain Lloyd
 // unless cfg.spherical.
 
+// 256 sample rows per sub-quantizer: the head of one shuffle each
+static std::vector<int64_t> first_codeword_rows(int64_t ns, int m_count, uint64_t seed)
+{
+    std::mt19937_64 gen(seed + 2);
+    std::vector<int64_t> rows((size_t)m_count * 256);
+    std::vector<uint32_t> pick((size_t)ns);   // half the memory to walk; the shuffle draws by position, whatever it moves
+    for (int m = 0; m < m_count; m++) {
+        std::iota(pick.begin(), pick.end(), 0u);
+        std::shuffle(pick.begin(), pick.end(), gen);
+        for (int k = 0; k < 256; k++) {
+            rows[(size_t)m * 256 + k] = (int64_t)pick[(size_t)(k % ns)];
+        }
+    }
+    return rows;
+}
+
 void IvfpqIndex::train(int64_t n, const float *x, bool on_device)
 {
     flush_stats();
@@ -1846,8 +1864,17 @@ void IvfpqIndex::train(int64_t n, const float *x, bool on_device)
         sample_dev.upload(sample.data(), sample.size(), stream_);
         sync_stream(stream_);   // the host copy is freed on leaving this block
     }
+    // The sample rows of the first codewords are drawn while the coarse quantizer trains on the device: M shuffles of ns
+    // numbers, 10.8 ms for 131072 samples and M = 32 when the stream waited for them (build of 1M x 128: 53.8 -> 41.5 ms).
+    auto draw = [ns, m = M_, seed = cfg_.seed] { return first_codeword_rows(ns, m, seed); };
+    std::future<std::vector<int64_t>> rows;
+    try {
+        rows = std::async(std::launch::async, draw);
+    } catch (const std::system_error &) {
+        rows = std::async(std::launch::deferred, draw);   // no thread to be had: drawn when they are asked for
+    }
     kmeans_coarse(sample_dev.data(), ns);
-    kmeans_pq(sample_dev.data(), ns);
+    kmeans_pq(sample_dev.data(), ns, rows.get());
     trained_ = true;
 }
 
@@ -1897,23 +1924,13 @@ void IvfpqIndex::kmeans_coarse(const float *sample_dev, int64_t ns)
     sync_stream(stream_);
 }
 
-void IvfpqIndex::kmeans_pq(const float *sample_dev, int64_t ns)
+void IvfpqIndex::kmeans_pq(const float *sample_dev, int64_t ns, const std::vector<int64_t> &rows_of)
 {
     const int niter = cfg_.pq_niter >= 0 ? cfg_.pq_niter : cfg_.niter;
     // the first codewords of sub-quantizer m are the m-th sub-vectors of 256 sample rows: those rows are gathered
     // on the device (M x 256 rows come to the host, not the sample)
     std::vector<float> cb((size_t)M_ * 256 * dsub_);
-    std::mt19937_64 gen(cfg_.seed + 2);
     {
-        std::vector<int64_t> rows_of((size_t)M_ * 256);
-        for (int m = 0; m < M_; m++) {
-            std::vector<int64_t> pick((size_t)ns);
-            std::iota(pick.begin(), pick.end(), 0);
-            std::shuffle(pick.begin(), pick.end(), gen);
-            for (int k = 0; k < 256; k++) {
-                rows_of[(size_t)m * 256 + k] = pick[(size_t)(k % ns)];
-            }
-        }
         DeviceBuffer<int64_t> rows_dev;
         DeviceBuffer<float> picked((size_t)M_ * 256 * d_);
         std::vector<float> h_picked((size_t)M_ * 256 * d_);
