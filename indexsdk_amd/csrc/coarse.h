@@ -147,11 +147,15 @@ constexpr int kSelectMaxK = 3072;
 // (ordered score << 32) | (col_base + column): its content takes part in the selection and is
 // replaced by the result, so calling this over successive column chunks keeps a streaming top-k.
 // Before the first chunk fill it with 0xff bytes, or pass fresh = true for that chunk (`running` is then
-// only written).
+// only written).  parts (may be null): select_parts_keys() keys of scratch with which few long rows are selected by several
+// workgroups each.
 void launch_select_rows(const float *scores, int64_t nrows, int64_t ld, int64_t nc, int ksel, int32_t *out_idx,
-                        int64_t col_base, unsigned long long *running, hipStream_t s, bool fresh = false);
+                        int64_t col_base, unsigned long long *running, hipStream_t s, bool fresh = false,
+                        unsigned long long *parts = nullptr);
 void launch_select_rows_i32(const int32_t *scores, int64_t nrows, int64_t ld, int64_t nc, int ksel, int32_t *out_idx,
-                            int64_t col_base, unsigned long long *running, hipStream_t s, bool fresh = false);
+                            int64_t col_base, unsigned long long *running, hipStream_t s, bool fresh = false,
+                            unsigned long long *parts = nullptr);
+size_t select_parts_keys(int64_t nrows, int64_t nc, int ksel);   // 0: no scratch wanted
 
 // Exact best-nout SET from approximately scored, sorted candidates (see refine_boundary_kernel):
 // re-evaluates only the candidates within 2 * err of the rank-nout score; a query whose list

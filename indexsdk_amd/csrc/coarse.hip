@@ -755,8 +755,17 @@ __device__ __forceinline__ void rank_select_256(key_t *src, int have, int n, key
 template <typename S, int G>
 __global__ __launch_bounds__(256, IXA_SELREG_WAVES) void select_rows_reg_kernel(
     const S *__restrict__ scores, int64_t ld, int64_t nc, int ksel, int cap, int32_t *__restrict__ out_idx,
-    int64_t col_base, key_t *__restrict__ running, bool fresh)
+    int64_t col_base, key_t *running, bool fresh, int64_t part_cols, key_t *parts)
 {
+    if (part_cols) {
+        // a stretch of the row per workgroup: its best keys go to parts[row][stretch], select_parts_kernel takes it from there
+        const int64_t c0 = (int64_t)blockIdx.y * part_cols;
+        scores += c0;
+        col_base += c0;
+        nc = nc - c0 < part_cols ? nc - c0 : part_cols;
+        fresh = true;
+        running = parts + ((int64_t)blockIdx.x * (gridDim.y - 1) + blockIdx.y) * ksel;   // + blockIdx.x * ksel below
+    }
     extern __shared__ __align__(16) unsigned char smem_raw[];
     key_t *cand = reinterpret_cast<key_t *>(smem_raw);            // kSelRegCap + 2
     key_t *best = cand + kSelRegCap + 2;                          // kSelRegMaxK
@@ -1115,6 +1124,68 @@ void launch_tau_from_minima(const float *gm, int G, int rank, int64_t nq, float 
     }
 }
 
+// Few rows of many columns: with one workgroup per row most of the GPU is idle (8 rows of 250000 columns, 128 keys: 205 of the
+// 260 us of a search's GPU time; the whole call 296 -> 145 us with this plan).  The rows are cut into stretches of whole segments, each selected from registers by a
+// workgroup of its own, and one more workgroup per row orders the stretches' keys and those of `running`.
+constexpr int kPartKeys = 4096;    // keys of a row that are ordered together
+constexpr int kPartRows = 64;      // above, a workgroup per row fills enough of the GPU
+
+__global__ __launch_bounds__(1024) void select_parts_kernel(const key_t *__restrict__ parts, int nparts, int ksel,
+                                                            int32_t *__restrict__ out_idx, key_t *__restrict__ running,
+                                                            bool fresh)
+{
+    __shared__ __align__(16) key_t buf[kPartKeys];
+    __shared__ int count;
+    const int tid = threadIdx.x;
+    const int64_t row = blockIdx.x;
+    if (tid == 0) {
+        count = 0;
+    }
+    __syncthreads();
+    const int own = nparts * ksel, all = own + (running && !fresh ? ksel : 0);
+    for (int i0 = 0; i0 < all; i0 += 1024) {
+        const int i = i0 + tid;
+        const key_t k = i < own ? parts[row * own + i] : (i < all ? running[row * ksel + i - own] : kEmptyKey);
+        const unsigned long long m = __ballot(k != kEmptyKey);
+        int at = 0;
+        if ((tid & 63) == 0 && m) {
+            at = atomicAdd(&count, __popcll(m));
+        }
+        at = __builtin_amdgcn_readfirstlane(at) +
+             (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0));
+        if (k != kEmptyKey) {
+            buf[at] = k;
+        }
+    }
+    __syncthreads();
+    const int n = count;
+    block_sort_keys<1024>(buf, n, tid);
+    for (int i = tid; i < ksel; i += 1024) {
+        const key_t k = i < n ? buf[i] : kEmptyKey;
+        if (out_idx) {
+            out_idx[row * ksel + i] = k == kEmptyKey ? -1 : (int32_t)key_index(k);
+        }
+        if (running) {
+            running[row * ksel + i] = k;
+        }
+    }
+}
+
+// stretches a row is cut into (1: not at all)
+static int select_parts(int64_t nrows, int64_t nc, int ksel)
+{
+    if (nrows > kPartRows || ksel > kSelRegMaxK || nc < 2 * kSelRegSeg) {
+        return 1;
+    }
+    return (int)std::min<int64_t>({(nc + kSelRegSeg - 1) / kSelRegSeg, kPartKeys / ksel - 1, 64});
+}
+
+size_t select_parts_keys(int64_t nrows, int64_t nc, int ksel)
+{
+    const int parts = select_parts(nrows, nc, ksel);
+    return parts > 1 ? (size_t)nrows * parts * ksel : 0;
+}
+
 // Few keys from short float rows (assignment during training and adding, small coarse stages): one wavefront per row, the row
 // in registers, and one extraction of the smallest key per result.  The pools above pay a workgroup, a merge and a sort per
 // row for the same few keys: 9 of 1024 columns 121 us per 12000 rows, 17 of the 40 ms of GPU time of building a 1M index.
@@ -1214,7 +1285,8 @@ __global__ __launch_bounds__(256) void select_rows_wave_kernel(const float *__re
 
 template <typename S>
 static void launch_select_rows_t(const S *scores, int64_t nrows, int64_t ld, int64_t nc, int ksel, int32_t *out_idx,
-                                 int64_t col_base, unsigned long long *running, bool fresh, hipStream_t s)
+                                 int64_t col_base, unsigned long long *running, bool fresh, hipStream_t s,
+                                 unsigned long long *parts)
 {
     if (nrows == 0) {
         return;
@@ -1242,13 +1314,20 @@ static void launch_select_rows_t(const S *scores, int64_t nrows, int64_t ld, int
     const bool vec4 = ld % 4 == 0 && reinterpret_cast<uintptr_t>(scores) % 16 == 0;
     // measured: the register kernel wins on rows of up to a few segments (16384 columns: 0.17 ms against
     // 0.27 ms for 10000 rows, ksel 88), the streaming kernel on rows of hundreds of thousands of columns
-    if (vec4 && ksel <= kSelRegMaxK && nc >= 2048 && nc <= 6 * kSelRegSeg) {
+    const int nparts = parts && vec4 ? select_parts(nrows, nc, ksel) : 1;
+    if (nparts > 1 || (vec4 && ksel <= kSelRegMaxK && nc >= 2048 && nc <= 6 * kSelRegSeg)) {
         smem = std::max(smem, (size_t)(kSelRegCap + 2 + kSelRegMaxK + 4 * kSelRegStage) * sizeof(key_t) + 4 * 64 * 4 * 4 + 64);
         // groups per lane: ksel / (256 G) stays near 1/3
         auto kern = ksel <= 96 ? select_rows_reg_kernel<S, 1>
                                : (ksel <= 192 ? select_rows_reg_kernel<S, 2> : select_rows_reg_kernel<S, 4>);
-        hipLaunchKernelGGL(kern, dim3((unsigned)nrows), dim3(256), smem, s, scores, ld, nc, ksel, cap, out_idx,
-                           col_base, running, fresh);
+        const int64_t part_cols = nparts > 1 ? round_up((nc + nparts - 1) / nparts, kSelRegSeg) : 0;
+        const unsigned used = part_cols ? (unsigned)((nc + part_cols - 1) / part_cols) : 1;   // <= nparts
+        hipLaunchKernelGGL(kern, dim3((unsigned)nrows, used), dim3(256), smem, s, scores, ld, nc, ksel, cap, part_cols ? nullptr : out_idx,
+                           col_base, running, fresh, part_cols, parts);
+        if (part_cols) {
+            hipLaunchKernelGGL(select_parts_kernel, dim3((unsigned)nrows), dim3(1024), 0, s, parts, (int)used, ksel, out_idx,
+                               running, fresh);
+        }
         return;
     }
     auto kern = active == 4 ? select_rows_kernel<S, 4> : (active == 2 ? select_rows_kernel<S, 2> : select_rows_kernel<S, 1>);
@@ -1258,15 +1337,16 @@ static void launch_select_rows_t(const S *scores, int64_t nrows, int64_t ld, int
 }
 
 void launch_select_rows(const float *scores, int64_t nrows, int64_t ld, int64_t nc, int ksel, int32_t *out_idx,
-                        int64_t col_base, unsigned long long *running, hipStream_t s, bool fresh)
+                        int64_t col_base, unsigned long long *running, hipStream_t s, bool fresh, unsigned long long *parts)
 {
-    launch_select_rows_t<float>(scores, nrows, ld, nc, ksel, out_idx, col_base, running, fresh, s);
+    launch_select_rows_t<float>(scores, nrows, ld, nc, ksel, out_idx, col_base, running, fresh, s, parts);
 }
 
 void launch_select_rows_i32(const int32_t *scores, int64_t nrows, int64_t ld, int64_t nc, int ksel, int32_t *out_idx,
-                            int64_t col_base, unsigned long long *running, hipStream_t s, bool fresh)
+                            int64_t col_base, unsigned long long *running, hipStream_t s, bool fresh,
+                            unsigned long long *parts)
 {
-    launch_select_rows_t<int32_t>(scores, nrows, ld, nc, ksel, out_idx, col_base, running, fresh, s);
+    launch_select_rows_t<int32_t>(scores, nrows, ld, nc, ksel, out_idx, col_base, running, fresh, s, parts);
 }
 
 // ------------------------------------------------------------------------------------------------

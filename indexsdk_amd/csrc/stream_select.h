@@ -10,6 +10,7 @@ struct StreamSelectWorkspace {
     DeviceBuffer<S> scores, tau, thr;
     DeviceBuffer<int32_t> cnt;                    // per-query admitted-candidate counters + overflow flag
     DeviceBuffer<unsigned long long> filter;
+    DeviceBuffer<unsigned long long> parts;       // keys of the stretches of few long rows (launch_select_rows)
     bool cnt_zero = false;                        // every counter is zero (the sampled-bound plan keeps them so)
 };
 

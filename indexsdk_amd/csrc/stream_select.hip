@@ -116,9 +116,9 @@ struct F32Ops {
         launch_score_tiles_filtered(Q, nq, B + b0 * d, nb, d, qn + q0, bn + b0, metric, flt, s);
     }
     void select(const S *sc, int64_t nq, int64_t ld, int64_t nc, int k, int64_t base, key_t *run, bool fresh,
-                hipStream_t s) const
+                hipStream_t s, key_t *parts) const
     {
-        launch_select_rows(sc, nq, ld, nc, k, nullptr, base, run, s, fresh);
+        launch_select_rows(sc, nq, ld, nc, k, nullptr, base, run, s, fresh, parts);
     }
     static constexpr bool kMergeKeepsThreshold = false;
     void merge(key_t *run, int k, ScoreFilter<S> flt, S *tau, int64_t nq, int64_t, int *ovf, hipStream_t s) const
@@ -129,12 +129,12 @@ struct F32Ops {
 
 // fp32 operands whose products run on the bf16 matrix cores: queries split once per call ([hi | hi | lo], by the caller),
 // base rows split ([hi | lo | hi]) stretch by stretch into a buffer small enough to stay in the memory-side cache until the
-// score launch reads it.  Three bf16 products per element run about 3.5 x as fast as one fp32 product; splitting a row costs
+// score launch reads it.  Three bf16 products per element run about 2.5 x as fast as one fp32 product; splitting a row costs
 // 10 bytes of traffic per element, whatever the number of queries, so large batches take this path (flat.hip has the line).
 //
 // At this rate an admitted key (an atomic each) costs as much as thousands of scores, so the bound is tightened early, as for
 // int8: a longer seed and chunks of twice what has been seen.  1M x 128, 1000 queries, k 100: fp32 scores 3.19 ms; splits with
-// the fp32 plan's seed of 2048 and chunks of 4 x 2.30 ms (the first 50000 rows alone 0.45 ms).
+// the fp32 plan's seed of 2048 and chunks of 4 x 2.30 ms (the first 50000 rows alone 0.45 ms), with these 1.84 ms.
 struct F32SplitOps : F32Ops {
     static constexpr int64_t kSeedRows = 16384, kMaxGrowth = 2;
     SplitBase sp;
@@ -205,9 +205,9 @@ struct Bf16Ops {
         IXA_REQUIRE(ok, kErrInner, "bf16 score kernel rejected a shape it had accepted");
     }
     void select(const S *sc, int64_t nq, int64_t ld, int64_t nc, int k, int64_t base, key_t *run, bool fresh,
-                hipStream_t s) const
+                hipStream_t s, key_t *parts) const
     {
-        launch_select_rows(sc, nq, ld, nc, k, nullptr, base, run, s, fresh);
+        launch_select_rows(sc, nq, ld, nc, k, nullptr, base, run, s, fresh, parts);
     }
     static constexpr bool kMergeKeepsThreshold = false;
     void merge(key_t *run, int k, ScoreFilter<S> flt, S *tau, int64_t nq, int64_t, int *ovf, hipStream_t s) const
@@ -245,9 +245,9 @@ struct I8Ops {
         launch_i8_scores_filtered(Q, nq, B, d, qn + q0, bn, b0, b0 + nb, flt, s);
     }
     void select(const S *sc, int64_t nq, int64_t ld, int64_t nc, int k, int64_t base, key_t *run, bool fresh,
-                hipStream_t s) const
+                hipStream_t s, key_t *parts) const
     {
-        launch_select_rows_i32(sc, nq, ld, nc, k, nullptr, base, run, s, fresh);
+        launch_select_rows_i32(sc, nq, ld, nc, k, nullptr, base, run, s, fresh, parts);
     }
     // the merge writes the next launch's thresholds along with the new bounds
     static constexpr bool kMergeKeepsThreshold = true;
@@ -352,7 +352,12 @@ int stream_select(const Ops &ops, const typename Ops::T *Q, int64_t nq_total, co
                     apply_mask(ws.scores.data(), nq, ldo, nbc, mask + q0 * mask_stride, mask_stride, nullptr, b0, s);
                 }
                 // the first chunk of a query block starts its running keys (whatever `running` held)
-                ops.select(ws.scores.data(), nq, ldo, nbc, ncand, b0, running + q0 * ncand, b0 == 0, s);
+                const size_t part_keys = select_parts_keys(nq, nbc, ncand);
+                if (part_keys > ws.parts.size()) {
+                    ws.parts.resize(part_keys);
+                }
+                ops.select(ws.scores.data(), nq, ldo, nbc, ncand, b0, running + q0 * ncand, b0 == 0, s,
+                           part_keys ? ws.parts.data() : nullptr);
                 launches++;
             }
             if (!fused) {

@@ -485,3 +485,25 @@ def test_flat_f32_base_with_values_out_of_range_keeps_the_fp32_plan(ix):
         D, I = index.search(q, k)
         Ds, Is = index.search(q[:100], k)
         assert np.array_equal(I[:100], Is) and np.array_equal(D[:100].view(np.uint32), Ds.view(np.uint32))
+
+
+# Up to 64 queries over 32768 rows and more: every row of scores is selected by several workgroups, whose keys one more orders.
+@pytest.mark.parametrize("nq,k,scratch", [(1, 1, 0), (8, 128, 0), (64, 300, 0), (65, 128, 0), (3, 384, 20 << 20), (3, 385, 0)])
+def test_flat_few_queries_over_a_long_base(ix, oracle, nq, k, scratch):
+    rng = np.random.default_rng(nq + k)
+    n, d = 100_003, 64
+    base = rng.integers(-20, 21, size=(n, d), dtype=np.int8)
+    base[50_000:50_400] = base[7]          # equal scores on both sides of a stretch's end
+    q = rng.integers(-20, 21, size=(nq, d), dtype=np.int8)
+    q[0] = base[7]
+    index = ix.AscendIndexInt8Flat(d, ix.METRIC_L2, scratch_bytes=scratch) if scratch else ix.AscendIndexInt8Flat(d, ix.METRIC_L2)
+    index.add(base)
+    D, I = index.search_int32(q, k)
+    Dr, Ir = oracle.flat_i8(base, q, k)
+    assert np.array_equal(D, Dr) and np.array_equal(I, Ir)
+    x, y = base.astype(np.float32), q.astype(np.float32)
+    index = ix.AscendIndexFlat(d, ix.METRIC_L2, scratch_bytes=scratch)
+    index.add(x)
+    D, I = index.search(y, k)
+    Dr, Ir = oracle.flat_f32(x, y, k, ix.METRIC_L2)
+    assert np.array_equal(D, Dr) and np.array_equal(I, Ir)

@@ -49,3 +49,22 @@ def test_sub_quantizer_update_with_remainders_and_empty_codewords(oracle, d, M, 
     for m in range(M):
         want = lloyd_step(x[:, m * dsub:(m + 1) * dsub], codes[:, m], books[0][m])
         assert np.array_equal(want.view(np.uint32), books[1][m].view(np.uint32)), m
+
+
+@pytest.mark.parametrize("nlist", [255, 256, 257, 512, 1024, 1025, 2047])
+def test_assignment_at_the_edges_of_the_row_widths(nlist):
+    """Assignment selects a few keys of nlist scores with one wavefront per row (4, 8, 16 or 32 values per lane); equal
+    centroids resolve to the smaller id."""
+    import indexsdk_amd as ix
+    from oracle import oracle as orc
+
+    rng = np.random.default_rng(nlist)
+    d, n = 32, 3001
+    cent = rng.standard_normal((nlist, d)).astype(np.float32)
+    cent[nlist - 1] = cent[3]
+    cent[64] = cent[0]
+    x = (cent[rng.integers(0, nlist, n)] + 0.2 * rng.standard_normal((n, d))).astype(np.float32)
+    x[0], x[1] = cent[3], cent[0]
+    gpu = ix.AscendIndexIVFPQ(d, ix.METRIC_L2, nlist, 8, 8)
+    gpu.set_trained(cent, orc.train_pq(x, 8, niter=1, seed=1))
+    assert np.array_equal(gpu.assign(x), orc.assign(x, cent))
