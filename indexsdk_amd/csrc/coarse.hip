@@ -1125,8 +1125,9 @@ void launch_tau_from_minima(const float *gm, int G, int rank, int64_t nq, float 
 }
 
 // Few rows of many columns: with one workgroup per row most of the GPU is idle (8 rows of 250000 columns, 128 keys: 205 of the
-// 260 us of a search's GPU time; the whole call 296 -> 145 us with this plan).  The rows are cut into stretches of whole segments, each selected from registers by a
-// workgroup of its own, and one more workgroup per row orders the stretches' keys and those of `running`.
+// 260 us of a search's GPU time; the whole call 296 -> 145 us with this plan).  The rows are cut into stretches of whole
+// segments, each selected from registers by a workgroup of its own, and one more workgroup per row orders the stretches' keys
+// and those of `running`.
 constexpr int kPartKeys = 4096;    // keys of a row that are ordered together
 constexpr int kPartRows = 64;      // above, a workgroup per row fills enough of the GPU
 
