@@ -131,6 +131,20 @@ void launch_split_bf16x3_rows(const float *x, int64_t n, int d, int dp, bool bas
 // launch_sqnorm_rows(x -> norms) and the query-side launch_split_bf16x3(x -> split) in one launch
 void launch_sqnorm_and_split_bf16x3(const float *x, int64_t n, int d, int dp, float *norms, uint16_t *split, hipStream_t s);
 
+// Largest difference between an approximate and the canonical score of a query with squared norm qnorm and any base vector no
+// longer than cmax: err_scale |q| cmax, and for L2 (round_scale > 0; 0 for inner product) round_scale (|q| + cmax)^2 on top.
+// Both lengths come from fp32 sums of squares, to which a square below 2^-126 may not contribute at all: a query of
+// components below 1e-19 has length 0 here and would be given a margin of 0.  So a margin exists only for lengths beside
+// which d lost squares, and d lost products, are nothing (1e-13: d * 2^-126 against 1e-26); for L2 it is enough that the sum
+// of the two is (1e-12), whose rounding term covers what the shorter one does.  Below, nothing is decided by approximate
+// scores: the margin is infinite.
+__device__ __forceinline__ float score_margin(float qnorm, float cmax, float err_scale, float round_scale)
+{
+    const float qlen = sqrtf(qnorm);
+    const bool lost = round_scale > 0.f ? qlen + cmax < 1e-12f : fminf(qlen, cmax) < 1e-13f;
+    return lost ? __builtin_inff() : err_scale * qlen * cmax + round_scale * (qlen + cmax) * (qlen + cmax);
+}
+
 // Sets *flag = 1 if some query's approximate candidate list (running[nq][ncand], ascending keys) is
 // not provably a superset of its best nout centroids; see score_ring.hip.  finite_only: a query whose norm is not
 // finite counts as unproven.

@@ -1443,7 +1443,7 @@ __global__ __launch_bounds__(256) void refine_kernel(const float *__restrict__ Q
 
 // Exact selection of the best `nout` candidates as a SET, touching only the candidates that the
 // approximate scores cannot decide.  `running` holds, per query, ncand keys sorted by approximate
-// score s, each within err = err_scale * |q| * cmax + round_scale * (|q| + cmax)^2 of the canonical score e.  With T = s at rank
+// score s, each within err = score_margin() of the canonical score e.  With T = s at rank
 // nout: a candidate with s < T - 2 err is certainly among the nout best (fewer than nout others have
 // s < T, and only those can have e below its e < T - err); one with s > T + 2 err certainly is not
 // (the nout candidates with s <= T all have e <= T + err).  Only the candidates in between are
@@ -1482,8 +1482,7 @@ __global__ __launch_bounds__(256) void refine_boundary_kernel(const float *__res
         return;
     }
     const float T = key_score(at_rank);
-    const float qlen = sqrtf(qn[row]);
-    const float err = err_scale * qlen * cmax + round_scale * (qlen + cmax) * (qlen + cmax);
+    const float err = score_margin(qn[row], cmax, err_scale, round_scale);
     const float lo = T - 2.0f * err, hi = T + 2.0f * err;
     const key_t last = run[ncand - 1];
     if (lane == 0 && !complete && last != kEmptyKey && !(key_score(last) > hi)) {   // a list of all rows is complete
@@ -1673,8 +1672,7 @@ __global__ __launch_bounds__(256) void fold_refine_boundary_kernel(
             p = below < nout ? c : p;
         }
         const float T = unordered_bits(p);
-        const float qlen = sqrtf(qnorm);
-        const float err = err_scale * qlen * cmax + round_scale * (qlen + cmax) * (qlen + cmax);
+        const float err = score_margin(qnorm, cmax, err_scale, round_scale);
         lo = T - 2.0f * err;
         hi = T + 2.0f * err;
         fail = !(tau > hi);

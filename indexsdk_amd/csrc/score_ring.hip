@@ -716,7 +716,7 @@ bool launch_score_ring_bf16_records(const uint16_t *Q, int64_t nq, const uint16_
 
 // Appends a query to the list flag[1 + flag[0]++] unless, for that query, no centroid outside its approximate candidate list can beat
 // its nout-th exact score: (approximate score of the last candidate) - err > (nout-th exact score),
-// err = err_scale * |q| * max|c| + round_scale * (|q| + max|c|)^2.  Rows whose candidate list is not full hold every centroid.
+// err = score_margin().  Rows whose candidate list is not full hold every centroid.
 __global__ __launch_bounds__(256) void verify_superset_kernel(const key_t *__restrict__ running, int ncand,
                                                               const float *__restrict__ exact_dist, int nout,
                                                               const float *__restrict__ qn, float cmax, float err_scale,
@@ -738,8 +738,7 @@ __global__ __launch_bounds__(256) void verify_superset_kernel(const key_t *__res
     const float a_last = key_score(last);
     const float d_out = exact_dist[i * nout + (nout - 1)];
     const float s_star = metric == kMetricL2 ? d_out : -d_out;
-    const float qlen = sqrtf(qn[i]);
-    const float err = err_scale * qlen * cmax + round_scale * (qlen + cmax) * (qlen + cmax);
+    const float err = score_margin(qn[i], cmax, err_scale, round_scale);
     if (!(a_last - err > s_star)) {
         flag[1 + atomicAdd(flag, 1)] = (int)i;   // the list of queries that need another plan
     }

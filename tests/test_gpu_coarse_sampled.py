@@ -133,3 +133,29 @@ def test_sampled_bound_with_centroids_in_an_adverse_order(ix, oracle, case, scra
     Dr, Ir = ref.search(q, 10, nprobe)
     assert stats["scanned_codes"] == ref.last_scanned
     assert_topk_parity(oracle, ref, q, D, I, Dr, Ir, 1e-4)
+
+
+@pytest.mark.parametrize("nlist,nq,sampled", [(8192, 2112, 1), (8192, 2112, 0), (2048, 1100, 1)])
+@pytest.mark.parametrize("scale", [1e-24, 1e-36])
+def test_queries_of_vanishing_norm_prove_nothing(ix, oracle, nlist, nq, sampled, scale):
+    """Inner product, components so small that the fp32 sum of their squares is 0: the proofs' margin is a multiple of that
+    length, and centroids around one point have products closer to each other than the scores' error.  Every plan (sampled
+    bound, score matrix with boundary refinement, score matrix with superset proof) gives the oracle's lists."""
+    d, M, nprobe = 64, 8, 16
+    rng = np.random.default_rng(9)
+    cent = (rng.standard_normal(d) + 1e-6 * rng.standard_normal((nlist, d))).astype(np.float32)
+    q = (scale * rng.standard_normal((nq, d))).astype(np.float32)
+    cb = rng.standard_normal((M, 256, d // M)).astype(np.float32)
+    x = rng.standard_normal((20000, d)).astype(np.float32)
+    gpu = ix.AscendIndexIVFPQ(d, ix.METRIC_INNER_PRODUCT, nlist, M, 8, ix.AscendIndexIVFPQConfig(coarse_sampled_bound=sampled))
+    gpu.set_trained(cent, cb)
+    gpu.setNumProbes(nprobe)
+    gi, gd = gpu.coarse_probe(q)
+    oi, od = oracle.coarse_probe(q, cent, nprobe, ix.METRIC_INNER_PRODUCT)
+    assert np.array_equal(gi, oi) and np.array_equal(gd.view(np.uint32), od.view(np.uint32))
+    ids = np.arange(len(x), dtype=np.int64)
+    gpu.add_with_ids(x, ids)
+    ref = oracle.CsrIndex.build(d, M, ix.METRIC_INNER_PRODUCT, cent, cb, x, ids)
+    D, I = gpu.search(q, 5)
+    ref.search(q, 5, nprobe)
+    assert gpu.last_search_stats()["scanned_codes"] == ref.last_scanned      # the same SET of lists for every query

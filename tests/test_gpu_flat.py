@@ -507,3 +507,24 @@ def test_flat_few_queries_over_a_long_base(ix, oracle, nq, k, scratch):
     D, I = index.search(y, k)
     Dr, Ir = oracle.flat_f32(x, y, k, ix.METRIC_L2)
     assert np.array_equal(D, Dr) and np.array_equal(I, Ir)
+
+
+# Vectors so short that fp32 sums of their squares lose everything (components below 1e-19): the length that the completeness
+# proof multiplies its error bound with is 0, so the proof may not be believed.  300 queries take the bf16 x 3 plan, 100 the fp32
+# one; the base lies so close around one point that its inner products differ by less than either plan's scores err.
+@pytest.mark.parametrize("metric_name", ["L2", "IP"])
+@pytest.mark.parametrize("qscale,bscale", [(1e-24, 1.0), (1e-30, 1.0), (1e-36, 1.0), (1.0, 1e-24), (1e-19, 1e-17)])
+def test_flat_f32_queries_and_bases_of_vanishing_norm(ix, oracle, metric_name, qscale, bscale):
+    metric = ix.METRIC_L2 if metric_name == "L2" else ix.METRIC_INNER_PRODUCT
+    rng = np.random.default_rng(24)
+    d, n, k = 64, 40000, 10
+    point = rng.standard_normal(d)
+    for spread in (1e-5, 1e-6):
+        base = (bscale * (point + spread * rng.standard_normal((n, d)))).astype(np.float32)
+        q = (qscale * rng.standard_normal((300, d))).astype(np.float32)
+        index = ix.AscendIndexFlat(d, metric)
+        index.add(base)
+        Dr, Ir = oracle.flat_f32(base, q[:40], k, metric)
+        for nq in (300, 100):
+            D, I = index.search(q[:nq], k)
+            assert np.array_equal(I[:40], Ir) and np.array_equal(D[:40].view(np.uint32), Dr.view(np.uint32)), (nq, spread)
