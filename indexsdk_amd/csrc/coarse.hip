@@ -1189,9 +1189,25 @@ size_t select_parts_keys(int64_t nrows, int64_t nc, int ksel)
 
 // Few keys from short float rows (assignment during training and adding, small coarse stages): one wavefront per row, the row
 // in registers, and one extraction of the smallest key per result.  The pools above pay a workgroup, a merge and a sort per
-// row for the same few keys: 9 of 1024 columns 121 us per 12000 rows, 17 of the 40 ms of GPU time of building a 1M index.
-// Beyond kSelWaveMaxK extractions their serial chain is longer than the pools' work.
+// row for the same few keys: 9 of 1024 columns 102 us per 12000 rows against 32 here.
 constexpr int kSelWaveMaxK = 24, kSelWaveMaxCols = 2048;
+
+// Most keys this kernel is given.  The extractions are a serial chain: 0.45 us each with 4 values per lane, 0.6 / 0.85 / 1.5 us
+// with 8 / 16 / 32, whatever the number of rows, while the pools' time hardly grows with ksel (6 - 14 us for up to 1000 rows).
+// Many rows hide the chain behind each other's (2048 columns, 4000 rows: 16 keys 45.1 us with the pools, 41.8 here; 24 keys
+// 45.9 / 49.8); few do not.  Up to 1000 rows, pools / here in us: 64 columns, 6 keys 7.6 / 6.8, 9 keys 7.8 / 8.3; 256 columns, 16
+// keys 11.7 / 11.7, 20 keys 11.7 / 13.4; 512 columns, 6 keys 11.9 / 8.9, 9 keys (257 columns) 10.3 / 10.8; 1000 columns, 4 keys
+// 12.1 / 10.2, 9 keys 12.7 / 16.4; 2048 columns, 2 keys 11.2 / 8.8, 4 keys 11.1 / 12.8, 24 keys 12.4 / 47.7.
+static int select_wave_max_k(int64_t nrows, int64_t nc)
+{
+    if (nc > kSelWaveMaxCols) {
+        return 0;
+    }
+    if (nrows >= 4000) {
+        return nc > 1024 ? 20 : kSelWaveMaxK;
+    }
+    return nc <= 128 ? 6 : (nc <= 256 ? 16 : (nc <= 512 ? 8 : (nc <= 1024 ? 3 : 2)));
+}
 
 template <int V>
 __global__ __launch_bounds__(256) void select_rows_wave_kernel(const float *__restrict__ scores, int64_t nrows, int64_t ld,
@@ -1295,7 +1311,7 @@ static void launch_select_rows_t(const S *scores, int64_t nrows, int64_t ld, int
     IXA_REQUIRE(ksel >= 1 && ksel <= kSelectMaxK, kErrInvalidParam, "selection size %d out of range [1, %d]", ksel,
                 kSelectMaxK);
     if constexpr (std::is_same<S, float>::value) {
-        if (ksel <= kSelWaveMaxK && nc <= kSelWaveMaxCols) {
+        if (ksel <= select_wave_max_k(nrows, nc)) {
             auto kern = nc <= 256 ? select_rows_wave_kernel<4>
                                   : (nc <= 512 ? select_rows_wave_kernel<8>
                                                : (nc <= 1024 ? select_rows_wave_kernel<16> : select_rows_wave_kernel<32>));

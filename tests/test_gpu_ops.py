@@ -68,6 +68,49 @@ def _p(b):
     return b.ptr
 
 
+def _topk_args(env, rows, n, k, seed=0):
+    hip, ix, _capi, lib = env
+    rng = np.random.default_rng(rows + n + k + seed)
+    d = np.round(rng.standard_normal((rows, n)) * 50).astype(np.float32) / 8     # many exact ties
+    return d, (_p(hip.put(d)), rows, n, n, k, 1), hip.empty((rows, k), np.float32), hip.empty((rows, k), np.int64)
+
+
+# Both sides of the lines between the selection by one wavefront per row and the pools: row widths of 4, 8, 16 and 32 values
+# per lane, the largest k each is given with few rows and the next one, and many rows.
+@pytest.mark.parametrize("rows", [3, 4000])
+@pytest.mark.parametrize("n,k", [(30, 6), (128, 7), (129, 16), (256, 17), (257, 8), (512, 9), (513, 3), (1024, 4), (1025, 2),
+                                 (2048, 3), (2048, 20), (1500, 21), (1024, 24), (700, 25), (2049, 1)])
+def test_topk_flat_fp32_of_few_keys(env, rows, n, k):
+    lib, _capi = env[3], env[2]
+    d, args, out_d, out_l = _topk_args(env, rows, n, k)
+    _capi.check(lib.ixa_op_topk_flat_fp32(*args, _p(out_d), _p(out_l), None))
+    want = np.argsort(d, axis=1, kind="stable")[:, :k]
+    assert np.array_equal(out_l.get(), want)
+    assert np.array_equal(out_d.get().view(np.uint32), np.take_along_axis(d, want, 1).view(np.uint32))
+
+
+@pytest.mark.parametrize("rows,n,k", [(64, 2048, 24), (8, 2048, 9), (64, 1024, 24), (8, 513, 24), (64, 64, 24)])
+def test_topk_of_few_rows_is_not_a_serial_chain(env, rows, n, k):
+    """Extracting the keys one after the other by a single wavefront is several times slower than the pools on few rows:
+    the call takes no longer than half as much again as the one of 25 keys, which the pools always serve."""
+    import time
+    hip, ix, _capi, lib = env
+
+    def seconds(kk):
+        d, args, out_d, out_l = _topk_args(env, rows, n, kk)
+        best = 1e9
+        for _ in range(5):
+            hip._ok(hip.rt.hipDeviceSynchronize())
+            t = time.perf_counter()
+            for _ in range(200):
+                lib.ixa_op_topk_flat_fp32(*args, _p(out_d), _p(out_l), None)
+            hip._ok(hip.rt.hipDeviceSynchronize())
+            best = min(best, time.perf_counter() - t)
+        return best
+
+    assert seconds(k) < 1.5 * seconds(25)
+
+
 @pytest.mark.parametrize("batch,n,d", [(37, 1013, 96), (5, 64, 128), (3, 7, 30), (20, 4096, 64)])
 def test_distance_flat_l2_mins(env, oracle, batch, n, d):
     hip, ix, _capi, lib = env

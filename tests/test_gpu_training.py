@@ -59,7 +59,7 @@ def test_assignment_at_the_edges_of_the_row_widths(nlist):
     from oracle import oracle as orc
 
     rng = np.random.default_rng(nlist)
-    d, n = 32, 3001
+    d, n = 32, 4001   # from 4000 rows on every width takes that kernel
     cent = rng.standard_normal((nlist, d)).astype(np.float32)
     cent[nlist - 1] = cent[3]
     cent[64] = cent[0]
