@@ -594,7 +594,39 @@ void FlatIndex::search_with_masks(int64_t n, const float *x, int64_t k, const ui
 
 namespace {
 constexpr int64_t kSplitBytes = (int64_t)256 << 20;   // split base rows in flight: what the memory-side cache holds
-constexpr int64_t kSplitMinQueries = 256, kSplitMinBase = 32768;
+
+// Whether a search forms its candidate scores from bf16 x 3 splits on the bf16 matrix cores.  Splitting the base costs 10 bytes
+// of traffic per element whatever the number of queries, and the split ring kernel scores 256 queries at a time, so a batch has
+// to bring more than one such tile and enough products.  fp32 / split, us per search, k 100:
+//   256 queries: 200k x 64 370 / 423, 200k x 128 440 / 482, 400k x 128 769 / 818, 65536 x 768 371 / 455; from 1M on 1627 / 1101
+//   (d 128), 2117 / 1654 (d 256), 1628 / 1612 (d 64, k 300).  128 queries: 1M x 128 1566 / 1639, 200k x 128 429 / 456.  (160 - 255
+//   queries over 1M rows and more would gain as well, 160 over 1M x 128 1587 / 1060; they have the fp32 plan all the same.)
+//   320 queries: 32768 x 128 171 / 166, 65536 x 128 238 / 223, 200k x 128 631 / 577, 400k x 128 1073 / 768, 32768 x 768 362 / 306;
+//   d 64, where a tile's products are few: 512 queries 32768 152 / 159, 100k 325 / 341, 200k 542 / 541, 400k 908 / 659; 1024
+//   queries 32768 200 / 198, 100k 487 / 469, 200k 805 / 580; and none with very many keys (300k, 1024 queries, k 500 1902 / 1819,
+//   k 1000 3760 / 4206).
+// Half of the scratch goes to the split base, with three consequences:
+//   Where the fp32 plan could still keep the whole score matrix and the split plan no longer can, the bound-filtered launches
+//   that take its place win with few keys (512 queries, 400k x 128, k 10: 1075 / 548, k 100: 1100 / 769) and lose with many
+//   (k 300: 1299 / 1534).
+//   Where the candidate buffers of the batch do not fit the other half, the queries go in blocks and the base is split for each
+//   (300k x 128, k 300, 1024 queries: 64 MB 2579 / 3008, 128 MB 2648 / 1772; k 100, 4096 queries: 32 MB 4400 / 4906, 64 MB
+//   4040 / 2938; k 300, 4096 queries: 128 MB 8300 / 6665).
+//   Short stretches of split rows pay a launch each (300k x 64, 1024 queries, k 10: 16 MB 769 / 994, 32 MB 747 / 704; d 128, 32
+//   MB: 1034 / 993).
+bool split_pays(int64_t nq, int64_t nb, int dp, int64_t k, int64_t ncand, int64_t scratch_bytes)
+{
+    const int64_t half = scratch_bytes - scratch_bytes / 2, mb = (int64_t)1 << 20;
+    const int64_t matrix = round_up(nq, 128) * round_up(nb, 128) * (int64_t)sizeof(float);
+    if (scratch_bytes < 30 * mb || (dp < 128 && k > 512) || (k > 128 && matrix <= scratch_bytes && matrix > half)) {
+        return false;
+    }
+    const int64_t candidates = std::min<int64_t>(round_up(nq, 128), 16384) * stream_select_candidates((int)ncand) * 8;
+    if (candidates > half && scratch_bytes < (k <= 128 ? 64 : 128) * mb) {
+        return false;
+    }
+    return nq >= 256 && nb >= (nq == 256 ? 1000000 : (dp >= 128 || nq >= 1024 ? 32768 : 250000));
+}
 }  // namespace
 
 void FlatIndex::search_masked(int64_t n, const float *x, int64_t k, float *dist, int64_t *labels, bool on_device,
@@ -616,16 +648,15 @@ void FlatIndex::search_masked(int64_t n, const float *x, int64_t k, float *dist,
         dd = ws_dist_.data();
         ld = ws_labels_.data();
     }
-    // Large batches form their candidate scores from bf16 x 3 splits on the bf16 matrix cores (three products at about ten
-    // times the fp32 rate), everything else on the fp32 ones.  Splitting the base costs 10 bytes of traffic per element and
-    // search: about what 140 queries save.  Short bases stay with one launch, and vectors so small that products of their
-    // parts leave the normal range stay with fp32.
+    // Large batches form their candidate scores from bf16 x 3 splits on the bf16 matrix cores, everything else on the fp32
+    // ones (split_pays).  Vectors so small that products of their parts leave the normal range stay with fp32.
     const int dp = (int)round_up(d_, 32);
     int64_t split_rows = std::min<int64_t>(scratch_bytes_ / 2, kSplitBytes) / (6 * dp) / 2048 * 2048;
     split_rows = std::min<int64_t>(split_rows, round_up(ntotal_, 2048));
-    const bool split = !mask_dev && n >= kSplitMinQueries && ntotal_ >= kSplitMinBase && split_rows >= 16384 && bmax_ >= 1e-6f &&
-                       finite_;
-    const int ncand = (int)std::min<int64_t>(std::max<int64_t>(ntotal_, 1), k + (split ? 16 : 8) + k / 8);
+    const int64_t split_cand = k + std::max<int64_t>(16, 8 + k / 8);
+    const bool split = !mask_dev && split_pays(n, ntotal_, dp, k, split_cand, scratch_bytes_) && split_rows >= 16384 &&
+                       bmax_ >= 1e-6f && finite_;
+    const int ncand = (int)std::min<int64_t>(std::max<int64_t>(ntotal_, 1), split ? split_cand : k + 8 + k / 8);
     ws_qn_.resize((size_t)n);
     ws_running_.resize((size_t)n * ncand);
     ws_cand_.resize((size_t)n * ncand);

@@ -1,6 +1,7 @@
 // Streaming brute-force selection: the best `ncand` base rows for every query row, kept as sorted
 // keys, without ever materialising more than a bounded stretch of the score matrix.
 #pragma once
+#include <algorithm>
 #include "coarse.h"
 
 namespace ixa {
@@ -30,6 +31,9 @@ struct StreamSelectWorkspace {
 int stream_select_f32(const float *Q, int64_t nq, const float *B, int64_t nb, int d, const float *qn, const float *bn,
                       int metric, int ncand, unsigned long long *running, StreamSelectWorkspace<float> &ws,
                       int64_t scratch_bytes, hipStream_t s, const uint8_t *mask = nullptr, int64_t mask_stride = 0);
+// Keys per query that the bound-filtered launches of a selection of ncand may admit.
+inline int stream_select_candidates(int ncand) { return pow2_ceil(std::max(1024, 16 * ncand)); }
+
 // The same selection with the scores of fp32 operands formed from their bf16 x 3 splits (approximate: the caller refines and
 // proves).  query: the split queries (rows of 3 dp elements); base: room for rows + kSplitMinRows split base rows, which are
 // written stretch by stretch on the stream.  No mask.

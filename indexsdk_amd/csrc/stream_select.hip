@@ -278,7 +278,7 @@ int stream_select(const Ops &ops, const typename Ops::T *Q, int64_t nq_total, co
     int64_t nb = scratch_bytes / (qb * (int64_t)sizeof(S));
     nb = std::max<int64_t>(128, nb / 128 * 128);
     nb = std::min<int64_t>(nb, round_up(std::max<int64_t>(nb_total, 1), 128));
-    const int cap = pow2_ceil((int)std::max<int64_t>(1024, 16 * (int64_t)ncand));
+    const int cap = stream_select_candidates(ncand);
     const int64_t seed_rows = std::min<int64_t>(nb_total, std::max<int64_t>(Ops::kSeedRows, 16 * (int64_t)ncand));
     // when the whole score matrix of a query block fits the scratch, one materialised pass is the
     // cheapest plan (measured on the IVFPQ coarse stage: 16384 centroids); the filtered plan is for

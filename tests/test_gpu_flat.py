@@ -443,19 +443,19 @@ def test_flat_int8_mask_precision_recipe(ix, oracle):
         assert passes[Im].all()
 
 
-# Batches of 256 queries and more over bases of 32768 rows and more form their candidate scores from bf16 x 3 splits; the
-# results are canonical scores all the same, so they equal the fp32 plan's bit for bit.
+# Batches of more than 256 queries (1024 where rows are short) over bases of 32768 rows and more form their candidate scores from
+# bf16 x 3 splits; the results are canonical scores all the same, so they equal the fp32 plan's bit for bit.
 @pytest.mark.parametrize("metric_name", ["L2", "IP"])
-@pytest.mark.parametrize("d,n,k,scratch", [(64, 32768, 1, 0), (100, 34817, 100, 0), (33, 70001, 20, 24 << 20),
-                                           (200, 50001, 300, 64 << 20)])
-def test_flat_f32_large_batches_equal_small_ones(ix, oracle, metric_name, d, n, k, scratch):
+@pytest.mark.parametrize("d,n,nq,k,scratch", [(64, 32768, 1027, 1, 0), (100, 34817, 259, 100, 0), (33, 70001, 1027, 20, 32 << 20),
+                                              (200, 50001, 259, 300, 64 << 20)])
+def test_flat_f32_large_batches_equal_small_ones(ix, oracle, metric_name, d, n, nq, k, scratch):
     metric = ix.METRIC_L2 if metric_name == "L2" else ix.METRIC_INNER_PRODUCT
     rng = np.random.default_rng(n + d)
     centres = rng.standard_normal((200, d)).astype(np.float32)
     base = (centres[rng.integers(0, 200, n)] + 0.4 * rng.standard_normal((n, d))).astype(np.float32)
     base[n - 3] = base[100]
     base[5] *= 50.0
-    q = (centres[rng.integers(0, 200, 259)] + 0.4 * rng.standard_normal((259, d))).astype(np.float32)
+    q = (centres[rng.integers(0, 200, nq)] + 0.4 * rng.standard_normal((nq, d))).astype(np.float32)
     q[0] = base[100]
     q[3] *= 1e-3
     q[7, 1] = np.nan
@@ -464,7 +464,7 @@ def test_flat_f32_large_batches_equal_small_ones(ix, oracle, metric_name, d, n, 
     index = ix.AscendIndexFlat(d, metric, scratch_bytes=scratch)
     index.add(base)
     D, I = index.search(q, k)
-    for s in range(0, 259, 130):
+    for s in range(0, nq, 130):
         Ds, Is = index.search(q[s:s + 130], k)
         assert np.array_equal(I[s:s + 130], Is)
         assert np.array_equal(D[s:s + 130].view(np.uint32), Ds.view(np.uint32))
@@ -478,7 +478,7 @@ def test_flat_f32_base_with_values_out_of_range_keeps_the_fp32_plan(ix):
     base = rng.standard_normal((n, d)).astype(np.float32)
     base[17, 3] = np.inf
     base[18, 3] = np.nan
-    q = rng.standard_normal((300, d)).astype(np.float32)
+    q = rng.standard_normal((1100, d)).astype(np.float32)
     for metric in (ix.METRIC_L2, ix.METRIC_INNER_PRODUCT):
         index = ix.AscendIndexFlat(d, metric)
         index.add(base)
@@ -510,7 +510,7 @@ def test_flat_few_queries_over_a_long_base(ix, oracle, nq, k, scratch):
 
 
 # Vectors so short that fp32 sums of their squares lose everything (components below 1e-19): the length that the completeness
-# proof multiplies its error bound with is 0, so the proof may not be believed.  300 queries take the bf16 x 3 plan, 100 the fp32
+# proof multiplies its error bound with is 0, so the proof may not be believed.  1100 queries take the bf16 x 3 plan, 100 the fp32
 # one; the base lies so close around one point that its inner products differ by less than either plan's scores err.
 @pytest.mark.parametrize("metric_name", ["L2", "IP"])
 @pytest.mark.parametrize("qscale,bscale", [(1e-24, 1.0), (1e-30, 1.0), (1e-36, 1.0), (1.0, 1e-24), (1e-19, 1e-17)])
@@ -521,10 +521,30 @@ def test_flat_f32_queries_and_bases_of_vanishing_norm(ix, oracle, metric_name, q
     point = rng.standard_normal(d)
     for spread in (1e-5, 1e-6):
         base = (bscale * (point + spread * rng.standard_normal((n, d)))).astype(np.float32)
-        q = (qscale * rng.standard_normal((300, d))).astype(np.float32)
+        q = (qscale * rng.standard_normal((1100, d))).astype(np.float32)
         index = ix.AscendIndexFlat(d, metric)
         index.add(base)
         Dr, Ir = oracle.flat_f32(base, q[:40], k, metric)
-        for nq in (300, 100):
+        for nq in (1100, 100):
             D, I = index.search(q[:nq], k)
             assert np.array_equal(I[:40], Ir) and np.array_equal(D[:40].view(np.uint32), Dr.view(np.uint32)), (nq, spread)
+
+
+def test_flat_f32_a_batch_that_splits_do_not_pay_for(ix):
+    """Splitting the base costs the same for every batch: 256 queries over 65536 rows bring too few products for it and keep
+    the plan of 255 queries (371 us; with splits 455)."""
+    rng = np.random.default_rng(1)
+    d, n, k = 768, 65536, 100
+    base = rng.standard_normal((n, d)).astype(np.float32)
+    q = rng.standard_normal((256, d)).astype(np.float32)
+    index = ix.AscendIndexFlat(d, ix.METRIC_L2)
+    index.add(base)
+
+    def milliseconds(nq):
+        best = 1e9
+        for _ in range(30):
+            index.search(q[:nq], k)
+            best = min(best, index.last_search_stats()["ms_total"])
+        return best
+
+    assert milliseconds(256) < 1.1 * milliseconds(255)
