@@ -595,6 +595,9 @@ void FlatIndex::search_with_masks(int64_t n, const float *x, int64_t k, const ui
 namespace {
 constexpr int64_t kSplitBytes = (int64_t)256 << 20;   // split base rows in flight: what the memory-side cache holds
 
+// candidates per query of the split plan: sixteen spare ones, or as many as the fp32 plan has
+int64_t split_spare(int64_t k) { return k + std::max<int64_t>(16, 8 + k / 8); }
+
 // Whether a search forms its candidate scores from bf16 x 3 splits on the bf16 matrix cores.  Splitting the base costs 10 bytes
 // of traffic per element whatever the number of queries, and the split ring kernel scores 256 queries at a time, so a batch has
 // to bring more than one such tile and enough products.  fp32 / split, us per search, k 100:
@@ -653,10 +656,66 @@ void FlatIndex::search_masked(int64_t n, const float *x, int64_t k, float *dist,
     const int dp = (int)round_up(d_, 32);
     int64_t split_rows = std::min<int64_t>(scratch_bytes_ / 2, kSplitBytes) / (6 * dp) / 2048 * 2048;
     split_rows = std::min<int64_t>(split_rows, round_up(ntotal_, 2048));
-    const int64_t split_cand = k + std::max<int64_t>(16, 8 + k / 8);
-    const bool split = !mask_dev && split_pays(n, ntotal_, dp, k, split_cand, scratch_bytes_) && split_rows >= 16384 &&
-                       bmax_ >= 1e-6f && finite_;
-    const int ncand = (int)std::min<int64_t>(std::max<int64_t>(ntotal_, 1), split ? split_cand : k + 8 + k / 8);
+    bool split = !mask_dev && split_pays(n, ntotal_, dp, k, split_spare(k), scratch_bytes_) && split_rows >= 16384 &&
+                 bmax_ >= 1e-6f && finite_;
+    if (split && split_rest_ > 0) {
+        split_rest_--;
+        split = false;
+    }
+    stats_ = FlatStats();
+    std::vector<int64_t> rows = search_plan(n, xd, k, dd, ld, mask_dev, mask_stride, split ? split_rows : 0);
+    if (split && !rows.empty()) {
+        // The error bound of the splits is two to three times that of fp32 scores: what they leave unproven, the fp32 plan may
+        // prove, at a fraction of what canonical scores of the whole base cost (200k x 128, 512 queries with a common offset
+        // that leaves 449 unproven by splits and 122 by fp32 as well: 10.7 ms with exact rows at once, 3.8 with fp32 before them;
+        // one undefined query of 1024 over 1M x 128: 2.27 ms against 2.07, 64 of them 10.7 against 2.28).
+        // The second plan costs about what a tile of 128 queries does (0.25 of 1.0 ms for 1024 queries, 0.25 of 0.63 for 512), so
+        // unproven queries make a small batch, or an eighth of them any batch, slower than fp32 alone: then the next sixteen batches
+        // that would take splits go without, and the one after them tries again.
+        if ((int64_t)rows.size() * 8 > n || n < 1024) {
+            split_rest_ = 16;
+        }
+        const int64_t m = (int64_t)rows.size();
+        DeviceBuffer<int64_t> rows_dev, lsub((size_t)m * k);
+        DeviceBuffer<float> xsub((size_t)m * d_), dsub((size_t)m * k);
+        rows_dev.upload(rows.data(), rows.size(), stream_);
+        hipLaunchKernelGGL(gather_rows_f32_kernel, dim3(blocks_for(m * d_)), dim3(256), 0, stream_, xd, rows_dev.data(), m, d_,
+                           xsub.data());
+        std::vector<int64_t> left = search_plan(m, xsub.data(), k, dsub.data(), lsub.data(), nullptr, 0, 0);
+        hipLaunchKernelGGL(scatter_result_rows_kernel, dim3(blocks_for(m * k)), dim3(256), 0, stream_, dsub.data(), lsub.data(),
+                           rows_dev.data(), m, (int)k, dd, ld);
+        sync_stream(stream_);   // the temporaries above are freed on leaving this block
+        for (int64_t &r : left) {
+            r = rows[(size_t)r];
+        }
+        rows = std::move(left);
+    }
+    if (!rows.empty()) {
+        IXA_HIP(hipEventRecord(ev_[1], stream_));
+        exact_rows(xd, rows, k, dd, ld, mask_dev, mask_stride);
+        IXA_HIP(hipEventRecord(ev_[2], stream_));
+        sync_stream(stream_);
+        float ms = 0;
+        IXA_HIP(hipEventElapsedTime(&ms, ev_[1], ev_[2]));
+        stats_.ms_select += ms;
+        stats_.exact_reruns = (double)rows.size();
+    }
+    if (!on_device) {
+        ws_dist_.download(dist, (size_t)n * k, stream_);
+        ws_labels_.download(labels, (size_t)n * k, stream_);
+    }
+    stats_.ms_total = stats_.ms_score + stats_.ms_select;
+}
+
+// One plan for n queries in device memory: candidates from approximate scores (split_rows > 0: of bf16 x 3 splits, that many
+// base rows at a time; 0: fp32 matrix cores), their canonical re-evaluation into dd / ld, and the proof.  Returns the queries
+// without proof, ascending; waits for the stream.  Adds its times and launches to stats_.
+std::vector<int64_t> FlatIndex::search_plan(int64_t n, const float *xd, int64_t k, float *dd, int64_t *ld,
+                                            const uint8_t *mask_dev, int64_t mask_stride, int64_t split_rows)
+{
+    const bool split = split_rows > 0;
+    const int dp = (int)round_up(d_, 32);
+    const int ncand = (int)std::min<int64_t>(std::max<int64_t>(ntotal_, 1), split ? split_spare(k) : k + 8 + k / 8);
     ws_qn_.resize((size_t)n);
     ws_running_.resize((size_t)n * ncand);
     ws_cand_.resize((size_t)n * ncand);
@@ -689,8 +748,8 @@ void FlatIndex::search_masked(int64_t n, const float *x, int64_t k, float *dist,
     // approximate scores are fp32 matrix-core sums: they and the canonical left-to-right sums are each
     // within (d + 1) 2^-24 sum |x_i y_i| of the exact dot product (a few units added for second-order
     // terms); an L2 score holds two dot products and three further roundings of numbers no larger
-    // than (|q| + |b|)^2.  Queries without proof are redone exactly.
-    stats_.exact_reruns = 0;
+    // than (|q| + |b|)^2.  Queries without proof are the caller's.
+    std::vector<int32_t> rows32;
     if (ncand < ntotal_) {
         const float u = 5.9604645e-8f;
         // (bf16 x 3: hi + lo misses at most 2^-18 of a value, so the three products kept miss at most 3 x 2^-18 sum |x_i y_i|;
@@ -705,27 +764,21 @@ void FlatIndex::search_masked(int64_t n, const float *x, int64_t k, float *dist,
         int32_t nfail = 0;
         ws_flag_.download(&nfail, 1, stream_);
         if (nfail > 0) {
-            std::vector<int32_t> rows32((size_t)nfail);
+            rows32.resize((size_t)nfail);
             IXA_HIP(hipMemcpyAsync(rows32.data(), ws_flag_.data() + 1, (size_t)nfail * 4, hipMemcpyDeviceToHost, stream_));
             sync_stream(stream_);
-            std::sort(rows32.begin(), rows32.end());
-            exact_rows(xd, std::vector<int64_t>(rows32.begin(), rows32.end()), k, dd, ld, mask_dev, mask_stride);
-            stats_.exact_reruns = nfail;
         }
     }
     IXA_HIP(hipEventRecord(ev_[2], stream_));
     sync_stream(stream_);
-    if (!on_device) {
-        ws_dist_.download(dist, (size_t)n * k, stream_);
-        ws_labels_.download(labels, (size_t)n * k, stream_);
-    }
+    std::sort(rows32.begin(), rows32.end());
     float a = 0, b = 0;
     IXA_HIP(hipEventElapsedTime(&a, ev_[0], ev_[1]));
     IXA_HIP(hipEventElapsedTime(&b, ev_[1], ev_[2]));
-    stats_.ms_score = a;
-    stats_.ms_select = b;
-    stats_.ms_total = a + b;
-    stats_.score_launches = launches;
+    stats_.ms_score += a;
+    stats_.ms_select += b;
+    stats_.score_launches += launches;
+    return std::vector<int64_t>(rows32.begin(), rows32.end());
 }
 
 // ---- int8 ---------------------------------------------------------------------------------------

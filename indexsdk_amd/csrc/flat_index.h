@@ -101,6 +101,8 @@ private:
                     const uint8_t *mask_dev, int64_t mask_stride);
     void search_masked(int64_t n, const float *x, int64_t k, float *dist, int64_t *labels, bool on_device,
                        const uint8_t *mask_dev, int64_t mask_stride);
+    std::vector<int64_t> search_plan(int64_t n, const float *xd, int64_t k, float *dd, int64_t *ld, const uint8_t *mask_dev,
+                                     int64_t mask_stride, int64_t split_rows);
     DeviceBuffer<float> norms_, ws_qn_, ws_dist_;
     DeviceBuffer<uint16_t> ws_qsplit_, ws_bsplit_;   // bf16 x 3 splits of a search's queries and of a stretch of the base
     StreamSelectWorkspace<float> ws_sel_;
@@ -108,6 +110,7 @@ private:
     DeviceBuffer<int64_t> ws_labels_;
     float bmax_ = 0.f;   // largest base vector norm
     bool finite_ = true; // no vector with an infinite or undefined norm was added
+    int split_rest_ = 0; // batches that go without splits, after one that splits left largely unproven
 };
 
 class FlatI8Index : public FlatBase<int8_t> {

@@ -548,3 +548,26 @@ def test_flat_f32_a_batch_that_splits_do_not_pay_for(ix):
         return best
 
     assert milliseconds(256) < 1.1 * milliseconds(255)
+
+
+@pytest.mark.parametrize("offset", [10.0, 14.0, 20.0, 28.0, 60.0])
+def test_flat_f32_queries_that_splits_leave_unproven(ix, offset):
+    """Vectors with a common offset: inner products grow against the gaps between distances, until first the splits' error bound
+    and then that of fp32 scores exceeds the gap behind the k-th.  Whatever the plan of the batch, a query is redone from
+    canonical scores only where fp32 scores do not prove it either, and the answers are those of small batches."""
+    rng = np.random.default_rng(3)
+    d, n, nq, k = 128, 60000, 510, 10
+    centres = rng.standard_normal((256, d))
+    base = (centres[rng.integers(0, 256, n)] + 0.5 * rng.standard_normal((n, d)) + offset).astype(np.float32)
+    q = (centres[rng.integers(0, 256, nq)] + 0.5 * rng.standard_normal((nq, d)) + offset).astype(np.float32)
+    index = ix.AscendIndexFlat(d, ix.METRIC_L2)
+    index.add(base)
+    parts, redone = [], 0
+    for s in range(0, nq, 255):
+        parts.append(index.search(q[s:s + 255], k))
+        redone += index.last_search_stats()["exact_reruns"]
+    for _ in range(20):   # also where batches of this base have stopped taking splits, and when one tries again
+        D, I = index.search(q, k)
+        assert index.last_search_stats()["exact_reruns"] <= redone   # (a few less: the splits' list has more spare candidates)
+        assert np.array_equal(I, np.concatenate([p[1] for p in parts]))
+        assert np.array_equal(D.view(np.uint32), np.concatenate([p[0] for p in parts]).view(np.uint32))
