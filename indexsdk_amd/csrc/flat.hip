@@ -73,20 +73,25 @@ __global__ __launch_bounds__(256) void finish_keys_kernel(const key_t *__restric
     out_labels[i] = ids[key_index(kk)];
 }
 
-// largest value of a non-negative float array: the bit patterns order like the values
+// out[0]: largest number of an array of non-negative floats and NaN (their bit patterns order like the values); out[1]: 1 if a
+// NaN is among them
 __global__ __launch_bounds__(256) void max_bits_kernel(const float *__restrict__ v, int64_t n, uint32_t *__restrict__ out)
 {
-    uint32_t m = 0;
+    uint32_t m = 0, nan = 0;
     for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) {
-        const uint32_t b = __float_as_uint(v[i]);
+        const float x = v[i];
+        const uint32_t b = x == x ? __float_as_uint(x) : 0;
         m = b > m ? b : m;
+        nan |= x != x;
     }
     for (int o = 32; o > 0; o >>= 1) {
         const uint32_t t = __shfl_down(m, o);
         m = t > m ? t : m;
+        nan |= __shfl_down(nan, o);
     }
     if ((threadIdx.x & 63) == 0) {
         atomicMax(out, m);
+        atomicMax(out + 1, nan);
     }
 }
 
@@ -485,17 +490,18 @@ void FlatIndex::add(int64_t n, const float *x, const int64_t *ids, bool on_devic
         IXA_HIP(hipMemcpyAsync(nn.data(), norms_.data(), (size_t)before * 4, hipMemcpyDeviceToDevice, stream_));
     }
     launch_sqnorm_rows(base_.data() + before * d_, n, d_, nn.data() + before, stream_);
-    // largest norm of the base (the error bound of the approximate scores is proportional to it)
-    DeviceBuffer<uint32_t> mx(1);
-    IXA_HIP(hipMemsetAsync(mx.data(), 0, 4, stream_));
+    // largest norm of the base (the error bound of the approximate scores is proportional to it): a vector with an undefined
+    // norm does not hide the others'
+    DeviceBuffer<uint32_t> mx(2);
+    IXA_HIP(hipMemsetAsync(mx.data(), 0, 8, stream_));
     hipLaunchKernelGGL(max_bits_kernel, dim3((unsigned)std::min<int64_t>(1024, (n + 255) / 256)), dim3(256), 0, stream_,
                        nn.data() + before, n, mx.data());
-    uint32_t bits = 0;
-    mx.download(&bits, 1, stream_);
+    uint32_t bits[2] = {0, 0};
+    mx.download(bits, 2, stream_);
     float sq;
-    std::memcpy(&sq, &bits, 4);
+    std::memcpy(&sq, &bits[0], 4);
     bmax_ = std::max(bmax_, std::sqrt(sq));
-    finite_ = finite_ && std::isfinite(sq);
+    finite_ = finite_ && std::isfinite(sq) && bits[1] == 0;
     norms_ = std::move(nn);
 }
 

@@ -571,3 +571,22 @@ def test_flat_f32_queries_that_splits_leave_unproven(ix, offset):
         assert index.last_search_stats()["exact_reruns"] <= redone   # (a few less: the splits' list has more spare candidates)
         assert np.array_equal(I, np.concatenate([p[1] for p in parts]))
         assert np.array_equal(D.view(np.uint32), np.concatenate([p[0] for p in parts]).view(np.uint32))
+
+
+@pytest.mark.parametrize("metric_name", ["L2", "IP"])
+def test_flat_f32_an_undefined_vector_does_not_hide_the_longest(ix, oracle, metric_name):
+    """The margin of the completeness proof grows with the longest vector of the base, also when a vector with an undefined
+    norm was added along with it: a base so close around one point that fp32 scores cannot order it is redone exactly."""
+    metric = ix.METRIC_L2 if metric_name == "L2" else ix.METRIC_INNER_PRODUCT
+    rng = np.random.default_rng(8)
+    d, n, k = 64, 40000, 10
+    short = (1e-3 * rng.standard_normal((100, d))).astype(np.float32)
+    base = (8.0 * rng.standard_normal(d) + 2e-5 * rng.standard_normal((n, d))).astype(np.float32)
+    undefined = np.full((1, d), np.nan, dtype=np.float32)
+    q = (8.0 * rng.standard_normal((40, d))).astype(np.float32)
+    index = ix.AscendIndexFlat(d, metric)
+    index.add(short)
+    index.add(np.concatenate([base, undefined]))
+    D, I = index.search(q, k)
+    Dr, Ir = oracle.flat_f32(np.concatenate([short, base]), q, k, metric)
+    assert np.array_equal(I, Ir) and np.array_equal(D.view(np.uint32), Dr.view(np.uint32))
