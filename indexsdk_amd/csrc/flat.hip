@@ -490,19 +490,39 @@ void FlatIndex::add(int64_t n, const float *x, const int64_t *ids, bool on_devic
         IXA_HIP(hipMemcpyAsync(nn.data(), norms_.data(), (size_t)before * 4, hipMemcpyDeviceToDevice, stream_));
     }
     launch_sqnorm_rows(base_.data() + before * d_, n, d_, nn.data() + before, stream_);
-    // largest norm of the base (the error bound of the approximate scores is proportional to it): a vector with an undefined
-    // norm does not hide the others'
+    measure_norms(nn.data() + before, n);
+    norms_ = std::move(nn);
+}
+
+// Takes n norms into the largest of the base (the error bound of the approximate scores is proportional to it) and into
+// whether all are finite; a vector with an undefined norm does not hide the others'.
+void FlatIndex::measure_norms(const float *norms, int64_t n)
+{
     DeviceBuffer<uint32_t> mx(2);
     IXA_HIP(hipMemsetAsync(mx.data(), 0, 8, stream_));
-    hipLaunchKernelGGL(max_bits_kernel, dim3((unsigned)std::min<int64_t>(1024, (n + 255) / 256)), dim3(256), 0, stream_,
-                       nn.data() + before, n, mx.data());
+    hipLaunchKernelGGL(max_bits_kernel, dim3((unsigned)std::min<int64_t>(1024, (n + 255) / 256)), dim3(256), 0, stream_, norms, n,
+                       mx.data());
     uint32_t bits[2] = {0, 0};
     mx.download(bits, 2, stream_);
     float sq;
     std::memcpy(&sq, &bits[0], 4);
     bmax_ = std::max(bmax_, std::sqrt(sq));
     finite_ = finite_ && std::isfinite(sq) && bits[1] == 0;
-    norms_ = std::move(nn);
+}
+
+// After vectors have left.  While all were finite the largest norm may stay what it was, a bound on what is left; a vector
+// without a finite norm would keep the index on plans that its remaining vectors do not need.
+void FlatIndex::forget_norms()
+{
+    if (ntotal_ > 0 && finite_) {
+        return;
+    }
+    bmax_ = 0.f;
+    finite_ = true;
+    split_rest_ = 0;
+    if (ntotal_ > 0) {
+        measure_norms(norms_.data(), ntotal_);
+    }
 }
 
 // Exact plan of last resort (queries whose candidate list cannot be proven complete): canonical scores
@@ -554,17 +574,22 @@ void FlatIndex::reset()
 {
     FlatBase<float>::reset();
     norms_.release();
+    forget_norms();
 }
 
 int64_t FlatIndex::remove_ids(int64_t n, const int64_t *ids)
 {
     IXA_REQUIRE(n >= 0 && (n == 0 || ids), kErrInvalidParam, "ids can not be nullptr.");
-    return remove_selected(n, ids, 0, 0, reinterpret_cast<uint32_t *>(norms_.data()));
+    const int64_t removed = remove_selected(n, ids, 0, 0, reinterpret_cast<uint32_t *>(norms_.data()));
+    forget_norms();
+    return removed;
 }
 
 int64_t FlatIndex::remove_range(int64_t imin, int64_t imax)
 {
-    return remove_selected(0, nullptr, imin, imax, reinterpret_cast<uint32_t *>(norms_.data()));
+    const int64_t removed = remove_selected(0, nullptr, imin, imax, reinterpret_cast<uint32_t *>(norms_.data()));
+    forget_norms();
+    return removed;
 }
 
 // search (FR/ascendhost/src/index/IndexFlatL2Aicpu.cpp:157-306): the base is walked in row chunks;

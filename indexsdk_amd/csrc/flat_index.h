@@ -101,6 +101,8 @@ private:
                     const uint8_t *mask_dev, int64_t mask_stride);
     void search_masked(int64_t n, const float *x, int64_t k, float *dist, int64_t *labels, bool on_device,
                        const uint8_t *mask_dev, int64_t mask_stride);
+    void measure_norms(const float *norms, int64_t n);
+    void forget_norms();
     std::vector<int64_t> search_plan(int64_t n, const float *xd, int64_t k, float *dd, int64_t *ld, const uint8_t *mask_dev,
                                      int64_t mask_stride, int64_t split_rows);
     DeviceBuffer<float> norms_, ws_qn_, ws_dist_;
@@ -109,7 +111,7 @@ private:
     DeviceBuffer<int32_t> ws_cand_, ws_idx_, ws_flag_;
     DeviceBuffer<int64_t> ws_labels_;
     float bmax_ = 0.f;   // largest base vector norm
-    bool finite_ = true; // no vector with an infinite or undefined norm was added
+    bool finite_ = true; // no vector of the base has an infinite or undefined norm
     int split_rest_ = 0; // batches that go without splits, after one that splits left largely unproven
 };
 

@@ -590,3 +590,34 @@ def test_flat_f32_an_undefined_vector_does_not_hide_the_longest(ix, oracle, metr
     D, I = index.search(q, k)
     Dr, Ir = oracle.flat_f32(np.concatenate([short, base]), q, k, metric)
     assert np.array_equal(I, Ir) and np.array_equal(D.view(np.uint32), Dr.view(np.uint32))
+
+
+@pytest.mark.parametrize("way", ["reset", "remove_ids", "remove_range", "remove all"])
+def test_flat_f32_forgets_a_vector_without_a_finite_norm(ix, way):
+    """An index that has lost an infinite and an undefined vector plans its searches like one that never had them: the same
+    launches, nothing redone exactly (with an infinite margin every query is)."""
+    rng = np.random.default_rng(6)
+    d, n, nq, k = 128, 60000, 512, 10
+    base = rng.standard_normal((n, d)).astype(np.float32)
+    q = rng.standard_normal((nq, d)).astype(np.float32)
+    odd = np.ones((2, d), dtype=np.float32)
+    odd[0, 3], odd[1, 4] = np.inf, np.nan
+    fresh = ix.AscendIndexFlat(d, ix.METRIC_L2, scratch_bytes=48 << 20)
+    fresh.add(base)
+    D, I = fresh.search(q, k)
+    index = ix.AscendIndexFlat(d, ix.METRIC_L2, scratch_bytes=48 << 20)
+    if way in ("reset", "remove all"):
+        index.add(np.concatenate([base[:100], odd]))
+        if way == "reset":
+            index.reset()
+        else:
+            assert index.remove_range(0, 102) == 102
+        index.add(base)
+    else:
+        index.add(np.concatenate([base, odd]))
+        assert (index.remove_ids(np.array([n, n + 1])) if way == "remove_ids" else index.remove_range(n, n + 2)) == 2
+    Dn, In = index.search(q, k)
+    got, want = index.last_search_stats(), fresh.last_search_stats()
+    assert got["exact_reruns"] == want["exact_reruns"] == 0
+    assert got["score_launches"] == want["score_launches"]
+    assert np.array_equal(In % n, I) and np.array_equal(Dn.view(np.uint32), D.view(np.uint32))
