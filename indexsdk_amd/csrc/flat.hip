@@ -625,6 +625,7 @@ void FlatIndex::search_with_masks(int64_t n, const float *x, int64_t k, const ui
 
 namespace {
 constexpr int64_t kSplitBytes = (int64_t)256 << 20;   // split base rows in flight: what the memory-side cache holds
+constexpr int64_t kSplitPage = 16384;                  // queries that are split together
 
 // candidates per query of the split plan: sixteen spare ones, or as many as the fp32 plan has
 int64_t split_spare(int64_t k) { return k + std::max<int64_t>(16, 8 + k / 8); }
@@ -684,9 +685,11 @@ void FlatIndex::search_masked(int64_t n, const float *x, int64_t k, float *dist,
     }
     // Large batches form their candidate scores from bf16 x 3 splits on the bf16 matrix cores, everything else on the fp32
     // ones (split_pays).  Vectors so small that products of their parts leave the normal range stay with fp32.
+    // Half of the scratch holds the split queries (of a page: one block of stream_select) and the split base rows.
     const int dp = (int)round_up(d_, 32);
-    int64_t split_rows = std::min<int64_t>(scratch_bytes_ / 2, kSplitBytes) / (6 * dp) / 2048 * 2048;
-    split_rows = std::min<int64_t>(split_rows, round_up(ntotal_, 2048));
+    const int64_t page = std::min<int64_t>(n, kSplitPage);
+    int64_t split_rows = std::min<int64_t>(scratch_bytes_ / 2 - page * 6 * dp, kSplitBytes) / (6 * dp) - kSplitMinRows;
+    split_rows = std::min<int64_t>(split_rows / 2048 * 2048, round_up(ntotal_, 2048));
     bool split = !mask_dev && split_pays(n, ntotal_, dp, k, split_spare(k), scratch_bytes_) && split_rows >= 16384 &&
                  bmax_ >= 1e-6f && finite_;
     if (split && split_rest_ > 0) {
@@ -694,7 +697,16 @@ void FlatIndex::search_masked(int64_t n, const float *x, int64_t k, float *dist,
         split = false;
     }
     stats_ = FlatStats();
-    std::vector<int64_t> rows = search_plan(n, xd, k, dd, ld, mask_dev, mask_stride, split ? split_rows : 0);
+    std::vector<int64_t> rows;   // without proof
+    if (split) {
+        for (int64_t q0 = 0; q0 < n; q0 += page) {
+            for (int64_t r : search_plan(std::min(page, n - q0), xd + q0 * d_, k, dd + q0 * k, ld + q0 * k, nullptr, 0, split_rows)) {
+                rows.push_back(q0 + r);
+            }
+        }
+    } else {
+        rows = search_plan(n, xd, k, dd, ld, mask_dev, mask_stride, 0);
+    }
     if (split && !rows.empty()) {
         // The error bound of the splits is two to three times that of fp32 scores: what they leave unproven, the fp32 plan may
         // prove, at a fraction of what canonical scores of the whole base cost (200k x 128, 512 queries with a common offset

@@ -621,3 +621,32 @@ def test_flat_f32_forgets_a_vector_without_a_finite_norm(ix, way):
     assert got["exact_reruns"] == want["exact_reruns"] == 0
     assert got["score_launches"] == want["score_launches"]
     assert np.array_equal(In % n, I) and np.array_equal(Dn.view(np.uint32), D.view(np.uint32))
+
+
+def test_flat_f32_split_queries_stay_within_the_scratch(ix, oracle):
+    """Queries are split a page at a time: a larger batch costs its own inputs, results and candidate lists in memory (here 12
+    bytes for each of 17 candidates), not 6 bytes per component for every query; the pages' results stand where the batch's do."""
+    import ctypes
+    rt = ctypes.CDLL("libamdhip64.so")
+
+    def free_bytes():
+        free, total = ctypes.c_size_t(), ctypes.c_size_t()
+        assert rt.hipDeviceSynchronize() == 0 and rt.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+        return free.value
+
+    rng = np.random.default_rng(12)
+    d, n, nq, k = 256, 33000, 70000, 1
+    base = rng.standard_normal((n, d)).astype(np.float32)
+    q = base[rng.integers(0, n, nq)] + np.float32(0.5) * rng.standard_normal((nq, d)).astype(np.float32)
+    q[16383, 0], q[16384, 0], q[nq - 1, 0] = np.nan, np.inf, np.nan     # redone: on both sides of a page's end
+    index = ix.AscendIndexFlat(d, ix.METRIC_L2)
+    index.add(base)
+    D, I = index.search(q[:16384], k)
+    before = free_bytes()
+    D, I = index.search(q, k)
+    assert before - free_bytes() < (nq - 16384) * (4 * d + 17 * 12 + 64) + (32 << 20)
+    for s in (0, 16300, 32700, 65500, nq - 200):
+        Ds, Is = index.search(q[s:s + 200], k)
+        assert np.array_equal(I[s:s + 200], Is) and np.array_equal(D[s:s + 200].view(np.uint32), Ds.view(np.uint32))
+    Dr, Ir = oracle.flat_f32(base, q[16385:16405], k, ix.METRIC_L2)
+    assert np.array_equal(I[16385:16405], Ir) and np.array_equal(D[16385:16405].view(np.uint32), Dr.view(np.uint32))
