@@ -536,7 +536,7 @@ __host__ __device__ inline int select_region_keys(int active, int cap, int extra
     return n;
 }
 
-template <typename S, int active = 4>
+template <typename S, int active = 4, bool LEAN = false>
 __device__ __forceinline__ void select_row_streaming(unsigned char *smem_raw, const S *__restrict__ scores, int64_t ld,
                                                      int64_t nc, int ksel, int cap, int32_t *__restrict__ out_idx,
                                                      int64_t col_base, key_t *__restrict__ running, bool fresh)
@@ -635,7 +635,7 @@ __device__ __forceinline__ void select_row_streaming(unsigned char *smem_raw, co
     if (lane == 0) {
         counts[wave] = scans ? pool.count : 0;
     }
-    const int total = block_merge_pools<4>(pools, cap, counts, run, (run && !fresh) ? ksel : 0, tid);
+    const int total = block_merge_pools<4, LEAN>(pools, cap, counts, run, (run && !fresh) ? ksel : 0, tid);
     for (int i = tid; i < ksel; i += 256) {
         key_t kk = i < total ? pools[i] : kEmptyKey;
         if (out_idx) {
@@ -752,12 +752,14 @@ __device__ __forceinline__ void rank_select_256(key_t *src, int have, int n, key
     __syncthreads();
 }
 
-template <typename S, int G>
+// (PARTS as a template parameter and the fallback's sort with few registers: every spilled register is one more round trip to
+// scratch in the common path.  The branch and the register sort together cost two to three of them.)
+template <typename S, int G, bool PARTS>
 __global__ __launch_bounds__(256, IXA_SELREG_WAVES) void select_rows_reg_kernel(
     const S *__restrict__ scores, int64_t ld, int64_t nc, int ksel, int cap, int32_t *__restrict__ out_idx,
-    int64_t col_base, key_t *running, bool fresh, int64_t part_cols, key_t *parts)
+    int64_t col_base, key_t *__restrict__ running, bool fresh, int64_t part_cols, key_t *__restrict__ parts)
 {
-    if (part_cols) {
+    if constexpr (PARTS) {
         // a stretch of the row per workgroup: its best keys go to parts[row][stretch], select_parts_kernel takes it from there
         const int64_t c0 = (int64_t)blockIdx.y * part_cols;
         scores += c0;
@@ -919,7 +921,7 @@ __global__ __launch_bounds__(256, IXA_SELREG_WAVES) void select_rows_reg_kernel(
         if (ctl[4]) {
             // too many equal scores for the list: the streaming selection redoes the row
             __syncthreads();
-            select_row_streaming<S>(smem_raw, scores, ld, nc, ksel, cap, out_idx, col_base, running, fresh);
+            select_row_streaming<S, 4, true>(smem_raw, scores, ld, nc, ksel, cap, out_idx, col_base, running, fresh);
             return;
         }
         int before = have, total = 0;
@@ -1335,8 +1337,10 @@ static void launch_select_rows_t(const S *scores, int64_t nrows, int64_t ld, int
     if (nparts > 1 || (vec4 && ksel <= kSelRegMaxK && nc >= 2048 && nc <= 6 * kSelRegSeg)) {
         smem = std::max(smem, (size_t)(kSelRegCap + 2 + kSelRegMaxK + 4 * kSelRegStage) * sizeof(key_t) + 4 * 64 * 4 * 4 + 64);
         // groups per lane: ksel / (256 G) stays near 1/3
-        auto kern = ksel <= 96 ? select_rows_reg_kernel<S, 1>
-                               : (ksel <= 192 ? select_rows_reg_kernel<S, 2> : select_rows_reg_kernel<S, 4>);
+        auto kern = nparts > 1 ? (ksel <= 96 ? select_rows_reg_kernel<S, 1, true>
+                                             : (ksel <= 192 ? select_rows_reg_kernel<S, 2, true> : select_rows_reg_kernel<S, 4, true>))
+                               : (ksel <= 96 ? select_rows_reg_kernel<S, 1, false>
+                                             : (ksel <= 192 ? select_rows_reg_kernel<S, 2, false> : select_rows_reg_kernel<S, 4, false>));
         const int64_t part_cols = nparts > 1 ? round_up((nc + nparts - 1) / nparts, kSelRegSeg) : 0;
         const unsigned used = part_cols ? (unsigned)((nc + part_cols - 1) / part_cols) : 1;   // <= nparts
         hipLaunchKernelGGL(kern, dim3((unsigned)nrows, used), dim3(256), smem, s, scores, ld, nc, ksel, cap, part_cols ? nullptr : out_idx,

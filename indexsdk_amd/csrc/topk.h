@@ -433,8 +433,8 @@ struct WavePool {
 // Workgroup epilogue: gathers the W pools (wave w owns pools[w*cap .. w*cap + counts[w])) to the
 // front of the pool region, appends `extra_n` further keys (may be 0), sorts ascending and
 // returns the number of valid keys; afterwards pools[0..result) is sorted.  The region must hold
-// pow2_ceil(W*cap + extra_n) keys.  Called by all threads of the workgroup.
-template <int W>
+// pow2_ceil(W*cap + extra_n) keys.  Called by all threads of the workgroup.  LEAN: by the sort with the fewest registers.
+template <int W, bool LEAN = false>
 __device__ inline int block_merge_pools(key_t *pools, int cap, const int *counts, const key_t *extra, int extra_n,
                                         int tid)
 {
@@ -471,7 +471,18 @@ __device__ inline int block_merge_pools(key_t *pools, int cap, const int *counts
         pools[total + i] = extra[i];
     }
     total += extra_n;
-    block_sort_keys<NT>(pools, total, tid);
+    if constexpr (LEAN) {
+        int n = 2;
+        while (n < total) {
+            n <<= 1;
+        }
+        for (int i = total + tid; i < n; i += NT) {
+            pools[i] = kEmptyKey;
+        }
+        block_bitonic_sort(pools, n, tid, NT);
+    } else {
+        block_sort_keys<NT>(pools, total, tid);
+    }
     return total;
 }
 

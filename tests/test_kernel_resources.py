@@ -1,0 +1,43 @@
+"""Registers of the built kernels (code object metadata of the library): the counts on which the number of resident workgroups
+depends, and spills."""
+import os
+import re
+import struct
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+LIB = os.path.join(ROOT, "indexsdk_amd", "libindexsdk_amd.so")
+READELF = "/opt/rocm/llvm/bin/llvm-readelf"
+
+
+@pytest.fixture(scope="module")
+def kernels(tmp_path_factory):
+    """{mangled name: (registers per lane, spilled registers)} of every gfx950 kernel in the library"""
+    if not (os.path.exists(LIB) and os.path.exists(READELF)):
+        pytest.skip("needs the built library and the ROCm toolchain")
+    data, found, at = open(LIB, "rb").read(), {}, 0
+    path = str(tmp_path_factory.mktemp("co") / "kernels.co")
+    while (at := data.find(b"__CLANG_OFFLOAD_BUNDLE__", at)) >= 0:
+        entry = at + 32
+        for _ in range(struct.unpack_from("<Q", data, at + 24)[0]):
+            offset, size, length = struct.unpack_from("<QQQ", data, entry)
+            target = data[entry + 24:entry + 24 + length].decode()
+            entry += 24 + length
+            if "gfx950" in target and size:
+                with open(path, "wb") as f:
+                    f.write(data[at + offset:at + offset + size])
+                notes = subprocess.run([READELF, "--notes", path], capture_output=True, text=True, check=True).stdout
+                for block in notes.split("- .agpr_count")[1:]:
+                    def field(key):
+                        return re.search(rf"\.{key}:\s+(\S+)", block).group(1)
+                    found[field("name")] = int(field("vgpr_count")), int(field("vgpr_spill_count"))
+        at = entry
+    assert len(found) > 100
+    return found
+
+
+def test_register_selection(kernels):
+    select = [v for n, v in kernels.items() if re.search("select_rows_reg_kernelI[fi]Li[124]ELb0EE", n)]
+    assert len(select) == 6 and all(spilled <= 8 for _, spilled in select)
