@@ -117,10 +117,13 @@ __device__ __forceinline__ uint32_t byte_times_pow2(uint32_t w, int j)
 // Short codes with the shared pool leave LDS room for four workgroups per CU and are bound by latency, not by registers'
 // worth of prefetch: those kernels are held to 64 registers (8 waves per SIMD).  Left alone the allocator takes a few more,
 // which halves the resident workgroups (64 queries x 128 lists of 16000 four-byte codes: 512 of 1024 workgroups at a time).
+// The same holds for private pools of short rows: at M 4 and 8 the allocator left alone took 65 with the sort of the epilogue
+// inlined, one more than four workgroups of eight wavefronts have.
 template <int MT, typename LutT, int LAYOUT, int W, bool SHARED>
 __global__ __launch_bounds__(W * 64, (LAYOUT == 1 && sizeof(LutT) == 2 && !SHARED) ? 4
                                      : (SHARED && W == 8 && MT > 0 && MT <= 8)    ? 8
-                                                                                   : 1) void ivfpq_scan_kernel(
+                                     : (!SHARED && LAYOUT == 0 && MT > 0 && MT <= 32) ? 8
+                                                                                      : 1) void ivfpq_scan_kernel(
     ScanParams p)
 {
     extern __shared__ __align__(16) unsigned char smem_raw[];
@@ -724,7 +727,8 @@ constexpr int kMergeSelectCap = 4096;
 constexpr int kMergeSelectThreads = 1024;
 constexpr int kMergeCountMax = 384;   // survivors ranked by counting; more are sorted
 
-__global__ __launch_bounds__(kMergeSelectThreads) void ivfpq_merge_kernel(
+// (held to 64 registers: two workgroups per CU; it takes 65 when left alone)
+__global__ __launch_bounds__(kMergeSelectThreads, 8) void ivfpq_merge_kernel(
     const key_t *__restrict__ partial, int nsplit, int k, int metric, const int64_t *__restrict__ ids,
     const int32_t *__restrict__ order, float *__restrict__ out_dist, int64_t *__restrict__ out_labels)
 {

@@ -10,6 +10,7 @@ import pytest
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 LIB = os.path.join(ROOT, "indexsdk_amd", "libindexsdk_amd.so")
 READELF = "/opt/rocm/llvm/bin/llvm-readelf"
+SCAN = re.compile(r"ivfpq_scan_kernelILi(\d+)E(f|6__half)Li(\d)ELi(\d+)ELb([01])EE")
 
 
 @pytest.fixture(scope="module")
@@ -41,3 +42,20 @@ def kernels(tmp_path_factory):
 def test_register_selection(kernels):
     select = [v for n, v in kernels.items() if re.search("select_rows_reg_kernelI[fi]Li[124]ELb0EE", n)]
     assert len(select) == 6 and all(spilled <= 8 for _, spilled in select)
+
+
+def test_scan_kernels_of_short_codes_leave_room_for_four_workgroups(kernels):
+    """Row layout, eight wavefronts: 64 registers let four workgroups share a CU (private pools up to M 32, the shared pool up
+    to M 8)."""
+    seen = 0
+    for name, (registers, spilled) in kernels.items():
+        m = SCAN.search(name)
+        if m and m.group(3) == "0" and m.group(4) == "8" and 0 < int(m.group(1)) <= (8 if m.group(5) == "1" else 32):
+            assert registers <= 64 and spilled == 0, (name, registers, spilled)
+            seen += 1
+    assert seen >= 16
+
+
+def test_merge_of_slices(kernels):
+    merge = [v for n, v in kernels.items() if "ivfpq_merge_kernel" in n]
+    assert merge and all(registers <= 64 and spilled == 0 for registers, spilled in merge)      # two workgroups per CU
