@@ -326,7 +326,12 @@ __global__ __launch_bounds__(W * 64, (LAYOUT == 1 && sizeof(LutT) == 2 && !SHARE
     // ---- stages 3 + 4: the probed lists form one sequence of 64-code groups; wavefront w takes
     // groups w, w + W, ... of that sequence, so the waves stay balanced whatever the list lengths.
     WavePool<float> pool;
-    BlockPool<W> bpool;
+    // With sixteen wavefronts the prune stands in every step of the loop, between codes in flight.  At M 96 that spills, and the
+    // sort of the prune decides how much: with the register network 23 registers (rot32, halves; 17 without), 199 (row; 102),
+    // but 62 with the fp32 rot32 table (66 without).  2000 queries over 2M x 96 bytes, 64 lists of 2048, k 300: halves 2.95
+    // against 2.34 ms, fp32 7.22 against 8.03.
+    constexpr bool kLeanPrune = W == 16 && (LAYOUT == 0 || (LAYOUT == 1 && sizeof(LutT) == 2));
+    BlockPool<W, kLeanPrune> bpool;
     if constexpr (SHARED) {
         bpool.init(pools, p.cap, p.k, reinterpret_cast<int *>(smem_raw + p.off_hist),
                    reinterpret_cast<BlockPoolCtl *>(counts + W), tid);

@@ -510,7 +510,8 @@ struct BlockPoolCtl {
     key_t bound_key;   // kEmptyKey, or the k-th smallest key once ties at the k-th score overflowed the pool
 };
 
-template <int W>
+// LEAN: the sort of a pool that one bucket fills is the one with the fewest registers.
+template <int W, bool LEAN = false>
 struct BlockPool {
     static constexpr int NT = W * kWave;
     static constexpr int kMaxPerThread = W >= 16 ? 4 : 8;   // cap <= kMaxPerThread * NT
@@ -724,7 +725,14 @@ struct BlockPool {
         float top = ScoreOps<float>::bucket_top((P << SH) | ((1u << SH) - 1u));
         if (kept > cap - NT) {
             // one bucket holds almost everything: exact selection by sorting
-            block_sort_keys<NT>((key_t *)buf, kept, tid);
+            if constexpr (LEAN) {
+                for (int i = kept + tid; i < cap; i += NT) {
+                    buf[i] = kEmptyKey;
+                }
+                block_bitonic_sort((key_t *)buf, cap, tid, NT);
+            } else {
+                block_sort_keys<NT>((key_t *)buf, kept, tid);
+            }
             kept = k;
             top = key_score(buf[k - 1]);
             if (tid == 0) {

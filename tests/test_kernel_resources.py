@@ -59,3 +59,12 @@ def test_scan_kernels_of_short_codes_leave_room_for_four_workgroups(kernels):
 def test_merge_of_slices(kernels):
     merge = [v for n, v in kernels.items() if "ivfpq_merge_kernel" in n]
     assert merge and all(registers <= 64 and spilled == 0 for registers, spilled in merge)      # two workgroups per CU
+
+
+def test_scan_kernels_of_sixteen_wavefronts_spill_only_at_96_bytes(kernels):
+    limit = {("f", "0"): 194, ("6__half", "0"): 194, ("f", "1"): 66, ("6__half", "1"): 17}
+    for name, (registers, spilled) in kernels.items():
+        m = SCAN.search(name)
+        if m and m.group(4) == "16":
+            allowed = limit[m.group(2), m.group(3)] if m.group(1) == "96" else 0
+            assert registers <= 128 and spilled <= allowed, (name, registers, spilled)
