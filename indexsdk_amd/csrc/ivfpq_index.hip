@@ -124,7 +124,9 @@ void parallel_copy(std::initializer_list<CopyJob> jobs)
         w.join();
     }
 }
-constexpr int64_t kPqTrainBytes = (int64_t)4 << 30;   // sub-vectors, codes and member lists of the sub-quantizers trained together
+// Least room for the sub-vectors, codes and member lists of the sub-quantizers that are trained together; the scratch budget
+// where that is larger.
+constexpr int64_t kPqTrainBytes = (int64_t)64 << 20;
 constexpr int64_t kCoarseExactMaxMacs = (int64_t)1 << 27;   // queries x centroids x dims up to which a search selects its lists exactly
 
 // ---- arena kernels ------------------------------------------------------------------------------
@@ -1949,9 +1951,9 @@ void IvfpqIndex::kmeans_pq(const float *sample_dev, int64_t ns, const std::vecto
     // From here on an iteration is queued without a wait: codes of the sample (sub-quantizer-major, as the update reads
     // them), the members of every codeword in sample order, their means (float64 sums in that order), empty codewords
     // re-seeded, all in device memory.  The sub-quantizers do not depend on each other: they are trained in groups whose
-    // sub-vectors, codes and member lists stay within kPqTrainBytes.
+    // sub-vectors, codes and member lists stay within the scratch budget.
     const int64_t per_m = ns * (4 * dsub_ + 1 + 4);
-    const int group = (int)std::max<int64_t>(1, std::min<int64_t>(M_, kPqTrainBytes / per_m));
+    const int group = (int)std::max<int64_t>(1, std::min<int64_t>(M_, std::max(cfg_.scratch_bytes, kPqTrainBytes) / per_m));
     DeviceBuffer<float> subs((size_t)ns * group * dsub_);
     DeviceBuffer<uint8_t> codes((size_t)ns * group);
     DeviceBuffer<unsigned long long> cnt((size_t)group * 256);

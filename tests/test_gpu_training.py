@@ -68,3 +68,19 @@ def test_assignment_at_the_edges_of_the_row_widths(nlist):
     gpu = ix.AscendIndexIVFPQ(d, ix.METRIC_L2, nlist, 8, 8)
     gpu.set_trained(cent, orc.train_pq(x, 8, niter=1, seed=1))
     assert np.array_equal(gpu.assign(x), orc.assign(x, cent))
+
+
+# dsub 16 and 72 (the two ways sub-vectors are gathered); with the smallest scratch groups of 3, 3 and 2 of 8 sub-quantizers, and of
+# one of 3
+@pytest.mark.parametrize("d,M,n", [(128, 8, 300_000), (216, 3, 120_000)])
+def test_sub_quantizers_trained_in_groups_equal_those_trained_together(d, M, n):
+    ix = _ix()
+    rng = np.random.default_rng(d)
+    x = rng.standard_normal((n, d), dtype=np.float32)
+    books = []
+    for scratch in (1 << 30, 1 << 20):
+        cfg = ix.AscendIndexIVFPQConfig(niter=1, pq_niter=2, train_samples_per_list=1 << 20, scratch_bytes=scratch)
+        gpu = ix.AscendIndexIVFPQ(d, ix.METRIC_L2, 4, M, 8, cfg)
+        gpu.train(x)
+        books.append(gpu.get_trained()[1])
+    assert np.array_equal(books[0].view(np.uint32), books[1].view(np.uint32))
