@@ -166,6 +166,28 @@ def test_flat_searches_side_by_side_equal_searches_alone(ix, oracle, kind):
     run_threads(4, lambda t: [np.testing.assert_array_equal(search(queries[(t + r) % 4], k)[1], want[(t + r) % 4][1]) for r in range(10)])
 
 
+def test_flat_large_batches_side_by_side_equal_searches_alone(ix):
+    """Batches whose candidate scores come from bf16 x 3 splits: every lane has split buffers of its own, for its queries and
+    for the stretch of the base in flight (a scratch that holds a sixth of the base: the stretches change under the others)."""
+    rng = np.random.default_rng(15)
+    d, n, k = 128, 200_000, 10
+    base = rng.standard_normal((n, d)).astype(np.float32)
+    index = ix.AscendIndexFlat(d, ix.METRIC_L2, scratch_bytes=64 << 20)
+    index.add(base)
+    queries = [(base[a:a + m] + np.float32(0.1)).astype(np.float32) for a, m in ((0, 600), (70_000, 1100), (150_000, 300), (5, 40))]
+    queries[1][17, 3] = np.nan      # redone with fp32 candidates, beside the others
+    want = [index.search(qq, k) for qq in queries]
+
+    def body(t):
+        for r in range(12):
+            j = (t + r) % len(queries)
+            D, I = index.search(queries[j], k)
+            assert np.array_equal(I, want[j][1]) and np.array_equal(D.view(np.uint32), want[j][0].view(np.uint32)), (t, r, j)
+
+    run_threads(4, body)
+    assert np.array_equal(want[0][1][:, 0], np.arange(600)) and (want[1][1][17] == -1).all()
+
+
 @pytest.fixture(scope="module")
 def ix():
     import indexsdk_amd

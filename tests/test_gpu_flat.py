@@ -650,3 +650,37 @@ def test_flat_f32_split_queries_stay_within_the_scratch(ix, oracle):
         assert np.array_equal(I[s:s + 200], Is) and np.array_equal(D[s:s + 200].view(np.uint32), Ds.view(np.uint32))
     Dr, Ir = oracle.flat_f32(base, q[16385:16405], k, ix.METRIC_L2)
     assert np.array_equal(I[16385:16405], Ir) and np.array_equal(D[16385:16405].view(np.uint32), Dr.view(np.uint32))
+
+
+# Masked searches write every chunk of the score matrix: with 20 MB of scratch chunks of 40960, 40960 and 18083 columns.  The second is
+# cut into stretches whose keys are ordered together with those the first has left.
+@pytest.mark.parametrize("kind", ["int8", "float"])
+@pytest.mark.parametrize("nq,k", [(1, 1), (5, 300), (64, 100)])
+def test_flat_masked_few_queries_over_several_long_chunks(ix, kind, nq, k):
+    rng = np.random.default_rng(nq)
+    n, d = 100_003, 64
+    base = rng.integers(-20, 21, size=(n, d), dtype=np.int8)
+    base[40_700:41_300] = base[7]                                       # equal scores on both sides of a chunk's end
+    q = rng.integers(-20, 21, size=(nq, d), dtype=np.int8)
+    q[0] = base[7]
+    passes = rng.random((nq, n)) < 0.5
+    if nq > 2:
+        passes[1] = False
+        passes[1, [3, 40_959, 40_960, 50_000, n - 1]] = True            # fewer vectors take part than are asked for
+        passes[2, :81_920] = False                                      # none of the first two chunks
+    mask = np.packbits(passes, axis=1, bitorder="little")
+    if kind == "int8":
+        index = ix.AscendIndexInt8Flat(d, ix.METRIC_L2, scratch_bytes=20 << 20)
+        index.add(base)
+        D, I = index.search_with_masks_int32(q, k, mask)
+    else:
+        index = ix.AscendIndexFlat(d, ix.METRIC_L2, scratch_bytes=20 << 20)
+        index.add(base.astype(np.float32))
+        D, I = index.search_with_masks(q.astype(np.float32), k, mask)
+    b = base.astype(np.float32)   # (sums of products up to 64 * 400: exact)
+    dist = (b * b).sum(1) - 2 * (q.astype(np.float32) @ b.T) + (q.astype(np.float32) ** 2).sum(1, keepdims=True)
+    dist[~passes] = np.inf
+    want = np.argsort(dist, axis=1, kind="stable")[:, :k]
+    best = np.take_along_axis(dist, want, 1)
+    assert np.array_equal(I, np.where(np.isinf(best), -1, want))
+    assert np.array_equal(D[np.isfinite(best)].astype(np.float32), best[np.isfinite(best)])

@@ -973,17 +973,19 @@ def test_host_batch_beyond_the_staging_buffer_equals_its_pieces(ix, oracle):
     assert_topk_parity(oracle, ref, q[:500], D[:500], I[:500], Dr, Ir, TOL_FP32)
 
 
+@pytest.mark.parametrize("lut_fp16", [0, 1])
 @pytest.mark.parametrize("M", [12, 20, 24, 40, 56, 36, 9, 3, 7, 33])
-def test_sub_quantizer_counts_off_the_powers_of_two(ix, oracle, M):
+def test_sub_quantizer_counts_off_the_powers_of_two(ix, oracle, M, lut_fp16):
     """Compile-time M (multiples of 4 up to 24, of 8 up to 64), run-time M by words (36) and by bytes (3 and 7 together, 9 and
-    33 one by one); a batch that is split over workgroups and one that is not, private pools and the shared pool."""
-    gpu, ref, x, q, ids = build_pair(ix, oracle, 300 + M, 9001, 70, 4 * M, 24, M, ix.METRIC_L2)
+    33 in eights and a remainder), either table; a batch that is split over workgroups and one that is not, private pools and
+    the shared pool."""
+    gpu, ref, x, q, ids = build_pair(ix, oracle, 300 + M, 9001, 70, 4 * M, 24, M, ix.METRIC_L2, lut_fp16=lut_fp16)
     gpu.setNumProbes(5)
     for k in (10, 300):
         for nq in (70, 1):
             D, I = gpu.search(q[:nq], k)
-            Dr, Ir = ref.search(q[:nq], k, 5)
-            assert_topk_parity(oracle, ref, q[:nq], D, I, Dr, Ir, TOL_FP32)
+            Dr, Ir = ref.search(q[:nq], k, 5, lut_fp16=bool(lut_fp16))
+            assert_topk_parity(oracle, ref, q[:nq], D, I, Dr, Ir, TOL_FP16 if lut_fp16 else TOL_FP32)
 
 
 @pytest.mark.parametrize("k", [1, 2, 255, 256, 257, 511, 512, 513, 1023, 1024, 1025, 2047, 2048])
