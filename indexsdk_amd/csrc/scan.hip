@@ -1349,8 +1349,9 @@ static size_t plan_scan_by_residency(ScanParams &p)
         }
         ScanParams q = p;
         const size_t smem = plan_with_waves(q, alt.waves, alt.shared);
-        // a shared-pool workgroup keeps its CU to itself: those kernels need more than the 64
-        // registers per lane that a second resident workgroup would leave them
+        // a shared-pool workgroup counts once per CU.  That is so with sixteen wavefronts (more than the 64 registers that
+        // would leave room for a second); with eight the registers admit two workgroups (M < 56, up to 128 registers) or four
+        // (M <= 8, held to 64), which this count leaves out: k 897 - 1920 at M <= 8, for one, is given to sixteen wavefronts.
         const int rw = smem <= 160 * 1024 ? (alt.shared ? alt.waves : resident_waves(smem, alt.waves)) : 0;
         if (rw > best_waves) {
             best = q;

@@ -127,10 +127,11 @@ struct F32Ops {
     }
 };
 
-// fp32 operands whose products run on the bf16 matrix cores: queries split once per call ([hi | hi | lo], by the caller),
+// fp32 operands whose products run on the bf16 matrix cores: queries split once ([hi | hi | lo], by the caller),
 // base rows split ([hi | lo | hi]) stretch by stretch into a buffer small enough to stay in the memory-side cache until the
-// score launch reads it.  Three bf16 products per element run about 2.5 x as fast as one fp32 product; splitting a row costs
-// 10 bytes of traffic per element, whatever the number of queries, so large batches take this path (flat.hip has the line).
+// score launch reads it.  1M x 128, 1000 queries: the score launches take 1.34 ms (0.57 PFLOP/s of bf16 products, 0.71 in the
+// longest) where the fp32 ones took 3.1; splitting the base takes 0.28 ms whatever the number of queries, so large batches take
+// this path (flat.hip has the line).
 //
 // At this rate an admitted key (an atomic each) costs as much as thousands of scores, so the bound is tightened early, as for
 // int8: a longer seed and chunks of twice what has been seen.  1M x 128, 1000 queries, k 100: fp32 scores 3.19 ms; splits with

@@ -244,8 +244,8 @@ __device__ inline void block_rank_sort(key_t *buf, int n, int tid)
     __syncthreads();
 }
 
-// Sorts buf[0 .. n) ascending; buf has room for the next power of two (at least two keys).  All NT threads of the workgroup
-// call it, barriers inside.  Up to 256 keys are ranked by counting; beyond, the squared number of comparisons costs more
+// Sorts buf[0 .. n) ascending.  buf has room for n + 1 keys, and where n > 256 for max(512, NT) or the next power of two, the
+// larger: that far it is filled up.  All NT threads of the workgroup call it, barriers inside.  Up to 256 keys are ranked by counting; beyond, the squared number of comparisons costs more
 // issue slots than the network's stages (400 keys at the end of every query of 10M x 32 bytes, nprobe 64: +1.5 %).
 template <int NT>
 __device__ inline void block_sort_keys(key_t *buf, int n, int tid)
