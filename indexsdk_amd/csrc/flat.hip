@@ -638,8 +638,9 @@ int64_t split_spare(int64_t k) { return k + std::max<int64_t>(16, 8 + k / 8); }
 //   queries over 1M rows and more would gain as well, 160 over 1M x 128 1587 / 1060; they have the fp32 plan all the same.)
 //   320 queries: 32768 x 128 171 / 166, 65536 x 128 238 / 223, 200k x 128 631 / 577, 400k x 128 1073 / 768, 32768 x 768 362 / 306;
 //   d 64, where a tile's products are few: 512 queries 32768 152 / 159, 100k 325 / 341, 200k 542 / 541, 400k 908 / 659; 1024
-//   queries 32768 200 / 198, 100k 487 / 469, 200k 805 / 580; and none with very many keys (300k, 1024 queries, k 500 1902 / 1819,
-//   k 1000 3760 / 4206).
+//   queries 32768 200 / 198, 100k 487 / 469, 200k 805 / 580.
+//   Very many keys, k 1000: d 64, 300k, 1024 queries 3760 / 4206 (k 500: 1902 / 1819); d 128 the same 4087 / 4360, but 300 queries
+//   2049 / 1908 and over 1M 8840 / 8643; d 256 4832 / 4758.
 // Half of the scratch goes to the split base, with three consequences:
 //   Where the fp32 plan could still keep the whole score matrix and the split plan no longer can, the bound-filtered launches
 //   that take its place win with few keys (512 queries, 400k x 128, k 10: 1075 / 548, k 100: 1100 / 769) and lose with many
@@ -653,7 +654,8 @@ bool split_pays(int64_t nq, int64_t nb, int dp, int64_t k, int64_t ncand, int64_
 {
     const int64_t half = scratch_bytes - scratch_bytes / 2, mb = (int64_t)1 << 20;
     const int64_t matrix = round_up(nq, 128) * round_up(nb, 128) * (int64_t)sizeof(float);
-    if (scratch_bytes < 30 * mb || (dp < 128 && k > 512) || (k > 128 && matrix <= scratch_bytes && matrix > half)) {
+    const bool many_keys = k > 512 && (dp < 128 || (dp < 256 && nq > 512 && nb < 1000000));
+    if (scratch_bytes < 30 * mb || many_keys || (k > 128 && matrix <= scratch_bytes && matrix > half)) {
         return false;
     }
     const int64_t candidates = std::min<int64_t>(round_up(nq, 128), 16384) * stream_select_candidates((int)ncand) * 8;
