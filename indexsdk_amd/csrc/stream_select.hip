@@ -129,7 +129,7 @@ struct F32Ops {
 
 // fp32 operands whose products run on the bf16 matrix cores: queries split once ([hi | hi | lo], by the caller),
 // base rows split ([hi | lo | hi]) stretch by stretch into a buffer small enough to stay in the memory-side cache until the
-// score launch reads it.  1M x 128, 1000 queries: the score launches take 1.34 ms (0.57 PFLOP/s of bf16 products, 0.71 in the
+// score launch reads it.  1M x 128, 1000 queries: the score launches take 1.33 ms (0.58 PFLOP/s of bf16 products, 0.71 in the
 // longest) where the fp32 ones took 3.1; splitting the base takes 0.28 ms whatever the number of queries, so large batches take
 // this path (flat.hip has the line).
 //
