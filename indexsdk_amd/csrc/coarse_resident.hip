@@ -256,19 +256,6 @@ __global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(2, 
     }
 }
 
-int device_cus()
-{
-    static std::atomic<int> known{0};
-    int cus = known.load(std::memory_order_relaxed);
-    if (cus == 0) {
-        int dev = 0;
-        IXA_HIP(hipGetDevice(&dev));
-        IXA_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-        known.store(cus, std::memory_order_relaxed);
-    }
-    return cus;
-}
-
 // rounds of work items x (loading the query tile + walking a segment), in units of one block-row of matrix work;
 // load = what a query tile costs to load, in tiles' time (measured inside the kernel: 1.6 where a tile has the record
 // epilogue behind it, about 3 where it has the minima's)

@@ -9,6 +9,7 @@
 #include "coarse.h"
 #include "flat_i8.h"
 #include "flat_index.h"
+#include "flat_resident.h"
 #include "stream_select.h"
 #include "topk.h"
 
@@ -485,7 +486,7 @@ void FlatIndex::add(int64_t n, const float *x, const int64_t *ids, bool on_devic
     const int64_t before = ntotal_;
     FlatBase<float>::add(n, x, ids, on_device);
     // norms of the whole base are kept in one array; recompute the tail (left-to-right fp32)
-    DeviceBuffer<float> nn((size_t)capacity_);
+    DeviceBuffer<float> nn((size_t)round_up(capacity_, 4));
     if (before > 0) {
         IXA_HIP(hipMemcpyAsync(nn.data(), norms_.data(), (size_t)before * 4, hipMemcpyDeviceToDevice, stream_));
     }
@@ -627,10 +628,7 @@ namespace {
 constexpr int64_t kSplitBytes = (int64_t)256 << 20;   // split base rows in flight: what the memory-side cache holds
 constexpr int64_t kSplitPage = 16384;                  // queries that are split together
 
-// candidates per query of the split plan: sixteen spare ones, or as many as the fp32 plan has
-int64_t split_spare(int64_t k) { return k + std::max<int64_t>(16, 8 + k / 8); }
-
-// Whether a search forms its candidate scores from bf16 x 3 splits on the bf16 matrix cores.  Splitting the base costs 10 bytes
+// Whether a search that resident_pays leaves splits its operands before the scores.  Splitting the base costs 10 bytes
 // of traffic per element whatever the number of queries, and the split ring kernel scores 256 queries at a time, so a batch has
 // to bring more than one such tile and enough products.  fp32 / split, us per search, k 100:
 //   256 queries: 200k x 64 370 / 423, 200k x 128 440 / 482, 400k x 128 769 / 818, 65536 x 768 371 / 455; from 1M on 1627 / 1101
@@ -664,6 +662,34 @@ bool split_pays(int64_t nq, int64_t nb, int dp, int64_t k, int64_t ncand, int64_
     }
     return nq >= 256 && nb >= (nq == 256 ? 1000000 : (dp >= 128 || nq >= 1024 ? 32768 : 250000));
 }
+
+// Candidates per query of the two plans that score with splits.  A query is proven when its list reaches past its k-th score by
+// the error bound, which for L2 grows with the dimension against the spread of the scores: on mixtures of 16 and 1024 components
+// with deviations of 0.2 to 1, a million vectors and k 10 / 100 / 300, the resident plan's lists have to hold up to 4 / 15 / 35
+// vectors more at 128 dimensions, 10 / 32 / 77 at 256, 11 / 55 / 117 at 384 and 40 / 174 / 380 at 768 (from a deviation of 0.25
+// on 23 / 75 / 180), the split plan's about half as many; inner products of unit vectors need up to 23 at 768.  384 keys are
+// what the register selection takes.
+int64_t split_candidates(int64_t k, int dp, int metric, bool resident)
+{
+    const int64_t least = std::max<int64_t>(16, 8 + k / 8);
+    int64_t spare = least;
+    if (metric == kMetricL2) {
+        spare = resident ? std::max<int64_t>({16 + dp / 24, k * dp / 768, least}) : std::max(least, k * dp / 1536);
+    }
+    return std::max<int64_t>(k + least, std::min<int64_t>(k + spare, 384));
+}
+
+// Whether the kernel that splits base rows in registers forms the scores.  It keeps 256 queries per tile up to 128 dimensions,
+// 128 up to 256, 64 up to 512, 32 above, and reads the base once per tile, so at large dimensions many queries are better served by
+// the split plan (or by fp32 products, for 257 to 384 queries).  1M x 384, k 100 and 10: 100 queries 2482 / 730 us (the other plan /
+// this one), 700 3186 / 2530, 1024 3338 / 2980, 2000 5424 / 5653; 800k x 512: 60 queries 1897 / 601, 700 3245 / 2656, 1000 4020 /
+// 3364; 700k x 768: 4 queries 2190 / 620, 300 5290 / 3033, 384 5293 / 3518, 700 5296 / 6933.  Elsewhere it wins with every number
+// of queries and rows (128 dimensions: 4096 queries over 10000 rows 229 / 174, 10 over 10000 120 / 89, one over 1M 651 / 208, 1000
+// over 1M 1763 / 964; 256: 100 over 1M 1993 / 528, 1000 2744 / 1524).
+bool resident_pays(int64_t nq, int64_t nb, int d)
+{
+    return nb >= 2048 && nq <= (d <= 256 ? INT64_MAX : (d <= 512 ? 1024 : 384));
+}
 }  // namespace
 
 void FlatIndex::search_masked(int64_t n, const float *x, int64_t k, float *dist, int64_t *labels, bool on_device,
@@ -685,31 +711,38 @@ void FlatIndex::search_masked(int64_t n, const float *x, int64_t k, float *dist,
         dd = ws_dist_.data();
         ld = ws_labels_.data();
     }
-    // Large batches form their candidate scores from bf16 x 3 splits on the bf16 matrix cores, everything else on the fp32
-    // ones (split_pays).  Vectors so small that products of their parts leave the normal range stay with fp32.
-    // Half of the scratch holds the split queries (of a page: one block of stream_select) and the split base rows.
+    // Candidate scores come from bf16 x 3 splits on the bf16 matrix cores, formed in the score kernel (resident_pays) or before it
+    // (split_pays), or from fp32 products.  Vectors so small that products of their parts leave the normal range stay with fp32.
+    // Where splits are formed beforehand, half of the scratch holds those of the queries (of a page: one block of
+    // stream_select) and of the base rows.
     const int dp = (int)round_up(d_, 32);
     const int64_t page = std::min<int64_t>(n, kSplitPage);
     int64_t split_rows = std::min<int64_t>(scratch_bytes_ / 2 - page * 6 * dp, kSplitBytes) / (6 * dp) - kSplitMinRows;
     split_rows = std::min<int64_t>(split_rows / 2048 * 2048, round_up(ntotal_, 2048));
-    bool split = !mask_dev && split_pays(n, ntotal_, dp, k, split_spare(k), scratch_bytes_) && split_rows >= 16384 &&
-                 bmax_ >= 1e-6f && finite_;
-    if (split && split_rest_ > 0) {
+    const bool can_split = !mask_dev && bmax_ >= 1e-6f && finite_;
+    Candidates from = Candidates::kFp32;
+    if (can_split && resident_f32_serves(d_) && reinterpret_cast<uintptr_t>(xd) % 16 == 0 && resident_pays(n, ntotal_, d_)) {
+        from = Candidates::kResident;
+    } else if (can_split && split_pays(n, ntotal_, dp, k, split_candidates(k, dp, metric_, false), scratch_bytes_) && split_rows >= 16384) {
+        from = Candidates::kSplit;
+    }
+    if (from != Candidates::kFp32 && split_rest_ > 0) {
         split_rest_--;
-        split = false;
+        from = Candidates::kFp32;
     }
     stats_ = FlatStats();
     std::vector<int64_t> rows;   // without proof
-    if (split) {
+    if (from == Candidates::kSplit) {
         for (int64_t q0 = 0; q0 < n; q0 += page) {
-            for (int64_t r : search_plan(std::min(page, n - q0), xd + q0 * d_, k, dd + q0 * k, ld + q0 * k, nullptr, 0, split_rows)) {
+            for (int64_t r : search_plan(std::min(page, n - q0), xd + q0 * d_, k, dd + q0 * k, ld + q0 * k, nullptr, 0, from,
+                                        split_rows)) {
                 rows.push_back(q0 + r);
             }
         }
     } else {
-        rows = search_plan(n, xd, k, dd, ld, mask_dev, mask_stride, 0);
+        rows = search_plan(n, xd, k, dd, ld, mask_dev, mask_stride, from, 0);
     }
-    if (split && !rows.empty()) {
+    if (from != Candidates::kFp32 && !rows.empty()) {
         // The error bound of the splits is two to three times that of fp32 scores: what they leave unproven, the fp32 plan may
         // prove, at a fraction of what canonical scores of the whole base cost (200k x 128, 512 queries with a common offset
         // that leaves 449 unproven by splits and 122 by fp32 as well: 10.7 ms with exact rows at once, 3.8 with fp32 before them;
@@ -726,7 +759,7 @@ void FlatIndex::search_masked(int64_t n, const float *x, int64_t k, float *dist,
         rows_dev.upload(rows.data(), rows.size(), stream_);
         hipLaunchKernelGGL(gather_rows_f32_kernel, dim3(blocks_for(m * d_)), dim3(256), 0, stream_, xd, rows_dev.data(), m, d_,
                            xsub.data());
-        std::vector<int64_t> left = search_plan(m, xsub.data(), k, dsub.data(), lsub.data(), nullptr, 0, 0);
+        std::vector<int64_t> left = search_plan(m, xsub.data(), k, dsub.data(), lsub.data(), nullptr, 0, Candidates::kFp32, 0);
         hipLaunchKernelGGL(scatter_result_rows_kernel, dim3(blocks_for(m * k)), dim3(256), 0, stream_, dsub.data(), lsub.data(),
                            rows_dev.data(), m, (int)k, dd, ld);
         sync_stream(stream_);   // the temporaries above are freed on leaving this block
@@ -752,15 +785,15 @@ void FlatIndex::search_masked(int64_t n, const float *x, int64_t k, float *dist,
     stats_.ms_total = stats_.ms_score + stats_.ms_select;
 }
 
-// One plan for n queries in device memory: candidates from approximate scores (split_rows > 0: of bf16 x 3 splits, that many
-// base rows at a time; 0: fp32 matrix cores), their canonical re-evaluation into dd / ld, and the proof.  Returns the queries
+// One plan for n queries in device memory: candidates from approximate scores (`from`; split_rows: base rows that are split at a
+// time where they are split beforehand), their canonical re-evaluation into dd / ld, and the proof.  Returns the queries
 // without proof, ascending; waits for the stream.  Adds its times and launches to stats_.
 std::vector<int64_t> FlatIndex::search_plan(int64_t n, const float *xd, int64_t k, float *dd, int64_t *ld,
-                                            const uint8_t *mask_dev, int64_t mask_stride, int64_t split_rows)
+                                            const uint8_t *mask_dev, int64_t mask_stride, Candidates from, int64_t split_rows)
 {
-    const bool split = split_rows > 0;
+    const bool split = from == Candidates::kSplit, resident = from == Candidates::kResident;
     const int dp = (int)round_up(d_, 32);
-    const int ncand = (int)std::min<int64_t>(std::max<int64_t>(ntotal_, 1), split ? split_spare(k) : k + 8 + k / 8);
+    const int ncand = (int)std::min<int64_t>(std::max<int64_t>(ntotal_, 1), split || resident ? split_candidates(k, dp, metric_, resident) : k + 8 + k / 8);
     ws_qn_.resize((size_t)n);
     ws_running_.resize((size_t)n * ncand);
     ws_cand_.resize((size_t)n * ncand);
@@ -775,6 +808,10 @@ std::vector<int64_t> FlatIndex::search_plan(int64_t n, const float *xd, int64_t 
         launches = stream_select_f32_split(xd, n, base_.data(), ntotal_, d_, ws_qn_.data(), norms_.data(), metric_, ncand,
                                            ws_running_.data(), ws_sel_, scratch_bytes_ - scratch_bytes_ / 2, stream_,
                                            SplitBase{ws_qsplit_.data(), ws_bsplit_.data(), split_rows, dp});
+    } else if (resident) {
+        launch_sqnorm_rows(xd, n, d_, ws_qn_.data(), stream_);
+        launches = stream_select_f32_resident(xd, n, base_.data(), ntotal_, d_, ws_qn_.data(), norms_.data(), metric_, ncand,
+                                              ws_running_.data(), ws_sel_, scratch_bytes_, stream_);
     } else {
         launch_sqnorm_rows(xd, n, d_, ws_qn_.data(), stream_);
         launches = stream_select_f32(xd, n, base_.data(), ntotal_, d_, ws_qn_.data(), norms_.data(), metric_, ncand,
@@ -800,12 +837,17 @@ std::vector<int64_t> FlatIndex::search_plan(int64_t n, const float *xd, int64_t 
         // (bf16 x 3: hi + lo misses at most 2^-18 of a value, so the three products kept miss at most 3 x 2^-18 sum |x_i y_i|;
         // their 3 dp terms are exact and summed in some order)
         const float dots = metric_ == kMetricL2 ? 2.0f : 1.0f;
-        const float err_scale = split ? dots * (3.0f / 262144.0f + (float)(3 * dp + d_ + 8) * u) : dots * (float)(2 * d_ + 8) * u;
-        const float round_scale = metric_ == kMetricL2 ? 4.0f * u : 0.0f;
+        float err_scale = split || resident ? dots * (3.0f / 262144.0f + (float)(3 * dp + d_ + 8) * u) : dots * (float)(2 * d_ + 8) * u;
+        float round_scale = metric_ == kMetricL2 ? 4.0f * u : 0.0f;
+        if (resident && metric_ == kMetricL2) {
+            // the 3 dp terms are added to -|b|^2 / 2: twice 3 dp roundings of numbers up to |b|^2 / 2 + |q| |b|
+            err_scale = dots * (3.0f / 262144.0f + (float)(d_ + 8) * u);
+            round_scale = (float)(3 * dp + 4) * u;
+        }
         ws_flag_.resize((size_t)n + 1);
         IXA_HIP(hipMemsetAsync(ws_flag_.data(), 0, sizeof(int32_t), stream_));
         launch_verify_superset(ws_running_.data(), ncand, dd, (int)k, ws_qn_.data(), bmax_, err_scale, round_scale, metric_,
-                               n, ws_flag_.data(), stream_, split);
+                               n, ws_flag_.data(), stream_, split || resident);
         int32_t nfail = 0;
         ws_flag_.download(&nfail, 1, stream_);
         if (nfail > 0) {

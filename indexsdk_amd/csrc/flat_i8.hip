@@ -538,19 +538,6 @@ __global__ __launch_bounds__(kResidentWaves * 64) __attribute__((amdgpu_waves_pe
     }
 }
 
-int device_cus()
-{
-    static std::atomic<int> known{0};
-    int cus = known.load(std::memory_order_relaxed);
-    if (cus == 0) {
-        int dev = 0;
-        IXA_HIP(hipGetDevice(&dev));
-        IXA_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-        known.store(cus, std::memory_order_relaxed);
-    }
-    return cus;
-}
-
 template <int NHS, int PF, int RA, bool FILTER>
 void launch_resident(const int8_t *Q, int64_t nq, const int8_t *tiled, const int32_t *qn, const int32_t *bn, int64_t r0,
                      int64_t r1, int32_t *out, int64_t ldo, ScoreFilter<int32_t> flt, hipStream_t s)

@@ -101,11 +101,13 @@ private:
                     const uint8_t *mask_dev, int64_t mask_stride);
     void search_masked(int64_t n, const float *x, int64_t k, float *dist, int64_t *labels, bool on_device,
                        const uint8_t *mask_dev, int64_t mask_stride);
+    // where the candidates' scores come from: fp32 products, bf16 x 3 splits formed in the score kernel, or splits formed before
+    enum class Candidates { kFp32, kResident, kSplit };
     void measure_norms(const float *norms, int64_t n);
     void forget_norms();
     std::vector<int64_t> search_plan(int64_t n, const float *xd, int64_t k, float *dd, int64_t *ld, const uint8_t *mask_dev,
-                                     int64_t mask_stride, int64_t split_rows);
-    DeviceBuffer<float> norms_, ws_qn_, ws_dist_;
+                                     int64_t mask_stride, Candidates from, int64_t split_rows);
+    DeviceBuffer<float> norms_, ws_qn_, ws_dist_;   // norms_: room up to a multiple of four
     DeviceBuffer<uint16_t> ws_qsplit_, ws_bsplit_;   // bf16 x 3 splits of a search's queries and of a stretch of the base
     StreamSelectWorkspace<float> ws_sel_;
     DeviceBuffer<int32_t> ws_cand_, ws_idx_, ws_flag_;

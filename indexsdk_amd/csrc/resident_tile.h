@@ -5,10 +5,26 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <atomic>
 #include <cstdint>
 #include <type_traits>
 
+#include "common.h"
+
 namespace ixa {
+
+inline int device_cus()
+{
+    static std::atomic<int> known{0};
+    int cus = known.load(std::memory_order_relaxed);
+    if (cus == 0) {
+        int dev = 0;
+        IXA_HIP(hipGetDevice(&dev));
+        IXA_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+        known.store(cus, std::memory_order_relaxed);
+    }
+    return cus;
+}
 
 template <int I, int N, typename F>
 __device__ __forceinline__ void static_for(F &&f)

@@ -47,6 +47,10 @@ struct SplitBase {
 int stream_select_f32_split(const float *Q, int64_t nq, const float *B, int64_t nb, int d, const float *qn, const float *bn,
                             int metric, int ncand, unsigned long long *running, StreamSelectWorkspace<float> &ws,
                             int64_t scratch_bytes, hipStream_t s, const SplitBase &split);
+// The same with the splits formed inside the score kernel (flat_resident.h says what it asks of the operands).  No mask.
+int stream_select_f32_resident(const float *Q, int64_t nq, const float *B, int64_t nb, int d, const float *qn, const float *bn,
+                               int metric, int ncand, unsigned long long *running, StreamSelectWorkspace<float> &ws,
+                               int64_t scratch_bytes, hipStream_t s);
 // Same selection with approximate scores: Qs / Bs are the bf16 x 3 splits of the operands (rows of d3
 // bf16 elements, see launch_split_bf16x3), qn / bn the exact fp32 norms.  Returns -1 without doing
 // anything when the shape does not qualify for the bf16 matrix-core kernel.

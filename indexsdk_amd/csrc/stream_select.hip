@@ -5,6 +5,7 @@
 #include <cmath>
 
 #include "flat_i8.h"
+#include "flat_resident.h"
 #include "topk.h"
 
 namespace ixa {
@@ -102,6 +103,7 @@ struct F32Ops {
     using S = float;
     static constexpr int64_t kMinChunk = 1;   // its score launchers serve any chunk of base rows
     static constexpr int64_t kSeedRows = 2048, kMaxGrowth = 1 << 20;
+    static constexpr int64_t kFuseScores = INT64_MAX;   // scores from which a matrix that fits the scratch is not stored all the same
     const float *qn, *bn;
     int metric;
     const S *threshold(StreamSelectWorkspace<S> &, int64_t, int64_t, hipStream_t) const { return nullptr; }
@@ -184,11 +186,35 @@ struct F32SplitOps : F32Ops {
     }
 };
 
+// fp32 operands scored by the resident-query kernel, which splits the base rows on their way in (flat_resident.hip).
+// Stored scores cost their write and the selection's reading of them; a bound-filtered search costs a seed and three to six more
+// pairs of launches: 32M scores over 1M x 128 297 / 294 us, 64M 368 / 418, 128M 1037 / 447.  Seeds of 8192, 16384 and 32768 rows
+// and chunks of two to four times what has been seen are within 4 % of each other.
+struct F32ResidentOps : F32Ops {
+    static constexpr int64_t kSeedRows = 16384, kMaxGrowth = 2;
+    static constexpr int64_t kFuseScores = (int64_t)64 << 20;
+    F32ResidentOps(const float *qn_, const float *bn_, int metric_) : F32Ops{qn_, bn_, metric_} {}
+    void scores(const T *Q, int64_t nq, int64_t q0, const T *B, int64_t nb, int64_t b0, int d, S *out, int64_t ldo,
+                hipStream_t s) const
+    {
+        if (!launch_resident_f32(Q, nq, B + b0 * d, nb, d, qn + q0, bn + b0, metric, out, ldo, false, ScoreFilter<float>{}, s)) {
+            F32Ops::scores(Q, nq, q0, B, nb, b0, d, out, ldo, s);
+        }
+    }
+    void filtered(const T *Q, int64_t nq, int64_t q0, const T *B, int64_t nb, int64_t b0, int d, ScoreFilter<S> flt,
+                  hipStream_t s) const
+    {
+        if (!launch_resident_f32(Q, nq, B + b0 * d, nb, d, qn + q0, bn + b0, metric, nullptr, 0, true, flt, s)) {
+            F32Ops::filtered(Q, nq, q0, B, nb, b0, d, flt, s);
+        }
+    }
+};
+
 struct Bf16Ops {
     using T = uint16_t;
     using S = float;
     static constexpr int64_t kMinChunk = 2048;   // the ring kernel is the only one for split operands
-    static constexpr int64_t kSeedRows = 2048, kMaxGrowth = 1 << 20;
+    static constexpr int64_t kSeedRows = 2048, kMaxGrowth = 1 << 20, kFuseScores = INT64_MAX;
     const float *qn, *bn;
     int metric;
     const S *threshold(StreamSelectWorkspace<S> &, int64_t, int64_t, hipStream_t) const { return nullptr; }
@@ -227,7 +253,7 @@ struct I8Ops {
     // pass, so the bound is tightened often: a longer seed stretch (a bound from 8192 rows admits a quarter of what
     // one from 2048 does) and chunks that only double what has been seen (10M x 512, 2048 queries, k 100, same box:
     // seed 2048 and chunks of 5 x seen 8.91 ms per search; 8192 and 5 x: 8.80; 8192 and 3 x: 8.54; 8192 and 2 x: 8.47)
-    static constexpr int64_t kSeedRows = 8192, kMaxGrowth = 2;
+    static constexpr int64_t kSeedRows = 8192, kMaxGrowth = 2, kFuseScores = INT64_MAX;
     const int32_t *qn, *bn;
     const S *threshold(StreamSelectWorkspace<S> &ws, int64_t q0, int64_t nq, hipStream_t s) const
     {
@@ -285,7 +311,8 @@ int stream_select(const Ops &ops, const typename Ops::T *Q, int64_t nq_total, co
     // cheapest plan (measured on the IVFPQ coarse stage: 16384 centroids); the filtered plan is for
     // long bases
     // (a masked search materialises every stretch: the mask is applied to the stored scores)
-    bool can_fuse = mask == nullptr && nb_total > nb && nb_total >= 4 * seed_rows &&
+    const bool long_base = nb_total > nb || std::min(nq_total, qb) * nb_total >= Ops::kFuseScores;
+    bool can_fuse = mask == nullptr && long_base && nb_total >= 4 * seed_rows &&
                     pow2_ceil(ncand + cap) * sizeof(key_t) <= 160 * 1024;
     if (can_fuse && qb * (int64_t)cap * (int64_t)sizeof(key_t) > scratch_bytes) {
         // the candidate buffers of a query block count against the scratch budget too: a narrower block
@@ -293,7 +320,7 @@ int stream_select(const Ops &ops, const typename Ops::T *Q, int64_t nq_total, co
         nb = scratch_bytes / (qb * (int64_t)sizeof(S));
         nb = std::max<int64_t>(128, nb / 128 * 128);
         nb = std::min<int64_t>(nb, round_up(std::max<int64_t>(nb_total, 1), 128));
-        can_fuse = nb_total > nb;
+        can_fuse = nb_total > nb || std::min(nq_total, qb) * nb_total >= Ops::kFuseScores;
     }
     // tau is fixed during a chunk, so a chunk admits about ncand * chunk / seen keys per query; keep
     // that expectation below a quarter of the candidate buffer
@@ -404,6 +431,13 @@ int stream_select_f32(const float *Q, int64_t nq, const float *B, int64_t nb, in
 {
     return stream_select(F32Ops{qn, bn, metric}, Q, nq, B, nb, d, ncand, running, ws, scratch_bytes, s, mask,
                          mask_stride);
+}
+
+int stream_select_f32_resident(const float *Q, int64_t nq, const float *B, int64_t nb, int d, const float *qn, const float *bn,
+                               int metric, int ncand, unsigned long long *running, StreamSelectWorkspace<float> &ws,
+                               int64_t scratch_bytes, hipStream_t s)
+{
+    return stream_select(F32ResidentOps(qn, bn, metric), Q, nq, B, nb, d, ncand, running, ws, scratch_bytes, s);
 }
 
 int stream_select_f32_split(const float *Q, int64_t nq, const float *B, int64_t nb, int d, const float *qn, const float *bn,

@@ -3,10 +3,14 @@
 int8: exact int32 distances and ids, bit for bit.  fp32: the final candidates are re-evaluated in
 the canonical scalar arithmetic, so distances and ids equal the oracle's bit for bit as well.
 """
+import ctypes
 import os
 
 import numpy as np
 import pytest
+import torch
+
+from indexsdk_amd import _capi
 
 pytestmark = pytest.mark.gpu
 GOLDEN = os.path.join(os.path.dirname(os.path.abspath(__file__)), "golden", "ivfpq_small.npz")
@@ -485,6 +489,39 @@ def test_flat_f32_base_with_values_out_of_range_keeps_the_fp32_plan(ix):
         D, I = index.search(q, k)
         Ds, Is = index.search(q[:100], k)
         assert np.array_equal(I[:100], Is) and np.array_equal(D[:100].view(np.uint32), Ds.view(np.uint32))
+
+
+# The kernel that keeps a tile of 256, 128, 64 or 32 queries in LDS and splits fp32 base rows in registers (dimensions that are a
+# multiple of 4): remainders of the dimension, of the 256-row tile, of a wavefront's 32 rows and of four rows, tiles that the batch
+# does not fill, scores stored and bound-filtered (scratch of 8 MB).  Canonical results: the oracle's, bit for bit.
+@pytest.mark.parametrize("metric_name", ["L2", "IP"])
+@pytest.mark.parametrize("d,n,nq,k,scratch", [(36, 2048, 1, 1, 0), (64, 2049, 257, 10, 0), (100, 2303, 33, 300, 0),
+                                              (128, 4095, 129, 100, 0), (132, 3001, 300, 20, 0), (256, 2050, 65, 5, 0),
+                                              (388, 2305, 64, 100, 0), (512, 2559, 31, 10, 0), (768, 2561, 40, 384, 0),
+                                              (1024, 2100, 3, 7, 0), (44, 65537, 300, 10, 8 << 20), (96, 65794, 385, 100, 8 << 20),
+                                              (200, 70001, 259, 3, 8 << 20), (384, 65567, 70, 60, 2 << 20)])
+def test_flat_f32_split_in_the_score_kernel(ix, oracle, metric_name, d, n, nq, k, scratch):
+    metric = ix.METRIC_L2 if metric_name == "L2" else ix.METRIC_INNER_PRODUCT
+    rng = np.random.default_rng(d + n)
+    centres = rng.standard_normal((50, d)).astype(np.float32)
+    base = (centres[rng.integers(0, 50, n)] + 0.5 * rng.standard_normal((n, d))).astype(np.float32)
+    base[n - 1] = base[0]
+    q = (centres[rng.integers(0, 50, nq)] + 0.5 * rng.standard_normal((nq, d))).astype(np.float32)
+    q[nq - 1] = base[0]
+    index = ix.AscendIndexFlat(d, metric, scratch_bytes=scratch)
+    index.add(base)
+    some = np.unique(np.concatenate([np.arange(min(nq, 3)), [nq - 1], np.arange(31, nq, 32), np.arange(32, nq, 32)]))
+    Dr, Ir = oracle.flat_f32(base, q[some], k, metric)
+    D, I = index.search(q, k)
+    assert np.array_equal(I[some], Ir) and np.array_equal(D[some].view(np.uint32), Dr.view(np.uint32))
+    # queries in device memory that are not 16-byte aligned keep the fp32 kernels
+    room = torch.zeros(nq * d + 1, device="cuda")
+    room[1:] = torch.from_numpy(q).reshape(-1)
+    Dd, Id = torch.empty(nq, k, device="cuda"), torch.empty(nq, k, device="cuda", dtype=torch.int64)
+    torch.cuda.synchronize()
+    _capi.check(_capi.load().flat_search_device(index._h, nq, ctypes.c_void_p(room.data_ptr() + 4), k,
+                                                ctypes.c_void_p(Dd.data_ptr()), ctypes.c_void_p(Id.data_ptr())))
+    assert np.array_equal(Id.cpu().numpy(), I) and np.array_equal(Dd.cpu().numpy().view(np.uint32), D.view(np.uint32))
 
 
 # Up to 64 queries over 32768 rows and more: every row of scores is selected by several workgroups, whose keys one more orders.

@@ -68,3 +68,9 @@ def test_scan_kernels_of_sixteen_wavefronts_spill_only_at_96_bytes(kernels):
         if m and m.group(4) == "16":
             allowed = limit[m.group(2), m.group(3)] if m.group(1) == "96" else 0
             assert registers <= 128 and spilled <= allowed, (name, registers, spilled)
+
+
+def test_flat_kernels_that_split_in_registers_do_not_spill(kernels):
+    """Their fragments are read by instructions whose arrival the compiler does not track: a spill would store them too early."""
+    resident = [v for n, v in kernels.items() if "resident_f32_kernel" in n]
+    assert len(resident) == 14 and all(registers <= 256 and spilled == 0 for registers, spilled in resident)
