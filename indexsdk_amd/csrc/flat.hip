@@ -9,7 +9,7 @@
 #include "coarse.h"
 #include "flat_i8.h"
 #include "flat_index.h"
-#include "flat_resident.h"
+#include "resident_f32.h"
 #include "stream_select.h"
 #include "topk.h"
 

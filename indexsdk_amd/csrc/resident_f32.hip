@@ -1,4 +1,5 @@
-// fp32 Flat scores on the bf16 matrix cores, the base read as it lies.
+// fp32 scores on the bf16 matrix cores, the streamed operand read as it lies: Flat search (queries in LDS, base streamed) and
+// assignment (centroids in LDS, vectors streamed).
 //
 // resident_f32_kernel has the structure of the int8 kernel (flat_i8.hip): a persistent workgroup of 8 wavefronts keeps a tile
 // of QT = 32 RA queries in LDS, wavefront w owns rows 32 w .. 32 w + 31 of every tile of 256 base rows, and no workgroup barrier
@@ -19,7 +20,8 @@
 //     batch's loads: they have SPB K-steps to arrive.
 //
 // 1M x 128, 1000 queries: 1.23 PFLOP/s of bf16 products in the longest launch (0.71 of the ring kernel that reads split rows); a
-// search 1763 -> 964 us.  What bounds it is what bounds the int8 kernel: the clock under dense matrix work, and LDS reads (85
+// search 1763 -> 964 us.  Assignment of 1M x 128 to 1024 centroids: 660 us of score launch at 1.19 PFLOP/s, 100 us for the tiles' best
+// and 26 us for what they leave open, where scores, selections and the refinement took 7.6 ms.  What bounds it is what bounds the int8 kernel: the clock under dense matrix work, and LDS reads (85
 // bytes per cycle and CU of 128); with few queries the base's bytes (512 MB in 100 us of the 207 of one query over 1M x 128).
 //
 // Score arithmetic: the accumulators start from -|b|^2 / 2 (L2; 0 for inner product) and end as u = q.b - |b|^2 / 2, and the
@@ -28,7 +30,7 @@
 #include <cmath>
 
 #include "coarse.h"
-#include "flat_resident.h"
+#include "resident_f32.h"
 #include "resident_tile.h"
 #include "topk.h"
 
@@ -46,8 +48,10 @@ constexpr int kWaves = 8;
 constexpr int kTileRows = 256;       // base rows of a tile
 constexpr int kQueueKeys = 128;      // per-wavefront queue of admitted keys (16 bytes each); flushed above 64
 constexpr float kNoRow = -__builtin_inff();   // accumulator start of a row outside the launch: it reaches no test value
+constexpr float kNoCentroid = -3e38f;   // of a centroid past the last one (a number: low bits are put into the sums)
 // LDS behind the query tile of a filtered launch: {bound, norm, test value, -} per query, the wavefronts' queues
 constexpr int filter_lds(int qt) { return qt * 16 + kWaves * kQueueKeys * 16; }
+constexpr int assign_lds(int qt) { return qt * 4; }   // -|c|^2 / 2 per centroid
 constexpr int kLdsLimit = 160 * 1024;
 
 // hi and lo of eight numbers
@@ -82,14 +86,49 @@ __device__ __forceinline__ float test_value(float qn, float tau, bool l2)
     return fmaxf(t, -3.402823466e+38f);
 }
 
-// RA: query blocks of 32 per tile; SPB: K-steps of 16 dimensions per batch; FILTER: append admitted keys, otherwise store
-// every score.  nbat >= 2 batches cover the d dimensions.
-template <int RA, int SPB, bool FILTER>
+// The larger of two numbers, or the number where the other is a NaN.  (fmaxf would make v a quiet number first, an instruction
+// each.  The operands are results of vector instructions, never of a matrix instruction, whose results an inline instruction
+// would not wait for.)
+__device__ __forceinline__ float max_number(float m, float v)
+{
+    float r;
+    asm("v_max_f32 %0, %1, %2" : "=v"(r) : "v"(m), "v"(v));
+    return r;
+}
+
+// Three largest values, the places of two.  (A NaN among the values is passed over: med3 of it and two numbers is the smaller.)
+struct Best {
+    float v1, v2, v3;
+    uint32_t p1, p2;
+    __device__ __forceinline__ void merge(const Best &o)
+    {
+        const bool first = o.v1 > v1;
+        const float a1 = first ? o.v1 : v1, a2 = first ? o.v2 : v2, a3 = first ? o.v3 : v3, b1 = first ? v1 : o.v1, b2 = first ? v2 : o.v2;
+        const uint32_t ap1 = first ? o.p1 : p1, ap2 = first ? o.p2 : p2, bp1 = first ? p1 : o.p1;
+        const bool second = b1 > a2;   // of the list with the smaller best
+        v1 = a1;
+        p1 = ap1;
+        v2 = second ? b1 : a2;
+        p2 = second ? bp1 : ap2;
+        v3 = second ? fmaxf(a2, b2) : fmaxf(a3, b1);
+    }
+};
+
+enum { kStore = 0, kFilter = 1, kAssign = 2 };
+
+// RA: query blocks of 32 per tile; SPB: K-steps of 16 dimensions per batch; nbat >= 2 batches cover the d dimensions.  MODE:
+//   kStore   every score is stored;
+//   kFilter  admitted keys are appended;
+//   kAssign  the "queries" are centroids, the base rows vectors: of every tile of centroids the best two of each vector and the
+//            third value.  The matrix operands change places, so that a lane owns ONE vector and 16 centroids per block, and
+//            the accumulators start from -|c|^2 / 2, kept in LDS.
+template <int RA, int SPB, int MODE>
 __global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) void resident_f32_kernel(
     const float *__restrict__ Q, int64_t nq, const float *__restrict__ B, int64_t nb, int d, int nbat,
     const float *__restrict__ qn, const float *__restrict__ bn, int metric, float *__restrict__ out, int64_t ldo,
-    ScoreFilter<float> flt, int tiles_m, int ntiles, int seg_tiles)
+    ScoreFilter<float> flt, float4 *__restrict__ top, int tiles_m, int ntiles, int seg_tiles, int own_resident)
 {
+    constexpr bool FILTER = MODE == kFilter, ASSIGN = MODE == kAssign;
     constexpr int QT = RA * 32;
     // LDS of a K-step: [half][RA blocks of hi, RA of lo][32 queries][16 B]
     constexpr int kStepLds = QT * 64;
@@ -106,7 +145,7 @@ __global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(2, 
     const bool l2 = metric == kMetricL2;
 
     const int xcd = blockIdx.x & 7, wi = blockIdx.x >> 3, wpx = gridDim.x >> 3;
-    const ResidentItems sched(tiles_m, ntiles, seg_tiles, xcd, wpx);
+    const ResidentItems sched(tiles_m, ntiles, seg_tiles, xcd, wpx, own_resident != 0);
     const int S = sched.S;
     const int first_item = sched.next(wi);
     if (first_item < 0) {
@@ -115,6 +154,7 @@ __global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(2, 
     const uint32_t lds_base = (uint32_t)reinterpret_cast<size_t>((__attribute__((address_space(3))) unsigned char *)lds);
     const uint32_t a_lane = lds_base + (uint32_t)(half * (QT * 32) + l32 * 16);
     float4 *meta = reinterpret_cast<float4 *>(lds + (size_t)nbat * kBatchLds);   // {tau, |q|^2, test value, -}
+    float *start = reinterpret_cast<float *>(meta);   // kAssign: -|c|^2 / 2 per centroid instead
     uint4 *queue = reinterpret_cast<uint4 *>(meta + QT) + wave * kQueueKeys;
     int qcount = 0;   // keys in this wavefront's queue (wave-uniform)
     // every queued key takes its place in its query's candidate buffer; 64 lanes, one key each
@@ -166,7 +206,9 @@ __global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(2, 
     sched.range(it_t, tm, j, jend);
     const float *cur = row_ptr(j);
     // Loads are issued in the same order here and in the loop: norms of a tile before its first batch.
-    load_norms(j);
+    if constexpr (!ASSIGN) {
+        load_norms(j);
+    }
     load_batch(cur, 0);
     bool staggered = false;
     while (true) {
@@ -218,6 +260,12 @@ __global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(2, 
                                          : make_float4(__builtin_nanf(""), 0.f, __builtin_inff(), 0.f);
                 }
             }
+            if constexpr (ASSIGN) {
+                if (tid < QT) {
+                    const int64_t c = (int64_t)tm * QT + tid;
+                    start[tid] = c < nq ? -0.5f * qn[c] : kNoCentroid;
+                }
+            }
             cur_tm = tm;
             __syncthreads();
             // The second wavefront of every SIMD starts half a tile late, once: from then on each one's epilogue runs under the
@@ -245,11 +293,25 @@ __global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(2, 
         const float *nxt = row_ptr(n_j);
         const int64_t row0 = block_row0(j);
         v16f c0;
+        if constexpr (ASSIGN) {
 #pragma unroll
-        for (int r = 0; r < 16; r++) {
-            c0[r] = l2 ? -0.5f * bnv[r >> 2][r & 3] : 0.f;
+            for (int ra = 0; ra < RA; ra++) {
+#pragma unroll
+                for (int g = 0; g < 4; g++) {
+                    const v4f c = *reinterpret_cast<const v4f *>(start + ra * 32 + 8 * g + 4 * half);
+#pragma unroll
+                    for (int t = 0; t < 4; t++) {
+                        acc[ra][4 * g + t] = c[t];
+                    }
+                }
+            }
+        } else {
+#pragma unroll
+            for (int r = 0; r < 16; r++) {
+                c0[r] = l2 ? -0.5f * bnv[r >> 2][r & 3] : 0.f;
+            }
         }
-        if (row0 + 32 > nb) {   // the last tile of the launch: rows past its end take no part
+        if (!ASSIGN && row0 + 32 > nb) {   // the last tile of the launch: rows past its end take no part
 #pragma unroll
             for (int r = 0; r < 16; r++) {
                 c0[r] = row0 + 4 * half + 8 * (r >> 2) + (r & 3) < nb ? c0[r] : kNoRow;
@@ -268,7 +330,7 @@ __global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(2, 
             for (int t = 0; t < SPB; t++) {
                 split8(raw[2 * t], raw[2 * t + 1], bh[t], bl[t]);
             }
-            if constexpr (LAST) {
+            if constexpr (LAST && !ASSIGN) {
                 load_norms(n_j);
             }
             load_batch(next_row, next_batch);
@@ -283,7 +345,9 @@ __global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(2, 
                 }
                 static_for<0, G>([&](auto tc) {
                     constexpr int t = decltype(tc)::value, f = p * G + t, ra = f % RA;
-                    if constexpr (FIRST && st == 0 && f < RA) {
+                    if constexpr (ASSIGN) {
+                        acc[ra] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[u & 1][t], bh[st], acc[ra], 0, 0, 0);
+                    } else if constexpr (FIRST && st == 0 && f < RA) {
                         acc[ra] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bh[st], fa[u & 1][t], c0, 0, 0, 0);
                     } else {
                         acc[ra] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bh[st], fa[u & 1][t], acc[ra], 0, 0, 0);
@@ -291,7 +355,9 @@ __global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(2, 
                 });
                 static_for<0, G>([&](auto tc) {
                     constexpr int t = decltype(tc)::value, f = p * G + t;
-                    if constexpr (f < RA) {
+                    if constexpr (f < RA && ASSIGN) {
+                        acc[f] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[u & 1][t], bl[st], acc[f], 0, 0, 0);
+                    } else if constexpr (f < RA) {
                         acc[f] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bl[st], fa[u & 1][t], acc[f], 0, 0, 0);
                     }
                 });
@@ -344,6 +410,36 @@ __global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(2, 
                         }
                     }
                 }
+            }
+        } else if constexpr (ASSIGN) {
+            // Largest, second and third u of four blocks at a time, their places 16 ra + r in the low six bits (which moves a value
+            // by at most 2^-17 of it); then of all blocks, and of both halves, which hold different centroids of the same vector.
+            constexpr int SETS = RA > 4 ? RA / 4 : 1, BLOCKS = RA / SETS;
+            Best best[SETS];
+#pragma unroll
+            for (int set = 0; set < SETS; set++) {
+                float m1 = kNoCentroid, m2 = kNoCentroid, m3 = kNoCentroid;
+#pragma unroll
+                for (int i = 0; i < BLOCKS * 16; i++) {
+                    const float v = __uint_as_float((__float_as_uint(acc[set * BLOCKS + i / 16][i % 16]) & ~63u) | (uint32_t)i);
+                    m3 = __builtin_amdgcn_fmed3f(m2, m3, v);
+                    m2 = __builtin_amdgcn_fmed3f(m1, m2, v);
+                    m1 = max_number(m1, v);
+                }
+                auto place = [&](float v) {
+                    const uint32_t i = __float_as_uint(v) & 63u;
+                    return set * (BLOCKS * 32) + (i >> 4) * 32 + ((i >> 2) & 3) * 8 + half * 4 + (i & 3);
+                };
+                best[set] = Best{m1, m2, m3, place(m1), place(m2)};
+            }
+            if constexpr (SETS == 2) {
+                best[0].merge(best[1]);
+            }
+            const Best &own = best[0];
+            best[0].merge(Best{__shfl_xor(own.v1, 32), __shfl_xor(own.v2, 32), __shfl_xor(own.v3, 32),
+                               (uint32_t)__shfl_xor((int)own.p1, 32), (uint32_t)__shfl_xor((int)own.p2, 32)});
+            if (half == 0 && row0 + l32 < nb) {
+                top[(int64_t)tm * nb + row0 + l32] = make_float4(own.v1, own.v2, own.v3, __uint_as_float(own.p1 | own.p2 << 16));
             }
         } else {
 #pragma unroll
@@ -398,15 +494,18 @@ struct Args {
     float *out;
     int64_t ldo;
     ScoreFilter<float> flt;
+    float4 *top;
     hipStream_t s;
 };
 
-template <int RA, int SPB, bool FILTER>
+constexpr int extra_lds(int mode, int qt) { return mode == kFilter ? filter_lds(qt) : (mode == kAssign ? assign_lds(qt) : 0); }
+
+template <int RA, int SPB, int MODE>
 void launch_shape(const Args &a, int nbat)
 {
     constexpr int QT = RA * 32;
-    const size_t smem = (size_t)nbat * SPB * QT * 64 + (FILTER ? filter_lds(QT) : 0);
-    auto kern = resident_f32_kernel<RA, SPB, FILTER>;
+    const size_t smem = (size_t)nbat * SPB * QT * 64 + extra_lds(MODE, QT);
+    auto kern = resident_f32_kernel<RA, SPB, MODE>;
     static std::atomic<bool> configured{false};   // per instantiation
     if (!configured) {
         hipFuncAttributes attr;
@@ -420,44 +519,192 @@ void launch_shape(const Args &a, int nbat)
     const int64_t tiles_m = (a.nq + QT - 1) / QT, ntiles = (a.nb + kTileRows - 1) / kTileRows;
     IXA_REQUIRE(tiles_m < (1 << 20) && ntiles < ((int64_t)1 << 30), kErrInvalidParam, "fp32 score launch too large");
     const unsigned grid = (unsigned)((device_cus() + 7) / 8 * 8);   // one persistent workgroup per CU
-    const int64_t wpx = grid / 8, own_n = (ntiles + 7) / 8;
+    const int64_t wpx = grid / 8;
+    // Which operand's tiles an XCD owns.  The streamed one's, so that its L2 serves a tile to every query tile; but where an
+    // XCD's share of few streamed tiles is uneven, the resident one's (both counted in rounds of tiles per workgroup).
+    const int64_t rounds_b = (tiles_m * ((ntiles + 7) / 8) + wpx - 1) / wpx, rounds_q = ((tiles_m + 7) / 8 * ntiles + wpx - 1) / wpx;
+    const bool own_q = MODE == kAssign && rounds_q < rounds_b;
+    const int64_t tm = own_q ? (tiles_m + 7) / 8 : tiles_m, tn = own_q ? ntiles : (ntiles + 7) / 8;
     // segments: enough items for an even share per workgroup, long enough to pay for a query tile that changes
-    const int seg = (int)std::min<int64_t>(16, std::max<int64_t>(1, (own_n * tiles_m + wpx * 8 - 1) / (wpx * 8)));
+    const int seg = (int)std::min<int64_t>(16, std::max<int64_t>(1, (tn * tm + wpx * 8 - 1) / (wpx * 8)));
     hipLaunchKernelGGL(kern, dim3(grid), dim3(kWaves * 64), smem, a.s, a.Q, a.nq, a.B, a.nb, a.d, nbat, a.qn, a.bn, a.metric,
-                       a.out, a.ldo, a.flt, (int)tiles_m, (int)ntiles, seg);
+                       a.out, a.ldo, a.flt, a.top, (int)tiles_m, (int)ntiles, seg, own_q ? 1 : 0);
 }
 
 // batches of a row: of four K-steps where that does not add padding, else of two
 int batch_steps(int d) { return (d + 31) / 32 % 2 == 0 && d > 64 ? 4 : 2; }
 int batches(int d, int spb) { return (d + 16 * spb - 1) / (16 * spb); }
-bool fits(int d, int ra)
-{
-    return (d + 31) / 32 * 32 * 4 * ra * 32 + filter_lds(ra * 32) <= kLdsLimit;
-}
+bool fits(int d, int ra) { return (d + 31) / 32 * 32 * 4 * ra * 32 + filter_lds(ra * 32) <= kLdsLimit; }
 
-template <bool FILTER>
-void launch_filter(const Args &a)
+// query blocks per tile: tiles x (blocks + 1), the one for loading and splitting a base row and for the epilogue
+int tile_blocks(int64_t nq, int d)
 {
-    // query blocks per tile: tiles x (blocks + 1), the one for loading and splitting a base row and for the epilogue
     int ra = 1;
     int64_t best = INT64_MAX;
     for (int c = 8; c >= 1; c /= 2) {
-        const int64_t cost = (a.nq + 32 * c - 1) / (32 * c) * (c + 1);
-        if (fits(a.d, c) && cost < best) {
+        const int64_t cost = (nq + 32 * c - 1) / (32 * c) * (c + 1);
+        if (fits(d, c) && cost < best) {
             best = cost;
             ra = c;
         }
     }
-    const int spb = ra == 8 ? 2 : batch_steps(a.d);
-    const int nbat = batches(a.d, spb);
+    return ra;
+}
+
+template <int MODE>
+void launch_mode(const Args &a)
+{
+    const int ra = tile_blocks(a.nq, a.d), spb = ra == 8 ? 2 : batch_steps(a.d), nbat = batches(a.d, spb);
     if (ra == 8) {
-        launch_shape<8, 2, FILTER>(a, nbat);
+        launch_shape<8, 2, MODE>(a, nbat);
     } else if (ra == 4) {
-        spb == 4 ? launch_shape<4, 4, FILTER>(a, nbat) : launch_shape<4, 2, FILTER>(a, nbat);
+        spb == 4 ? launch_shape<4, 4, MODE>(a, nbat) : launch_shape<4, 2, MODE>(a, nbat);
     } else if (ra == 2) {
-        spb == 4 ? launch_shape<2, 4, FILTER>(a, nbat) : launch_shape<2, 2, FILTER>(a, nbat);
+        spb == 4 ? launch_shape<2, 4, MODE>(a, nbat) : launch_shape<2, 2, MODE>(a, nbat);
     } else {
-        spb == 4 ? launch_shape<1, 4, FILTER>(a, nbat) : launch_shape<1, 2, FILTER>(a, nbat);
+        spb == 4 ? launch_shape<1, 4, MODE>(a, nbat) : launch_shape<1, 2, MODE>(a, nbat);
+    }
+}
+
+// ---- what the tiles' best become ------------------------------------------------------------------------------------------
+
+// By how much a u has to lead another for the canonical scores to be in that order.  Both scores |x|^2 - 2 u are within E of the
+// canonical ones, and the places in the low bits have moved each u by at most 2^-17 |u|, |u| <= |x| cmax + cmax^2 / 2.  Infinite
+// or undefined where nothing can be decided.
+__device__ __forceinline__ float assign_need(float norm, float cmax, float err_scale, float round_scale)
+{
+    return score_margin(norm, cmax, err_scale, round_scale) + 1.6e-5f * (sqrtf(norm) * cmax + cmax * cmax);
+}
+
+// The best two of every vector over all tiles and the third value; a lead of more than the error bound decides, a tie of two
+// goes to `pairs` (vector, two centroids), of more (or an undefined length) to `rows`.  count: the two lists' lengths.
+__global__ __launch_bounds__(256) void assign_combine_kernel(const float4 *__restrict__ top, int tiles, int tile_centroids, int64_t n,
+                                                             const float *__restrict__ xn, float cmax, float err_scale,
+                                                             float round_scale, int32_t *__restrict__ out, int4 *__restrict__ pairs,
+                                                             int32_t *__restrict__ rows, int32_t *__restrict__ count)
+{
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    const int lane = threadIdx.x & 63;
+    Best best{kNoCentroid, kNoCentroid, kNoCentroid, 0u, 0u};
+    if (i < n) {
+        for (int t = 0; t < tiles; t++) {
+            const float4 v = top[(int64_t)t * n + i];
+            const uint32_t p = __float_as_uint(v.w), c0 = (uint32_t)(t * tile_centroids);
+            best.merge(Best{v.x, v.y, v.z, c0 + (p & 0xffffu), c0 + (p >> 16)});
+        }
+    }
+    const float need = assign_need(i < n ? xn[i] : 0.f, cmax, err_scale, round_scale);
+    const bool decided = i >= n || best.v1 - best.v2 > need, pair = !decided && best.v1 - best.v3 > need;
+    if (i < n) {
+        out[i] = (int32_t)best.p1;
+    }
+    const unsigned long long mp = __ballot(pair), mr = __ballot(!decided && !pair);
+    if ((mp | mr) != 0) {
+        int at = 0;
+        if (lane == 0 && mp) {
+            at = atomicAdd(count, (int)__popcll(mp));
+        }
+        if (lane == 1 && mr) {
+            at = atomicAdd(count + 1, (int)__popcll(mr));
+        }
+        const int at_p = __builtin_amdgcn_readlane(at, 0), at_r = __builtin_amdgcn_readlane(at, 1);
+        const unsigned long long below = (1ull << lane) - 1;
+        if (pair) {
+            pairs[at_p + __popcll(mp & below)] = make_int4((int)i, (int)best.p1, (int)best.p2, 0);
+        } else if (!decided) {
+            rows[at_r + __popcll(mr & below)] = (int32_t)i;
+        }
+    }
+}
+
+// the score of the exact plans: dot product left to right without FMA, then (|x|^2 + |c|^2) - g - g
+__device__ __forceinline__ float canonical_l2(const float *__restrict__ x, const float *__restrict__ c, int d, float xn, float cn)
+{
+    float g = 0.f;
+#pragma unroll 8
+    for (int t = 0; t < d; t += 4) {
+        const float4 a = *reinterpret_cast<const float4 *>(x + t), b = *reinterpret_cast<const float4 *>(c + t);
+        g = __fadd_rn(g, __fmul_rn(a.x, b.x));
+        g = __fadd_rn(g, __fmul_rn(a.y, b.y));
+        g = __fadd_rn(g, __fmul_rn(a.z, b.z));
+        g = __fadd_rn(g, __fmul_rn(a.w, b.w));
+    }
+    return __fsub_rn(__fsub_rn(__fadd_rn(xn, cn), g), g);
+}
+
+// What assign_combine_kernel has left open, from canonical scores: first the pairs, a lane for each of the two centroids, then
+// the vectors with more, a wavefront for each.  Of every tile whose best is within reach of the vector's best the best and the
+// second are evaluated where they are within reach themselves, and all centroids where the third is (100000 vectors, 16384
+// centroids, sixteen to a component of the mixture: 1.6 ms when such a vector was scored against every centroid).
+// Equal scores: the smaller number.  A NaN is never chosen; -1 where nothing else is left.
+__global__ __launch_bounds__(256) void assign_resolve_kernel(const float *__restrict__ X, const float *__restrict__ xn, int64_t n,
+                                                             const float *__restrict__ C, const float *__restrict__ cn, int64_t nc,
+                                                             int d, float cmax, float err_scale, float round_scale,
+                                                             const float4 *__restrict__ top, int tiles, int tile_centroids,
+                                                             const int4 *__restrict__ pairs, const int32_t *__restrict__ rows,
+                                                             const int32_t *__restrict__ count, int32_t *__restrict__ out)
+{
+    const int lane = threadIdx.x & 63;
+    const int64_t wave = (int64_t)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), waves = (int64_t)gridDim.x * 4;
+    const int npairs = count[0], nrows = count[1];
+    auto key_of = [&](int64_t row, int64_t c) {
+        const float v = canonical_l2(X + row * d, C + c * d, d, xn[row], cn[c]);
+        return v == v ? make_key(v, (uint32_t)c) : kEmptyKey;
+    };
+    for (int64_t p0 = wave * 32; p0 < npairs; p0 += waves * 32) {
+        const int64_t p = p0 + (lane >> 1);
+        const int4 e = pairs[p < npairs ? p : npairs - 1];
+        const key_t mine = key_of(e.x, lane & 1 ? e.z : e.y), other = __shfl_xor(mine, 1);
+        const key_t best = mine < other ? mine : other;
+        if (p < npairs && (lane & 1) == 0) {
+            out[e.x] = best == kEmptyKey ? -1 : (int32_t)key_index(best);
+        }
+    }
+    for (int64_t r = wave; r < nrows; r += waves) {
+        const int64_t row = rows[r];
+        float lead = kNoCentroid;
+        for (int t = lane; t < tiles; t += 64) {
+            lead = fmaxf(lead, top[(int64_t)t * n + row].x);
+        }
+        for (int o = 32; o > 0; o >>= 1) {
+            lead = fmaxf(lead, __shfl_xor(lead, o));
+        }
+        const float reach = lead - assign_need(xn[row], cmax, err_scale, round_scale);
+        key_t best = kEmptyKey;
+        for (int t0 = 0; t0 < tiles; t0 += 64) {
+            const int t = t0 + lane;
+            const float4 v = top[(int64_t)(t < tiles ? t : tiles - 1) * n + row];
+            // (written so that an undefined reach leaves nothing out)
+            const bool one = t < tiles && !(v.x < reach), two = t < tiles && !(v.y < reach);
+            const unsigned long long whole = __ballot(t < tiles && !(v.z < reach));
+            if ((whole >> lane & 1) == 0) {
+                const uint32_t p = __float_as_uint(v.w);
+                const int64_t c1 = (int64_t)t * tile_centroids + (p & 0xffffu), c2 = (int64_t)t * tile_centroids + (p >> 16);
+                if (one && c1 < nc) {
+                    const key_t k = key_of(row, c1);
+                    best = k < best ? k : best;
+                }
+                if (two && c2 < nc) {
+                    const key_t k = key_of(row, c2);
+                    best = k < best ? k : best;
+                }
+            }
+            for (unsigned long long w = whole; w != 0; w &= w - 1) {
+                const int64_t c0 = (int64_t)(t0 + __builtin_ctzll(w)) * tile_centroids;
+                const int64_t c_end = c0 + tile_centroids < nc ? c0 + tile_centroids : nc;
+                for (int64_t c = c0 + lane; c < c_end; c += 64) {
+                    const key_t k = key_of(row, c);
+                    best = k < best ? k : best;
+                }
+            }
+        }
+        for (int o = 32; o > 0; o >>= 1) {
+            const key_t k = __shfl_xor(best, o);
+            best = k < best ? k : best;
+        }
+        if (lane == 0) {
+            out[row] = best == kEmptyKey ? -1 : (int32_t)key_index(best);
+        }
     }
 }
 
@@ -473,13 +720,47 @@ bool launch_resident_f32(const float *Q, int64_t nq, const float *B, int64_t nb,
         (!filter && (ldo % 4 != 0 || reinterpret_cast<uintptr_t>(out) % 16 != 0))) {
         return false;
     }
-    const Args a{Q, nq, B, nb, d, qn, bn, metric, out, ldo, flt, s};
+    const Args a{Q, nq, B, nb, d, qn, bn, metric, out, ldo, flt, nullptr, s};
     if (filter) {
-        launch_filter<true>(a);
+        launch_mode<kFilter>(a);
     } else {
-        launch_filter<false>(a);
+        launch_mode<kStore>(a);
     }
     return true;
+}
+
+bool resident_assign_serves(const float *X, const float *C, int d)
+{
+    return resident_f32_serves(d) && reinterpret_cast<uintptr_t>(X) % 16 == 0 && reinterpret_cast<uintptr_t>(C) % 16 == 0;
+}
+
+void launch_resident_assign(const float *X, int64_t n, const float *C, int64_t nc, int d, const float *xn, const float *cn, float cmax,
+                            int32_t *out, AssignWorkspace &ws, int64_t scratch_bytes, hipStream_t s)
+{
+    if (n <= 0) {
+        return;
+    }
+    IXA_REQUIRE(resident_assign_serves(X, C, d) && nc >= 1 && n < ((int64_t)1 << 31), kErrInner, "assignment kernel does not serve these operands");
+    const int qt = 32 * tile_blocks(nc, d);
+    const int64_t tiles = (nc + qt - 1) / qt;
+    // vectors per pass: 16 bytes per vector and tile of centroids, 20 for what is left open
+    const int64_t page = std::min<int64_t>(n, std::max<int64_t>(kTileRows, scratch_bytes / (16 * tiles + 20) / kTileRows * kTileRows));
+    ws.top.resize((size_t)(page * tiles));
+    ws.pairs.resize((size_t)page);
+    ws.rows.resize((size_t)page + 2);
+    int32_t *count = ws.rows.data() + page;
+    // (the bound of resident_f32.h for L2: 3 dp products, dp the dimension rounded up to 32)
+    const float u = 5.9604645e-8f;
+    const float err_scale = 2.0f * (3.0f / 262144.0f + (float)(d + 8) * u), round_scale = (float)(3 * ((d + 31) / 32 * 32) + 4) * u;
+    for (int64_t i0 = 0; i0 < n; i0 += page) {
+        const int64_t m = std::min(page, n - i0);
+        IXA_HIP(hipMemsetAsync(count, 0, 8, s));
+        launch_mode<kAssign>(Args{C, nc, X + i0 * d, m, d, cn, nullptr, kMetricL2, nullptr, 0, ScoreFilter<float>{}, ws.top.data(), s});
+        hipLaunchKernelGGL(assign_combine_kernel, dim3((unsigned)((m + 255) / 256)), dim3(256), 0, s, ws.top.data(), (int)tiles, qt, m,
+                           xn + i0, cmax, err_scale, round_scale, out + i0, ws.pairs.data(), ws.rows.data(), count);
+        hipLaunchKernelGGL(assign_resolve_kernel, dim3((unsigned)std::min<int64_t>(m, device_cus() * 2)), dim3(256), 0, s, X + i0 * d,
+                           xn + i0, m, C, cn, nc, d, cmax, err_scale, round_scale, ws.top.data(), (int)tiles, qt, ws.pairs.data(), ws.rows.data(), count, out + i0);
+    }
 }
 
 }  // namespace ixa

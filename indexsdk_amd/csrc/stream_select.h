@@ -47,7 +47,7 @@ struct SplitBase {
 int stream_select_f32_split(const float *Q, int64_t nq, const float *B, int64_t nb, int d, const float *qn, const float *bn,
                             int metric, int ncand, unsigned long long *running, StreamSelectWorkspace<float> &ws,
                             int64_t scratch_bytes, hipStream_t s, const SplitBase &split);
-// The same with the splits formed inside the score kernel (flat_resident.h says what it asks of the operands).  No mask.
+// The same with the splits formed inside the score kernel (resident_f32.h says what it asks of the operands).  No mask.
 int stream_select_f32_resident(const float *Q, int64_t nq, const float *B, int64_t nb, int d, const float *qn, const float *bn,
                                int metric, int ncand, unsigned long long *running, StreamSelectWorkspace<float> &ws,
                                int64_t scratch_bytes, hipStream_t s);

@@ -5,7 +5,7 @@
 #include <cmath>
 
 #include "flat_i8.h"
-#include "flat_resident.h"
+#include "resident_f32.h"
 #include "topk.h"
 
 namespace ixa {
@@ -186,7 +186,7 @@ struct F32SplitOps : F32Ops {
     }
 };
 
-// fp32 operands scored by the resident-query kernel, which splits the base rows on their way in (flat_resident.hip).
+// fp32 operands scored by the resident-query kernel, which splits the base rows on their way in (resident_f32.hip).
 // Stored scores cost their write and the selection's reading of them; a bound-filtered search costs a seed and three to six more
 // pairs of launches: 32M scores over 1M x 128 297 / 294 us, 64M 368 / 418, 128M 1037 / 447.  Seeds of 8192, 16384 and 32768 rows
 // and chunks of two to four times what has been seen are within 4 % of each other.

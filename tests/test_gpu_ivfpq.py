@@ -1019,3 +1019,35 @@ def test_odd_sub_quantizer_counts_scan_about_as_fast_as_their_neighbours(ix):
             times.append(gpu.last_search_stats()["ms_scan"])
         best[M] = min(times)
     assert best[33] < 2.0 * best[36], best
+
+
+# The assignment kernel (a tile of 256, 128, 64 or 32 centroids in LDS, the best two and the third value of each): remainders of
+# the dimension, of a tile of centroids or vectors, of a wavefront's 32; one centroid and two; centroids that tie exactly or within
+# the error bound, two and more of them, inside a tile and across tiles.
+@pytest.mark.parametrize("d,nlist,n", [(36, 2, 1), (64, 33, 257), (100, 255, 300), (128, 1, 5), (128, 257, 511), (200, 129, 1000),
+                                       (256, 513, 255), (384, 100, 600), (768, 70, 130), (1024, 33, 65), (128, 4100, 300),
+                                       (96, 2049, 5000)])
+def test_assignment_decides_every_tie_exactly(ix, oracle, d, nlist, n):
+    rng = np.random.default_rng(d + nlist)
+    cent = rng.standard_normal((nlist, d)).astype(np.float32)
+    if nlist >= 33:
+        cent[5] = cent[3]                                     # two equal, in one tile
+        cent[nlist - 1] = cent[10]                            # and in two
+        for i, c in enumerate((7, 8, 9, 20, nlist - 2, nlist // 2)):
+            cent[c] = cent[7] * np.float32(1 + i * 1e-7)      # six within the bound
+    x = (cent[rng.integers(0, nlist, n)] + 0.3 * rng.standard_normal((n, d))).astype(np.float32)
+    if nlist >= 33:
+        x[0:n:9] = cent[7] + np.float32(1e-3) * rng.standard_normal(x[0:n:9].shape).astype(np.float32)
+        x[1:n:9] = cent[3]
+        x[2:n:9] = cent[10]
+        x[4:n:9] = 0.5 * (cent[0] + cent[nlist - 3])          # halfway between two
+        x[5:n:9] = 0.0
+    book = rng.standard_normal((4, 256, d // 4)).astype(np.float32)
+    for scratch in (0, 1 << 20):                              # the second: in pages of vectors
+        cfg = ix.AscendIndexIVFPQConfig(**({"scratch_bytes": scratch} if scratch else {}))
+        gpu = ix.AscendIndexIVFPQ(d, ix.METRIC_L2, nlist, 4, 8, cfg)
+        gpu.set_trained(cent, book)
+        assert np.array_equal(gpu.assign(x), oracle.assign(x, cent))
+    x[0, 1] = np.nan
+    got = gpu.assign(x)
+    assert got[0] == -1 and np.array_equal(got[1:], oracle.assign(x[1:], cent))
