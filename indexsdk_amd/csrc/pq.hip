@@ -2,53 +2,266 @@
 // (FR/ascend/impl/AscendIndexIVFPQImpl.cpp:879-921: encodeSingleVectorPQ /
 // findCentroidInSubQuantizer / calDistance): the RAW vector is encoded (by_residual = false),
 // distance = sum (a-b)^2 accumulated left to right in fp32 without FMA, strict '<' so the first
-// minimum wins.  This is plain VALU work: the arithmetic order is the contract, so it is not
-// reshaped into a GEMM.
+// minimum wins.  That arithmetic decides every code; the matrix cores only say which 16 of a sub-quantizer's 256
+// codewords it has to be applied to.
 #include "pq.h"
 
 #include <algorithm>
 
+#include "resident_tile.h"
+
 namespace ixa {
 
-// One workgroup finds the codes of 256 vectors for ONE sub-quantizer (blockIdx.y): its 256 x dsub codeword
-// slab is staged in LDS and every lane walks all 256 codewords for its own vector (all lanes read the same
-// LDS address per step: a broadcast, no bank conflicts).  A small batch still fills the GPU this way: the
-// walk is a serial chain per lane, and 10000 vectors x 32 sub-quantizers are 1280 workgroups instead of 40.
-//
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef float v16f __attribute__((ext_vector_type(16)));
+
 // Sub-vector m of vector i starts at x + i * xi + m * xm, its code is codes[i * ci + m * cm].
 struct PqStrides {
     int64_t xi, xm, ci, cm;
 };
 
+constexpr float kPqFar = 3.402823466e+38f;   // a codeword at this distance or farther is never chosen
+
+// A workgroup of four wavefronts encodes one sub-quantizer of a block of vectors, 32 vectors of a wavefront at a time.
+//   1. u = x.c - |c|^2 / 2 of 32 vectors and all 256 codewords on the bf16 matrix cores.  Vectors and codewords are split into
+//      hi + lo (x = hi + lo + rest, |rest| <= 2^-18 |x|) and laid side by side in K: [hi | hi | lo | 1 1 1] against
+//      [hi | lo | hi | the three parts of -|c|^2 / 2], so up to four dimensions are ONE matrix instruction per 32 codewords.
+//      The codewords' fragments are made once per workgroup and stay in registers (in LDS above eight dimensions).
+//   2. A lane owns one vector and 16 codewords of each block of 32 (the other half of the wavefront the others): it keeps the
+//      largest u of every 16, the best 16 and the runner-up, then the two halves compare.
+//   3. The winning 16 are decided by the reference's arithmetic, eight by either half.  Where the runner-up is within the error
+//      bound, the wavefront evaluates all 256 codewords of that vector.
+// Per 32 vectors: KS matrix instructions and a maximum over 16 per block, and 16 distances, where every lane walking 256
+// codewords for its own vector took 256 of them: 20000 x 32 sub-quantizers of 4 dimensions 55 -> 20 us,
+//   131072 x 32 280 -> 70, 20000 x 4 of 32 dimensions 75 -> 34.
+//   The bound: distances decide by |x|^2 - 2 u, so a lead of u decides when twice it exceeds the errors of both sides:
+//   a u misses at most 3 x 2^-18 |x||c| and its K + dsub sums (2^-24 of at most |x||c| + |c|^2 / 2 each), a canonical
+//   distance (dsub + 2) 2^-24 of itself, at most (|x| + |c|)^2.  Lengths below 1e-15, where products may vanish, decide nothing.
 template <int DSUB>
-__global__ __launch_bounds__(256) void pq_encode_kernel(const float *__restrict__ x, int64_t n, PqStrides st,
-                                                        const float *__restrict__ codebook,
-                                                        uint8_t *__restrict__ codes)
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DSUB > 24 ? 1 : 2))) void pq_encode_kernel(const float *__restrict__ x, int64_t n, PqStrides st, int M,
+                                                        const float *__restrict__ codebook, uint8_t *__restrict__ codes,
+                                                        int64_t per_block)
 {
-    __shared__ float cb[256 * DSUB];
-    const int tid = threadIdx.x;
-    const int m = blockIdx.y;
-    const int64_t i = (int64_t)blockIdx.x * 256 + tid;
-    const float *src = codebook + (int64_t)m * 256 * DSUB;
-    for (int e = tid; e < 256 * DSUB; e += 256) {
-        cb[e] = src[e];
+    constexpr int K = 3 * DSUB + 3, KS = (K + 15) / 16;
+    constexpr bool kInRegisters = KS <= 2;
+    __shared__ __align__(16) float cb[256 * DSUB];
+    __shared__ __align__(16) bf16x8 frag[8][KS][64];   // [block of 32 codewords][K-step][lane]
+    __shared__ float wave_max[4];
+    const int tid = threadIdx.x, lane = tid & 63, half = lane >> 5, l32 = lane & 31;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    // the sub-quantizers of a block of vectors run on one XCD, whose L2 then has the lines their sub-vectors share
+    const int64_t vb = (blockIdx.x >> 3) / M * 8 + (blockIdx.x & 7), i_first = vb * per_block;
+    const int m = (blockIdx.x >> 3) % M;
+    if (i_first >= n) {
+        return;
     }
-    __syncthreads();
-    if (i < n) {
-        float sub[DSUB];
+    const int64_t i_end = i_first + per_block < n ? i_first + per_block : n;
+    // element `slot` of K for a vector (hi, hi, lo, ones) or codeword (hi, lo, hi, parts of the norm)
+    auto slot_of = [](int slot, const __bf16 *first, const __bf16 *second, const __bf16 *third, const __bf16 *tail) {
+        return slot < DSUB ? first[slot] : (slot < 2 * DSUB ? second[slot - DSUB]
+               : (slot < 3 * DSUB ? third[slot - 2 * DSUB] : (slot < K ? tail[slot - 3 * DSUB] : (__bf16)0.f)));
+    };
+    {
+        const float *src = codebook + ((int64_t)m * 256 + tid) * DSUB;
+        __bf16 hi[DSUB], lo[DSUB], part[3];
+        float sq = 0.f;
 #pragma unroll
         for (int t = 0; t < DSUB; t++) {
-            sub[t] = x[i * st.xi + m * st.xm + t];
+            const float c = src[t];
+            cb[tid * DSUB + t] = c;
+            sq += c * c;
+            hi[t] = (__bf16)c;
+            lo[t] = (__bf16)(c - (float)hi[t]);
         }
-        float best = 3.402823466e+38f;
+        float rest = -0.5f * sq;
+#pragma unroll
+        for (int t = 0; t < 3; t++) {
+            part[t] = (__bf16)rest;
+            rest -= (float)part[t];
+        }
+#pragma unroll
+        for (int ks = 0; ks < KS; ks++) {
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                bf16x8 f;
+#pragma unroll
+                for (int t = 0; t < 8; t++) {
+                    f[t] = slot_of(ks * 16 + h * 8 + t, hi, lo, hi, part);
+                }
+                frag[tid >> 5][ks][h * 32 + (tid & 31)] = f;
+            }
+        }
+        for (int o = 32; o > 0; o >>= 1) {
+            sq = fmaxf(sq, __shfl_xor(sq, o));
+        }
+        if (lane == 0) {
+            wave_max[wave] = sq;
+        }
+    }
+    __syncthreads();
+    const float cmax = sqrtf(fmaxf(fmaxf(wave_max[0], wave_max[1]), fmaxf(wave_max[2], wave_max[3])));
+    bf16x8 own[kInRegisters ? 8 : 1][KS];
+    if constexpr (kInRegisters) {
+#pragma unroll
+        for (int b = 0; b < 8; b++) {
+#pragma unroll
+            for (int ks = 0; ks < KS; ks++) {
+                own[b][ks] = frag[b][ks][lane];
+            }
+        }
+    }
+    const float *xm = x + m * st.xm;
+    float next[DSUB];
+    auto fetch = [&](int64_t i0) {
+        const float *src = xm + (i0 + l32 < n ? i0 + l32 : n - 1) * st.xi;
+#pragma unroll
+        for (int t = 0; t < DSUB; t++) {
+            next[t] = src[t];
+        }
+    };
+    fetch(i_first + wave * 32);
+    for (int64_t i0 = i_first + wave * 32; i0 < i_end; i0 += 128) {
+        float sub[DSUB];
+        __bf16 hi[DSUB], lo[DSUB];
+        const __bf16 ones[3] = {(__bf16)1.f, (__bf16)1.f, (__bf16)1.f};
+        float sq = 0.f;
+#pragma unroll
+        for (int t = 0; t < DSUB; t++) {
+            sub[t] = next[t];
+            sq += sub[t] * sub[t];
+            hi[t] = (__bf16)sub[t];
+            lo[t] = (__bf16)(sub[t] - (float)hi[t]);
+        }
+        fetch(i0 + 128);
+        bf16x8 vec[KS];
+#pragma unroll
+        for (int ks = 0; ks < KS; ks++) {
+            bf16x8 f0, f1;
+#pragma unroll
+            for (int t = 0; t < 8; t++) {
+                f0[t] = slot_of(ks * 16 + t, hi, hi, lo, ones);
+                f1[t] = slot_of(ks * 16 + 8 + t, hi, hi, lo, ones);
+            }
+            vec[ks] = half ? f1 : f0;
+        }
+        // the largest u of the lane's 16 codewords of each block: the best, its block, and the next
+        float m1 = -kPqFar, m2 = -kPqFar;
+        int blk = 0;
+#pragma unroll
+        for (int b = 0; b < 8; b++) {
+            if constexpr (!kInRegisters) {
+                asm volatile("" ::: "memory");   // the fragments stay in LDS
+            }
+            v16f acc{};
+#pragma unroll
+            for (int ks = 0; ks < KS; ks++) {
+                acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kInRegisters ? own[kInRegisters ? b : 0][ks] : frag[b][ks][lane], vec[ks],
+                                                              acc, 0, 0, 0);
+            }
+            float top = acc[0];
+#pragma unroll
+            for (int r = 1; r < 16; r++) {
+                top = fmaxf(top, acc[r]);
+            }
+            m2 = __builtin_amdgcn_fmed3f(m1, m2, top);
+            blk = top > m1 ? b : blk;
+            m1 = fmaxf(m1, top);
+        }
+        const float o1 = __shfl_xor(m1, 32), o2 = __shfl_xor(m2, 32);
+        const int oblk = __shfl_xor(blk, 32);
+        const float len = sqrtf(sq), mag = len * cmax + 0.5f * cmax * cmax, far = len + cmax;
+        const float need = 2.f * (3.f / 262144.f * len * cmax + (float)(K + DSUB + 4) * 5.9604645e-8f * mag) +
+                           (float)(DSUB + 4) * 5.9604645e-8f * far * far;
+        // (an undefined or infinite bound decides nothing)
+        const bool decided = fmaxf(m1, o1) - fmaxf(fminf(m1, o1), fmaxf(m2, o2)) > need && far > 1e-15f;
+        const bool mine = m1 > o1;
+        const int first = (mine ? blk : oblk) * 32 + (mine ? half : 1 - half) * 4;   // the 16: first + 8 g + t, t < 4
+        float best = kPqFar;
+        int arg = 0;
+#pragma unroll
+        for (int g = 0; g < 2; g++) {
+#pragma unroll
+            for (int t = 0; t < 4; t++) {
+                const int k = first + 8 * (2 * half + g) + t;
+                float dist = 0.f;
+#pragma unroll
+                for (int j = 0; j < DSUB; j++) {
+                    const float diff = __fsub_rn(sub[j], cb[k * DSUB + j]);
+                    dist = __fadd_rn(dist, __fmul_rn(diff, diff));
+                }
+                if (dist < best) {
+                    best = dist;
+                    arg = k;
+                }
+            }
+        }
+        {   // the other half's eight; of equal distances the smaller codeword (half 0 has those)
+            const float ob = __shfl_xor(best, 32);
+            const int oa = __shfl_xor(arg, 32);
+            arg = ob < best || (ob == best && half == 1) ? oa : arg;
+        }
+        unsigned long long open = __ballot(!decided && half == 0 && i0 + l32 < i_end);
+        for (; open != 0; open &= open - 1) {
+            const int v = __builtin_ctzll(open);
+            float near = kPqFar;
+            int at = 0;
+            float one[DSUB];
+#pragma unroll
+            for (int j = 0; j < DSUB; j++) {
+                one[j] = __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(sub[j]), v));
+            }
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                const int k = q * 64 + lane;
+                float dist = 0.f;
+#pragma unroll
+                for (int j = 0; j < DSUB; j++) {
+                    const float diff = __fsub_rn(one[j], cb[k * DSUB + j]);
+                    dist = __fadd_rn(dist, __fmul_rn(diff, diff));
+                }
+                if (dist < near) {
+                    near = dist;
+                    at = k;
+                }
+            }
+            float least = near;
+            for (int o = 32; o > 0; o >>= 1) {
+                least = fminf(least, __shfl_xor(least, o));
+            }
+            int low = near == least ? at : 256;
+            if (__popcll(__ballot(near == least)) > 1) {
+                for (int o = 32; o > 0; o >>= 1) {
+                    const int other = __shfl_xor(low, o);
+                    low = other < low ? other : low;
+                }
+            } else {
+                low = __builtin_amdgcn_readlane(low, __builtin_ctzll(__ballot(near == least)));
+            }
+            arg = l32 == v ? low : arg;
+        }
+        if (half == 0 && i0 + l32 < i_end) {
+            codes[(i0 + l32) * st.ci + m * st.cm] = (uint8_t)arg;
+        }
+    }
+}
+
+// One dimension: a lane walks the 256 codewords for its own vector (three instructions each; 3000 x 64 sub-quantizers 12 us,
+// with the kernel above 27).
+__global__ __launch_bounds__(256) void pq_encode_scalar_kernel(const float *__restrict__ x, int64_t n, PqStrides st,
+                                                               const float *__restrict__ codebook, uint8_t *__restrict__ codes)
+{
+    __shared__ float cb[256];
+    const int m = blockIdx.y;
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    cb[threadIdx.x] = codebook[(int64_t)m * 256 + threadIdx.x];
+    __syncthreads();
+    if (i < n) {
+        const float v = x[i * st.xi + m * st.xm];
+        float best = kPqFar;
         int arg = 0;
         for (int k = 0; k < 256; k++) {
-            float dist = 0.f;
-#pragma unroll
-            for (int t = 0; t < DSUB; t++) {
-                float diff = __fsub_rn(sub[t], cb[k * DSUB + t]);
-                dist = __fadd_rn(dist, __fmul_rn(diff, diff));
-            }
+            const float diff = __fsub_rn(v, cb[k]);
+            const float dist = __fmul_rn(diff, diff);
             if (dist < best) {
                 best = dist;
                 arg = k;
@@ -95,12 +308,18 @@ void launch_encode(const float *x, int64_t n, int M, int dsub, PqStrides st, con
         return;
     }
     dim3 grid((unsigned)((n + 255) / 256), (unsigned)M), block(256);
+    // vectors per workgroup: 2048 (16 per wavefront and codeword fragment made), fewer while that leaves CUs without four
+    const int64_t per_block = std::min<int64_t>(2048, std::max<int64_t>(128, round_up(n * M / (4 * device_cus()), 128)));
+    const int64_t blocks = round_up((n + per_block - 1) / per_block, 8) * M;
+    IXA_REQUIRE(blocks < (int64_t)1 << 31, kErrInvalidParam, "encode grid too large");
 #define IXA_ENC(D)                                                                                             \
     case D:                                                                                                    \
-        hipLaunchKernelGGL(pq_encode_kernel<D>, grid, block, 0, s, x, n, st, codebook, codes);                \
+        hipLaunchKernelGGL(pq_encode_kernel<D>, dim3((unsigned)blocks), block, 0, s, x, n, st, M, codebook, codes, per_block); \
         break;
     switch (dsub) {
-        IXA_ENC(1)
+    case 1:
+        hipLaunchKernelGGL(pq_encode_scalar_kernel, grid, block, 0, s, x, n, st, codebook, codes);
+        break;
         IXA_ENC(2)
         IXA_ENC(3)
         IXA_ENC(4)

@@ -84,3 +84,39 @@ def test_sub_quantizers_trained_in_groups_equal_those_trained_together(d, M, n):
         gpu.train(x)
         books.append(gpu.get_trained()[1])
     assert np.array_equal(books[0].view(np.uint32), books[1].view(np.uint32))
+
+
+# The encoder finds a vector's 16 candidate codewords on the matrix cores and decides among them in the reference's arithmetic:
+# codewords that tie exactly or within the error bound (the first one wins), in one group of 16 and in several, undefined and
+# infinite values (codeword 0), lengths at both ends of the range, remainders of the 32 vectors of a wavefront.
+@pytest.mark.parametrize("dsub", [1, 2, 3, 4, 5, 6, 7, 8, 10, 12, 16, 24, 32])
+@pytest.mark.parametrize("n,scale", [(1, 1.0), (33, 1.0), (2600, 1.0), (257, 1e-12), (257, 1e-16), (257, 1e-30), (257, 1e17)])
+def test_codes_are_the_first_nearest_codewords(oracle, dsub, n, scale):
+    import indexsdk_amd as ix
+
+    rng = np.random.default_rng(dsub + n)
+    m = 3 if n > 1000 else 9
+    d = m * dsub
+    book = (scale * rng.standard_normal((m, 256, dsub))).astype(np.float32)
+    book[0, 7] = book[0, 3]
+    book[1, 200] = book[1, 100]
+    book[2, 5:40] = book[2, 4]
+    for i in range(30, 60):
+        book[0, i] = book[0, 30] * np.float32(1 + (i % 7) * 1e-7)
+    x = (scale * rng.standard_normal((n, d))).astype(np.float32)
+    picked = np.concatenate([book[j][rng.integers(0, 256, n)] for j in range(m)], axis=1)
+    x[::3] = picked[::3]
+    x[1::7] = 0.5 * (picked[1::7] + np.roll(picked, 1, axis=0)[1::7])
+    x[2::11] = 0.0
+    if n > 40:
+        x[20, 0] = np.nan
+        x[21, d - 1] = np.inf
+        x[22, 0] = -np.inf
+    cent = rng.standard_normal((2, d)).astype(np.float32)
+    index = ix.AscendIndexIVFPQ(d, ix.METRIC_L2, 2, m, 8)
+    index.set_trained(cent, book)
+    assert np.array_equal(index.encode(x), oracle.pq_encode(x, book))
+    book[0, 9, 0] = np.nan
+    book[1, 17, 0] = np.inf
+    index.set_trained(cent, book)
+    assert np.array_equal(index.encode(x), oracle.pq_encode(x, book))
