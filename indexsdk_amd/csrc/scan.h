@@ -40,6 +40,7 @@ struct ScanParams {
     const int32_t *order;      // optional permutation of the queries (execution order), may be null
     int xcd_chunks;            // 1: deal contiguous chunks of the execution order to the 8 XCDs
     int64_t nq;                // filled by launch_scan()
+    int by_groups;             // 1: a split query is divided by groups of codes, 0: by lists (filled by launch_scan())
     // filled by plan_scan()
     int waves, shared_pool, cap, merge_n, table_n, off_query, off_pools, off_merge, off_table, off_hist, off_misc;
 };

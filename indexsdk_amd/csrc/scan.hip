@@ -127,7 +127,7 @@ __global__ __launch_bounds__(W * 64, (LAYOUT == 1 && sizeof(LutT) == 2 && !SHARE
     ScanParams p)
 {
     extern __shared__ __align__(16) unsigned char smem_raw[];
-    constexpr int NT = W * 64;
+    constexpr int NT = W * 64, kWavesLog2 = W == 16 ? 4 : (W == 8 ? 3 : 2);
     const int M = MT > 0 ? MT : p.M;
     LutT *lut = reinterpret_cast<LutT *>(smem_raw);
     float *qs = reinterpret_cast<float *>(smem_raw + p.off_query);
@@ -156,8 +156,9 @@ __global__ __launch_bounds__(W * 64, (LAYOUT == 1 && sizeof(LutT) == 2 && !SHARE
     const int64_t q = p.order ? p.order[qslot] : qslot;
     const int split = blockIdx.x % p.nsplit;
 
-    // ---- list table of this workgroup: local list i = probe rank split + i * nsplit
-    const int nlocal = (p.nprobe - split + p.nsplit - 1) / p.nsplit;
+    // ---- list table of this workgroup: local list i = probe rank first + i * step
+    const int list_first = p.by_groups ? 0 : split, list_step = p.by_groups ? 1 : p.nsplit;
+    const int nlocal = (p.nprobe - list_first + list_step - 1) / list_step;
     for (int j = tid; j < p.d; j += NT) {
         qs[j] = p.queries[q * p.d + j];
     }
@@ -165,7 +166,7 @@ __global__ __launch_bounds__(W * 64, (LAYOUT == 1 && sizeof(LutT) == 2 && !SHARE
         share[tid] = __builtin_inff();
     }
     for (int i = tid; i < nlocal; i += NT) {
-        const int l = p.probes[q * p.nprobe + split + i * p.nsplit];
+        const int l = p.probes[q * p.nprobe + list_first + i * list_step];
         const bool has = (uint32_t)l < (uint32_t)p.nlist;   // anything else is "no list", whatever the caller left there
         const int len = has ? p.list_len[l] : 0;
         t_len[i] = len;
@@ -340,16 +341,35 @@ __global__ __launch_bounds__(W * 64, (LAYOUT == 1 && sizeof(LutT) == 2 && !SHARE
         pool.init(pools + wave * p.cap, p.cap, p.k);
     }
     const int l32 = lane & 31;
-    const int total = nlocal > 0 ? __builtin_amdgcn_readfirstlane(t_gend[nlocal - 1]) : 0;
+    // A query split by groups: its slices take the groups of ALL its lists in turn, W at a time.  The wavefront counts its own
+    // groups as G = wave, wave + W, ...; group G of the sequence is G plus what the other slices take in between.
+    const int all_groups = nlocal > 0 ? __builtin_amdgcn_readfirstlane(t_gend[nlocal - 1]) : 0;
+    // (Workgroups of sixteen wavefronts are not divided so: their kernels have no registers to spare for it.)
+    constexpr bool kByGroups = W < 16;
+    const int g_first = kByGroups && p.by_groups ? split * W : 0, g_skip = kByGroups && p.by_groups ? (p.nsplit - 1) * W : 0;
+    // one past the last of the wavefront's own count
+    const int total = g_skip == 0 ? all_groups
+                                  : (all_groups > g_first + wave ? wave + ((all_groups - g_first - wave - 1) / (g_skip + W) + 1) * W : 0);
     int li = 0;          // list the current group belongs to (monotone, wave-uniform)
     int gstart = 0;      // first group of that list
     int gend = nlocal > 0 ? __builtin_amdgcn_readfirstlane(t_gend[0]) : 0;
 
-    auto locate = [&](int G) -> GroupRef {
+    auto locate = [&](int own) -> GroupRef {
+        const int G = kByGroups ? own + g_first + (own >> kWavesLog2) * g_skip : own;
         while (G >= gend) {
-            gstart = gend;
-            li++;
-            gend = __builtin_amdgcn_readfirstlane(t_gend[li]);
+            if (!kByGroups || g_skip == 0) {   // the next list, or the one behind it
+                gstart = gend;
+                li++;
+                gend = __builtin_amdgcn_readfirstlane(t_gend[li]);
+            } else {   // lists are skipped: the first of the next 64 that ends behind G
+                const int at = li + 1 + lane;
+                const int ends = t_gend[at < nlocal ? at : nlocal - 1];
+                const unsigned long long behind = __ballot(ends > G);
+                const int hop = behind ? __builtin_ctzll(behind) : 63;
+                gstart = hop ? __builtin_amdgcn_readlane(ends, hop - 1) : gend;
+                gend = __builtin_amdgcn_readlane(ends, hop);
+                li += 1 + hop;
+            }
         }
         const int pos = ((G - gstart) << 6) + lane;
         GroupRef r;
@@ -1278,7 +1298,7 @@ static size_t plan_with_waves(ScanParams &p, int waves, bool shared)
     p.shared_pool = shared ? 1 : 0;
     p.cap = shared ? block_pool_capacity(p.k, waves) : wave_pool_capacity(p.k);
     p.merge_n = shared ? p.cap : waves * p.cap;
-    p.table_n = (p.nprobe + p.nsplit - 1) / p.nsplit;
+    p.table_n = p.by_groups ? p.nprobe : (p.nprobe + p.nsplit - 1) / p.nsplit;
     size_t off = round_up((int64_t)lut_bytes, 16);
     p.off_query = (int)off;
     off += round_up((int64_t)p.d * 4, 16);
@@ -1390,13 +1410,22 @@ size_t scan_lds_plan(int d, int M, int lut_fp16, int code_layout, int nprobe, in
     return smem;
 }
 
+// How a query that is split over workgroups is divided: by groups of 64 codes, every slice taking its share of every list, up
+// to this many lists (their table is 12 bytes of LDS each); by whole lists above.
+constexpr int kSplitGroupsMaxLists = 512;
+
 void launch_scan(ScanParams p, int64_t nq, hipStream_t s)
 {
     if (nq == 0) {
         return;
     }
     p.nq = nq;
-    const size_t smem = plan_scan(p);
+    p.by_groups = p.nsplit > 1 && p.nprobe <= kSplitGroupsMaxLists ? 1 : 0;
+    size_t smem = plan_scan(p);
+    if (p.by_groups && (smem > 160 * 1024 || p.waves == 16)) {   // (the longer list table may be what no longer fits)
+        p.by_groups = 0;
+        smem = plan_scan(p);
+    }
     IXA_REQUIRE(smem <= 160 * 1024, kErrInvalidParam,
                 "IVFPQ scan needs at least %zu bytes of LDS (M=%d, k=%d, %s LUT); the limit is 163840", smem, p.M, p.k,
                 p.lut_fp16 ? "fp16" : "fp32");
