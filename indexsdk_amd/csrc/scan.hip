@@ -120,11 +120,14 @@ __device__ __forceinline__ uint32_t byte_times_pow2(uint32_t w, int j)
 // The same holds for private pools of short rows: at M 4 and 8 the allocator left alone took 65 with the sort of the epilogue
 // inlined, one more than four workgroups of eight wavefronts have.
 template <int MT, typename LutT, int LAYOUT, int W, bool SHARED>
-__global__ __launch_bounds__(W * 64, (LAYOUT == 1 && sizeof(LutT) == 2 && !SHARED) ? 4
-                                     : (SHARED && W == 8 && MT > 0 && MT <= 8)    ? 8
-                                     : (!SHARED && LAYOUT == 0 && MT > 0 && MT <= 32) ? 8
-                                                                                      : 1) void ivfpq_scan_kernel(
-    ScanParams p)
+constexpr int kScanWavesPerSimd = (LAYOUT == 1 && sizeof(LutT) == 2 && !SHARED) ? 4
+                                  : (SHARED && W == 8 && MT > 0 && MT <= 8)    ? 8
+                                  : (!SHARED && LAYOUT == 0 && MT > 0 && MT <= 32) ? 8
+                                                                                   : 1;
+
+// BY_GROUPS: the query is split over workgroups by groups of codes (below); otherwise by lists, or not at all.
+template <int MT, typename LutT, int LAYOUT, int W, bool SHARED, bool BY_GROUPS>
+__device__ __forceinline__ void scan_body(const ScanParams &p)
 {
     extern __shared__ __align__(16) unsigned char smem_raw[];
     constexpr int NT = W * 64, kWavesLog2 = W == 16 ? 4 : (W == 8 ? 3 : 2);
@@ -157,7 +160,7 @@ __global__ __launch_bounds__(W * 64, (LAYOUT == 1 && sizeof(LutT) == 2 && !SHARE
     const int split = blockIdx.x % p.nsplit;
 
     // ---- list table of this workgroup: local list i = probe rank first + i * step
-    const int list_first = p.by_groups ? 0 : split, list_step = p.by_groups ? 1 : p.nsplit;
+    const int list_first = BY_GROUPS ? 0 : split, list_step = BY_GROUPS ? 1 : p.nsplit;
     const int nlocal = (p.nprobe - list_first + list_step - 1) / list_step;
     for (int j = tid; j < p.d; j += NT) {
         qs[j] = p.queries[q * p.d + j];
@@ -344,24 +347,20 @@ __global__ __launch_bounds__(W * 64, (LAYOUT == 1 && sizeof(LutT) == 2 && !SHARE
     // A query split by groups: its slices take the groups of ALL its lists in turn, W at a time.  The wavefront counts its own
     // groups as G = wave, wave + W, ...; group G of the sequence is G plus what the other slices take in between.
     const int all_groups = nlocal > 0 ? __builtin_amdgcn_readfirstlane(t_gend[nlocal - 1]) : 0;
-    // (Workgroups of sixteen wavefronts are not divided so: their kernels have no registers to spare for it.)
-    constexpr bool kByGroups = W < 16;
-    const int g_first = kByGroups && p.by_groups ? split * W : 0, g_skip = kByGroups && p.by_groups ? (p.nsplit - 1) * W : 0;
-    // one past the last of the wavefront's own count
-    const int total = g_skip == 0 ? all_groups
-                                  : (all_groups > g_first + wave ? wave + ((all_groups - g_first - wave - 1) / (g_skip + W) + 1) * W : 0);
+    int g_first = 0, g_skip = 0, total = all_groups;   // total: one past the last of the wavefront's own count
+    if constexpr (BY_GROUPS) {
+        g_first = split * W;
+        g_skip = (p.nsplit - 1) * W;
+        total = all_groups > g_first + wave ? wave + ((all_groups - g_first - wave - 1) / (g_skip + W) + 1) * W : 0;
+    }
     int li = 0;          // list the current group belongs to (monotone, wave-uniform)
     int gstart = 0;      // first group of that list
     int gend = nlocal > 0 ? __builtin_amdgcn_readfirstlane(t_gend[0]) : 0;
 
     auto locate = [&](int own) -> GroupRef {
-        const int G = kByGroups ? own + g_first + (own >> kWavesLog2) * g_skip : own;
+        const int G = BY_GROUPS ? own + g_first + (own >> kWavesLog2) * g_skip : own;
         while (G >= gend) {
-            if (!kByGroups || g_skip == 0) {   // the next list, or the one behind it
-                gstart = gend;
-                li++;
-                gend = __builtin_amdgcn_readfirstlane(t_gend[li]);
-            } else {   // lists are skipped: the first of the next 64 that ends behind G
+            if constexpr (BY_GROUPS) {   // lists are skipped: the first of the next 64 that ends behind G
                 const int at = li + 1 + lane;
                 const int ends = t_gend[at < nlocal ? at : nlocal - 1];
                 const unsigned long long behind = __ballot(ends > G);
@@ -369,6 +368,10 @@ __global__ __launch_bounds__(W * 64, (LAYOUT == 1 && sizeof(LutT) == 2 && !SHARE
                 gstart = hop ? __builtin_amdgcn_readlane(ends, hop - 1) : gend;
                 gend = __builtin_amdgcn_readlane(ends, hop);
                 li += 1 + hop;
+            } else {
+                gstart = gend;
+                li++;
+                gend = __builtin_amdgcn_readfirstlane(t_gend[li]);
             }
         }
         const int pos = ((G - gstart) << 6) + lane;
@@ -748,6 +751,19 @@ __global__ __launch_bounds__(W * 64, (LAYOUT == 1 && sizeof(LutT) == 2 && !SHARE
         p.out_dist[q * p.k + i] = ok ? (p.metric == kMetricL2 ? v : -v) : pad;
         p.out_labels[q * p.k + i] = ok ? p.ids[key_index(kk)] : -1;
     }
+}
+
+template <int MT, typename LutT, int LAYOUT, int W, bool SHARED>
+__global__ __launch_bounds__(W * 64, (kScanWavesPerSimd<MT, LutT, LAYOUT, W, SHARED>)) void ivfpq_scan_kernel(ScanParams p)
+{
+    scan_body<MT, LutT, LAYOUT, W, SHARED, false>(p);
+}
+
+// (a kernel of its own: in the one above the other way of counting groups cost 2 % of 1000 queries over 16 lists of 390 codes)
+template <int MT, typename LutT, int LAYOUT, bool SHARED>
+__global__ __launch_bounds__(512, (kScanWavesPerSimd<MT, LutT, LAYOUT, 8, SHARED>)) void ivfpq_scan_groups_kernel(ScanParams p)
+{
+    scan_body<MT, LutT, LAYOUT, 8, SHARED, true>(p);
 }
 
 // Merges the nsplit sorted partial lists of a query (tile merge, the role of op TopkIvfpqL3).
@@ -1220,8 +1236,13 @@ template <int MT, typename LutT, int LAYOUT>
 static void launch_one(const ScanParams &p, int64_t nq, size_t smem, hipStream_t s)
 {
     const int64_t slots = p.xcd_chunks ? (nq + 7) / 8 * 8 : nq;
-    static std::atomic<bool> lds_checked[4] = {{false}, {false}, {false}, {false}};
-    if (p.shared_pool && p.waves == 16) {
+    static std::atomic<bool> lds_checked[6] = {{false}, {false}, {false}, {false}, {false}, {false}};
+    if (p.by_groups) {
+        auto kern = p.shared_pool ? ivfpq_scan_groups_kernel<MT, LutT, LAYOUT, true> : ivfpq_scan_groups_kernel<MT, LutT, LAYOUT, false>;
+        require_no_static_lds(reinterpret_cast<const void *>(kern), lds_checked[p.shared_pool ? 4 : 5]);
+        require_dynamic_lds(reinterpret_cast<const void *>(kern), smem);
+        hipLaunchKernelGGL(kern, dim3((unsigned)(slots * p.nsplit)), dim3(512), smem, s, p);
+    } else if (p.shared_pool && p.waves == 16) {
         auto kern = ivfpq_scan_kernel<MT, LutT, LAYOUT, 16, true>;
         require_no_static_lds(reinterpret_cast<const void *>(kern), lds_checked[0]);
         require_dynamic_lds(reinterpret_cast<const void *>(kern), smem);
@@ -1411,7 +1432,8 @@ size_t scan_lds_plan(int d, int M, int lut_fp16, int code_layout, int nprobe, in
 }
 
 // How a query that is split over workgroups is divided: by groups of 64 codes, every slice taking its share of every list, up
-// to this many lists (their table is 12 bytes of LDS each); by whole lists above.
+// to this many lists (their table is 12 bytes of LDS each); by whole lists above, and by workgroups of four or sixteen wavefronts
+// (plans for LUTs and pools of the largest sizes; with sixteen the way of counting spills).
 constexpr int kSplitGroupsMaxLists = 512;
 
 void launch_scan(ScanParams p, int64_t nq, hipStream_t s)
@@ -1422,7 +1444,7 @@ void launch_scan(ScanParams p, int64_t nq, hipStream_t s)
     p.nq = nq;
     p.by_groups = p.nsplit > 1 && p.nprobe <= kSplitGroupsMaxLists ? 1 : 0;
     size_t smem = plan_scan(p);
-    if (p.by_groups && (smem > 160 * 1024 || p.waves == 16)) {   // (the longer list table may be what no longer fits)
+    if (p.by_groups && (smem > 160 * 1024 || p.waves != 8)) {   // (the longer list table may be what no longer fits)
         p.by_groups = 0;
         smem = plan_scan(p);
     }
