@@ -183,6 +183,11 @@ void launch_refine_boundary(const float *Q, int64_t nq, const float *C, int d, c
 // Canonical scores of all nc centroids for every row (one lane per score; the exact plan of last resort).
 void launch_canonical_scores(const float *Q, int64_t nq, const float *C, int64_t nc, int d, const float *qn,
                              const float *cn, int metric, float *out, int64_t ldo, hipStream_t s);
+// out_ids[nq][nout] = the lists with the smallest canonical scores, best first (-1 where fewer have one), in one launch without a
+// score matrix.  Q: device memory, or page-locked host memory whose rows are then left in `copy` (device, may be null).
+bool nearest_lists_serves(const float *Q, int64_t nq, const float *C, int64_t nc, int d, int nout);
+void launch_nearest_lists(const float *Q, int64_t nq, const float *C, int64_t nc, int d, const float *cn, int metric, int nout,
+                          int32_t *out_ids, float *copy, hipStream_t s);
 // dist[n][k] = public distances of the columns idx[n][k] of a score matrix (-1 -> +-FLT_MAX).
 void launch_gather_scores(const float *scores, int64_t ld, const int32_t *idx, int64_t n, int k, int metric, float *dist,
                           hipStream_t s);

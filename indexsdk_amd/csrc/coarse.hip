@@ -1887,6 +1887,120 @@ void launch_canonical_scores(const float *Q, int64_t nq, const float *C, int64_t
     }
 }
 
+// The nout nearest lists of a small batch in ONE launch, where a quantizer has at most as many lists as a workgroup threads: a
+// thread scores one centroid against QB queries in the arithmetic above (the queries in LDS, a centroid read once for all of
+// them), and the workgroup sorts each query's keys.  Scores that never leave the chip, and one launch where
+// canonical_scores_kernel, which reads every centroid once per query, and a selection from its matrix are two.  What bounds it: the
+// round trips to L2 for a centroid's row, the chain of d additions, the sort (1024 keys).
+// Q may be page-locked host memory: every row is read once, and written to `copy` (may be null) for the kernels that follow.
+template <int NT, int QB>
+__global__ __launch_bounds__(NT) void nearest_lists_kernel(const float *__restrict__ Q, int64_t nq, const float *__restrict__ C,
+                                                           int nc, int d, const float *__restrict__ cn, int metric, int nout,
+                                                           int32_t *__restrict__ out_ids, float *__restrict__ copy)
+{
+    __shared__ __align__(16) key_t keys[(NT < 512 ? 512 : NT) + 2];
+    __shared__ float norm[QB];
+    extern __shared__ __align__(16) float qs[];   // [QB][d]
+    const int tid = threadIdx.x;
+    const int64_t q0 = (int64_t)blockIdx.x * QB;
+    for (int e = tid * 4; e < QB * d; e += NT * 4) {
+        const int64_t row = q0 + e / d;
+        float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (row < nq) {   // d % 4 == 0: the four belong to one row
+            v = *reinterpret_cast<const float4 *>(Q + q0 * d + e);
+            if (copy) {
+                *reinterpret_cast<float4 *>(copy + q0 * d + e) = v;
+            }
+        }
+        *reinterpret_cast<float4 *>(qs + e) = v;
+    }
+    __syncthreads();
+    if (metric == kMetricL2 && (tid & 63) == 0 && (tid >> 6) < QB) {   // left to right, as sqnorm_rows_kernel
+        const float *q = qs + (tid >> 6) * d;
+        float sum = 0.f;
+#pragma unroll 4
+        for (int t = 0; t < d; t += 4) {
+            const float4 a = *reinterpret_cast<const float4 *>(q + t);
+            sum = __fadd_rn(sum, __fmul_rn(a.x, a.x));
+            sum = __fadd_rn(sum, __fmul_rn(a.y, a.y));
+            sum = __fadd_rn(sum, __fmul_rn(a.z, a.z));
+            sum = __fadd_rn(sum, __fmul_rn(a.w, a.w));
+        }
+        norm[tid >> 6] = sum;
+    }
+    float g[QB];
+#pragma unroll
+    for (int q = 0; q < QB; q++) {
+        g[q] = 0.f;
+    }
+    const float *c = C + (int64_t)(tid < nc ? tid : nc - 1) * d;
+#pragma unroll 8
+    for (int t = 0; t < d; t += 4) {
+        const float4 b = *reinterpret_cast<const float4 *>(c + t);
+#pragma unroll
+        for (int q = 0; q < QB; q++) {
+            const float4 a = *reinterpret_cast<const float4 *>(qs + q * d + t);
+            g[q] = __fadd_rn(g[q], __fmul_rn(a.x, b.x));
+            g[q] = __fadd_rn(g[q], __fmul_rn(a.y, b.y));
+            g[q] = __fadd_rn(g[q], __fmul_rn(a.z, b.z));
+            g[q] = __fadd_rn(g[q], __fmul_rn(a.w, b.w));
+        }
+    }
+    __syncthreads();   // norm[]
+    const float cnorm = tid < nc ? cn[tid] : 0.f;
+#pragma unroll
+    for (int q = 0; q < QB; q++) {
+        if (q0 + q >= nq) {
+            break;   // the same for the whole workgroup
+        }
+        float v = -g[q];
+        if (metric == kMetricL2) {
+            v = __fsub_rn(__fsub_rn(__fadd_rn(norm[q], cnorm), g[q]), g[q]);
+        }
+        if (tid < nc) {
+            keys[tid] = v == v ? make_key(v, (uint32_t)tid) : kEmptyKey;   // a NaN is never selected
+        }
+        block_sort_keys<NT>(keys, nc, tid);
+        if (tid < nout) {
+            const key_t k = tid < nc ? keys[tid] : kEmptyKey;
+            out_ids[(q0 + q) * nout + tid] = k == kEmptyKey ? -1 : (int32_t)key_index(k);
+        }
+        __syncthreads();
+    }
+}
+
+// Where it is the faster way.  One CU reads every centroid, and the lines of many long rows do not stay in its cache while they
+// are wanted, so lists x dimensions is bounded (two launches / one, us per search: one query 1000 x 768 96 / 160, 500 x 384 109 / 114,
+// 1024 x 128 70 / 64, 400 x 96 38 / 37).  From 768 queries on four share a centroid's read (1024 lists, 1000 queries 193 / 152;
+// 400 lists, 2000 queries 131 / 92); up to 256 lists the two launches are as good from 500 queries on and better from 1000.
+bool nearest_lists_serves(const float *Q, int64_t nq, const float *C, int64_t nc, int d, int nout)
+{
+    return nc <= 1024 && nc * d <= 1024 * 128 && (nc > 256 || nq < 500) && nout <= nc && d % 4 == 0 && d <= 1024 &&
+           reinterpret_cast<uintptr_t>(Q) % 16 == 0 && reinterpret_cast<uintptr_t>(C) % 16 == 0;
+}
+
+void launch_nearest_lists(const float *Q, int64_t nq, const float *C, int64_t nc, int d, const float *cn, int metric, int nout,
+                          int32_t *out_ids, float *copy, hipStream_t s)
+{
+    IXA_REQUIRE(nearest_lists_serves(Q, nq, C, nc, d, nout) && nq < ((int64_t)1 << 31), kErrInner,
+                "%ld queries for %ld lists of %d dimensions in one launch", (long)nq, (long)nc, d);
+    if (nq <= 0) {
+        return;
+    }
+    const bool four = nq >= 768;
+    auto launch = [&](auto kern, int threads, int qb) {
+        hipLaunchKernelGGL(kern, dim3((unsigned)((nq + qb - 1) / qb)), dim3((unsigned)threads), (size_t)qb * d * sizeof(float), s, Q, nq, C,
+                           (int)nc, d, cn, metric, nout, out_ids, copy);
+    };
+    if (nc <= 256) {
+        launch(nearest_lists_kernel<256, 1>, 256, 1);
+    } else if (nc <= 512) {
+        four ? launch(nearest_lists_kernel<512, 4>, 512, 4) : launch(nearest_lists_kernel<512, 1>, 512, 1);
+    } else {
+        four ? launch(nearest_lists_kernel<1024, 4>, 1024, 4) : launch(nearest_lists_kernel<1024, 1>, 1024, 1);
+    }
+}
+
 // dist[row * k + t] = the score at column idx[row * k + t], as the public distance (inner products are
 // stored negated in the score matrix); (+-FLT_MAX where idx is -1).
 __global__ __launch_bounds__(256) void gather_scores_kernel(const float *__restrict__ scores, int64_t ld,

@@ -141,6 +141,7 @@ private:
     // best `nout` lists of every row of device matrix x (canonical arithmetic), device outputs
     void coarse_select(const float *x_dev, int64_t n, int nout, int select_metric, int32_t *out_ids,
                        float *out_dist, bool set_only = false, bool defer_check = false);
+    bool coarse_exact_serves(int64_t n) const;
     float bf16x3_err_scale(int select_metric) const;
     // redone (may be null): receives the rows that were redone, ascending
     int coarse_finish(const float *x_dev, int nout, int select_metric, int32_t *out_ids, float *out_dist,

@@ -127,6 +127,7 @@ void parallel_copy(std::initializer_list<CopyJob> jobs)
 // Least room for the sub-vectors, codes and member lists of the sub-quantizers that are trained together; the scratch budget
 // where that is larger.
 constexpr int64_t kPqTrainBytes = (int64_t)64 << 20;
+constexpr size_t kReadInPlaceBytes = 32 << 10;   // queries in page-locked memory that the first kernel reads where they lie
 constexpr int64_t kCoarseExactMaxMacs = (int64_t)1 << 27;   // queries x centroids x dims up to which a search selects its lists exactly
 
 // ---- arena kernels ------------------------------------------------------------------------------
@@ -780,6 +781,13 @@ void IvfpqIndex::coarse_exact_rows(const float *x_dev, const std::vector<int64_t
     sync_stream(stream_);   // the temporaries above are freed on return
 }
 
+// Whether the probed set of n queries is selected from canonical scores of every centroid.
+bool IvfpqIndex::coarse_exact_serves(int64_t n) const
+{
+    return cfg_.coarse_exact_small != 0 && n * nlist_ * d_ <= kCoarseExactMaxMacs && n <= 65535 &&
+           n * nlist_ * (int64_t)sizeof(float) <= cfg_.scratch_bytes;
+}
+
 // Candidate generation with matrix-core products -- bf16 x 3 (error bound below, 16 spare candidates)
 // or, where that kernel does not serve the shape or is switched off, fp32 (8 spare candidates) -- then
 // either the canonical re-evaluation of every candidate plus a proof that nothing outside the list can
@@ -797,11 +805,14 @@ void IvfpqIndex::coarse_select(const float *x_dev, int64_t n, int nout, int sele
     // nothing to prove and no verdict for the host to read, where the matrix-core plans queue seven and a round
     // trip; worth it while the work is small (the canonical kernel reads every centroid once per query: 10M x 128
     // in 16384 lists, 32 queries: 106 us per search against 133; 20M x 768 in 32768 lists, 4 queries: 166 / 224).
-    last_coarse_exact_ = cfg_.coarse_exact_small != 0 && set_only && !out_dist && n * nlist_ * d_ <= kCoarseExactMaxMacs &&
-                         n <= 65535 && n * nlist_ * (int64_t)sizeof(float) <= cfg_.scratch_bytes;
+    last_coarse_exact_ = set_only && !out_dist && coarse_exact_serves(n);
     if (last_coarse_exact_) {
         last_coarse_plan_ = 0;
         last_coarse_n_ = n;
+        if (nearest_lists_serves(x_dev, n, centroids_.data(), nlist_, d_, nout)) {
+            launch_nearest_lists(x_dev, n, centroids_.data(), nlist_, d_, cnorm_.data(), select_metric, nout, out_ids, nullptr, stream_);
+            return;
+        }
         ws_exact_.resize((size_t)n * nlist_);
         launch_canonical_scores(x_dev, n, centroids_.data(), nlist_, d_, nullptr, cnorm_.data(), select_metric,
                                 ws_exact_.data(), nlist_, stream_);   // without row norms: the kernel adds them up itself
@@ -1681,13 +1692,25 @@ void IvfpqIndex::search_page(int64_t n, const float *x, int64_t k, float *dist, 
     const bool staged_io = !on_device && label_at + label_bytes <= kPipelinedIoBytes;
     const bool pipelined_io = staged_io && label_at + label_bytes > kStagedIoBytes;
     unsigned char *io = nullptr;
+    unsigned char *mapped = nullptr;   // the staging buffer as the GPU addresses it
+    const float *x_first = nullptr;    // what the coarse stage reads instead of xd
     if (staged_io) {
         io = static_cast<unsigned char *>(io_stage_.reserve(label_at + label_bytes));
+        void *mapped_io = nullptr;
+        IXA_HIP(hipHostGetDevicePointer(&mapped_io, io, 0));
+        mapped = static_cast<unsigned char *>(mapped_io);
         ws_x_.resize((size_t)n * d_);
+        if (coarse_exact_serves(n) && in_bytes <= kReadInPlaceBytes &&
+            nearest_lists_serves(reinterpret_cast<const float *>(mapped), n, centroids_.data(), nlist_, d_, nprobe_)) {
+            // a few queries: the one launch of the coarse stage reads them over the link and leaves them in device memory, and
+            // there is no copy to wait for
+            std::memcpy(io, x, in_bytes);
+            x_first = reinterpret_cast<const float *>(mapped);
+        }
         // the queries go up in two halves when there is much of them: the second half is copied into the staging
         // buffer while the first is on its way
         const size_t half = pipelined_io ? (in_bytes / 2 + 4095) / 4096 * 4096 : in_bytes;
-        for (size_t off = 0; off < in_bytes; off += half) {
+        for (size_t off = 0; off < in_bytes && !x_first; off += half) {
             const size_t bytes = std::min(half, in_bytes - off);
             parallel_copy({{io + off, reinterpret_cast<const unsigned char *>(x) + off, bytes}});
             IXA_HIP(hipMemcpyAsync(reinterpret_cast<unsigned char *>(ws_x_.data()) + off, io + off, bytes,
@@ -1704,10 +1727,8 @@ void IvfpqIndex::search_page(int64_t n, const float *x, int64_t k, float *dist, 
         // The kernels that finish a query write its distances and labels straight into the page-locked staging buffer,
         // which the GPU addresses over PCIe: the results travel while other queries are still being scanned, and no
         // copy engine has to be waited for once the last kernel is done.  (Nothing reads the results back.)
-        void *mapped = nullptr;
-        IXA_HIP(hipHostGetDevicePointer(&mapped, io, 0));
-        dd = reinterpret_cast<float *>(static_cast<unsigned char *>(mapped) + dist_at);
-        ld = reinterpret_cast<int64_t *>(static_cast<unsigned char *>(mapped) + label_at);
+        dd = reinterpret_cast<float *>(mapped + dist_at);
+        ld = reinterpret_cast<int64_t *>(mapped + label_at);
     } else if (!on_device) {
         ws_dist_.resize((size_t)n * k);
         ws_labels_.resize((size_t)n * k);
@@ -1722,7 +1743,15 @@ void IvfpqIndex::search_page(int64_t n, const float *x, int64_t k, float *dist, 
         IXA_HIP(hipEventRecord(ev_[0], stream_));
     }
     last_coarse_reruns_ = 0;
-    coarse_select(xd, n, nprobe_, metric_, ws_probes_.data(), nullptr, true, true);
+    if (x_first) {
+        last_coarse_exact_ = true;
+        last_coarse_plan_ = 0;
+        last_coarse_n_ = n;
+        launch_nearest_lists(x_first, n, centroids_.data(), nlist_, d_, cnorm_.data(), metric_, nprobe_, ws_probes_.data(), ws_x_.data(),
+                             stream_);
+    } else {
+        coarse_select(xd, n, nprobe_, metric_, ws_probes_.data(), nullptr, true, true);
+    }
     if (timed) {
         IXA_HIP(hipEventRecord(ev_[1], stream_));
     }

@@ -1051,3 +1051,65 @@ def test_assignment_decides_every_tie_exactly(ix, oracle, d, nlist, n):
     x[0, 1] = np.nan
     got = gpu.assign(x)
     assert got[0] == -1 and np.array_equal(got[1:], oracle.assign(x[1:], cent))
+
+
+# A query split over workgroups deals groups of 64 codes to its slices in turn: lists without codes, of one code and of a remainder,
+# several groups per list and (nprobe 512: a slice skips more than 64 lists at a time) far fewer; private pools, the shared pool,
+# kernels for a compile-time number of sub-quantizers and not.  As in one workgroup per query (a large batch), bit for bit.
+@pytest.mark.parametrize("M,k,layout", [(4, 300, 0), (8, 20, 0), (32, 100, 0), (32, 100, 1), (28, 30, 0), (9, 200, 0)])
+@pytest.mark.parametrize("nlist,nprobe,n", [(512, 512, 3000), (600, 512, 9000), (40, 17, 60000), (3, 3, 700), (700, 600, 9000)])
+def test_slices_of_a_query_take_groups_of_codes_in_turn(ix, oracle, M, k, layout, nlist, nprobe, n):
+    rng = np.random.default_rng(nlist + M)
+    d = 4 * M
+    cent = rng.standard_normal((nlist, d)).astype(np.float32)
+    book = (0.7 * rng.standard_normal((M, 256, 4))).astype(np.float32)
+    index = ix.AscendIndexIVFPQ(d, ix.METRIC_L2, nlist, M, 8, ix.AscendIndexIVFPQConfig(code_layout=layout))
+    index.set_trained(cent, book)
+    # lengths from none to several groups, most vectors in a few lists
+    weight = rng.random(nlist) ** 6
+    weight[rng.integers(0, nlist, nlist // 3)] = 0.0
+    lists = np.sort(rng.choice(nlist, n, p=weight / weight.sum()))
+    for l in np.unique(lists):
+        count = int((lists == l).sum())
+        index.add_codes(int(l), rng.integers(0, 256, (count, M)).astype(np.uint8), np.arange(count, dtype=np.int64) + 100000 * int(l))
+    index.setNumProbes(nprobe)
+    q = rng.standard_normal((2000, d)).astype(np.float32)
+    D, I = index.search(q, k)
+    assert index.last_search_stats()["nsplit"] == 1
+    for nq in (1, 7, 60):
+        Ds, Is = index.search(q[:nq], k)
+        assert index.last_search_stats()["nsplit"] > 1
+        assert np.array_equal(Is, I[:nq]) and np.array_equal(Ds.view(np.uint32), D[:nq].view(np.uint32))
+
+
+# The coarse stage of a small batch in one launch (up to 1024 lists): list counts around 256, 512 and 1024, batches around a
+# workgroup's four queries, equal centroids and undefined queries, queries read from page-locked memory and from the device.
+@pytest.mark.parametrize("metric_name", ["L2", "IP"])
+@pytest.mark.parametrize("nlist,d,nq,nprobe", [(1, 8, 1, 1), (2, 64, 3, 2), (255, 32, 499, 16), (256, 36, 5, 256), (257, 64, 767, 5),
+                                               (512, 64, 769, 100), (513, 32, 770, 513), (1023, 128, 2, 64), (1024, 128, 801, 3),
+                                               (1024, 32, 1, 1024)])
+def test_small_batches_find_their_lists_in_one_launch(ix, oracle, metric_name, nlist, d, nq, nprobe):
+    metric = ix.METRIC_L2 if metric_name == "L2" else ix.METRIC_INNER_PRODUCT
+    rng = np.random.default_rng(nlist + nq)
+    cent = rng.standard_normal((nlist, d)).astype(np.float32)
+    if nlist > 100:
+        cent[40] = cent[30]
+        cent[nlist - 1] = cent[50]
+    q = (cent[rng.integers(0, nlist, nq)] + 0.5 * rng.standard_normal((nq, d))).astype(np.float32)
+    if nq > 4:
+        q[3, 1] = np.nan
+    book = rng.standard_normal((2, 256, d // 2)).astype(np.float32)
+    # one vector per list, found if and only if its list is probed
+    index = ix.AscendIndexIVFPQ(d, metric, nlist, 2, 8)
+    index.set_trained(cent, book)
+    for l in range(nlist):
+        index.add_codes(l, np.array([[l % 256, l // 256]], dtype=np.uint8), np.array([l], dtype=np.int64))
+    index.setNumProbes(nprobe)
+    want, _ = oracle.coarse_probe(q, cent, nprobe, metric)
+    keep = np.arange(nq) != (3 if nq > 4 else -1)
+    for rows in (np.arange(nq), np.arange(min(nq, 2))):      # the whole batch, and one small enough to be read in place
+        D, I = index.search(q[rows], nprobe)
+        good = keep[rows]
+        assert np.array_equal(np.sort(I, axis=1)[good], np.sort(want[rows], axis=1)[good])
+        if not good.all():
+            assert (I[~good] == -1).all()
