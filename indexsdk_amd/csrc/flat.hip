@@ -458,6 +458,30 @@ int64_t FlatBase<T>::remove_selected(int64_t nv, const int64_t *victims, int64_t
     return (int64_t)hits;
 }
 
+constexpr size_t kFlatStagedBytes = (size_t)8 << 20;
+
+template <typename T>
+typename FlatBase<T>::StagedIo FlatBase<T>::stage_in(int64_t n, const T *x, int64_t k, size_t dist_size)
+{
+    const size_t in_bytes = (size_t)n * d_ * sizeof(T), cells = (size_t)n * k;
+    StagedIo io;
+    io.dist_at = (in_bytes + 255) / 256 * 256;
+    io.label_at = io.dist_at + (cells * dist_size + 255) / 256 * 256;
+    const size_t bytes = io.label_at + cells * sizeof(int64_t);
+    if (bytes > kFlatStagedBytes) {
+        ws_x_.upload(x, (size_t)n * d_, stream_);
+        return io;
+    }
+    io.host = static_cast<unsigned char *>(io_stage_.reserve(bytes));
+    void *mapped = nullptr;
+    IXA_HIP(hipHostGetDevicePointer(&mapped, io.host, 0));
+    io.mapped = static_cast<unsigned char *>(mapped);
+    std::memcpy(io.host, x, in_bytes);
+    ws_x_.resize((size_t)n * d_);
+    IXA_HIP(hipMemcpyAsync(ws_x_.data(), io.host, in_bytes, hipMemcpyHostToDevice, stream_));
+    return io;
+}
+
 template <typename T>
 void FlatBase<T>::move_rows(const int64_t *moves, int64_t nmoves, uint32_t *norms)
 {
@@ -699,13 +723,12 @@ void FlatIndex::search_masked(int64_t n, const float *x, int64_t k, float *dist,
     IXA_REQUIRE(n > 0 && n < kMaxN, kErrInvalidParam, "n must be > 0 and < %ld", (long)kMaxN);
     IXA_REQUIRE(k > 0 && k <= kMaxK, kErrInvalidParam, "k must be > 0 and <= %ld", (long)kMaxK);
     const float *xd = x;
-    if (!on_device) {
-        ws_x_.upload(x, (size_t)n * d_, stream_);
-        xd = ws_x_.data();
-    }
     float *dd = dist;
     int64_t *ld = labels;
+    StagedIo io;
     if (!on_device) {
+        io = stage_in(n, x, k, sizeof(float));
+        xd = ws_x_.data();
         ws_dist_.resize((size_t)n * k);
         ws_labels_.resize((size_t)n * k);
         dd = ws_dist_.data();
@@ -778,7 +801,13 @@ void FlatIndex::search_masked(int64_t n, const float *x, int64_t k, float *dist,
         stats_.ms_select += ms;
         stats_.exact_reruns = (double)rows.size();
     }
-    if (!on_device) {
+    if (io.host) {   // (the proof reads the distances back, so they are not written straight to host memory)
+        IXA_HIP(hipMemcpyAsync(io.host + io.dist_at, dd, (size_t)n * k * sizeof(float), hipMemcpyDeviceToHost, stream_));
+        IXA_HIP(hipMemcpyAsync(io.host + io.label_at, ld, (size_t)n * k * sizeof(int64_t), hipMemcpyDeviceToHost, stream_));
+        sync_stream(stream_);
+        std::memcpy(dist, io.host + io.dist_at, (size_t)n * k * sizeof(float));
+        std::memcpy(labels, io.host + io.label_at, (size_t)n * k * sizeof(int64_t));
+    } else if (!on_device) {
         ws_dist_.download(dist, (size_t)n * k, stream_);
         ws_labels_.download(labels, (size_t)n * k, stream_);
     }
@@ -848,8 +877,10 @@ std::vector<int64_t> FlatIndex::search_plan(int64_t n, const float *xd, int64_t 
         IXA_HIP(hipMemsetAsync(ws_flag_.data(), 0, sizeof(int32_t), stream_));
         launch_verify_superset(ws_running_.data(), ncand, dd, (int)k, ws_qn_.data(), bmax_, err_scale, round_scale, metric_,
                                n, ws_flag_.data(), stream_, split || resident);
-        int32_t nfail = 0;
-        ws_flag_.download(&nfail, 1, stream_);
+        int32_t *verdict = static_cast<int32_t *>(verdict_.reserve(sizeof(int32_t)));
+        IXA_HIP(hipMemcpyAsync(verdict, ws_flag_.data(), sizeof(int32_t), hipMemcpyDeviceToHost, stream_));
+        sync_stream(stream_);
+        const int32_t nfail = *verdict;
         if (nfail > 0) {
             rows32.resize((size_t)nfail);
             IXA_HIP(hipMemcpyAsync(rows32.data(), ws_flag_.data() + 1, (size_t)nfail * 4, hipMemcpyDeviceToHost, stream_));
@@ -999,17 +1030,21 @@ void FlatI8Index::search_masked(int64_t n, const int8_t *x, int64_t k, int32_t *
     IXA_REQUIRE(n > 0 && n < kMaxN, kErrInvalidParam, "n must be > 0 and < %ld", (long)kMaxN);
     IXA_REQUIRE(k > 0 && k <= kMaxK, kErrInvalidParam, "k must be > 0 and <= %ld", (long)kMaxK);
     const int8_t *xd = x;
-    if (!on_device) {
-        ws_x_.upload(x, (size_t)n * d_, stream_);
-        xd = ws_x_.data();
-    }
     int32_t *dd = dist;
     int64_t *ld = labels;
+    StagedIo io;
     if (!on_device) {
-        ws_dist_.resize((size_t)n * k);
-        ws_labels_.resize((size_t)n * k);
-        dd = ws_dist_.data();
-        ld = ws_labels_.data();
+        io = stage_in(n, x, k, sizeof(int32_t));
+        xd = ws_x_.data();
+        if (io.host) {   // the last kernel writes the results where the host reads them
+            dd = reinterpret_cast<int32_t *>(io.mapped + io.dist_at);
+            ld = reinterpret_cast<int64_t *>(io.mapped + io.label_at);
+        } else {
+            ws_dist_.resize((size_t)n * k);
+            ws_labels_.resize((size_t)n * k);
+            dd = ws_dist_.data();
+            ld = ws_labels_.data();
+        }
     }
     ws_qn_.resize((size_t)n);
     ws_running_.resize((size_t)n * k);
@@ -1025,7 +1060,10 @@ void FlatI8Index::search_masked(int64_t n, const int8_t *x, int64_t k, int32_t *
                        ws_running_.data(), n * k, kMetricL2, ids_.data(), (int32_t)0x7fffffff, dd, ld);
     IXA_HIP(hipEventRecord(ev_[1], stream_));
     sync_stream(stream_);
-    if (!on_device) {
+    if (io.host) {
+        std::memcpy(dist, io.host + io.dist_at, (size_t)n * k * sizeof(int32_t));
+        std::memcpy(labels, io.host + io.label_at, (size_t)n * k * sizeof(int64_t));
+    } else if (!on_device) {
         ws_dist_.download(dist, (size_t)n * k, stream_);
         ws_labels_.download(labels, (size_t)n * k, stream_);
     }

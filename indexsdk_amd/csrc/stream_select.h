@@ -12,6 +12,7 @@ struct StreamSelectWorkspace {
     DeviceBuffer<int32_t> cnt;                    // per-query admitted-candidate counters + overflow flag
     DeviceBuffer<unsigned long long> filter;
     DeviceBuffer<unsigned long long> parts;       // keys of the stretches of few long rows (launch_select_rows)
+    PinnedBuffer overflow;                        // the overflow flag as the host reads it
     bool cnt_zero = false;                        // every counter is zero (the sampled-bound plan keeps them so)
 };
 

@@ -412,10 +412,10 @@ int stream_select(const Ops &ops, const typename Ops::T *Q, int64_t nq_total, co
         if (!fused) {
             break;   // nothing can overflow: no host synchronisation, the caller's stream carries on
         }
-        int ovf = 0;
-        IXA_HIP(hipMemcpyAsync(&ovf, overflow, sizeof(int), hipMemcpyDeviceToHost, s));
+        int *ovf = static_cast<int *>(ws.overflow.reserve(sizeof(int)));
+        IXA_HIP(hipMemcpyAsync(ovf, overflow, sizeof(int), hipMemcpyDeviceToHost, s));
         sync_stream(s);
-        if (!ovf) {
+        if (!*ovf) {
             break;
         }
         fused = false;
