@@ -285,6 +285,12 @@ __device__ __forceinline__ void scan_body(const ScanParams &p)
             build(std::integral_constant<int, 2>{});
         } else if (dsub == 1) {
             build(std::integral_constant<int, 1>{});
+        } else if (dsub == 3) {
+            build(std::integral_constant<int, 3>{});
+        } else if (dsub == 5) {
+            build(std::integral_constant<int, 5>{});
+        } else if (dsub == 6) {
+            build(std::integral_constant<int, 6>{});
         } else if (dsub % 16 == 0) {
             // long sub-vectors (128 dimensions in 2, 4 or 8 sub-quantizers): sixteen codeword floats per memory
             // round trip instead of one, accumulated in the same order
