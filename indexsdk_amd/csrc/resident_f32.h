@@ -25,7 +25,7 @@ struct AssignWorkspace {
     DeviceBuffer<int4> pairs;     // {vector, two centroids}
     DeviceBuffer<int32_t> rows;   // vectors with more than two; behind them the lengths of the two lists
 };
-bool resident_assign_serves(const float *X, const float *C, int d);
+bool resident_assign_serves(const float *X, const float *C, int64_t nc, int d);
 void launch_resident_assign(const float *X, int64_t n, const float *C, int64_t nc, int d, const float *xn, const float *cn, float cmax,
                             int32_t *out, AssignWorkspace &ws, int64_t scratch_bytes, hipStream_t s);
 

@@ -729,9 +729,11 @@ bool launch_resident_f32(const float *Q, int64_t nq, const float *B, int64_t nb,
     return true;
 }
 
-bool resident_assign_serves(const float *X, const float *C, int d)
+// (Above 512 dimensions a tile holds 32 centroids and every vector is read once per tile: adding 40000 x 768, score matrix / this in
+// us: 1500 lists 2271 / 1125, 2048 1887 / 1308, 8192 3121 / 3794; 512 dimensions, 4096 lists 1909 / 997, 384, 8192 1769 / 1272.)
+bool resident_assign_serves(const float *X, const float *C, int64_t nc, int d)
 {
-    return resident_f32_serves(d) && reinterpret_cast<uintptr_t>(X) % 16 == 0 && reinterpret_cast<uintptr_t>(C) % 16 == 0;
+    return resident_f32_serves(d) && (d <= 512 || nc <= 4096) && reinterpret_cast<uintptr_t>(X) % 16 == 0 && reinterpret_cast<uintptr_t>(C) % 16 == 0;
 }
 
 void launch_resident_assign(const float *X, int64_t n, const float *C, int64_t nc, int d, const float *xn, const float *cn, float cmax,
@@ -740,7 +742,7 @@ void launch_resident_assign(const float *X, int64_t n, const float *C, int64_t n
     if (n <= 0) {
         return;
     }
-    IXA_REQUIRE(resident_assign_serves(X, C, d) && nc >= 1 && n < ((int64_t)1 << 31), kErrInner, "assignment kernel does not serve these operands");
+    IXA_REQUIRE(resident_assign_serves(X, C, nc, d) && nc >= 1 && n < ((int64_t)1 << 31), kErrInner, "assignment kernel does not serve these operands");
     const int qt = 32 * tile_blocks(nc, d);
     const int64_t tiles = (nc + qt - 1) / qt;
     // vectors per pass: 16 bytes per vector and tile of centroids, 20 for what is left open
