@@ -1973,9 +1973,10 @@ __global__ __launch_bounds__(NT) void nearest_lists_kernel(const float *__restri
 // are wanted, so lists x dimensions is bounded (two launches / one, us per search: one query 1000 x 768 96 / 160, 500 x 384 109 / 114,
 // 1024 x 128 70 / 64, 400 x 96 38 / 37).  From 768 queries on four share a centroid's read (1024 lists, 1000 queries 193 / 152;
 // 400 lists, 2000 queries 131 / 92); up to 256 lists the two launches are as good from 500 queries on and better from 1000.
+// A few queries over more than 512 lists: 24 us on one CU each against 15 for the two launches, which use four.
 bool nearest_lists_serves(const float *Q, int64_t nq, const float *C, int64_t nc, int d, int nout)
 {
-    return nc <= 1024 && nc * d <= 1024 * 128 && (nc > 256 || nq < 500) && nout <= nc && d % 4 == 0 && d <= 1024 &&
+    return nc <= 1024 && nc * d <= 1024 * 128 && (nc > 256 || nq < 500) && (nc <= 512 || nq >= 32) && nout <= nc && d % 4 == 0 && d <= 1024 &&
            reinterpret_cast<uintptr_t>(Q) % 16 == 0 && reinterpret_cast<uintptr_t>(C) % 16 == 0;
 }
 
