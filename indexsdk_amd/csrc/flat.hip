@@ -657,7 +657,8 @@ constexpr int64_t kSplitPage = 16384;                  // queries that are split
 // to bring more than one such tile and enough products.  fp32 / split, us per search, k 100:
 //   256 queries: 200k x 64 370 / 423, 200k x 128 440 / 482, 400k x 128 769 / 818, 65536 x 768 371 / 455; from 1M on 1627 / 1101
 //   (d 128), 2117 / 1654 (d 256), 1628 / 1612 (d 64, k 300).  128 queries: 1M x 128 1566 / 1639, 200k x 128 429 / 456.  (160 - 255
-//   queries over 1M rows and more would gain as well, 160 over 1M x 128 1587 / 1060; they have the fp32 plan all the same.)
+//   queries over 1M rows and more would gain as well, 160 over 1M x 128 1587 / 1060.)  The figures of 64 to 256 dimensions
+//   are from before resident_pays took these dimensions where they are multiples of 4; others still come here.
 //   320 queries: 32768 x 128 171 / 166, 65536 x 128 238 / 223, 200k x 128 631 / 577, 400k x 128 1073 / 768, 32768 x 768 362 / 306;
 //   d 64, where a tile's products are few: 512 queries 32768 152 / 159, 100k 325 / 341, 200k 542 / 541, 400k 908 / 659; 1024
 //   queries 32768 200 / 198, 100k 487 / 469, 200k 805 / 580.
