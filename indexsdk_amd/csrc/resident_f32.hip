@@ -88,7 +88,7 @@ __device__ __forceinline__ float test_value(float qn, float tau, bool l2)
 
 // The larger of two numbers, or the number where the other is a NaN.  (fmaxf would make v a quiet number first, an instruction
 // each.  The operands are results of vector instructions, never of a matrix instruction, whose results an inline instruction
-// would not wait for.)
+// would not wait for.  A signalling NaN takes m away instead: assign_need rules the sums out that could become one.)
 __device__ __forceinline__ float max_number(float m, float v)
 {
     float r;
@@ -570,10 +570,13 @@ void launch_mode(const Args &a)
 
 // By how much a u has to lead another for the canonical scores to be in that order.  Both scores |x|^2 - 2 u are within E of the
 // canonical ones, and the places in the low bits have moved each u by at most 2^-17 |u|, |u| <= |x| cmax + cmax^2 / 2.  Infinite
-// or undefined where nothing can be decided.
+// or undefined where nothing can be decided: so for lengths whose products come near the start of a padding centroid (-3e38),
+// where a sum may overflow.  An infinite sum with a place in its low bits is a signalling NaN, which makes max_number forget the
+// best so far; and a number below -3e38 would be passed over.
 __device__ __forceinline__ float assign_need(float norm, float cmax, float err_scale, float round_scale)
 {
-    return score_margin(norm, cmax, err_scale, round_scale) + 1.6e-5f * (sqrtf(norm) * cmax + cmax * cmax);
+    const float reach = sqrtf(norm) * cmax + cmax * cmax;
+    return reach < 1e37f ? score_margin(norm, cmax, err_scale, round_scale) + 1.6e-5f * reach : __builtin_inff();
 }
 
 // The best two of every vector over all tiles and the third value; a lead of more than the error bound decides, a tie of two

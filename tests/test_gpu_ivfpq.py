@@ -1053,6 +1053,30 @@ def test_assignment_decides_every_tie_exactly(ix, oracle, d, nlist, n):
     assert got[0] == -1 and np.array_equal(got[1:], oracle.assign(x[1:], cent))
 
 
+# Lengths near the end of the range, where the sum of a padding centroid (it starts from -3e38) overflows and a tile's best two are
+# not to be trusted: the nearest centroid lies in the last tile, which is padded with copies of the one most distant from the vectors.
+@pytest.mark.parametrize("d,nlist", [(128, 300), (128, 257), (36, 129), (256, 140), (768, 50)])
+@pytest.mark.parametrize("length", [1e18, 3e18, 5e18, 6.4e18, 9e18, 1.2e19])
+def test_assignment_of_vectors_near_the_end_of_the_range(ix, oracle, d, nlist, length):
+    rng = np.random.default_rng(d + nlist)
+
+    def unit(rows):
+        return rows / np.linalg.norm(rows, axis=1, keepdims=True)
+
+    way = unit(rng.standard_normal((1, d)))
+    cent = unit(rng.standard_normal((nlist, d)) + 0.5 * np.sqrt(d) * way * (np.arange(nlist) % 2)[:, None])
+    cent[nlist - 1] = -way
+    cent[nlist - 3] = unit(way + 0.05 * rng.standard_normal((1, d)) / np.sqrt(d))
+    cent[2] = unit(way + 0.6 * rng.standard_normal((1, d)) / np.sqrt(d))
+    x = unit(way + 0.1 * rng.standard_normal((70, d)) / np.sqrt(d))
+    cent, x = (length * cent).astype(np.float32), (length * x).astype(np.float32)
+    gpu = ix.AscendIndexIVFPQ(d, ix.METRIC_L2, nlist, 4, 8)
+    gpu.set_trained(cent, rng.standard_normal((4, 256, d // 4)).astype(np.float32))
+    want = oracle.assign(x, cent)
+    assert (want == nlist - 3).all()
+    assert np.array_equal(gpu.assign(x), want)
+
+
 # A query split over workgroups deals groups of 64 codes to its slices in turn: lists without codes, of one code and of a remainder,
 # several groups per list and (nprobe 512: a slice skips more than 64 lists at a time) far fewer; private pools, the shared pool,
 # kernels for a compile-time number of sub-quantizers and not.  As in one workgroup per query (a large batch), bit for bit.
