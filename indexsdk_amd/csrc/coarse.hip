@@ -1969,14 +1969,29 @@ __global__ __launch_bounds__(NT) void nearest_lists_kernel(const float *__restri
     }
 }
 
-// Where it is the faster way.  One CU reads every centroid, and the lines of many long rows do not stay in its cache while they
-// are wanted, so lists x dimensions is bounded (two launches / one, us per search: one query 1000 x 768 96 / 160, 500 x 384 109 / 114,
-// 1024 x 128 70 / 64, 400 x 96 38 / 37).  From 768 queries on four share a centroid's read (1024 lists, 1000 queries 193 / 152;
-// 400 lists, 2000 queries 131 / 92); up to 256 lists the two launches are as good from 500 queries on and better from 1000.
-// A few queries over more than 512 lists: 24 us on one CU each against 15 for the two launches, which use four.
+// Where it is the faster way.  A selection of a few of up to 2048 scores is one wavefront's work and cheaper than the sort here, so
+// it depends on the number of lists asked for (two launches / one, us per search, queries in device memory):
+//   up to 128 lists of centroids: 100 x 128, 8 queries, 16 lists asked for 42 / 38, 1 list 26 / 26; from 500 queries on the two launches
+//     are as good, with many dimensions from 256 on (128 x 512, 300 queries, 1 list 67 / 70);
+//   up to 512: 256 x 128, 8 queries: 1 list 23 / 28, 3 lists 30 / 35, 16 lists 44 / 43, 128 lists 77 / 58; 512 x 256, 8 queries, 16
+//     lists 47 / 48, 32 lists 50 / 50, 128 lists 93 / 69; above 256 from 400 queries on with any number (400 x 256, 400 queries, 8 lists
+//     81 / 69), below it is the two launches from 500 on;
+//   above: one CU reads every centroid for a query or four.  1024 x 128, 32 queries: 1 list 22 / 31, 32 lists 46 / 49, 128 lists
+//     72 / 64; 400 queries, 16 lists 86 / 80, 1 list 65 / 65; 800 queries (four share a centroid's read) 1 list 126 / 98, but 1024 x
+//     64 62 / 64.  A few queries: 24 us on one CU each against 15 for the two launches, which use four.
+// The lines of many long rows do not stay in a CU's cache while they are wanted, so lists x dimensions is bounded (one query: 1000 x
+// 768 96 / 160, 500 x 384 109 / 114).
 bool nearest_lists_serves(const float *Q, int64_t nq, const float *C, int64_t nc, int d, int nout)
 {
-    return nc <= 1024 && nc * d <= 1024 * 128 && (nc > 256 || nq < 500) && (nc <= 512 || nq >= 32) && nout <= nc && d % 4 == 0 && d <= 1024 &&
+    bool faster;
+    if (nc <= 128) {
+        faster = nq < (d <= 256 ? 500 : 256);
+    } else if (nc <= 512) {
+        faster = (nout > (nc * d <= 98304 ? 8 : 16) && (nc > 256 || nq < 500)) || (nc > 256 && nq >= 400);
+    } else {
+        faster = (nout > 64 && nq >= 32) || (nout > 8 && nq >= 400) || (d >= 96 && nq >= 768);
+    }
+    return faster && nc <= 1024 && nc * d <= 1024 * 128 && nout <= nc && d % 4 == 0 && d <= 1024 &&
            reinterpret_cast<uintptr_t>(Q) % 16 == 0 && reinterpret_cast<uintptr_t>(C) % 16 == 0;
 }
 

@@ -1078,11 +1078,12 @@ def test_assignment_of_vectors_near_the_end_of_the_range(ix, oracle, d, nlist, l
 
 
 # A query split over workgroups deals groups of 64 codes to its slices in turn: lists without codes, of one code and of a remainder,
-# several groups per list and (nprobe 512: a slice skips more than 64 lists at a time) far fewer; private pools, the shared pool,
+# several groups per list and (nprobe 512: a slice skips more than 64 lists at a time) far fewer; 8 to 20 slices; private pools, the shared pool,
 # kernels for a compile-time number of sub-quantizers and not.  As in one workgroup per query (a large batch), bit for bit.
 @pytest.mark.parametrize("M,k,layout", [(4, 300, 0), (8, 20, 0), (32, 100, 0), (32, 100, 1), (28, 30, 0), (9, 200, 0)])
-@pytest.mark.parametrize("nlist,nprobe,n", [(512, 512, 3000), (600, 512, 9000), (40, 17, 60000), (3, 3, 700), (700, 600, 9000)])
-def test_slices_of_a_query_take_groups_of_codes_in_turn(ix, oracle, M, k, layout, nlist, nprobe, n):
+@pytest.mark.parametrize("nlist,nprobe,n,groups", [(512, 512, 3000, True), (600, 512, 9000, True), (40, 17, 60000, True),
+                                                   (130, 120, 90000, True), (3, 3, 700, False), (700, 600, 9000, False)])
+def test_slices_of_a_query_take_groups_of_codes_in_turn(ix, oracle, M, k, layout, nlist, nprobe, n, groups):
     rng = np.random.default_rng(nlist + M)
     d = 4 * M
     cent = rng.standard_normal((nlist, d)).astype(np.float32)
@@ -1102,16 +1103,22 @@ def test_slices_of_a_query_take_groups_of_codes_in_turn(ix, oracle, M, k, layout
     assert index.last_search_stats()["nsplit"] == 1
     for nq in (1, 7, 60):
         Ds, Is = index.search(q[:nq], k)
-        assert index.last_search_stats()["nsplit"] > 1
+        # (groups from two lists per slice to 512 lists, by workgroups of eight wavefronts; whole lists otherwise)
+        stats = index.last_search_stats()
+        assert stats["nsplit"] >= (16 if n == 90000 else 2)
+        assert (2 * stats["nsplit"] <= nprobe <= 512 and stats["scan_waves"] == 8) == groups
         assert np.array_equal(Is, I[:nq]) and np.array_equal(Ds.view(np.uint32), D[:nq].view(np.uint32))
 
 
-# The coarse stage of a small batch in one launch (up to 1024 lists): list counts around 256, 512 and 1024, batches around a
-# workgroup's four queries, equal centroids and undefined queries, queries read from page-locked memory and from the device.
+# The coarse stage of a small batch in one launch (up to 1024 lists): list counts around 256, 512 and 1024 and off them, with one
+# query per workgroup and (from 768 on) with four and their remainders, equal centroids and undefined queries, queries read from
+# page-locked memory (the two-row repeats of up to 512 lists) and from the device.  The last four take the two launches.
 @pytest.mark.parametrize("metric_name", ["L2", "IP"])
-@pytest.mark.parametrize("nlist,d,nq,nprobe", [(1, 8, 1, 1), (2, 64, 3, 2), (255, 32, 499, 16), (256, 36, 5, 256), (257, 64, 767, 5),
-                                               (512, 64, 769, 100), (513, 32, 770, 513), (1023, 128, 2, 64), (1024, 128, 801, 3),
-                                               (1024, 32, 1, 1024)])
+@pytest.mark.parametrize("nlist,d,nq,nprobe", [(1, 8, 1, 1), (2, 64, 3, 2), (100, 128, 60, 3), (128, 1024, 40, 9), (255, 32, 499, 16),
+                                               (256, 36, 5, 256), (257, 64, 767, 5), (300, 100, 40, 20), (512, 64, 769, 100),
+                                               (512, 256, 771, 3), (513, 32, 770, 513), (513, 32, 33, 65), (700, 64, 767, 9),
+                                               (1023, 128, 40, 100), (1023, 128, 769, 1), (1024, 128, 801, 3), (1024, 96, 500, 64),
+                                               (200, 64, 5, 3), (1023, 128, 2, 64), (1024, 32, 1, 1024), (1024, 64, 800, 3)])
 def test_small_batches_find_their_lists_in_one_launch(ix, oracle, metric_name, nlist, d, nq, nprobe):
     metric = ix.METRIC_L2 if metric_name == "L2" else ix.METRIC_INNER_PRODUCT
     rng = np.random.default_rng(nlist + nq)
