@@ -318,7 +318,8 @@ int ivfpq_ntotal(const ivfpq_index_t *h, int64_t *out);
  * regions the kernel addresses inside its dynamic LDS, and the total.  Host code only (no GPU is touched; it
  * works without one): what a test holds against the regions' sizes to prove that no region ends outside the
  * allocation.  waves = 0 asks for the plan the launcher would choose; 4, 8 or 16 with shared_pool 0 / 1 for
- * the layout of that workgroup size and pool kind.  No counterpart in the reference. */
+ * the layout of that workgroup size and pool kind.  nsplit > 1: of slices that take whole lists; slices that share every
+ * list have the layout of nsplit = 1.  No counterpart in the reference. */
 typedef struct ivfpq_scan_lds_plan {
     int32_t waves, shared_pool; /* wavefronts per workgroup; 1 = one workgroup-wide candidate pool */
     int32_t cap;                /* keys per pool */

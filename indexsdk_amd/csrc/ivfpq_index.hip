@@ -1593,7 +1593,7 @@ void IvfpqIndex::search_probes(int64_t n, const float *x_dev, const int32_t *pro
     stats_.nsplit = p.nsplit;
     stats_.scan_launches = p.nsplit > 1 ? 2 : 1;
     stats_.ordered = p.order ? (p.xcd_chunks ? 2 : 1) : 0;   // 1 = heaviest first, 2 = by locality
-    plan_scan(p);
+    plan_launch(p);
     stats_.scan_waves = p.waves;
     stats_.shared_pool = p.shared_pool;
 }
@@ -1775,7 +1775,7 @@ void IvfpqIndex::search_page(int64_t n, const float *x, int64_t k, float *dist, 
     stats_.ordered = p.order ? (p.xcd_chunks ? 2 : 1) : 0;   // 1 = heaviest first, 2 = by locality
     {
         ScanParams planned = p;
-        plan_scan(planned);
+        plan_launch(planned);
         stats_.scan_waves = planned.waves;
         stats_.shared_pool = planned.shared_pool;
     }

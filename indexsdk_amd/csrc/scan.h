@@ -40,18 +40,19 @@ struct ScanParams {
     const int32_t *order;      // optional permutation of the queries (execution order), may be null
     int xcd_chunks;            // 1: deal contiguous chunks of the execution order to the 8 XCDs
     int64_t nq;                // filled by launch_scan()
-    int by_groups;             // 1: a split query is divided by groups of codes, 0: by lists (filled by launch_scan())
-    // filled by plan_scan()
+    // filled by plan_launch()
+    int by_groups;             // 1: a split query is divided by groups of codes, 0: by lists
     int waves, shared_pool, cap, merge_n, table_n, off_query, off_pools, off_merge, off_table, off_hist, off_misc;
 };
 
-// Computes the LDS plan of a launch; returns the dynamic LDS bytes it needs.
-size_t plan_scan(ScanParams &p);
+// How launch_scan() would launch: the way a split query is divided, the workgroup and the LDS plan; returns the dynamic LDS bytes.
+size_t plan_launch(ScanParams &p);
 
 void launch_scan(ScanParams p, int64_t nq, hipStream_t s);
 
-// The LDS plan of a launch (host only).  waves = 0: the plan plan_scan() chooses; else the layout for that
-// workgroup size (4, 8, 16 wavefronts) and pool kind.  Returns the dynamic LDS bytes; *ctl_bytes = size of the
+// The LDS plan of a launch whose slices take whole lists (host only; slices that take groups have the table, and with it the
+// layout, of nsplit = 1).  waves = 0: the plan the launcher chooses; else the layout for that workgroup size (4, 8, 16
+// wavefronts) and pool kind.  Returns the dynamic LDS bytes; *ctl_bytes = size of the
 // shared pool's control block, which follows the 2 x waves words at off_misc.
 size_t scan_lds_plan(int d, int M, int lut_fp16, int code_layout, int nprobe, int nsplit, int k, int waves,
                      int shared_pool, ScanParams *out, int *ctl_bytes);

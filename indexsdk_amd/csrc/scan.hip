@@ -1360,7 +1360,7 @@ static int resident_waves(size_t smem, int waves)
 // pools -- in 1.68 / 2.61 ms; one query over 32 lists of 9800 four-byte codes, k = 300: 209 / 99 us).
 static size_t plan_scan_by_residency(ScanParams &p);
 
-size_t plan_scan(ScanParams &p)
+static size_t plan_scan(ScanParams &p)
 {
     const ScanParams asked = p;
     const size_t smem = plan_scan_by_residency(p);
@@ -1418,7 +1418,7 @@ static size_t plan_scan_by_residency(ScanParams &p)
     return best_smem;
 }
 
-// The LDS plan of a launch as plain numbers (host only: no device is touched).  waves = 0 lets plan_scan()
+// The LDS plan of a launch by whole lists as plain numbers (host only: no device is touched).  waves = 0 lets plan_scan()
 // choose; otherwise the plan for that workgroup size and pool kind is returned as it would be laid out.
 size_t scan_lds_plan(int d, int M, int lut_fp16, int code_layout, int nprobe, int nsplit, int k, int waves,
                      int shared_pool, ScanParams *out, int *ctl_bytes)
@@ -1444,18 +1444,24 @@ size_t scan_lds_plan(int d, int M, int lut_fp16, int code_layout, int nprobe, in
 // (plans for LUTs and pools of the largest sizes; with sixteen the way of counting spills).
 constexpr int kSplitGroupsMaxLists = 512;
 
-void launch_scan(ScanParams p, int64_t nq, hipStream_t s)
+size_t plan_launch(ScanParams &p)
 {
-    if (nq == 0) {
-        return;
-    }
-    p.nq = nq;
     p.by_groups = p.nsplit > 1 && p.nprobe >= 2 * p.nsplit && p.nprobe <= kSplitGroupsMaxLists ? 1 : 0;
     size_t smem = plan_scan(p);
     if (p.by_groups && (smem > 160 * 1024 || p.waves != 8)) {   // (the longer list table may be what no longer fits)
         p.by_groups = 0;
         smem = plan_scan(p);
     }
+    return smem;
+}
+
+void launch_scan(ScanParams p, int64_t nq, hipStream_t s)
+{
+    if (nq == 0) {
+        return;
+    }
+    p.nq = nq;
+    const size_t smem = plan_launch(p);
     IXA_REQUIRE(smem <= 160 * 1024, kErrInvalidParam,
                 "IVFPQ scan needs at least %zu bytes of LDS (M=%d, k=%d, %s LUT); the limit is 163840", smem, p.M, p.k,
                 p.lut_fp16 ? "fp16" : "fp32");

@@ -11,6 +11,7 @@ ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 LIB = os.path.join(ROOT, "indexsdk_amd", "libindexsdk_amd.so")
 READELF = "/opt/rocm/llvm/bin/llvm-readelf"
 SCAN = re.compile(r"ivfpq_scan_kernelILi(\d+)E(f|6__half)Li(\d)ELi(\d+)ELb([01])EE")
+GROUPS = re.compile(r"ivfpq_scan_groups_kernelILi(n?\d+)E(f|6__half)Li(\d)ELb([01])EE")
 
 
 @pytest.fixture(scope="module")
@@ -54,6 +55,28 @@ def test_scan_kernels_of_short_codes_leave_room_for_four_workgroups(kernels):
             assert registers <= 64 and spilled == 0, (name, registers, spilled)
             seen += 1
     assert seen >= 16
+
+
+def test_scan_kernels_by_groups_have_the_registers_of_those_by_lists(kernels):
+    """Eight wavefronts; row layout: 64 registers for private pools up to M 32 and the shared pool up to M 8, as above."""
+    seen = 0
+    for name, (registers, spilled) in kernels.items():
+        m = GROUPS.search(name)
+        if m:
+            assert spilled == 0 and registers <= 256, (name, registers, spilled)
+            if m.group(3) == "0" and not m.group(1).startswith("n") and 0 < int(m.group(1)) <= (8 if m.group(4) == "1" else 32):
+                assert registers <= 64, (name, registers)
+                seen += 1
+    assert seen >= 16
+
+
+def test_encoders_do_not_spill(kernels):
+    """32 vectors and the fragments of 256 codewords per wavefront: two wavefronts per SIMD up to 24 dimensions, one at 32."""
+    encoders = {n: v for n, v in kernels.items() if "pq_encode_kernelILi" in n}
+    assert len(encoders) == 11
+    for name, (registers, spilled) in encoders.items():
+        dsub = int(re.search(r"pq_encode_kernelILi(\d+)E", name).group(1))
+        assert spilled == 0 and registers <= (256 if dsub <= 24 else 512), (name, registers, spilled)
 
 
 def test_merge_of_slices(kernels):
