@@ -23,20 +23,27 @@ struct PqStrides {
 constexpr float kPqFar = 3.402823466e+38f;   // a codeword at this distance or farther is never chosen
 
 // A workgroup of four wavefronts encodes one sub-quantizer of a block of vectors, 32 vectors of a wavefront at a time.
-//   1. u = x.c - |c|^2 / 2 of 32 vectors and all 256 codewords on the bf16 matrix cores.  Vectors and codewords are split into
-//      hi + lo (x = hi + lo + rest, |rest| <= 2^-18 |x|) and laid side by side in K: [hi | hi | lo | 1 1 1] against
+//   1. u = x.c - |c|^2 / 2 of 32 vectors and all 256 codewords on the bf16 matrix cores, both relative to a centre (the mean of
+//      eight codewords), so that what sub-vectors have in common does not widen the error bound.  Vectors and codewords are split
+//      into hi + lo (x = hi + lo + rest, |rest| <= 2^-18 |x|) and laid side by side in K: [hi | hi | lo | 1 1 1] against
 //      [hi | lo | hi | the three parts of -|c|^2 / 2], so up to four dimensions are ONE matrix instruction per 32 codewords.
 //      The codewords' fragments are made once per workgroup and stay in registers (in LDS above eight dimensions).
 //   2. A lane owns one vector and 16 codewords of each block of 32 (the other half of the wavefront the others): it keeps the
-//      largest u of every 16, the best 16 and the runner-up, then the two halves compare.
-//   3. The winning 16 are decided by the reference's arithmetic, eight by either half.  Where the runner-up is within the error
-//      bound, the wavefront evaluates all 256 codewords of that vector.
+//      largest u of every 16.  A group of 16 whose largest u is within the error bound of the vector's largest is in reach.
+//   3. The reference's arithmetic decides among the groups in reach, one (eight codewords by either half) in most vectors.  Where
+//      some vector of the wavefront has more than kPqWalk of its 16 groups in reach (codewords that are equal, or nearly so), the
+//      wavefront walks through all 256 instead, and through those of its next kPqWalks steps without asking the matrix cores.
+// The bound: distances decide by |x|^2 - 2 u, so a lead of u decides when twice it exceeds the errors of both sides:
+//   a u misses at most 3 x 2^-18 |x||c| and its K + dsub sums (2^-24 of at most |x||c| + |c|^2 / 2 each), a canonical
+//   distance (dsub + 2) 2^-24 of itself, at most (|x| + |c|)^2, and the differences from the centre, rounded once, move a squared
+//   distance by 2 x 2^-24 (|x| + |c|)^2.  Lengths below 1e-15, where products may vanish, decide nothing.
 // Per 32 vectors: KS matrix instructions and a maximum over 16 per block, and 16 distances, where every lane walking 256
 // codewords for its own vector took 256 of them: 20000 x 32 sub-quantizers of 4 dimensions 55 -> 20 us,
-//   131072 x 32 280 -> 70, 20000 x 4 of 32 dimensions 75 -> 34.
-//   The bound: distances decide by |x|^2 - 2 u, so a lead of u decides when twice it exceeds the errors of both sides:
-//   a u misses at most 3 x 2^-18 |x||c| and its K + dsub sums (2^-24 of at most |x||c| + |c|^2 / 2 each), a canonical
-//   distance (dsub + 2) 2^-24 of itself, at most (|x| + |c|)^2.  Lengths below 1e-15, where products may vanish, decide nothing.
+//   131072 x 32 280 -> 70, 20000 x 4 of 32 dimensions 75 -> 34.  Adding 100000 x 64 of 2 dimensions to two lists, every lane walking
+//   / this: 864 / 303 us; an offset of 30 851 / 305; codewords in runs of eight equal ones 920 / 395 (4 of 32 dimensions: 858 / 352,
+//   805 / 290, 832 / 368).
+constexpr int kPqWalk = 11, kPqWalks = 7;
+
 template <int DSUB>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DSUB > 24 ? 1 : 2))) void pq_encode_kernel(const float *__restrict__ x, int64_t n, PqStrides st, int M,
                                                         const float *__restrict__ codebook, uint8_t *__restrict__ codes,
@@ -61,14 +68,25 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DSUB > 24 ?
         return slot < DSUB ? first[slot] : (slot < 2 * DSUB ? second[slot - DSUB]
                : (slot < 3 * DSUB ? third[slot - 2 * DSUB] : (slot < K ? tail[slot - 3 * DSUB] : (__bf16)0.f)));
     };
+    float centre[DSUB];   // the same in every lane: scalar registers
+#pragma unroll
+    for (int t = 0; t < DSUB; t++) {
+        float sum = 0.f;
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            sum += codebook[((int64_t)m * 256 + 32 * j) * DSUB + t];
+        }
+        sum = fabsf(sum) < 1e38f ? 0.125f * sum : 0.f;
+        centre[t] = __uint_as_float((uint32_t)__builtin_amdgcn_readfirstlane((int)__float_as_uint(sum)));
+    }
     {
         const float *src = codebook + ((int64_t)m * 256 + tid) * DSUB;
         __bf16 hi[DSUB], lo[DSUB], part[3];
         float sq = 0.f;
 #pragma unroll
         for (int t = 0; t < DSUB; t++) {
-            const float c = src[t];
-            cb[tid * DSUB + t] = c;
+            cb[tid * DSUB + t] = src[t];
+            const float c = src[t] - centre[t];
             sq += c * c;
             hi[t] = (__bf16)c;
             lo[t] = (__bf16)(c - (float)hi[t]);
@@ -120,124 +138,127 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DSUB > 24 ?
         }
     };
     fetch(i_first + wave * 32);
+    int walks = 0;   // steps that are walked without asking first (the same in every lane)
     for (int64_t i0 = i_first + wave * 32; i0 < i_end; i0 += 128) {
         float sub[DSUB];
-        __bf16 hi[DSUB], lo[DSUB];
-        const __bf16 ones[3] = {(__bf16)1.f, (__bf16)1.f, (__bf16)1.f};
-        float sq = 0.f;
 #pragma unroll
         for (int t = 0; t < DSUB; t++) {
             sub[t] = next[t];
-            sq += sub[t] * sub[t];
-            hi[t] = (__bf16)sub[t];
-            lo[t] = (__bf16)(sub[t] - (float)hi[t]);
         }
         fetch(i0 + 128);
-        bf16x8 vec[KS];
-#pragma unroll
-        for (int ks = 0; ks < KS; ks++) {
-            bf16x8 f0, f1;
-#pragma unroll
-            for (int t = 0; t < 8; t++) {
-                f0[t] = slot_of(ks * 16 + t, hi, hi, lo, ones);
-                f1[t] = slot_of(ks * 16 + 8 + t, hi, hi, lo, ones);
-            }
-            vec[ks] = half ? f1 : f0;
-        }
-        // the largest u of the lane's 16 codewords of each block: the best, its block, and the next
-        float m1 = -kPqFar, m2 = -kPqFar;
-        int blk = 0;
-#pragma unroll
-        for (int b = 0; b < 8; b++) {
-            if constexpr (!kInRegisters) {
-                asm volatile("" ::: "memory");   // the fragments stay in LDS
-            }
-            v16f acc{};
-#pragma unroll
-            for (int ks = 0; ks < KS; ks++) {
-                acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kInRegisters ? own[kInRegisters ? b : 0][ks] : frag[b][ks][lane], vec[ks],
-                                                              acc, 0, 0, 0);
-            }
-            float top = acc[0];
-#pragma unroll
-            for (int r = 1; r < 16; r++) {
-                top = fmaxf(top, acc[r]);
-            }
-            m2 = __builtin_amdgcn_fmed3f(m1, m2, top);
-            blk = top > m1 ? b : blk;
-            m1 = fmaxf(m1, top);
-        }
-        const float o1 = __shfl_xor(m1, 32), o2 = __shfl_xor(m2, 32);
-        const int oblk = __shfl_xor(blk, 32);
-        const float len = sqrtf(sq), mag = len * cmax + 0.5f * cmax * cmax, far = len + cmax;
-        const float need = 2.f * (3.f / 262144.f * len * cmax + (float)(K + DSUB + 4) * 5.9604645e-8f * mag) +
-                           (float)(DSUB + 4) * 5.9604645e-8f * far * far;
-        // (an undefined or infinite bound decides nothing)
-        const bool decided = fmaxf(m1, o1) - fmaxf(fminf(m1, o1), fmaxf(m2, o2)) > need && far > 1e-15f;
-        const bool mine = m1 > o1;
-        const int first = (mine ? blk : oblk) * 32 + (mine ? half : 1 - half) * 4;   // the 16: first + 8 g + t, t < 4
         float best = kPqFar;
         int arg = 0;
+        auto distance = [&](int k) {
+            float dist = 0.f;
 #pragma unroll
-        for (int g = 0; g < 2; g++) {
+            for (int j = 0; j < DSUB; j++) {
+                const float diff = __fsub_rn(sub[j], cb[k * DSUB + j]);
+                dist = __fadd_rn(dist, __fmul_rn(diff, diff));
+            }
+            return dist;
+        };
+        bool walk = walks > 0;
+        walks -= walk ? 1 : 0;
+        if (!walk) {
+            __bf16 hi[DSUB], lo[DSUB];
+            const __bf16 ones[3] = {(__bf16)1.f, (__bf16)1.f, (__bf16)1.f};
+            float sq = 0.f;
 #pragma unroll
-            for (int t = 0; t < 4; t++) {
-                const int k = first + 8 * (2 * half + g) + t;
-                float dist = 0.f;
+            for (int t = 0; t < DSUB; t++) {
+                const float v = sub[t] - centre[t];
+                sq += v * v;
+                hi[t] = (__bf16)v;
+                lo[t] = (__bf16)(v - (float)hi[t]);
+            }
+            bf16x8 vec[KS];
 #pragma unroll
-                for (int j = 0; j < DSUB; j++) {
-                    const float diff = __fsub_rn(sub[j], cb[k * DSUB + j]);
-                    dist = __fadd_rn(dist, __fmul_rn(diff, diff));
+            for (int ks = 0; ks < KS; ks++) {
+                bf16x8 f0, f1;
+#pragma unroll
+                for (int t = 0; t < 8; t++) {
+                    f0[t] = slot_of(ks * 16 + t, hi, hi, lo, ones);
+                    f1[t] = slot_of(ks * 16 + 8 + t, hi, hi, lo, ones);
                 }
+                vec[ks] = half ? f1 : f0;
+            }
+            float top[8];   // the largest u of the lane's 16 codewords of each block
+#pragma unroll
+            for (int b = 0; b < 8; b++) {
+                if constexpr (!kInRegisters) {
+                    asm volatile("" ::: "memory");   // the fragments stay in LDS
+                }
+                v16f acc{};
+#pragma unroll
+                for (int ks = 0; ks < KS; ks++) {
+                    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kInRegisters ? own[kInRegisters ? b : 0][ks] : frag[b][ks][lane], vec[ks],
+                                                                  acc, 0, 0, 0);
+                }
+                top[b] = acc[0];
+#pragma unroll
+                for (int r = 1; r < 16; r++) {
+                    top[b] = fmaxf(top[b], acc[r]);
+                }
+            }
+            float lead = top[0];
+#pragma unroll
+            for (int b = 1; b < 8; b++) {
+                lead = fmaxf(lead, top[b]);
+            }
+            lead = fmaxf(lead, __shfl_xor(lead, 32));
+            const float len = sqrtf(sq), mag = len * cmax + 0.5f * cmax * cmax, far = len + cmax;
+            const float need = 2.f * (3.f / 262144.f * len * cmax + (float)(K + DSUB + 4) * 5.9604645e-8f * mag) +
+                               (float)(DSUB + 7) * 5.9604645e-8f * far * far;
+            // (written so that a bound or a u that is undefined, and a bound that is infinite, leave no group out)
+            const float reach = far > 1e-15f ? lead - need : -__builtin_inff();
+            uint32_t todo = 0;   // groups in reach: bit = block, + 8 where the upper half of the wavefront has them
+#pragma unroll
+            for (int b = 0; b < 8; b++) {
+                todo |= top[b] < reach ? 0u : 1u << b;
+            }
+            todo = i0 + l32 < i_end ? todo << (8 * half) : 0u;
+            todo |= (uint32_t)__shfl_xor((int)todo, 32);
+            walk = __ballot(__popc(todo) > kPqWalk) != 0;
+            walks = walk ? kPqWalks : 0;
+            while (!walk && __ballot(todo != 0) != 0) {
+                if (todo != 0) {
+                    const int at = __builtin_ctz(todo);
+                    const int first = (at & 7) * 32 + (at >> 3) * 4;   // the 16: first + 8 g + t, g < 4, t < 4
+                    float near = kPqFar;
+                    int k_near = 256;
+#pragma unroll
+                    for (int g = 0; g < 2; g++) {
+#pragma unroll
+                        for (int t = 0; t < 4; t++) {
+                            const int k = first + 8 * (2 * half + g) + t;
+                            const float dist = distance(k);
+                            if (dist < near) {
+                                near = dist;
+                                k_near = k;
+                            }
+                        }
+                    }
+                    const bool nearer = near < best || (near == best && k_near < arg);
+                    best = nearer ? near : best;
+                    arg = nearer ? k_near : arg;
+                    todo &= todo - 1;
+                }
+            }
+        }
+        if (walk) {   // all codewords, the even ones by the lower half of the wavefront
+#pragma unroll 4
+            for (int j = 0; j < 128; j++) {
+                const int k = 2 * j + half;
+                const float dist = distance(k);
                 if (dist < best) {
                     best = dist;
                     arg = k;
                 }
             }
         }
-        {   // the other half's eight; of equal distances the smaller codeword (half 0 has those)
+        {   // what the other half found; of equal distances the smaller codeword
             const float ob = __shfl_xor(best, 32);
             const int oa = __shfl_xor(arg, 32);
-            arg = ob < best || (ob == best && half == 1) ? oa : arg;
-        }
-        unsigned long long open = __ballot(!decided && half == 0 && i0 + l32 < i_end);
-        for (; open != 0; open &= open - 1) {
-            const int v = __builtin_ctzll(open);
-            float near = kPqFar;
-            int at = 0;
-            float one[DSUB];
-#pragma unroll
-            for (int j = 0; j < DSUB; j++) {
-                one[j] = __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(sub[j]), v));
-            }
-#pragma unroll
-            for (int q = 0; q < 4; q++) {
-                const int k = q * 64 + lane;
-                float dist = 0.f;
-#pragma unroll
-                for (int j = 0; j < DSUB; j++) {
-                    const float diff = __fsub_rn(one[j], cb[k * DSUB + j]);
-                    dist = __fadd_rn(dist, __fmul_rn(diff, diff));
-                }
-                if (dist < near) {
-                    near = dist;
-                    at = k;
-                }
-            }
-            float least = near;
-            for (int o = 32; o > 0; o >>= 1) {
-                least = fminf(least, __shfl_xor(least, o));
-            }
-            int low = near == least ? at : 256;
-            if (__popcll(__ballot(near == least)) > 1) {
-                for (int o = 32; o > 0; o >>= 1) {
-                    const int other = __shfl_xor(low, o);
-                    low = other < low ? other : low;
-                }
-            } else {
-                low = __builtin_amdgcn_readlane(low, __builtin_ctzll(__ballot(near == least)));
-            }
-            arg = l32 == v ? low : arg;
+            arg = ob < best || (ob == best && oa < arg) ? oa : arg;
         }
         if (half == 0 && i0 + l32 < i_end) {
             codes[(i0 + l32) * st.ci + m * st.cm] = (uint8_t)arg;
