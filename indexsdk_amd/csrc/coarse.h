@@ -6,6 +6,8 @@ namespace ixa {
 
 // out[i] = |x_i|^2, accumulated left to right in fp32.
 void launch_sqnorm_rows(const float *x, int64_t n, int d, float *out, hipStream_t s);
+// the same, and centred[i] = |x_i - centre|^2 added up in some order; d % 4 == 0, operands 16-byte aligned
+void launch_sqnorm_rows_centred(const float *x, int64_t n, int d, const float *centre, float *out, float *centred, hipStream_t s);
 
 // Filtered epilogue of the score kernels: instead of storing the scores, every score <= tau[row]
 // is appended as a key (ordered score << 32 | col_base + col) to cand[row * cap + cnt[row]++].

@@ -41,8 +41,12 @@ __global__ __launch_bounds__(256) void sqnorm_rows_kernel(const float *__restric
 // them at a time (four 128-bit loads per lane, 256 contiguous bytes per row), transpose the chunk
 // through LDS, and lanes 0..15 each add their own row's 64 squares in column order; the next chunk's
 // loads are in flight meanwhile.  The order of additions per row is unchanged.
+// CENTRED: centred[i] = |x_i - centre|^2 as well, added up in some order.
+template <bool CENTRED = false>
 __device__ __forceinline__ void sqnorm_rows_tiled_block(const float *__restrict__ x, int64_t n, int d,
-                                                        float *__restrict__ out, int64_t block)
+                                                        float *__restrict__ out, int64_t block,
+                                                        const float *__restrict__ centre = nullptr,
+                                                        float *__restrict__ centred = nullptr)
 {
     __shared__ float tile[4][16][65];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -62,9 +66,20 @@ __device__ __forceinline__ void sqnorm_rows_tiled_block(const float *__restrict_
     float4 cur[4], nxt[4];
     fetch(0, cur);
     float s = 0.0f;
+    float sq[4] = {0.f, 0.f, 0.f, 0.f};
     for (int c0 = 0; c0 < d; c0 += 64) {
         if (c0 + 64 < d) {
             fetch(c0 + 64, nxt);
+        }
+        if constexpr (CENTRED) {
+            if (c0 + 4 * cg < d) {
+                const float4 m = *reinterpret_cast<const float4 *>(centre + c0 + 4 * cg);
+#pragma unroll
+                for (int t = 0; t < 4; t++) {
+                    const float a = cur[t].x - m.x, b = cur[t].y - m.y, c = cur[t].z - m.z, e = cur[t].w - m.w;
+                    sq[t] += a * a + b * b + (c * c + e * e);
+                }
+            }
         }
 #pragma unroll
         for (int t = 0; t < 4; t++) {
@@ -91,12 +106,39 @@ __device__ __forceinline__ void sqnorm_rows_tiled_block(const float *__restrict_
     if (lane < 16 && row0 + lane < n) {
         out[row0 + lane] = s;
     }
+    if constexpr (CENTRED) {
+#pragma unroll
+        for (int t = 0; t < 4; t++) {
+            for (int o = 8; o > 0; o >>= 1) {
+                sq[t] += __shfl_xor(sq[t], o);
+            }
+            const int64_t r = row0 + rsub + 4 * t;
+            if (cg == 0 && r < n) {
+                centred[r] = sq[t];
+            }
+        }
+    }
 }
 
 __global__ __launch_bounds__(256) void sqnorm_rows_tiled_kernel(const float *__restrict__ x, int64_t n, int d,
                                                                 float *__restrict__ out)
 {
     sqnorm_rows_tiled_block(x, n, d, out, blockIdx.x);
+}
+
+__global__ __launch_bounds__(256) void sqnorm_rows_centred_kernel(const float *__restrict__ x, int64_t n, int d,
+                                                                  const float *__restrict__ centre, float *__restrict__ out,
+                                                                  float *__restrict__ centred)
+{
+    sqnorm_rows_tiled_block<true>(x, n, d, out, blockIdx.x, centre, centred);
+}
+
+void launch_sqnorm_rows_centred(const float *x, int64_t n, int d, const float *centre, float *out, float *centred, hipStream_t s)
+{
+    IXA_REQUIRE(d % 4 == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0, kErrInner, "centred lengths of unaligned rows");
+    if (n > 0) {
+        hipLaunchKernelGGL(sqnorm_rows_centred_kernel, dim3((unsigned)((n + 63) / 64)), dim3(256), 0, s, x, n, d, centre, out, centred);
+    }
 }
 
 void launch_sqnorm_rows(const float *x, int64_t n, int d, float *out, hipStream_t s)

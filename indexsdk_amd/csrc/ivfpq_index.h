@@ -196,6 +196,7 @@ private:
             stats();
         }
     }
+    AssignCentroids centroids_centred_;                    // where resident_assign_serves
     float cmax_ = 0.f;                                      // largest centroid norm
     int dp_ = 0;                                            // d rounded up to a multiple of 32
     // arena

@@ -643,6 +643,10 @@ void IvfpqIndex::borrow_from(const IvfpqIndex &o)
     centroids_split_.borrow(o.centroids_split_);
     centroids_tiled_.borrow(o.centroids_tiled_);
     cnorm_pad_.borrow(o.cnorm_pad_);
+    centroids_centred_.centre.borrow(o.centroids_centred_.centre);
+    centroids_centred_.rows.borrow(o.centroids_centred_.rows);
+    centroids_centred_.norms.borrow(o.centroids_centred_.norms);
+    centroids_centred_.longest.borrow(o.centroids_centred_.longest);
     codes_.borrow(o.codes_);
     ids_.borrow(o.ids_);
     list_off_dev_.borrow(o.list_off_dev_);
@@ -687,6 +691,9 @@ void IvfpqIndex::derive_from_centroids()
     dp_ = (int)round_up(d_, 32);
     centroids_split_.resize((size_t)nlist_ * 3 * dp_);
     launch_split_bf16x3(centroids_.data(), nlist_, d_, dp_, true, centroids_split_.data(), stream_);
+    if (resident_assign_serves(nullptr, centroids_.data(), nlist_, d_)) {
+        launch_centre_centroids(centroids_.data(), nlist_, d_, cnorm_.data(), centroids_centred_, stream_);
+    }
     std::vector<float> cn((size_t)nlist_);
     cnorm_.download(cn.data(), cn.size(), stream_);
     cmax_ = std::sqrt(*std::max_element(cn.begin(), cn.end()));
@@ -819,7 +826,6 @@ void IvfpqIndex::coarse_select(const float *x_dev, int64_t n, int nout, int sele
         launch_select_rows(ws_exact_.data(), n, nlist_, nlist_, nout, out_ids, 0, nullptr, stream_);
         return;
     }
-    ws_qn_.resize((size_t)n);
     // The nearest list of every vector (training, adding): decided on the device, no score written, no verdict to read.  Adding,
     // us (score matrix or sampled bound / this): 1M x 128 to 1024 lists 10996 / 4175, 20000 to 4096 590 / 221, 100000 to 16384
     // 2508 / 1524, 100 to 1000 116 / 91; 50000 x 200 to 1500 1165 / 422; 20000 x 768 to 1024 898 / 650.
@@ -828,11 +834,11 @@ void IvfpqIndex::coarse_select(const float *x_dev, int64_t n, int nout, int sele
         last_coarse_exact_ = true;
         last_coarse_plan_ = 0;
         last_coarse_n_ = n;
-        launch_sqnorm_rows(x_dev, n, d_, ws_qn_.data(), stream_);
-        launch_resident_assign(x_dev, n, centroids_.data(), nlist_, d_, ws_qn_.data(), cnorm_.data(), cmax_, out_ids, ws_assign_,
+        launch_resident_assign(x_dev, n, centroids_.data(), nlist_, d_, cnorm_.data(), cmax_, centroids_centred_, out_ids, ws_assign_,
                                cfg_.scratch_bytes, stream_);
         return;
     }
+    ws_qn_.resize((size_t)n);
     if (cfg_.coarse_bf16) {   // the queries' norms and their bf16 x 3 split in one launch
         ws_xsplit_.resize((size_t)n * 3 * dp_);
         launch_sqnorm_and_split_bf16x3(x_dev, n, d_, dp_, ws_qn_.data(), ws_xsplit_.data(), stream_);

@@ -51,7 +51,7 @@ constexpr float kNoRow = -__builtin_inff();   // accumulator start of a row outs
 constexpr float kNoCentroid = -3e38f;   // of a centroid past the last one (a number: low bits are put into the sums)
 // LDS behind the query tile of a filtered launch: {bound, norm, test value, -} per query, the wavefronts' queues
 constexpr int filter_lds(int qt) { return qt * 16 + kWaves * kQueueKeys * 16; }
-constexpr int assign_lds(int qt) { return qt * 4; }   // -|c|^2 / 2 per centroid
+constexpr int assign_lds(int qt, int k) { return (qt + k) * 4; }   // a start per centroid; the centre, k = dimensions of whole batches
 constexpr int kLdsLimit = 160 * 1024;
 
 // hi and lo of eight numbers
@@ -121,7 +121,8 @@ enum { kStore = 0, kFilter = 1, kAssign = 2 };
 //   kFilter  admitted keys are appended;
 //   kAssign  the "queries" are centroids, the base rows vectors: of every tile of centroids the best two of each vector and the
 //            third value.  The matrix operands change places, so that a lane owns ONE vector and 16 centroids per block, and
-//            the accumulators start from -|c|^2 / 2, kept in LDS.
+//            the accumulators start from -qn / 2 of the centroid, kept in LDS.  The centroids are relative to a centre (bn: its
+//            d numbers), which is taken from the vectors between their load and their split.
 template <int RA, int SPB, int MODE>
 __global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) void resident_f32_kernel(
     const float *__restrict__ Q, int64_t nq, const float *__restrict__ B, int64_t nb, int d, int nbat,
@@ -154,7 +155,8 @@ __global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(2, 
     const uint32_t lds_base = (uint32_t)reinterpret_cast<size_t>((__attribute__((address_space(3))) unsigned char *)lds);
     const uint32_t a_lane = lds_base + (uint32_t)(half * (QT * 32) + l32 * 16);
     float4 *meta = reinterpret_cast<float4 *>(lds + (size_t)nbat * kBatchLds);   // {tau, |q|^2, test value, -}
-    float *start = reinterpret_cast<float *>(meta);   // kAssign: -|c|^2 / 2 per centroid instead
+    float *start = reinterpret_cast<float *>(meta);   // kAssign: the starts of the centroids' sums, and the centre
+    float *centre = start + QT;
     uint4 *queue = reinterpret_cast<uint4 *>(meta + QT) + wave * kQueueKeys;
     int qcount = 0;   // keys in this wavefront's queue (wave-uniform)
     // every queued key takes its place in its query's candidate buffer; 64 lanes, one key each
@@ -265,6 +267,11 @@ __global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(2, 
                     const int64_t c = (int64_t)tm * QT + tid;
                     start[tid] = c < nq ? -0.5f * qn[c] : kNoCentroid;
                 }
+                if (cur_tm < 0) {
+                    for (int k = tid; k < nbat * SPB * 16; k += kWaves * 64) {
+                        centre[k] = k < d ? bn[k] : 0.f;
+                    }
+                }
             }
             cur_tm = tm;
             __syncthreads();
@@ -318,6 +325,7 @@ __global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(2, 
             }
         }
         uint32_t addr = a_lane;
+        const float *centre_at = centre + 4 * half;
         // one batch: its rows are split, the loads that follow it sent for, the products added
         auto batch = [&](auto first, auto last, const float *next_row, int next_batch) {
             constexpr bool FIRST = decltype(first)::value, LAST = decltype(last)::value;
@@ -328,8 +336,13 @@ __global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(2, 
             bf16x8 bh[SPB], bl[SPB];
 #pragma unroll
             for (int t = 0; t < SPB; t++) {
+                if constexpr (ASSIGN) {
+                    raw[2 * t] -= *reinterpret_cast<const v4f *>(centre_at + 16 * t);
+                    raw[2 * t + 1] -= *reinterpret_cast<const v4f *>(centre_at + 16 * t + 8);
+                }
                 split8(raw[2 * t], raw[2 * t + 1], bh[t], bl[t]);
             }
+            centre_at += 16 * SPB;
             if constexpr (LAST && !ASSIGN) {
                 load_norms(n_j);
             }
@@ -498,13 +511,13 @@ struct Args {
     hipStream_t s;
 };
 
-constexpr int extra_lds(int mode, int qt) { return mode == kFilter ? filter_lds(qt) : (mode == kAssign ? assign_lds(qt) : 0); }
+constexpr int extra_lds(int mode, int qt, int k) { return mode == kFilter ? filter_lds(qt) : (mode == kAssign ? assign_lds(qt, k) : 0); }
 
 template <int RA, int SPB, int MODE>
 void launch_shape(const Args &a, int nbat)
 {
     constexpr int QT = RA * 32;
-    const size_t smem = (size_t)nbat * SPB * QT * 64 + extra_lds(MODE, QT);
+    const size_t smem = (size_t)nbat * SPB * QT * 64 + extra_lds(MODE, QT, nbat * SPB * 16);
     auto kern = resident_f32_kernel<RA, SPB, MODE>;
     static std::atomic<bool> configured{false};   // per instantiation
     if (!configured) {
@@ -568,22 +581,36 @@ void launch_mode(const Args &a)
 
 // ---- what the tiles' best become ------------------------------------------------------------------------------------------
 
-// By how much a u has to lead another for the canonical scores to be in that order.  Both scores |x|^2 - 2 u are within E of the
-// canonical ones, and the places in the low bits have moved each u by at most 2^-17 |u|, |u| <= |x| cmax + cmax^2 / 2.  Infinite
-// or undefined where nothing can be decided: so for lengths whose products come near the start of a padding centroid (-3e38),
-// where a sum may overflow.  An infinite sum with a place in its low bits is a signalling NaN, which makes max_number forget the
-// best so far; and a number below -3e38 would be passed over.
-__device__ __forceinline__ float assign_need(float norm, float cmax, float err_scale, float round_scale)
-{
-    const float reach = sqrtf(norm) * cmax + cmax * cmax;
-    return reach < 1e37f ? score_margin(norm, cmax, err_scale, round_scale) + 1.6e-5f * reach : __builtin_inff();
-}
+// By how much a u has to lead another for the canonical scores to be in that order.  With a = |x - centre|, b = the largest
+// |c - centre|, L = |x| and cmax the largest |c|, what separates -2 u from the canonical score of the same centroid, but for
+// what all centroids share:
+//   the canonical score  (|x|^2 + |c|^2) - g - g: g's d products and sums, 2 (d + 1) 2^-24 L cmax, and three roundings,
+//                        3 x 2^-24 (L + cmax)^2.  Its |c|^2, which is rounded itself, is the one that u starts from
+//                        (launch_centre_centroids), so that makes no difference;
+//   u                    the products that the splits miss, 2 x 3 x 2^-18 a b, and 3 dp sums of numbers up to a b + b^2 / 2;
+//   the differences from the centre, rounded once: 2 x 2^-24 (a + b)^2 of a squared distance;
+//   the places in the low bits: 2^-17 |u| for either of two, |u| <= a b + b^2 / 2.
+// What vectors and centroids have in common is in L and cmax only.  Infinite or undefined where nothing can be decided: so for
+// lengths that lost squares (score_margin has the line), and for lengths beside which the start of a padding centroid (-3e38) is
+// not far off.  There a sum may overflow, and an infinite sum with a place in its low bits is a signalling NaN, which makes
+// max_number forget the best so far.
+struct AssignBound {
+    const float *xn, *xc;   // |x|^2 and |x - centre|^2 per vector
+    const float *cc;        // the largest |c - centre|^2
+    float cmax, exact_scale, split_scale, sum_scale;
+    __device__ __forceinline__ float need(int64_t i) const
+    {
+        const float l = sqrtf(xn[i]), a = sqrtf(xc[i]), b = sqrtf(*cc), far = l + cmax, near = a + b;
+        const float e = exact_scale * l * cmax + 4.f * 5.9604645e-8f * far * far + split_scale * a * b + sum_scale * near * near +
+                        1.6e-5f * b * near;
+        return far > 1e-12f && near > 1e-12f && far * far < 1e36f ? 1.001f * e : __builtin_inff();
+    }
+};
 
 // The best two of every vector over all tiles and the third value; a lead of more than the error bound decides, a tie of two
 // goes to `pairs` (vector, two centroids), of more (or an undefined length) to `rows`.  count: the two lists' lengths.
 __global__ __launch_bounds__(256) void assign_combine_kernel(const float4 *__restrict__ top, int tiles, int tile_centroids, int64_t n,
-                                                             const float *__restrict__ xn, float cmax, float err_scale,
-                                                             float round_scale, int32_t *__restrict__ out, int4 *__restrict__ pairs,
+                                                             AssignBound bound, int32_t *__restrict__ out, int4 *__restrict__ pairs,
                                                              int32_t *__restrict__ rows, int32_t *__restrict__ count)
 {
     const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
@@ -596,7 +623,7 @@ __global__ __launch_bounds__(256) void assign_combine_kernel(const float4 *__res
             best.merge(Best{v.x, v.y, v.z, c0 + (p & 0xffffu), c0 + (p >> 16)});
         }
     }
-    const float need = assign_need(i < n ? xn[i] : 0.f, cmax, err_scale, round_scale);
+    const float need = bound.need(i < n ? i : n - 1);
     const bool decided = i >= n || best.v1 - best.v2 > need, pair = !decided && best.v1 - best.v3 > need;
     if (i < n) {
         out[i] = (int32_t)best.p1;
@@ -640,10 +667,9 @@ __device__ __forceinline__ float canonical_l2(const float *__restrict__ x, const
 // second are evaluated where they are within reach themselves, and all centroids where the third is (100000 vectors, 16384
 // centroids, sixteen to a component of the mixture: 1.6 ms when such a vector was scored against every centroid).
 // Equal scores: the smaller number.  A NaN is never chosen; -1 where nothing else is left.
-__global__ __launch_bounds__(256) void assign_resolve_kernel(const float *__restrict__ X, const float *__restrict__ xn, int64_t n,
+__global__ __launch_bounds__(256) void assign_resolve_kernel(const float *__restrict__ X, int64_t n,
                                                              const float *__restrict__ C, const float *__restrict__ cn, int64_t nc,
-                                                             int d, float cmax, float err_scale, float round_scale,
-                                                             const float4 *__restrict__ top, int tiles, int tile_centroids,
+                                                             int d, AssignBound bound, const float4 *__restrict__ top, int tiles, int tile_centroids,
                                                              const int4 *__restrict__ pairs, const int32_t *__restrict__ rows,
                                                              const int32_t *__restrict__ count, int32_t *__restrict__ out)
 {
@@ -651,7 +677,7 @@ __global__ __launch_bounds__(256) void assign_resolve_kernel(const float *__rest
     const int64_t wave = (int64_t)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), waves = (int64_t)gridDim.x * 4;
     const int npairs = count[0], nrows = count[1];
     auto key_of = [&](int64_t row, int64_t c) {
-        const float v = canonical_l2(X + row * d, C + c * d, d, xn[row], cn[c]);
+        const float v = canonical_l2(X + row * d, C + c * d, d, bound.xn[row], cn[c]);
         return v == v ? make_key(v, (uint32_t)c) : kEmptyKey;
     };
     for (int64_t p0 = wave * 32; p0 < npairs; p0 += waves * 32) {
@@ -672,7 +698,7 @@ __global__ __launch_bounds__(256) void assign_resolve_kernel(const float *__rest
         for (int o = 32; o > 0; o >>= 1) {
             lead = fmaxf(lead, __shfl_xor(lead, o));
         }
-        const float reach = lead - assign_need(xn[row], cmax, err_scale, round_scale);
+        const float reach = lead - bound.need(row);
         key_t best = kEmptyKey;
         for (int t0 = 0; t0 < tiles; t0 += 64) {
             const int t = t0 + lane;
@@ -739,8 +765,79 @@ bool resident_assign_serves(const float *X, const float *C, int64_t nc, int d)
     return resident_f32_serves(d) && (d <= 512 || nc <= 4096) && reinterpret_cast<uintptr_t>(X) % 16 == 0 && reinterpret_cast<uintptr_t>(C) % 16 == 0;
 }
 
-void launch_resident_assign(const float *X, int64_t n, const float *C, int64_t nc, int d, const float *xn, const float *cn, float cmax,
-                            int32_t *out, AssignWorkspace &ws, int64_t scratch_bytes, hipStream_t s)
+// out[0 .. d) = the mean of up to 1024 of the centroids (a component without one: 0); *longest = 0
+__global__ __launch_bounds__(1024) void centroid_mean_kernel(const float *__restrict__ C, int64_t nc, int d, float *__restrict__ out,
+                                                             float *__restrict__ longest)
+{
+    __shared__ float part[16][64];
+    const int col = blockIdx.x * 64 + (threadIdx.x & 63), slice = threadIdx.x >> 6;
+    const int64_t count = nc < 1024 ? nc : 1024;
+    float sum = 0.f;
+    if (col < d) {
+#pragma unroll 8
+        for (int64_t r = slice; r < count; r += 16) {
+            sum += C[r * nc / count * d + col];
+        }
+    }
+    part[slice][threadIdx.x & 63] = sum;
+    __syncthreads();
+    if (slice == 0 && col < d) {
+        for (int t = 1; t < 16; t++) {
+            sum += part[t][threadIdx.x];
+        }
+        sum /= (float)count;
+        out[col] = fabsf(sum) < 1e38f ? sum : 0.f;
+    }
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        *longest = 0.f;
+    }
+}
+
+// A wavefront per centroid: rows = c - centre, norms = the number that a sum of products with it starts from, times -2: |rows|^2
+// plus what the rounding of cn = |c|^2 has added to it.
+__global__ __launch_bounds__(256) void centre_centroids_kernel(const float *__restrict__ C, int64_t nc, int d, const float *__restrict__ cn,
+                                                               const float *__restrict__ centre, float *__restrict__ rows,
+                                                               float *__restrict__ norms, float *__restrict__ longest)
+{
+    const int64_t c = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+    const int lane = threadIdx.x & 63;
+    if (c >= nc) {
+        return;
+    }
+    double apart = 0.0, whole = 0.0;
+    for (int t = lane; t < d; t += 64) {
+        const float v = C[c * d + t], r = v - centre[t];
+        rows[c * d + t] = r;
+        apart += (double)r * r;
+        whole += (double)v * v;
+    }
+    for (int o = 32; o > 0; o >>= 1) {
+        apart += __shfl_xor(apart, o);
+        whole += __shfl_xor(whole, o);
+    }
+    if (lane == 0) {
+        norms[c] = (float)(apart + ((double)cn[c] - whole));
+        const float len = (float)apart;
+        if (len == len) {   // a centroid with a NaN is nobody's nearest; (of numbers >= 0 the bits have their order)
+            atomicMax(reinterpret_cast<unsigned int *>(longest), __float_as_uint(len));
+        }
+    }
+}
+
+void launch_centre_centroids(const float *C, int64_t nc, int d, const float *cn, AssignCentroids &out, hipStream_t s)
+{
+    out.centre.resize((size_t)d);
+    out.rows.resize((size_t)nc * d);
+    out.norms.resize((size_t)nc);
+    out.longest.resize(1);
+    hipLaunchKernelGGL(centroid_mean_kernel, dim3((unsigned)((d + 63) / 64)), dim3(1024), 0, s, C, nc, d, out.centre.data(),
+                       out.longest.data());
+    hipLaunchKernelGGL(centre_centroids_kernel, dim3((unsigned)((nc + 3) / 4)), dim3(256), 0, s, C, nc, d, cn, out.centre.data(),
+                       out.rows.data(), out.norms.data(), out.longest.data());
+}
+
+void launch_resident_assign(const float *X, int64_t n, const float *C, int64_t nc, int d, const float *cn, float cmax,
+                            const AssignCentroids &centred, int32_t *out, AssignWorkspace &ws, int64_t scratch_bytes, hipStream_t s)
 {
     if (n <= 0) {
         return;
@@ -748,23 +845,28 @@ void launch_resident_assign(const float *X, int64_t n, const float *C, int64_t n
     IXA_REQUIRE(resident_assign_serves(X, C, nc, d) && nc >= 1 && n < ((int64_t)1 << 31), kErrInner, "assignment kernel does not serve these operands");
     const int qt = 32 * tile_blocks(nc, d);
     const int64_t tiles = (nc + qt - 1) / qt;
-    // vectors per pass: 16 bytes per vector and tile of centroids, 20 for what is left open
-    const int64_t page = std::min<int64_t>(n, std::max<int64_t>(kTileRows, scratch_bytes / (16 * tiles + 20) / kTileRows * kTileRows));
+    // vectors per pass: 16 bytes per vector and tile of centroids, 28 for lengths and what is left open
+    const int64_t page = std::min<int64_t>(n, std::max<int64_t>(kTileRows, scratch_bytes / (16 * tiles + 28) / kTileRows * kTileRows));
     ws.top.resize((size_t)(page * tiles));
     ws.pairs.resize((size_t)page);
+    ws.xn.resize((size_t)page);
+    ws.xc.resize((size_t)page);
     ws.rows.resize((size_t)page + 2);
     int32_t *count = ws.rows.data() + page;
-    // (the bound of resident_f32.h for L2: 3 dp products, dp the dimension rounded up to 32)
     const float u = 5.9604645e-8f;
-    const float err_scale = 2.0f * (3.0f / 262144.0f + (float)(d + 8) * u), round_scale = (float)(3 * ((d + 31) / 32 * 32) + 4) * u;
+    AssignBound bound{ws.xn.data(), ws.xc.data(), centred.longest.data(), cmax, 2.f * (float)(d + 8) * u, 6.f / 262144.f,
+                      (float)(3 * ((d + 31) / 32 * 32) + 6) * u};
     for (int64_t i0 = 0; i0 < n; i0 += page) {
         const int64_t m = std::min(page, n - i0);
         IXA_HIP(hipMemsetAsync(count, 0, 8, s));
-        launch_mode<kAssign>(Args{C, nc, X + i0 * d, m, d, cn, nullptr, kMetricL2, nullptr, 0, ScoreFilter<float>{}, ws.top.data(), s});
+        const float *xi = X + i0 * d;
+        launch_sqnorm_rows_centred(xi, m, d, centred.centre.data(), ws.xn.data(), ws.xc.data(), s);
+        launch_mode<kAssign>(Args{centred.rows.data(), nc, xi, m, d, centred.norms.data(), centred.centre.data(), kMetricL2, nullptr, 0,
+                                  ScoreFilter<float>{}, ws.top.data(), s});
         hipLaunchKernelGGL(assign_combine_kernel, dim3((unsigned)((m + 255) / 256)), dim3(256), 0, s, ws.top.data(), (int)tiles, qt, m,
-                           xn + i0, cmax, err_scale, round_scale, out + i0, ws.pairs.data(), ws.rows.data(), count);
-        hipLaunchKernelGGL(assign_resolve_kernel, dim3((unsigned)std::min<int64_t>(m, device_cus() * 2)), dim3(256), 0, s, X + i0 * d,
-                           xn + i0, m, C, cn, nc, d, cmax, err_scale, round_scale, ws.top.data(), (int)tiles, qt, ws.pairs.data(), ws.rows.data(), count, out + i0);
+                           bound, out + i0, ws.pairs.data(), ws.rows.data(), count);
+        hipLaunchKernelGGL(assign_resolve_kernel, dim3((unsigned)std::min<int64_t>(m, device_cus() * 2)), dim3(256), 0, s, xi, m, C, cn, nc,
+                           d, bound, ws.top.data(), (int)tiles, qt, ws.pairs.data(), ws.rows.data(), count, out + i0);
     }
 }
 

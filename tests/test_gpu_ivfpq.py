@@ -1077,6 +1077,60 @@ def test_assignment_of_vectors_near_the_end_of_the_range(ix, oracle, d, nlist, l
     assert np.array_equal(gpu.assign(x), want)
 
 
+# Vectors with a common offset, and components of a mixture that lie far apart beside their widths: bit for bit.
+@pytest.mark.parametrize("d,nlist", [(128, 300), (36, 1030), (260, 64), (640, 200)])
+@pytest.mark.parametrize("offset,spread", [(5.0, 1.0), (300.0, 1.0), (0.0, 20.0), (-1e6, 1.0), (1e-3, 1e-6)])
+def test_assignment_of_offset_vectors(ix, oracle, d, nlist, offset, spread):
+    rng = np.random.default_rng(d)
+    centres = spread * rng.standard_normal((13, d))
+    cent = (centres[rng.integers(0, 13, nlist)] + 0.25 * rng.standard_normal((nlist, d)) + offset).astype(np.float32)
+    x = (centres[rng.integers(0, 13, 3001)] + 0.25 * rng.standard_normal((3001, d)) + offset).astype(np.float32)
+    cent[nlist // 2] = cent[7]
+    x[::50] = cent[7]
+    gpu = ix.AscendIndexIVFPQ(d, ix.METRIC_L2, nlist, 4, 8)
+    gpu.set_trained(cent, rng.standard_normal((4, 256, d // 4)).astype(np.float32))
+    assert np.array_equal(gpu.assign(x), oracle.assign(x, cent))
+
+
+def _adding_times(ix, case):
+    """Least seconds of adding 100000 x 128 vectors of 64 components to 1024 lists, sixteen to a component: the vectors as they are, and
+    as case() makes them from the components, the widths and the offset."""
+    import ctypes
+    import time
+
+    import torch
+
+    from indexsdk_amd import _capi
+
+    rng = np.random.default_rng(11)
+    d, n, nlist = 128, 100000, 1024
+    centres, which, near = rng.standard_normal((64, d)), rng.integers(0, 64, n), 0.25 * rng.standard_normal((n, d))
+    best = []
+    for spread, offset in ((1.0, 0.0), case):
+        vectors = (spread * centres[which] + near + offset).astype(np.float32)
+        index = ix.AscendIndexIVFPQ(d, ix.METRIC_L2, nlist, 4, 8, ix.AscendIndexIVFPQConfig(niter=4))
+        index.train(vectors)
+        x = torch.from_numpy(vectors).cuda()
+        ids = torch.arange(n, device="cuda")
+        times = []
+        for _ in range(5):
+            torch.cuda.synchronize()
+            t = time.perf_counter()
+            _capi.check(_capi.load().ivfpq_add_with_ids_device(index._h, n, ctypes.c_void_p(x.data_ptr()),
+                                                               ctypes.c_void_p(ids.data_ptr())))
+            times.append(time.perf_counter() - t)
+            index.remove_range(0, n)
+        best.append(min(times))
+    return best
+
+
+def test_adding_vectors_with_an_offset_takes_about_as_long(ix):
+    """The error bound is of lengths relative to a centre: an offset of 5 in every component made adding nine times as long when it was
+    of the lengths themselves (1.5 times now)."""
+    plain, offset = _adding_times(ix, (1.0, 5.0))
+    assert offset < 3.0 * plain, (plain, offset)
+
+
 # A query split over workgroups deals groups of 64 codes to its slices in turn: lists without codes, of one code and of a remainder,
 # several groups per list and (nprobe 512: a slice skips more than 64 lists at a time) far fewer; 8 to 20 slices; private pools, the shared pool,
 # kernels for a compile-time number of sub-quantizers and not.  As in one workgroup per query (a large batch), bit for bit.
