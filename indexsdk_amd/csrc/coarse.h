@@ -6,8 +6,6 @@ namespace ixa {
 
 // out[i] = |x_i|^2, accumulated left to right in fp32.
 void launch_sqnorm_rows(const float *x, int64_t n, int d, float *out, hipStream_t s);
-// the same, and centred[i] = |x_i - centre|^2 added up in some order; d % 4 == 0, operands 16-byte aligned
-void launch_sqnorm_rows_centred(const float *x, int64_t n, int d, const float *centre, float *out, float *centred, hipStream_t s);
 
 // Filtered epilogue of the score kernels: instead of storing the scores, every score <= tau[row]
 // is appended as a key (ordered score << 32 | col_base + col) to cand[row * cap + cnt[row]++].
@@ -146,6 +144,35 @@ __device__ __forceinline__ float score_margin(float qnorm, float cmax, float err
     const bool lost = round_scale > 0.f ? qlen + cmax < 1e-12f : fminf(qlen, cmax) < 1e-13f;
     return lost ? __builtin_inff() : err_scale * qlen * cmax + round_scale * (qlen + cmax) * (qlen + cmax);
 }
+
+// By how much a u of the assignment kernel (resident_f32.hip) has to lead another for the canonical scores to be in that order.  With a = |x - centre|, b = the largest
+// |c - centre|, L = |x| and cmax the largest |c|, what separates -2 u from the canonical score of the same centroid, but for
+// what all centroids share:
+//   the canonical score  (|x|^2 + |c|^2) - g - g: g's d products and sums, 2 (d + 1) 2^-24 L cmax, and three roundings,
+//                        3 x 2^-24 (L + cmax)^2.  Its |c|^2, which is rounded itself, is the one that u starts from
+//                        (launch_centre_centroids), so that makes no difference;
+//   u                    the products that the splits miss, 2 x 3 x 2^-18 a b, and 3 dp sums of numbers up to a b + b^2 / 2;
+//   the differences from the centre, rounded once: 2 x 2^-24 (a + b)^2 of a squared distance;
+//   the places in the low bits: 2^-17 |u| for either of two, |u| <= a b + b^2 / 2.
+// What vectors and centroids have in common is in L and cmax only.  Infinite or undefined where nothing can be decided: so for
+// lengths that lost squares (score_margin has the line), and for lengths beside which the start of a padding centroid (-3e38) is
+// not far off.  There a sum may overflow, and an infinite sum with a place in its low bits is a signalling NaN, which makes
+// max_number forget the best so far.
+struct AssignBound {
+    float cmax, longest;   // the largest |c| and |c - centre|
+    float exact_scale, split_scale, sum_scale;
+    // xn = |x|^2, xc = |x - centre|^2
+    __device__ __forceinline__ float need(float xn, float xc) const
+    {
+        const float l = sqrtf(xn), a = sqrtf(xc), b = longest, far = l + cmax, near = a + b;
+        const float e = exact_scale * l * cmax + 4.f * 5.9604645e-8f * far * far + split_scale * a * b + sum_scale * near * near +
+                        1.6e-5f * b * near;
+        return far > 1e-12f && near > 1e-12f && far * far < 1e36f ? 1.001f * e : __builtin_inff();
+    }
+};
+// xn[i] = |x_i|^2 as launch_sqnorm_rows has it, need[i] = the bound above, count[0 .. 1] = 0; d % 4 == 0, operands 16-byte aligned.
+void launch_assign_bounds(const float *x, int64_t n, int d, const float *centre, AssignBound bound, float *xn, float *need,
+                          int32_t *count, hipStream_t s);
 
 // Sets *flag = 1 if some query's approximate candidate list (running[nq][ncand], ascending keys) is
 // not provably a superset of its best nout centroids; see score_ring.hip.  finite_only: a query whose norm is not

@@ -41,12 +41,12 @@ __global__ __launch_bounds__(256) void sqnorm_rows_kernel(const float *__restric
 // them at a time (four 128-bit loads per lane, 256 contiguous bytes per row), transpose the chunk
 // through LDS, and lanes 0..15 each add their own row's 64 squares in column order; the next chunk's
 // loads are in flight meanwhile.  The order of additions per row is unchanged.
-// CENTRED: centred[i] = |x_i - centre|^2 as well, added up in some order.
-template <bool CENTRED = false>
+// BOUNDS: need[i] = the bound of the assignment kernel as well, from these sums and |x_i - centre|^2 (in some order).
+template <bool BOUNDS = false>
 __device__ __forceinline__ void sqnorm_rows_tiled_block(const float *__restrict__ x, int64_t n, int d,
                                                         float *__restrict__ out, int64_t block,
-                                                        const float *__restrict__ centre = nullptr,
-                                                        float *__restrict__ centred = nullptr)
+                                                        const float *__restrict__ centre = nullptr, AssignBound bound = {},
+                                                        float *__restrict__ need = nullptr)
 {
     __shared__ float tile[4][16][65];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -71,7 +71,7 @@ __device__ __forceinline__ void sqnorm_rows_tiled_block(const float *__restrict_
         if (c0 + 64 < d) {
             fetch(c0 + 64, nxt);
         }
-        if constexpr (CENTRED) {
+        if constexpr (BOUNDS) {
             if (c0 + 4 * cg < d) {
                 const float4 m = *reinterpret_cast<const float4 *>(centre + c0 + 4 * cg);
 #pragma unroll
@@ -103,19 +103,21 @@ __device__ __forceinline__ void sqnorm_rows_tiled_block(const float *__restrict_
             cur[t] = nxt[t];
         }
     }
-    if (lane < 16 && row0 + lane < n) {
-        out[row0 + lane] = s;
-    }
-    if constexpr (CENTRED) {
+    float away = 0.f;   // |x - centre|^2 of row `lane` (lanes 0..15)
+    if constexpr (BOUNDS) {
 #pragma unroll
         for (int t = 0; t < 4; t++) {
             for (int o = 8; o > 0; o >>= 1) {
                 sq[t] += __shfl_xor(sq[t], o);
             }
-            const int64_t r = row0 + rsub + 4 * t;
-            if (cg == 0 && r < n) {
-                centred[r] = sq[t];
-            }
+            const float v = __shfl(sq[t], 16 * (lane & 3));
+            away = lane >> 2 == t ? v : away;
+        }
+    }
+    if (lane < 16 && row0 + lane < n) {
+        out[row0 + lane] = s;
+        if constexpr (BOUNDS) {
+            need[row0 + lane] = bound.need(s, away);
         }
     }
 }
@@ -126,19 +128,21 @@ __global__ __launch_bounds__(256) void sqnorm_rows_tiled_kernel(const float *__r
     sqnorm_rows_tiled_block(x, n, d, out, blockIdx.x);
 }
 
-__global__ __launch_bounds__(256) void sqnorm_rows_centred_kernel(const float *__restrict__ x, int64_t n, int d,
-                                                                  const float *__restrict__ centre, float *__restrict__ out,
-                                                                  float *__restrict__ centred)
+__global__ __launch_bounds__(256) void assign_bounds_kernel(const float *__restrict__ x, int64_t n, int d,
+                                                            const float *__restrict__ centre, AssignBound bound,
+                                                            float *__restrict__ xn, float *__restrict__ need, int32_t *__restrict__ count)
 {
-    sqnorm_rows_tiled_block<true>(x, n, d, out, blockIdx.x, centre, centred);
+    if (blockIdx.x == 0 && threadIdx.x < 2) {
+        count[threadIdx.x] = 0;
+    }
+    sqnorm_rows_tiled_block<true>(x, n, d, xn, blockIdx.x, centre, bound, need);
 }
 
-void launch_sqnorm_rows_centred(const float *x, int64_t n, int d, const float *centre, float *out, float *centred, hipStream_t s)
+void launch_assign_bounds(const float *x, int64_t n, int d, const float *centre, AssignBound bound, float *xn, float *need,
+                          int32_t *count, hipStream_t s)
 {
-    IXA_REQUIRE(d % 4 == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0, kErrInner, "centred lengths of unaligned rows");
-    if (n > 0) {
-        hipLaunchKernelGGL(sqnorm_rows_centred_kernel, dim3((unsigned)((n + 63) / 64)), dim3(256), 0, s, x, n, d, centre, out, centred);
-    }
+    IXA_REQUIRE(n > 0 && d % 4 == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0, kErrInner, "bounds of unaligned rows");
+    hipLaunchKernelGGL(assign_bounds_kernel, dim3((unsigned)((n + 63) / 64)), dim3(256), 0, s, x, n, d, centre, bound, xn, need, count);
 }
 
 void launch_sqnorm_rows(const float *x, int64_t n, int d, float *out, hipStream_t s)

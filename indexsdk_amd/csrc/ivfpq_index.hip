@@ -643,10 +643,7 @@ void IvfpqIndex::borrow_from(const IvfpqIndex &o)
     centroids_split_.borrow(o.centroids_split_);
     centroids_tiled_.borrow(o.centroids_tiled_);
     cnorm_pad_.borrow(o.cnorm_pad_);
-    centroids_centred_.centre.borrow(o.centroids_centred_.centre);
-    centroids_centred_.rows.borrow(o.centroids_centred_.rows);
-    centroids_centred_.norms.borrow(o.centroids_centred_.norms);
-    centroids_centred_.longest.borrow(o.centroids_centred_.longest);
+    centroids_centred_.borrow(o.centroids_centred_);
     codes_.borrow(o.codes_);
     ids_.borrow(o.ids_);
     list_off_dev_.borrow(o.list_off_dev_);
@@ -686,17 +683,26 @@ void IvfpqIndex::sync_list_tables()
 // from centroids_ as it stands in device memory.
 void IvfpqIndex::derive_from_centroids()
 {
-    cnorm_.resize((size_t)nlist_);
+    const bool centred = resident_assign_serves(nullptr, centroids_.data(), nlist_, d_);
+    cnorm_.resize((size_t)nlist_ * (centred ? 2 : 1));   // behind the norms: the lengths relative to the centre, read along with them
     launch_sqnorm_rows(centroids_.data(), nlist_, d_, cnorm_.data(), stream_);
     dp_ = (int)round_up(d_, 32);
     centroids_split_.resize((size_t)nlist_ * 3 * dp_);
     launch_split_bf16x3(centroids_.data(), nlist_, d_, dp_, true, centroids_split_.data(), stream_);
-    if (resident_assign_serves(nullptr, centroids_.data(), nlist_, d_)) {
-        launch_centre_centroids(centroids_.data(), nlist_, d_, cnorm_.data(), centroids_centred_, stream_);
+    if (centred) {
+        launch_centre_centroids(centroids_.data(), nlist_, d_, cnorm_.data(), centroids_centred_, cnorm_.data() + nlist_, stream_);
     }
-    std::vector<float> cn((size_t)nlist_);
+    std::vector<float> cn(cnorm_.size());
     cnorm_.download(cn.data(), cn.size(), stream_);
-    cmax_ = std::sqrt(*std::max_element(cn.begin(), cn.end()));
+    cmax_ = std::sqrt(*std::max_element(cn.begin(), cn.begin() + nlist_));
+    if (centred) {   // (a centroid with a NaN is nobody's nearest)
+        float longest = 0.f;
+        for (auto it = cn.begin() + nlist_; it != cn.end(); ++it) {
+            longest = std::max(longest, *it);
+        }
+        centroids_centred_.longest = std::sqrt(longest);
+        cn.resize((size_t)nlist_);
+    }
     // The split centroids a second time, in matrix-core order, for the resident-query score kernel
     // (coarse_resident.hip), with their norms padded to whole tiles: +inf behind the last centroid, so that a
     // padding row never passes a bound; for inner product the kernel wants zeros in their place.

@@ -19,23 +19,31 @@ bool launch_resident_f32(const float *Q, int64_t nq, const float *B, int64_t nb,
 // The centroids as the assignment kernel reads them: relative to a centre (about their mean), so that what vectors and centroids
 // have in common does not widen its error bound.
 struct AssignCentroids {
-    DeviceBuffer<float> centre;    // [d]
-    DeviceBuffer<float> rows;      // [nc][d]
-    DeviceBuffer<float> norms;     // [nc]
-    DeviceBuffer<float> longest;   // the largest |c - centre|^2
+    DeviceBuffer<float> centre;   // [d]
+    DeviceBuffer<float> rows;     // [nc][d]
+    DeviceBuffer<float> norms;    // [nc]
+    float longest = 0.f;          // the largest |c - centre|
+    void borrow(const AssignCentroids &o)
+    {
+        centre.borrow(o.centre);
+        rows.borrow(o.rows);
+        norms.borrow(o.norms);
+        longest = o.longest;
+    }
 };
-// cn: canonical squared norms
-void launch_centre_centroids(const float *C, int64_t nc, int d, const float *cn, AssignCentroids &out, hipStream_t s);
+// cn: canonical squared norms.  lengths[nc] (device): |c - centre|^2, from which the caller sets `longest`.
+void launch_centre_centroids(const float *C, int64_t nc, int d, const float *cn, AssignCentroids &out, float *lengths, hipStream_t s);
 
 // out[i] = the centroid with the smallest canonical L2 score of vector i (the smallest number among equal ones; -1 where every
 // score is a NaN).  The score kernel keeps each tile's best two centroids and its third value per vector, so nothing of the
 // n x nc scores is written; what its error bound cannot decide is decided by canonical scores, all on the stream, with nothing
 // for the host to read.  cn: canonical squared norms; cmax: the largest centroid length.
 struct AssignWorkspace {
-    DeviceBuffer<float4> top;     // [tile][vector] {best, second, third u, places}
-    DeviceBuffer<float> xn, xc;   // canonical |x|^2, and |x - centre|^2
-    DeviceBuffer<int4> pairs;     // {vector, two centroids}
-    DeviceBuffer<int32_t> rows;   // vectors with more than two; behind them the lengths of the two lists
+    DeviceBuffer<float4> top;        // [tile][vector] {best, second, third u, places}
+    DeviceBuffer<uint32_t> within;   // centroids of the tiles where more than two are in reach
+    DeviceBuffer<float> xn, need;    // canonical |x|^2, and the bound
+    DeviceBuffer<int4> pairs;        // {vector, two centroids}
+    DeviceBuffer<int32_t> rows;      // vectors with more than two; behind them the lengths of the two lists
 };
 bool resident_assign_serves(const float *X, const float *C, int64_t nc, int d);
 void launch_resident_assign(const float *X, int64_t n, const float *C, int64_t nc, int d, const float *cn, float cmax,

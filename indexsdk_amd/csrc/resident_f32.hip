@@ -116,6 +116,19 @@ struct Best {
 
 enum { kStore = 0, kFilter = 1, kAssign = 2 };
 
+// Words of a (tile, vector) that say which of the tile's centroids are within the vector's bound of the tile's best: half of them from
+// either half of the wavefront, bit 16 (ra % 2) + r of word ra / 2 for the half's centroid of block ra in accumulator r.
+constexpr int within_words(int qt) { return qt >= 64 ? qt / 32 : 2; }
+
+// What a kAssign launch reads and writes per vector: the bound; the best two centroids of every tile and the third value; and, where
+// the third value is within the bound of the best (crowded), all centroids that are.
+struct AssignTiles {
+    const float *need;
+    float4 *top;        // [tile][vector] {best, second, third u, places}
+    uint32_t *within;   // [tile][vector][within_words]
+};
+__device__ __forceinline__ bool crowded(float best, float third, float need) { return !(best - third > need); }
+
 // RA: query blocks of 32 per tile; SPB: K-steps of 16 dimensions per batch; nbat >= 2 batches cover the d dimensions.  MODE:
 //   kStore   every score is stored;
 //   kFilter  admitted keys are appended;
@@ -127,7 +140,7 @@ template <int RA, int SPB, int MODE>
 __global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) void resident_f32_kernel(
     const float *__restrict__ Q, int64_t nq, const float *__restrict__ B, int64_t nb, int d, int nbat,
     const float *__restrict__ qn, const float *__restrict__ bn, int metric, float *__restrict__ out, int64_t ldo,
-    ScoreFilter<float> flt, float4 *__restrict__ top, int tiles_m, int ntiles, int seg_tiles, int own_resident)
+    ScoreFilter<float> flt, AssignTiles assign, int tiles_m, int ntiles, int seg_tiles, int own_resident)
 {
     constexpr bool FILTER = MODE == kFilter, ASSIGN = MODE == kAssign;
     constexpr int QT = RA * 32;
@@ -318,6 +331,10 @@ __global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(2, 
                 c0[r] = l2 ? -0.5f * bnv[r >> 2][r & 3] : 0.f;
             }
         }
+        float need = 0.f;
+        if constexpr (ASSIGN) {
+            need = assign.need[row0 + l32 < nb ? row0 + l32 : nb - 1];
+        }
         if (!ASSIGN && row0 + 32 > nb) {   // the last tile of the launch: rows past its end take no part
 #pragma unroll
             for (int r = 0; r < 16; r++) {
@@ -451,8 +468,27 @@ __global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(2, 
             const Best &own = best[0];
             best[0].merge(Best{__shfl_xor(own.v1, 32), __shfl_xor(own.v2, 32), __shfl_xor(own.v3, 32),
                                (uint32_t)__shfl_xor((int)own.p1, 32), (uint32_t)__shfl_xor((int)own.p2, 32)});
-            if (half == 0 && row0 + l32 < nb) {
-                top[(int64_t)tm * nb + row0 + l32] = make_float4(own.v1, own.v2, own.v3, __uint_as_float(own.p1 | own.p2 << 16));
+            const int64_t at = (int64_t)tm * nb + row0 + l32;
+            const bool there = row0 + l32 < nb;
+            if (half == 0 && there) {
+                assign.top[at] = make_float4(own.v1, own.v2, own.v3, __uint_as_float(own.p1 | own.p2 << 16));
+            }
+            if (__builtin_amdgcn_ballot_w64(there && crowded(own.v1, own.v3, need)) != 0) {
+                constexpr int WORDS = within_words(QT) / 2;
+                const float reach = own.v1 - need;
+                uint32_t *out_words = assign.within + (at * 2 + half) * WORDS;
+#pragma unroll
+                for (int w = 0; w < WORDS; w++) {
+                    uint32_t word = 0;
+                    // (written so that an undefined reach or u leaves nothing out)
+#pragma unroll
+                    for (int i = (RA > 1 ? 31 : 15); i >= 0; i--) {
+                        word = word << 1 | (acc[2 * w + i / 16][i % 16] < reach ? 0u : 1u);
+                    }
+                    if (there) {
+                        out_words[w] = word;
+                    }
+                }
             }
         } else {
 #pragma unroll
@@ -507,7 +543,7 @@ struct Args {
     float *out;
     int64_t ldo;
     ScoreFilter<float> flt;
-    float4 *top;
+    AssignTiles assign;
     hipStream_t s;
 };
 
@@ -541,7 +577,7 @@ void launch_shape(const Args &a, int nbat)
     // segments: enough items for an even share per workgroup, long enough to pay for a query tile that changes
     const int seg = (int)std::min<int64_t>(16, std::max<int64_t>(1, (tn * tm + wpx * 8 - 1) / (wpx * 8)));
     hipLaunchKernelGGL(kern, dim3(grid), dim3(kWaves * 64), smem, a.s, a.Q, a.nq, a.B, a.nb, a.d, nbat, a.qn, a.bn, a.metric,
-                       a.out, a.ldo, a.flt, a.top, (int)tiles_m, (int)ntiles, seg, own_q ? 1 : 0);
+                       a.out, a.ldo, a.flt, a.assign, (int)tiles_m, (int)ntiles, seg, own_q ? 1 : 0);
 }
 
 // batches of a row: of four K-steps where that does not add padding, else of two
@@ -581,36 +617,11 @@ void launch_mode(const Args &a)
 
 // ---- what the tiles' best become ------------------------------------------------------------------------------------------
 
-// By how much a u has to lead another for the canonical scores to be in that order.  With a = |x - centre|, b = the largest
-// |c - centre|, L = |x| and cmax the largest |c|, what separates -2 u from the canonical score of the same centroid, but for
-// what all centroids share:
-//   the canonical score  (|x|^2 + |c|^2) - g - g: g's d products and sums, 2 (d + 1) 2^-24 L cmax, and three roundings,
-//                        3 x 2^-24 (L + cmax)^2.  Its |c|^2, which is rounded itself, is the one that u starts from
-//                        (launch_centre_centroids), so that makes no difference;
-//   u                    the products that the splits miss, 2 x 3 x 2^-18 a b, and 3 dp sums of numbers up to a b + b^2 / 2;
-//   the differences from the centre, rounded once: 2 x 2^-24 (a + b)^2 of a squared distance;
-//   the places in the low bits: 2^-17 |u| for either of two, |u| <= a b + b^2 / 2.
-// What vectors and centroids have in common is in L and cmax only.  Infinite or undefined where nothing can be decided: so for
-// lengths that lost squares (score_margin has the line), and for lengths beside which the start of a padding centroid (-3e38) is
-// not far off.  There a sum may overflow, and an infinite sum with a place in its low bits is a signalling NaN, which makes
-// max_number forget the best so far.
-struct AssignBound {
-    const float *xn, *xc;   // |x|^2 and |x - centre|^2 per vector
-    const float *cc;        // the largest |c - centre|^2
-    float cmax, exact_scale, split_scale, sum_scale;
-    __device__ __forceinline__ float need(int64_t i) const
-    {
-        const float l = sqrtf(xn[i]), a = sqrtf(xc[i]), b = sqrtf(*cc), far = l + cmax, near = a + b;
-        const float e = exact_scale * l * cmax + 4.f * 5.9604645e-8f * far * far + split_scale * a * b + sum_scale * near * near +
-                        1.6e-5f * b * near;
-        return far > 1e-12f && near > 1e-12f && far * far < 1e36f ? 1.001f * e : __builtin_inff();
-    }
-};
-
 // The best two of every vector over all tiles and the third value; a lead of more than the error bound decides, a tie of two
 // goes to `pairs` (vector, two centroids), of more (or an undefined length) to `rows`.  count: the two lists' lengths.
 __global__ __launch_bounds__(256) void assign_combine_kernel(const float4 *__restrict__ top, int tiles, int tile_centroids, int64_t n,
-                                                             AssignBound bound, int32_t *__restrict__ out, int4 *__restrict__ pairs,
+                                                             const float *__restrict__ bound, int32_t *__restrict__ out,
+                                                             int4 *__restrict__ pairs,
                                                              int32_t *__restrict__ rows, int32_t *__restrict__ count)
 {
     const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
@@ -623,7 +634,7 @@ __global__ __launch_bounds__(256) void assign_combine_kernel(const float4 *__res
             best.merge(Best{v.x, v.y, v.z, c0 + (p & 0xffffu), c0 + (p >> 16)});
         }
     }
-    const float need = bound.need(i < n ? i : n - 1);
+    const float need = bound[i < n ? i : n - 1];
     const bool decided = i >= n || best.v1 - best.v2 > need, pair = !decided && best.v1 - best.v3 > need;
     if (i < n) {
         out[i] = (int32_t)best.p1;
@@ -662,22 +673,29 @@ __device__ __forceinline__ float canonical_l2(const float *__restrict__ x, const
     return __fsub_rn(__fsub_rn(__fadd_rn(xn, cn), g), g);
 }
 
-// What assign_combine_kernel has left open, from canonical scores: first the pairs, a lane for each of the two centroids, then
-// the vectors with more, a wavefront for each.  Of every tile whose best is within reach of the vector's best the best and the
-// second are evaluated where they are within reach themselves, and all centroids where the third is (100000 vectors, 16384
-// centroids, sixteen to a component of the mixture: 1.6 ms when such a vector was scored against every centroid).
+constexpr int kResolveRows = 16;   // vectors that a wavefront of the next kernel takes at a time, at most
+
+// What assign_combine_kernel has left open, from canonical scores: first the pairs, a lane for each of the two centroids; then the
+// vectors with more.  A wavefront takes up to sixteen of them, and a lane a word of a tile's centroids: where the tile's best is
+// within reach of the vector's best, the best and the second if they are, or all that are within reach of the tile's best where
+// the third is.  The (vector, centroid) items are gathered in LDS and scored 64 at a time, a lane for each, whatever vectors they
+// belong to; the least key of every vector is kept in LDS.  Adding 200000 x 128 of 64 components of deviation 0.25 to 1024 lists, us
+// (every centroid of a crowded tile scored / this): component centres of deviation 1 691 / 671, 3 3643 / 860, 10 9329 / 980; of
+// deviation 1 with an offset of 24 9036 / 897.
 // Equal scores: the smaller number.  A NaN is never chosen; -1 where nothing else is left.
-__global__ __launch_bounds__(256) void assign_resolve_kernel(const float *__restrict__ X, int64_t n,
+__global__ __launch_bounds__(256) void assign_resolve_kernel(const float *__restrict__ X, const float *__restrict__ xn, int64_t n,
                                                              const float *__restrict__ C, const float *__restrict__ cn, int64_t nc,
-                                                             int d, AssignBound bound, const float4 *__restrict__ top, int tiles, int tile_centroids,
+                                                             int d, AssignTiles assign, int tiles, int tile_centroids,
                                                              const int4 *__restrict__ pairs, const int32_t *__restrict__ rows,
                                                              const int32_t *__restrict__ count, int32_t *__restrict__ out)
 {
-    const int lane = threadIdx.x & 63;
-    const int64_t wave = (int64_t)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), waves = (int64_t)gridDim.x * 4;
+    __shared__ unsigned long long least_all[4][kResolveRows];
+    __shared__ uint2 items_all[4][128];   // {vector among the wavefront's, centroid}
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int64_t wave = (int64_t)blockIdx.x * 4 + wv, waves = (int64_t)gridDim.x * 4;
     const int npairs = count[0], nrows = count[1];
     auto key_of = [&](int64_t row, int64_t c) {
-        const float v = canonical_l2(X + row * d, C + c * d, d, bound.xn[row], cn[c]);
+        const float v = canonical_l2(X + row * d, C + c * d, d, xn[row], cn[c]);
         return v == v ? make_key(v, (uint32_t)c) : kEmptyKey;
     };
     for (int64_t p0 = wave * 32; p0 < npairs; p0 += waves * 32) {
@@ -689,50 +707,85 @@ __global__ __launch_bounds__(256) void assign_resolve_kernel(const float *__rest
             out[e.x] = best == kEmptyKey ? -1 : (int32_t)key_index(best);
         }
     }
-    for (int64_t r = wave; r < nrows; r += waves) {
-        const int64_t row = rows[r];
-        float lead = kNoCentroid;
-        for (int t = lane; t < tiles; t += 64) {
-            lead = fmaxf(lead, top[(int64_t)t * n + row].x);
+    unsigned long long *least = least_all[wv];
+    uint2 *items = items_all[wv];
+    const int words = within_words(tile_centroids), words_log2 = __builtin_ctz(words), all_words = tiles * words;
+    // few vectors: a wavefront takes fewer at a time
+    const int64_t per_wave = (nrows + waves - 1) / waves;
+    const int take = (int)(per_wave < kResolveRows ? per_wave : kResolveRows);
+    for (int64_t r0 = wave * take; r0 < nrows; r0 += waves * take) {
+        const int here = (int)(nrows - r0 < take ? nrows - r0 : take);
+        const int my_row = rows[r0 + (lane < here ? lane : here - 1)];
+        if (lane < kResolveRows) {
+            least[lane] = kEmptyKey;
         }
-        for (int o = 32; o > 0; o >>= 1) {
-            lead = fmaxf(lead, __shfl_xor(lead, o));
-        }
-        const float reach = lead - bound.need(row);
-        key_t best = kEmptyKey;
-        for (int t0 = 0; t0 < tiles; t0 += 64) {
-            const int t = t0 + lane;
-            const float4 v = top[(int64_t)(t < tiles ? t : tiles - 1) * n + row];
-            // (written so that an undefined reach leaves nothing out)
-            const bool one = t < tiles && !(v.x < reach), two = t < tiles && !(v.y < reach);
-            const unsigned long long whole = __ballot(t < tiles && !(v.z < reach));
-            if ((whole >> lane & 1) == 0) {
-                const uint32_t p = __float_as_uint(v.w);
-                const int64_t c1 = (int64_t)t * tile_centroids + (p & 0xffffu), c2 = (int64_t)t * tile_centroids + (p >> 16);
-                if (one && c1 < nc) {
-                    const key_t k = key_of(row, c1);
-                    best = k < best ? k : best;
+        int queued = 0;   // the same in every lane
+        auto score = [&](int m) {   // the first m items, at most 64; those behind them move up
+            wave_lds_fence();
+            const uint2 e = items[lane];
+            const uint2 behind = items[64 + lane];
+            const int row = __shfl(my_row, lane < m ? (int)e.x : 0);
+            if (lane < m) {
+                atomicMin(least + e.x, key_of(row, e.y));
+            }
+            wave_lds_fence();
+            items[lane] = behind;
+            queued -= m;
+        };
+        for (int v = 0; v < here; v++) {
+            const int64_t row = __builtin_amdgcn_readlane(my_row, v);
+            const float need = assign.need[row];
+            float lead = kNoCentroid;
+            for (int t = lane; t < tiles; t += 64) {
+                lead = fmaxf(lead, assign.top[(int64_t)t * n + row].x);
+            }
+            for (int o = 32; o > 0; o >>= 1) {
+                lead = fmaxf(lead, __shfl_xor(lead, o));
+            }
+            const float reach = lead - need;
+            for (int w0 = 0; w0 < all_words; w0 += 64) {
+                const int w = w0 + lane, t = w >> words_log2, j = w & (words - 1);
+                const int jh = j / (words / 2), jw = j % (words / 2);   // half of the wavefront, its word
+                uint32_t bits = 0;
+                // (written so that an undefined reach leaves nothing out)
+                if (w < all_words) {
+                    const int64_t at = (int64_t)t * n + row;
+                    const float4 best = assign.top[at];
+                    if (!(best.x < reach)) {
+                        if (crowded(best.x, best.z, need)) {
+                            bits = assign.within[at * words + j];
+                        } else {
+                            const uint32_t p = __float_as_uint(best.w);
+                            auto bit_of = [&](uint32_t place) {   // 32 ra + 8 (r / 4) + 4 half + r % 4
+                                const bool mine = (int)(place >> 6) == jw && (int)(place >> 2 & 1) == jh;
+                                return mine ? 1u << ((place >> 5 & 1) * 16 + (place >> 3 & 3) * 4 + (place & 3)) : 0u;
+                            };
+                            bits = bit_of(p & 0xffffu) | (best.y < reach ? 0u : bit_of(p >> 16));
+                        }
+                    }
                 }
-                if (two && c2 < nc) {
-                    const key_t k = key_of(row, c2);
-                    best = k < best ? k : best;
+                while (__ballot(bits != 0) != 0) {
+                    const int bit = bits != 0 ? __builtin_ctz(bits) : 0;
+                    const int64_t c = (int64_t)t * tile_centroids + (2 * jw + (bit >> 4)) * 32 + (bit >> 2 & 3) * 8 + jh * 4 + (bit & 3);
+                    const bool has = bits != 0 && c < nc;
+                    const unsigned long long m = __ballot(has);
+                    if (has) {
+                        items[queued + __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0))] =
+                            make_uint2((uint32_t)v, (uint32_t)c);
+                    }
+                    queued += __popcll(m);
+                    if (queued >= 64) {
+                        score(64);
+                    }
+                    bits &= bits - 1;
                 }
             }
-            for (unsigned long long w = whole; w != 0; w &= w - 1) {
-                const int64_t c0 = (int64_t)(t0 + __builtin_ctzll(w)) * tile_centroids;
-                const int64_t c_end = c0 + tile_centroids < nc ? c0 + tile_centroids : nc;
-                for (int64_t c = c0 + lane; c < c_end; c += 64) {
-                    const key_t k = key_of(row, c);
-                    best = k < best ? k : best;
-                }
-            }
         }
-        for (int o = 32; o > 0; o >>= 1) {
-            const key_t k = __shfl_xor(best, o);
-            best = k < best ? k : best;
-        }
-        if (lane == 0) {
-            out[row] = best == kEmptyKey ? -1 : (int32_t)key_index(best);
+        score(queued);
+        wave_lds_fence();
+        if (lane < here) {
+            const unsigned long long best = least[lane];
+            out[my_row] = best == kEmptyKey ? -1 : (int32_t)key_index(best);
         }
     }
 }
@@ -749,7 +802,7 @@ bool launch_resident_f32(const float *Q, int64_t nq, const float *B, int64_t nb,
         (!filter && (ldo % 4 != 0 || reinterpret_cast<uintptr_t>(out) % 16 != 0))) {
         return false;
     }
-    const Args a{Q, nq, B, nb, d, qn, bn, metric, out, ldo, flt, nullptr, s};
+    const Args a{Q, nq, B, nb, d, qn, bn, metric, out, ldo, flt, AssignTiles{}, s};
     if (filter) {
         launch_mode<kFilter>(a);
     } else {
@@ -765,75 +818,58 @@ bool resident_assign_serves(const float *X, const float *C, int64_t nc, int d)
     return resident_f32_serves(d) && (d <= 512 || nc <= 4096) && reinterpret_cast<uintptr_t>(X) % 16 == 0 && reinterpret_cast<uintptr_t>(C) % 16 == 0;
 }
 
-// out[0 .. d) = the mean of up to 1024 of the centroids (a component without one: 0); *longest = 0
-__global__ __launch_bounds__(1024) void centroid_mean_kernel(const float *__restrict__ C, int64_t nc, int d, float *__restrict__ out,
-                                                             float *__restrict__ longest)
+// Every workgroup adds up the mean of up to 64 of the centroids for itself (a component without one: 0), then takes the centroids
+// wave by wave: rows = c - centre, lengths = |rows|^2, norms = the number that a sum of products with it starts from, times -2:
+// |rows|^2 plus what the rounding of cn = |c|^2 has added to it.  Bound by the round trips of the mean's loads: 6 us for 1024
+// centroids of 128 dimensions.
+__global__ __launch_bounds__(256) void centre_centroids_kernel(const float *__restrict__ C, int64_t nc, int d, const float *__restrict__ cn,
+                                                               float *__restrict__ centre, float *__restrict__ rows,
+                                                               float *__restrict__ norms, float *__restrict__ lengths)
 {
-    __shared__ float part[16][64];
-    const int col = blockIdx.x * 64 + (threadIdx.x & 63), slice = threadIdx.x >> 6;
-    const int64_t count = nc < 1024 ? nc : 1024;
-    float sum = 0.f;
-    if (col < d) {
-#pragma unroll 8
-        for (int64_t r = slice; r < count; r += 16) {
-            sum += C[r * nc / count * d + col];
-        }
-    }
-    part[slice][threadIdx.x & 63] = sum;
-    __syncthreads();
-    if (slice == 0 && col < d) {
-        for (int t = 1; t < 16; t++) {
-            sum += part[t][threadIdx.x];
+    extern __shared__ float mean[];   // [d]
+    const int count = nc < 64 ? (int)nc : 64;
+    const int64_t step = nc / count * d;
+    for (int t = threadIdx.x; t < d; t += 256) {
+        float sum = 0.f;
+#pragma unroll 16
+        for (int r = 0; r < count; r++) {
+            sum += C[r * step + t];
         }
         sum /= (float)count;
-        out[col] = fabsf(sum) < 1e38f ? sum : 0.f;
+        sum = fabsf(sum) < 1e38f ? sum : 0.f;
+        mean[t] = sum;
+        if (blockIdx.x == 0) {
+            centre[t] = sum;
+        }
     }
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        *longest = 0.f;
-    }
-}
-
-// A wavefront per centroid: rows = c - centre, norms = the number that a sum of products with it starts from, times -2: |rows|^2
-// plus what the rounding of cn = |c|^2 has added to it.
-__global__ __launch_bounds__(256) void centre_centroids_kernel(const float *__restrict__ C, int64_t nc, int d, const float *__restrict__ cn,
-                                                               const float *__restrict__ centre, float *__restrict__ rows,
-                                                               float *__restrict__ norms, float *__restrict__ longest)
-{
-    const int64_t c = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+    __syncthreads();
     const int lane = threadIdx.x & 63;
-    if (c >= nc) {
-        return;
-    }
-    double apart = 0.0, whole = 0.0;
-    for (int t = lane; t < d; t += 64) {
-        const float v = C[c * d + t], r = v - centre[t];
-        rows[c * d + t] = r;
-        apart += (double)r * r;
-        whole += (double)v * v;
-    }
-    for (int o = 32; o > 0; o >>= 1) {
-        apart += __shfl_xor(apart, o);
-        whole += __shfl_xor(whole, o);
-    }
-    if (lane == 0) {
-        norms[c] = (float)(apart + ((double)cn[c] - whole));
-        const float len = (float)apart;
-        if (len == len) {   // a centroid with a NaN is nobody's nearest; (of numbers >= 0 the bits have their order)
-            atomicMax(reinterpret_cast<unsigned int *>(longest), __float_as_uint(len));
+    for (int64_t c = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6); c < nc; c += (int64_t)gridDim.x * 4) {
+        double apart = 0.0, whole = 0.0;
+        for (int t = lane; t < d; t += 64) {
+            const float v = C[c * d + t], r = v - mean[t];
+            rows[c * d + t] = r;
+            apart += (double)r * r;
+            whole += (double)v * v;
+        }
+        for (int o = 32; o > 0; o >>= 1) {
+            apart += __shfl_xor(apart, o);
+            whole += __shfl_xor(whole, o);
+        }
+        if (lane == 0) {
+            norms[c] = (float)(apart + ((double)cn[c] - whole));
+            lengths[c] = (float)apart;
         }
     }
 }
 
-void launch_centre_centroids(const float *C, int64_t nc, int d, const float *cn, AssignCentroids &out, hipStream_t s)
+void launch_centre_centroids(const float *C, int64_t nc, int d, const float *cn, AssignCentroids &out, float *lengths, hipStream_t s)
 {
     out.centre.resize((size_t)d);
     out.rows.resize((size_t)nc * d);
     out.norms.resize((size_t)nc);
-    out.longest.resize(1);
-    hipLaunchKernelGGL(centroid_mean_kernel, dim3((unsigned)((d + 63) / 64)), dim3(1024), 0, s, C, nc, d, out.centre.data(),
-                       out.longest.data());
-    hipLaunchKernelGGL(centre_centroids_kernel, dim3((unsigned)((nc + 3) / 4)), dim3(256), 0, s, C, nc, d, cn, out.centre.data(),
-                       out.rows.data(), out.norms.data(), out.longest.data());
+    hipLaunchKernelGGL(centre_centroids_kernel, dim3((unsigned)std::min<int64_t>((nc + 3) / 4, device_cus() * 4)), dim3(256),
+                       (size_t)d * sizeof(float), s, C, nc, d, cn, out.centre.data(), out.rows.data(), out.norms.data(), lengths);
 }
 
 void launch_resident_assign(const float *X, int64_t n, const float *C, int64_t nc, int d, const float *cn, float cmax,
@@ -845,28 +881,30 @@ void launch_resident_assign(const float *X, int64_t n, const float *C, int64_t n
     IXA_REQUIRE(resident_assign_serves(X, C, nc, d) && nc >= 1 && n < ((int64_t)1 << 31), kErrInner, "assignment kernel does not serve these operands");
     const int qt = 32 * tile_blocks(nc, d);
     const int64_t tiles = (nc + qt - 1) / qt;
-    // vectors per pass: 16 bytes per vector and tile of centroids, 28 for lengths and what is left open
-    const int64_t page = std::min<int64_t>(n, std::max<int64_t>(kTileRows, scratch_bytes / (16 * tiles + 28) / kTileRows * kTileRows));
+    // vectors per pass: the tiles' best and crowds, and 28 bytes for lengths, bounds and what is left open
+    const int words = within_words(qt);
+    const int64_t page = std::min<int64_t>(n, std::max<int64_t>(kTileRows, scratch_bytes / ((16 + 4 * words) * tiles + 28) / kTileRows * kTileRows));
     ws.top.resize((size_t)(page * tiles));
+    ws.within.resize((size_t)(page * tiles * words));
     ws.pairs.resize((size_t)page);
     ws.xn.resize((size_t)page);
-    ws.xc.resize((size_t)page);
+    ws.need.resize((size_t)page);
     ws.rows.resize((size_t)page + 2);
     int32_t *count = ws.rows.data() + page;
+    const AssignTiles assign{ws.need.data(), ws.top.data(), ws.within.data()};
     const float u = 5.9604645e-8f;
-    AssignBound bound{ws.xn.data(), ws.xc.data(), centred.longest.data(), cmax, 2.f * (float)(d + 8) * u, 6.f / 262144.f,
-                      (float)(3 * ((d + 31) / 32 * 32) + 6) * u};
+    const AssignBound bound{cmax, centred.longest, 2.f * (float)(d + 8) * u, 6.f / 262144.f,
+                            (float)(3 * ((d + 31) / 32 * 32) + 6) * u};
     for (int64_t i0 = 0; i0 < n; i0 += page) {
         const int64_t m = std::min(page, n - i0);
-        IXA_HIP(hipMemsetAsync(count, 0, 8, s));
         const float *xi = X + i0 * d;
-        launch_sqnorm_rows_centred(xi, m, d, centred.centre.data(), ws.xn.data(), ws.xc.data(), s);
+        launch_assign_bounds(xi, m, d, centred.centre.data(), bound, ws.xn.data(), ws.need.data(), count, s);
         launch_mode<kAssign>(Args{centred.rows.data(), nc, xi, m, d, centred.norms.data(), centred.centre.data(), kMetricL2, nullptr, 0,
-                                  ScoreFilter<float>{}, ws.top.data(), s});
+                                  ScoreFilter<float>{}, assign, s});
         hipLaunchKernelGGL(assign_combine_kernel, dim3((unsigned)((m + 255) / 256)), dim3(256), 0, s, ws.top.data(), (int)tiles, qt, m,
-                           bound, out + i0, ws.pairs.data(), ws.rows.data(), count);
-        hipLaunchKernelGGL(assign_resolve_kernel, dim3((unsigned)std::min<int64_t>(m, device_cus() * 2)), dim3(256), 0, s, xi, m, C, cn, nc,
-                           d, bound, ws.top.data(), (int)tiles, qt, ws.pairs.data(), ws.rows.data(), count, out + i0);
+                           ws.need.data(), out + i0, ws.pairs.data(), ws.rows.data(), count);
+        hipLaunchKernelGGL(assign_resolve_kernel, dim3((unsigned)std::min<int64_t>(m, device_cus() * 4)), dim3(256), 0, s, xi, ws.xn.data(), m, C, cn,
+                           nc, d, assign, (int)tiles, qt, ws.pairs.data(), ws.rows.data(), count, out + i0);
     }
 }
 

@@ -1131,6 +1131,37 @@ def test_adding_vectors_with_an_offset_takes_about_as_long(ix):
     assert offset < 3.0 * plain, (plain, offset)
 
 
+def test_adding_vectors_of_components_far_apart_takes_about_as_long(ix):
+    """A vector whose error bound leaves many of the centroids of its component open is scored against those: with components four
+    times as far apart adding took nine times as long when whole tiles of centroids were scored (1.2 times now)."""
+    plain, spread = _adding_times(ix, (4.0, 0.0))
+    assert spread < 3.0 * plain, (plain, spread)
+
+
+# Most vectors open, with dozens to all of the centroids in reach, in every tile size: all of a tile's centroids tie, some of its
+# halves' do; batches of vectors that a wavefront takes, fewer and more than sixteen.
+@pytest.mark.parametrize("d,nlist", [(128, 700), (128, 100), (64, 256), (256, 300), (512, 130), (768, 70), (1024, 33)])
+@pytest.mark.parametrize("n", [1, 15, 257, 40000])
+def test_assignment_of_crowds(ix, oracle, d, nlist, n):
+    rng = np.random.default_rng(d + nlist)
+    n = min(n, 40000 * 64 // d)
+    centres = 30.0 * rng.standard_normal((5, d))
+    which = rng.integers(0, 5, nlist)
+    cent = (centres[which] + np.where(which == 0, 1e-5, 0.05)[:, None] * rng.standard_normal((nlist, d))).astype(np.float32)
+    cent[which == 1] = cent[np.argmax(which == 1)]
+    x = (centres[rng.integers(0, 5, n)] + 0.05 * rng.standard_normal((n, d))).astype(np.float32)
+    x[::7] = cent[rng.integers(0, nlist, len(x[::7]))]
+    gpu = ix.AscendIndexIVFPQ(d, ix.METRIC_L2, nlist, 4, 8)
+    gpu.set_trained(cent, rng.standard_normal((4, 256, d // 4)).astype(np.float32))
+    assert np.array_equal(gpu.assign(x), oracle.assign(x, cent))
+    if n > 10:
+        x[3, 5], x[9, 1] = np.nan, np.inf
+        want = oracle.assign(x, cent)
+        got = gpu.assign(x)
+        keep = np.isfinite(x).all(axis=1)
+        assert np.array_equal(got[keep], want[keep]) and got[3] == -1
+
+
 # A query split over workgroups deals groups of 64 codes to its slices in turn: lists without codes, of one code and of a remainder,
 # several groups per list and (nprobe 512: a slice skips more than 64 lists at a time) far fewer; 8 to 20 slices; private pools, the shared pool,
 # kernels for a compile-time number of sub-quantizers and not.  As in one workgroup per query (a large batch), bit for bit.
