@@ -220,7 +220,6 @@ private:
     // search workspaces (grown on demand, reused between calls)
     DeviceBuffer<float> ws_x_, ws_qn_, ws_dist_, ws_exact_;
     StreamSelectWorkspace<float> ws_sel_;
-    AssignWorkspace ws_assign_;
     DeviceBuffer<unsigned long long> ws_running_;
     DeviceBuffer<int32_t> ws_cand_, ws_probes_;
     DeviceBuffer<int64_t> ws_labels_;

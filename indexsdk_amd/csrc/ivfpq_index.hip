@@ -840,7 +840,7 @@ void IvfpqIndex::coarse_select(const float *x_dev, int64_t n, int nout, int sele
         last_coarse_exact_ = true;
         last_coarse_plan_ = 0;
         last_coarse_n_ = n;
-        launch_resident_assign(x_dev, n, centroids_.data(), nlist_, d_, cnorm_.data(), cmax_, centroids_centred_, out_ids, ws_assign_,
+        launch_resident_assign(x_dev, n, centroids_.data(), nlist_, d_, cnorm_.data(), cmax_, centroids_centred_, out_ids, ws_sel_.scores,
                                cfg_.scratch_bytes, stream_);
         return;
     }

@@ -37,16 +37,10 @@ void launch_centre_centroids(const float *C, int64_t nc, int d, const float *cn,
 // out[i] = the centroid with the smallest canonical L2 score of vector i (the smallest number among equal ones; -1 where every
 // score is a NaN).  The score kernel keeps each tile's best two centroids and its third value per vector, so nothing of the
 // n x nc scores is written; what its error bound cannot decide is decided by canonical scores, all on the stream, with nothing
-// for the host to read.  cn: canonical squared norms; cmax: the largest centroid length.
-struct AssignWorkspace {
-    DeviceBuffer<float4> top;        // [tile][vector] {best, second, third u, places}
-    DeviceBuffer<uint32_t> within;   // centroids of the tiles where more than two are in reach
-    DeviceBuffer<float> xn, need;    // canonical |x|^2, and the bound
-    DeviceBuffer<int4> pairs;        // {vector, two centroids}
-    DeviceBuffer<int32_t> rows;      // vectors with more than two; behind them the lengths of the two lists
-};
+// for the host to read.  cn: canonical squared norms; cmax: the largest centroid length; scratch: memory that nothing queued behind
+// the call relies on, resized to at most scratch_bytes (or what 256 vectors take).
 bool resident_assign_serves(const float *X, const float *C, int64_t nc, int d);
 void launch_resident_assign(const float *X, int64_t n, const float *C, int64_t nc, int d, const float *cn, float cmax,
-                            const AssignCentroids &centred, int32_t *out, AssignWorkspace &ws, int64_t scratch_bytes, hipStream_t s);
+                            const AssignCentroids &centred, int32_t *out, DeviceBuffer<float> &scratch, int64_t scratch_bytes, hipStream_t s);
 
 }  // namespace ixa

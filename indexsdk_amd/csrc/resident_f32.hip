@@ -873,7 +873,7 @@ void launch_centre_centroids(const float *C, int64_t nc, int d, const float *cn,
 }
 
 void launch_resident_assign(const float *X, int64_t n, const float *C, int64_t nc, int d, const float *cn, float cmax,
-                            const AssignCentroids &centred, int32_t *out, AssignWorkspace &ws, int64_t scratch_bytes, hipStream_t s)
+                            const AssignCentroids &centred, int32_t *out, DeviceBuffer<float> &scratch, int64_t scratch_bytes, hipStream_t s)
 {
     if (n <= 0) {
         return;
@@ -881,30 +881,31 @@ void launch_resident_assign(const float *X, int64_t n, const float *C, int64_t n
     IXA_REQUIRE(resident_assign_serves(X, C, nc, d) && nc >= 1 && n < ((int64_t)1 << 31), kErrInner, "assignment kernel does not serve these operands");
     const int qt = 32 * tile_blocks(nc, d);
     const int64_t tiles = (nc + qt - 1) / qt;
-    // vectors per pass: the tiles' best and crowds, and 28 bytes for lengths, bounds and what is left open
+    // vectors per pass, and what the scratch holds of them, the widest first: of every tile the best two centroids and its crowd; what
+    // is left open (pairs: {vector, two centroids}; rows: vectors with more; the lengths of the two lists); |x|^2 and the bounds
     const int words = within_words(qt);
-    const int64_t page = std::min<int64_t>(n, std::max<int64_t>(kTileRows, scratch_bytes / ((16 + 4 * words) * tiles + 28) / kTileRows * kTileRows));
-    ws.top.resize((size_t)(page * tiles));
-    ws.within.resize((size_t)(page * tiles * words));
-    ws.pairs.resize((size_t)page);
-    ws.xn.resize((size_t)page);
-    ws.need.resize((size_t)page);
-    ws.rows.resize((size_t)page + 2);
-    int32_t *count = ws.rows.data() + page;
-    const AssignTiles assign{ws.need.data(), ws.top.data(), ws.within.data()};
+    const int64_t per_vector = (16 + 4 * words) * tiles + 28;
+    const int64_t page = std::min<int64_t>(n, std::max<int64_t>(kTileRows, (scratch_bytes - 8) / per_vector / kTileRows * kTileRows));
+    scratch.resize((size_t)(page * per_vector + 8) / 4);
+    float4 *top = reinterpret_cast<float4 *>(scratch.data());
+    int4 *pairs = reinterpret_cast<int4 *>(top + page * tiles);
+    uint32_t *within = reinterpret_cast<uint32_t *>(pairs + page);
+    float *xn = reinterpret_cast<float *>(within + page * tiles * words), *need = xn + page;
+    int32_t *rows = reinterpret_cast<int32_t *>(need + page), *count = rows + page;
+    const AssignTiles assign{need, top, within};
     const float u = 5.9604645e-8f;
     const AssignBound bound{cmax, centred.longest, 2.f * (float)(d + 8) * u, 6.f / 262144.f,
                             (float)(3 * ((d + 31) / 32 * 32) + 6) * u};
     for (int64_t i0 = 0; i0 < n; i0 += page) {
         const int64_t m = std::min(page, n - i0);
         const float *xi = X + i0 * d;
-        launch_assign_bounds(xi, m, d, centred.centre.data(), bound, ws.xn.data(), ws.need.data(), count, s);
+        launch_assign_bounds(xi, m, d, centred.centre.data(), bound, xn, need, count, s);
         launch_mode<kAssign>(Args{centred.rows.data(), nc, xi, m, d, centred.norms.data(), centred.centre.data(), kMetricL2, nullptr, 0,
                                   ScoreFilter<float>{}, assign, s});
-        hipLaunchKernelGGL(assign_combine_kernel, dim3((unsigned)((m + 255) / 256)), dim3(256), 0, s, ws.top.data(), (int)tiles, qt, m,
-                           ws.need.data(), out + i0, ws.pairs.data(), ws.rows.data(), count);
-        hipLaunchKernelGGL(assign_resolve_kernel, dim3((unsigned)std::min<int64_t>(m, device_cus() * 4)), dim3(256), 0, s, xi, ws.xn.data(), m, C, cn,
-                           nc, d, assign, (int)tiles, qt, ws.pairs.data(), ws.rows.data(), count, out + i0);
+        hipLaunchKernelGGL(assign_combine_kernel, dim3((unsigned)((m + 255) / 256)), dim3(256), 0, s, top, (int)tiles, qt, m, need,
+                           out + i0, pairs, rows, count);
+        hipLaunchKernelGGL(assign_resolve_kernel, dim3((unsigned)std::min<int64_t>(m, device_cus() * 4)), dim3(256), 0, s, xi, xn, m, C, cn, nc, d, assign,
+                           (int)tiles, qt, pairs, rows, count, out + i0);
     }
 }
 

@@ -1162,6 +1162,26 @@ def test_assignment_of_crowds(ix, oracle, d, nlist, n):
         assert np.array_equal(got[keep], want[keep]) and got[3] == -1
 
 
+def test_assignment_and_search_share_the_scratch(ix):
+    """What an assignment keeps per vector lies in the memory that a search writes its scores to: after a search that has used up the
+    scratch, assigning takes no more than the vectors and the answers themselves (beside a scratch of its own it took 50 MB more)."""
+    import torch
+
+    rng = np.random.default_rng(2)
+    d, nlist, n = 64, 2048, 400000
+    cent = rng.standard_normal((nlist, d)).astype(np.float32)
+    index = ix.AscendIndexIVFPQ(d, ix.METRIC_L2, nlist, 4, 8, ix.AscendIndexIVFPQConfig(scratch_bytes=64 << 20, coarse_sampled_bound=0))
+    index.set_trained(cent, rng.standard_normal((4, 256, d // 4)).astype(np.float32))
+    x = np.tile(rng.standard_normal((n // 10, d)).astype(np.float32), (10, 1))
+    index.add(x[:1000])
+    index.setNumProbes(8)
+    index.search(x[:30000], 1)
+    before = torch.cuda.mem_get_info()[0]
+    index.assign(x)
+    taken = before - torch.cuda.mem_get_info()[0]
+    assert taken < n * (d + 1) * 4 + (16 << 20), taken
+
+
 # A query split over workgroups deals groups of 64 codes to its slices in turn: lists without codes, of one code and of a remainder,
 # several groups per list and (nprobe 512: a slice skips more than 64 lists at a time) far fewer; 8 to 20 slices; private pools, the shared pool,
 # kernels for a compile-time number of sub-quantizers and not.  As in one workgroup per query (a large batch), bit for bit.
