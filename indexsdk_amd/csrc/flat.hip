@@ -544,7 +544,7 @@ void FlatIndex::forget_norms()
     }
     bmax_ = 0.f;
     finite_ = true;
-    split_rest_ = 0;
+    split_rest_ = resident_rest_ = resident_misses_ = 0;
     if (ntotal_ > 0) {
         measure_norms(norms_.data(), ntotal_);
     }
@@ -746,13 +746,19 @@ void FlatIndex::search_masked(int64_t n, const float *x, int64_t k, float *dist,
     const bool can_split = !mask_dev && bmax_ >= 1e-6f && finite_;
     Candidates from = Candidates::kFp32;
     if (can_split && resident_f32_serves(d_) && reinterpret_cast<uintptr_t>(xd) % 16 == 0 && resident_pays(n, ntotal_, d_)) {
-        from = Candidates::kResident;
-    } else if (can_split && split_pays(n, ntotal_, dp, k, split_candidates(k, dp, metric_, false), scratch_bytes_) && split_rows >= 16384) {
-        from = Candidates::kSplit;
+        if (resident_rest_ == 0) {
+            from = Candidates::kResident;
+        } else {
+            resident_rest_--;
+        }
     }
-    if (from != Candidates::kFp32 && split_rest_ > 0) {
-        split_rest_--;
-        from = Candidates::kFp32;
+    if (from == Candidates::kFp32 && can_split && split_rows >= 16384 &&
+        split_pays(n, ntotal_, dp, k, split_candidates(k, dp, metric_, false), scratch_bytes_)) {
+        if (split_rest_ == 0) {
+            from = Candidates::kSplit;
+        } else {
+            split_rest_--;
+        }
     }
     stats_ = FlatStats();
     std::vector<int64_t> rows;   // without proof
@@ -766,17 +772,14 @@ void FlatIndex::search_masked(int64_t n, const float *x, int64_t k, float *dist,
     } else {
         rows = search_plan(n, xd, k, dd, ld, mask_dev, mask_stride, from, 0);
     }
+    if (from == Candidates::kResident && rows.empty()) {
+        resident_misses_ = 0;
+    }
     if (from != Candidates::kFp32 && !rows.empty()) {
         // The error bound of the splits is two to three times that of fp32 scores: what they leave unproven, the fp32 plan may
         // prove, at a fraction of what canonical scores of the whole base cost (200k x 128, 512 queries with a common offset
         // that leaves 449 unproven by splits and 122 by fp32 as well: 10.7 ms with exact rows at once, 3.8 with fp32 before them;
         // one undefined query of 1024 over 1M x 128: 2.27 ms against 2.07, 64 of them 10.7 against 2.28).
-        // The second plan costs about what a tile of 128 queries does (0.25 of 1.0 ms for 1024 queries, 0.25 of 0.63 for 512), so
-        // unproven queries make a small batch, or an eighth of them any batch, slower than fp32 alone: then the next sixteen batches
-        // that would take splits go without, and the one after them tries again.
-        if ((int64_t)rows.size() * 8 > n || n < 1024) {
-            split_rest_ = 16;
-        }
         const int64_t m = (int64_t)rows.size();
         DeviceBuffer<int64_t> rows_dev, lsub((size_t)m * k);
         DeviceBuffer<float> xsub((size_t)m * d_), dsub((size_t)m * k);
@@ -786,11 +789,28 @@ void FlatIndex::search_masked(int64_t n, const float *x, int64_t k, float *dist,
         std::vector<int64_t> left = search_plan(m, xsub.data(), k, dsub.data(), lsub.data(), nullptr, 0, Candidates::kFp32, 0);
         hipLaunchKernelGGL(scatter_result_rows_kernel, dim3(blocks_for(m * k)), dim3(256), 0, stream_, dsub.data(), lsub.data(),
                            rows_dev.data(), m, (int)k, dd, ld);
-        sync_stream(stream_);   // the temporaries above are freed on leaving this block
+        std::vector<float> norms((size_t)m);   // as the second plan has found them
+        ws_qn_.download(norms.data(), (size_t)m, stream_);   // (waits: the temporaries above are freed on leaving this block)
         for (int64_t &r : left) {
             r = rows[(size_t)r];
         }
         rows = std::move(left);
+        // What the second plan costs decides whether the next batches go without the first.  Queries with an undefined norm do not
+        // count: nothing proves them, and they say nothing about the others.
+        const int64_t open = std::count_if(norms.begin(), norms.end(), [](float v) { return std::isfinite(v); });
+        if (from == Candidates::kSplit) {
+            // It costs about what a tile of 128 queries does (0.25 of 1.0 ms for 1024 queries, 0.25 of 0.63 for 512), so
+            // unproven queries make a small batch, or an eighth of them any batch, slower than fp32 alone: then the next
+            // sixteen batches that would take splits go without, and the one after them tries again.
+            split_rest_ = open * 8 > n || (open > 0 && n < 1024) ? 16 : split_rest_;
+        } else {
+            // (resident_pays has the times.)  A batch of up to 128 queries is slower than the older plans alone when one of them is
+            // unproven, larger ones when about half are.  One such batch may be its queries' own affair; after two in a row, and
+            // after each that follows without a proven one between, sixteen go without.
+            const bool missed = 2 * ((open + 127) / 128) > (n + 127) / 128;
+            resident_misses_ = missed ? std::min(resident_misses_ + 1, 2) : 0;
+            resident_rest_ = resident_misses_ == 2 ? 16 : 0;
+        }
     }
     if (!rows.empty()) {
         IXA_HIP(hipEventRecord(ev_[1], stream_));

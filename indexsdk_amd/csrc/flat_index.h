@@ -126,7 +126,8 @@ private:
     DeviceBuffer<int64_t> ws_labels_;
     float bmax_ = 0.f;   // largest base vector norm
     bool finite_ = true; // no vector of the base has an infinite or undefined norm
-    int split_rest_ = 0; // batches that go without splits, after one that splits left largely unproven
+    int split_rest_ = 0;   // batches that go without splits formed beforehand, after one that they left largely unproven
+    int resident_rest_ = 0, resident_misses_ = 0;   // the same for splits formed in the score kernel, and such batches in a row
 };
 
 class FlatI8Index : public FlatBase<int8_t> {

@@ -721,3 +721,58 @@ def test_flat_masked_few_queries_over_several_long_chunks(ix, kind, nq, k):
     best = np.take_along_axis(dist, want, 1)
     assert np.array_equal(I, np.where(np.isinf(best), -1, want))
     assert np.array_equal(D[np.isfinite(best)].astype(np.float32), best[np.isfinite(best)])
+
+
+def _flat_on_device(ix, base, k):
+    """An index over rows in device memory, and the seconds of one search of it."""
+    import time
+
+    index = ix.AscendIndexFlat(base.shape[1], ix.METRIC_L2)
+    torch.cuda.synchronize()
+    _capi.check(_capi.load().flat_add_with_ids_device(index._h, len(base), ctypes.c_void_p(base.data_ptr()), None))
+
+    def search(q):
+        D, I = torch.empty(len(q), k, device="cuda"), torch.empty(len(q), k, device="cuda", dtype=torch.int64)
+        torch.cuda.synchronize()
+        t = time.perf_counter()
+        _capi.check(_capi.load().flat_search_device(index._h, len(q), ctypes.c_void_p(q.data_ptr()), k, ctypes.c_void_p(D.data_ptr()),
+                                                    ctypes.c_void_p(I.data_ptr())))
+        return time.perf_counter() - t
+    search.index = index   # (lives as long as the function)
+    return search
+
+
+def test_flat_queries_without_proof_do_not_change_the_plan_of_the_next_batch(ix):
+    """An undefined query, or one amid more near ties than its candidate list has room for, is served by other plans; the next
+    batches keep the fast one (sixteen of them took up to three times as long when one such query was enough)."""
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    base = torch.randn(500000, 128, generator=gen, device="cuda")
+    base[:2000] = base[0] + 1e-5 * torch.randn(2000, 128, generator=gen, device="cuda")
+    search = _flat_on_device(ix, base, 10)
+    for nq in (1, 10, 300):
+        q = torch.randn(nq, 128, generator=gen, device="cuda")
+        undefined, tied = q.clone(), q.clone()
+        undefined[0, 5] = float("nan")
+        tied[0] = base[0]
+        best = min(search(q) for _ in range(10))
+        for odd in (undefined, tied):
+            search(odd)
+            assert min(search(q) for _ in range(10)) < 1.6 * best, nq
+
+
+def test_flat_batches_with_some_unproven_queries_keep_the_faster_plan(ix):
+    """An offset of 2 leaves a few of 300 queries unproven by splits: their second plan is cheaper than the older plan for all of them
+    (2.4 times as long when any such batch sent the next sixteen there)."""
+    gen = torch.Generator(device="cuda").manual_seed(4)
+    centres = torch.randn(1024, 128, generator=gen, device="cuda")
+
+    def rows(n):
+        which = torch.randint(0, 1024, (n,), generator=gen, device="cuda")
+        return centres[which] + 0.25 * torch.randn(n, 128, generator=gen, device="cuda")
+
+    base, batches, mean = rows(500000), [rows(300) for _ in range(24)], []
+    for offset in (0, 2):
+        search = _flat_on_device(ix, base + offset, 100)
+        times = [search(q + offset) for q in batches]
+        mean.append(sum(times[4:]) / len(times[4:]))
+    assert mean[1] < 1.8 * mean[0], mean
