@@ -836,7 +836,7 @@ void IvfpqIndex::coarse_select(const float *x_dev, int64_t n, int nout, int sele
     // us (score matrix or sampled bound / this): 1M x 128 to 1024 lists 10996 / 4175, 20000 to 4096 590 / 221, 100000 to 16384
     // 2508 / 1524, 100 to 1000 116 / 91; 50000 x 200 to 1500 1165 / 422; 20000 x 768 to 1024 898 / 650.
     if (cfg_.coarse_bf16 && nout == 1 && !out_dist && select_metric == kMetricL2 &&
-        resident_assign_serves(x_dev, centroids_.data(), nlist_, d_)) {
+        resident_assign_serves(x_dev, centroids_.data(), nlist_, d_) && resident_assign_pays(n, nlist_, d_)) {
         last_coarse_exact_ = true;
         last_coarse_plan_ = 0;
         last_coarse_n_ = n;

@@ -40,6 +40,7 @@ void launch_centre_centroids(const float *C, int64_t nc, int d, const float *cn,
 // for the host to read.  cn: canonical squared norms; cmax: the largest centroid length; scratch: memory that nothing queued behind
 // the call relies on, resized to at most scratch_bytes (or what 256 vectors take).
 bool resident_assign_serves(const float *X, const float *C, int64_t nc, int d);
+bool resident_assign_pays(int64_t n, int64_t nc, int d);
 void launch_resident_assign(const float *X, int64_t n, const float *C, int64_t nc, int d, const float *cn, float cmax,
                             const AssignCentroids &centred, int32_t *out, DeviceBuffer<float> &scratch, int64_t scratch_bytes, hipStream_t s);
 

@@ -811,11 +811,25 @@ bool launch_resident_f32(const float *Q, int64_t nq, const float *B, int64_t nb,
     return true;
 }
 
-// (Above 512 dimensions a tile holds 32 centroids and every vector is read once per tile: adding 40000 x 768, score matrix / this in
-// us: 1500 lists 2271 / 1125, 2048 1887 / 1308, 8192 3121 / 3794; 512 dimensions, 4096 lists 1909 / 997, 384, 8192 1769 / 1272.)
+// Above 512 dimensions a tile holds 32 centroids and every vector is read once per tile (adding 40000 x 768, score matrix / this in us:
+// 1500 lists 2271 / 1125, 2048 1887 / 1308, 8192 3121 / 3794; 512 dimensions, 4096 lists 1909 / 997, 384, 8192 1769 / 1272).
 bool resident_assign_serves(const float *X, const float *C, int64_t nc, int d)
 {
     return resident_f32_serves(d) && (d <= 512 || nc <= 4096) && reinterpret_cast<uintptr_t>(X) % 16 == 0 && reinterpret_cast<uintptr_t>(C) % 16 == 0;
+}
+
+// Whether n vectors are assigned faster than from the score matrix, or by the sampled bound.  Many centroids of many dimensions are
+// read for every tile of vectors, and some thousand vectors are too few to share that (adding, us, the older plans / this):
+//   16384 x 512: 30 vectors 145 / 155, 1000 203 / 274, 5000 537 / 557, 20000 1753 / 1670, 100000 8292 / 7020;
+//   50000 x 128: 30 104 / 117, 1000 166 / 186, 5000 378 / 380, 20000 1236 / 973; 16384 x 256: 30 114 / 101, 1000 161 / 156;
+//   4096 x 1024, with 32 centroids to a tile: 300 235 / 210, 1000 250 / 283, 5000 538 / 579, 20000 1598 / 1644, 100000 7470 / 6553;
+//   4096 x 768: 300 204 / 176, 1000 216 / 232, 5000 458 / 462, 20000 1299 / 1261.
+bool resident_assign_pays(int64_t n, int64_t nc, int d)
+{
+    if (d > 512 && nc * d > 2500000) {
+        return n <= 512 || n >= 32768;
+    }
+    return nc * d <= 5000000 || n >= 16384;
 }
 
 // Every workgroup adds up the mean of up to 64 of the centroids for itself (a component without one: 0), then takes the centroids

@@ -1162,6 +1162,21 @@ def test_assignment_of_crowds(ix, oracle, d, nlist, n):
         assert np.array_equal(got[keep], want[keep]) and got[3] == -1
 
 
+# Many centroids of many dimensions: batches on both sides of the lines where the assignment kernel takes over from the older plans.
+@pytest.mark.parametrize("d,nlist,few,many", [(128, 40000, 700, 16384), (1024, 2600, 513, 32768), (1024, 2600, 512, 600)])
+def test_assignment_is_the_same_by_either_plan(ix, oracle, d, nlist, few, many):
+    rng = np.random.default_rng(d)
+    cent = rng.standard_normal((nlist, d)).astype(np.float32)
+    cent[nlist // 2] = cent[3]
+    x = (cent[rng.integers(0, nlist, many)] + 0.5 * rng.standard_normal((many, d)).astype(np.float32))
+    x[5] = cent[3]
+    index = ix.AscendIndexIVFPQ(d, ix.METRIC_L2, nlist, 4, 8)
+    index.set_trained(cent, rng.standard_normal((4, 256, d // 4)).astype(np.float32))
+    got = index.assign(x)
+    assert np.array_equal(index.assign(x[:few]), got[:few])
+    assert np.array_equal(got[:40], oracle.assign(x[:40], cent))
+
+
 def test_assignment_and_search_share_the_scratch(ix):
     """What an assignment keeps per vector lies in the memory that a search writes its scores to: after a search that has used up the
     scratch, assigning takes no more than the vectors and the answers themselves (beside a scratch of its own it took 50 MB more)."""
