@@ -745,11 +745,13 @@ void FlatIndex::search_masked(int64_t n, const float *x, int64_t k, float *dist,
     split_rows = std::min<int64_t>(split_rows / 2048 * 2048, round_up(ntotal_, 2048));
     const bool can_split = !mask_dev && bmax_ >= 1e-6f && finite_;
     Candidates from = Candidates::kFp32;
+    bool resting = false;
     if (can_split && resident_f32_serves(d_) && reinterpret_cast<uintptr_t>(xd) % 16 == 0 && resident_pays(n, ntotal_, d_)) {
         if (resident_rest_ == 0) {
             from = Candidates::kResident;
         } else {
             resident_rest_--;
+            resting = true;
         }
     }
     if (from == Candidates::kFp32 && can_split && split_rows >= 16384 &&
@@ -804,13 +806,18 @@ void FlatIndex::search_masked(int64_t n, const float *x, int64_t k, float *dist,
             // sixteen batches that would take splits go without, and the one after them tries again.
             split_rest_ = open * 8 > n || (open > 0 && n < 1024) ? 16 : split_rest_;
         } else {
-            // (resident_pays has the times.)  A batch of up to 128 queries is slower than the older plans alone when one of them is
-            // unproven, larger ones when about half are.  One such batch may be its queries' own affair; after two in a row, and
-            // after each that follows without a proven one between, sixteen go without.
-            const bool missed = 2 * ((open + 127) / 128) > (n + 127) / 128;
+            // What the older plans take for such a batch is known once they have served one.  A batch that was not proven at once and
+            // took longer, or nobody knows, is a miss; one may be its queries' own affair, but after two in a row, and after each that
+            // follows without a better batch between, sixteen go to the older plans.
+            const double ms = stats_.ms_score + stats_.ms_select;
+            const bool known = older_.n == n && older_.k == k && older_.ntotal == ntotal_;
+            const bool missed = open > 0 && !(known && 1.1 * ms <= older_.ms);   // (a tenth for the host between the plans)
             resident_misses_ = missed ? std::min(resident_misses_ + 1, 2) : 0;
             resident_rest_ = resident_misses_ == 2 ? 16 : 0;
         }
+    }
+    if (resting) {
+        older_ = {n, k, ntotal_, stats_.ms_score + stats_.ms_select};
     }
     if (!rows.empty()) {
         IXA_HIP(hipEventRecord(ev_[1], stream_));

@@ -128,6 +128,10 @@ private:
     bool finite_ = true; // no vector of the base has an infinite or undefined norm
     int split_rest_ = 0;   // batches that go without splits formed beforehand, after one that they left largely unproven
     int resident_rest_ = 0, resident_misses_ = 0;   // the same for splits formed in the score kernel, and such batches in a row
+    struct {
+        int64_t n = 0, k = 0, ntotal = 0;
+        double ms = 0.0;
+    } older_;   // device time of the last batch that went without, before what no plan proved
 };
 
 class FlatI8Index : public FlatBase<int8_t> {
