@@ -145,9 +145,9 @@ __device__ __forceinline__ float score_margin(float qnorm, float cmax, float err
     return lost ? __builtin_inff() : err_scale * qlen * cmax + round_scale * (qlen + cmax) * (qlen + cmax);
 }
 
-// By how much a u of the assignment kernel (resident_f32.hip) has to lead another for the canonical scores to be in that order.  With a = |x - centre|, b = the largest
-// |c - centre|, L = |x| and cmax the largest |c|, what separates -2 u from the canonical score of the same centroid, but for
-// what all centroids share:
+// By how much a u of the assignment kernel (resident_f32.hip) has to lead another for the canonical scores to be in that order.
+// With a = |x - centre|, b = the largest |c - centre|, L = |x| and cmax the largest |c|, what separates -2 u from the canonical
+// score of the same centroid, but for what all centroids share:
 //   the canonical score  (|x|^2 + |c|^2) - g - g: g's d products and sums, 2 (d + 1) 2^-24 L cmax, and three roundings,
 //                        3 x 2^-24 (L + cmax)^2.  Its |c|^2, which is rounded itself, is the one that u starts from
 //                        (launch_centre_centroids), so that makes no difference;

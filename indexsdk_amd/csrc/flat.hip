@@ -850,7 +850,8 @@ std::vector<int64_t> FlatIndex::search_plan(int64_t n, const float *xd, int64_t 
 {
     const bool split = from == Candidates::kSplit, resident = from == Candidates::kResident;
     const int dp = (int)round_up(d_, 32);
-    const int ncand = (int)std::min<int64_t>(std::max<int64_t>(ntotal_, 1), split || resident ? split_candidates(k, dp, metric_, resident) : k + 8 + k / 8);
+    const int ncand = (int)std::min<int64_t>(std::max<int64_t>(ntotal_, 1),
+                                             split || resident ? split_candidates(k, dp, metric_, resident) : k + 8 + k / 8);
     ws_qn_.resize((size_t)n);
     ws_running_.resize((size_t)n * ncand);
     ws_cand_.resize((size_t)n * ncand);

@@ -42,6 +42,7 @@ void launch_centre_centroids(const float *C, int64_t nc, int d, const float *cn,
 bool resident_assign_serves(const float *X, const float *C, int64_t nc, int d);
 bool resident_assign_pays(int64_t n, int64_t nc, int d);
 void launch_resident_assign(const float *X, int64_t n, const float *C, int64_t nc, int d, const float *cn, float cmax,
-                            const AssignCentroids &centred, int32_t *out, DeviceBuffer<float> &scratch, int64_t scratch_bytes, hipStream_t s);
+                            const AssignCentroids &centred, int32_t *out, DeviceBuffer<float> &scratch, int64_t scratch_bytes,
+                            hipStream_t s);
 
 }  // namespace ixa

@@ -19,10 +19,12 @@
 //     sees to it that every base element is finite).  A batch is converted at once, which frees its registers for the next
 //     batch's loads: they have SPB K-steps to arrive.
 //
-// 1M x 128, 1000 queries: 1.23 PFLOP/s of bf16 products in the longest launch (0.71 of the ring kernel that reads split rows); a
-// search 1763 -> 964 us.  Assignment of 1M x 128 to 1024 centroids: 660 us of score launch at 1.19 PFLOP/s, 100 us for the tiles' best
-// and 26 us for what they leave open, where scores, selections and the refinement took 7.6 ms.  What bounds it is what bounds the int8 kernel: the clock under dense matrix work, and LDS reads (85
-// bytes per cycle and CU of 128); with few queries the base's bytes (512 MB in 100 us of the 207 of one query over 1M x 128).
+// 1M x 128, 1000 queries: a search 1763 -> 964 us on the device; 1.23 PFLOP/s of bf16 products in the longest launch (the ring kernel
+// that reads split rows: 0.71), matrix cores busy 70 % of the CU's cycles at the 1.9 GHz that they hold, the LDS pipe 28 %, wavefronts
+// waiting a quarter of theirs; with few queries the base's bytes (512 MB in 100 us of the 207 of one query).  Assignment of 1M x 128 to
+// 1024 centroids, where scores, selections and the refinement took 7.6 ms: norms and bounds 94 us, the score launch 655 us (1.20 PFLOP/s,
+// matrix cores busy 65 %: five vector instructions per matrix instruction, most of them the three largest of every sum), the tiles' best
+// 96 us, what they leave open 17 us.
 //
 // Score arithmetic: the accumulators start from -|b|^2 / 2 (L2; 0 for inner product) and end as u = q.b - |b|^2 / 2, and the
 // score is fma(-2, u, |q|^2), or -u.  The admission test of a block of 16 rows is one compare of the largest u with a value
@@ -811,11 +813,12 @@ bool launch_resident_f32(const float *Q, int64_t nq, const float *B, int64_t nb,
     return true;
 }
 
-// Above 512 dimensions a tile holds 32 centroids and every vector is read once per tile (adding 40000 x 768, score matrix / this in us:
-// 1500 lists 2271 / 1125, 2048 1887 / 1308, 8192 3121 / 3794; 512 dimensions, 4096 lists 1909 / 997, 384, 8192 1769 / 1272).
+// Above 512 dimensions a tile holds 32 centroids and every vector is read once per tile (adding 40000 x 768, score matrix / this in
+// us: 1500 lists 2271 / 1125, 2048 1887 / 1308, 8192 3121 / 3794; 512 dimensions, 4096 lists 1909 / 997, 384, 8192 1769 / 1272).
 bool resident_assign_serves(const float *X, const float *C, int64_t nc, int d)
 {
-    return resident_f32_serves(d) && (d <= 512 || nc <= 4096) && reinterpret_cast<uintptr_t>(X) % 16 == 0 && reinterpret_cast<uintptr_t>(C) % 16 == 0;
+    return resident_f32_serves(d) && (d <= 512 || nc <= 4096) && reinterpret_cast<uintptr_t>(X) % 16 == 0 &&
+           reinterpret_cast<uintptr_t>(C) % 16 == 0;
 }
 
 // Whether n vectors are assigned faster than from the score matrix, or by the sampled bound.  Many centroids of many dimensions are
@@ -887,7 +890,8 @@ void launch_centre_centroids(const float *C, int64_t nc, int d, const float *cn,
 }
 
 void launch_resident_assign(const float *X, int64_t n, const float *C, int64_t nc, int d, const float *cn, float cmax,
-                            const AssignCentroids &centred, int32_t *out, DeviceBuffer<float> &scratch, int64_t scratch_bytes, hipStream_t s)
+                            const AssignCentroids &centred, int32_t *out, DeviceBuffer<float> &scratch, int64_t scratch_bytes,
+                            hipStream_t s)
 {
     if (n <= 0) {
         return;
@@ -918,8 +922,8 @@ void launch_resident_assign(const float *X, int64_t n, const float *C, int64_t n
                                   ScoreFilter<float>{}, assign, s});
         hipLaunchKernelGGL(assign_combine_kernel, dim3((unsigned)((m + 255) / 256)), dim3(256), 0, s, top, (int)tiles, qt, m, need,
                            out + i0, pairs, rows, count);
-        hipLaunchKernelGGL(assign_resolve_kernel, dim3((unsigned)std::min<int64_t>(m, device_cus() * 4)), dim3(256), 0, s, xi, xn, m, C, cn, nc, d, assign,
-                           (int)tiles, qt, pairs, rows, count, out + i0);
+        hipLaunchKernelGGL(assign_resolve_kernel, dim3((unsigned)std::min<int64_t>(m, device_cus() * 4)), dim3(256), 0, s, xi, xn, m, C,
+                           cn, nc, d, assign, (int)tiles, qt, pairs, rows, count, out + i0);
     }
 }
 

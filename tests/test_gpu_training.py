@@ -152,7 +152,7 @@ def test_codes_of_offset_and_tied_sub_vectors(oracle, dsub, offset):
 
 def test_tied_and_offset_sub_vectors_are_encoded_about_as_fast_as_others():
     """Adding to two lists is mostly encoding: equal codewords took 4.3 times the time of distinct ones, an offset of 30 three times,
-    when vectors whose bound does not decide were handled one at a time (1.3 times and the same now)."""
+    when vectors whose bound does not decide were handled one at a time (1.1 times now)."""
     import ctypes
     import time
 
