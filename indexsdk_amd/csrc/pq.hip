@@ -39,9 +39,9 @@ constexpr float kPqFar = 3.402823466e+38f;   // a codeword at this distance or f
 //   distance by 2 x 2^-24 (|x| + |c|)^2.  Lengths below 1e-15, where products may vanish, decide nothing.
 // Per 32 vectors: KS matrix instructions and a maximum over 16 per block, and 16 distances, where every lane walking 256
 // codewords for its own vector took 256 of them: 20000 x 32 sub-quantizers of 4 dimensions 55 -> 20 us,
-//   131072 x 32 280 -> 70 (88 on the sub-vectors of a training), 20000 x 4 of 32 dimensions 75 -> 34.  Adding 100000 x 64 of 2 dimensions to two lists, every lane walking
-//   / this: 864 / 303 us; an offset of 30 851 / 305; codewords in runs of eight equal ones 920 / 395 (4 of 32 dimensions: 858 / 352,
-//   805 / 290, 832 / 368).
+//   131072 x 32 280 -> 70 (88 on the sub-vectors of a training), 20000 x 4 of 32 dimensions 75 -> 34.  Adding 100000 x 64 of 2
+//   dimensions to two lists, every lane walking / this: 864 / 303 us; an offset of 30 851 / 305; codewords in runs of eight equal
+//   ones 920 / 395 (4 of 32 dimensions: 858 / 352, 805 / 290, 832 / 368).
 // What bounds it at 4 dimensions: the LDS pipe, active in 71 % of a CU's cycles, three quarters of that with bank conflicts of the lanes'
 // codewords (each lane reads those of its own group); matrix cores busy 21 %, 45 vector instructions to a matrix instruction.
 constexpr int kPqWalk = 11, kPqWalks = 7;

@@ -90,7 +90,7 @@ __device__ __forceinline__ float test_value(float qn, float tau, bool l2)
 
 // The larger of two numbers, or the number where the other is a NaN.  (fmaxf would make v a quiet number first, an instruction
 // each.  The operands are results of vector instructions, never of a matrix instruction, whose results an inline instruction
-// would not wait for.  A signalling NaN takes m away instead: assign_need rules the sums out that could become one.)
+// would not wait for.  A signalling NaN takes m away instead: AssignBound rules the sums out that could become one.)
 __device__ __forceinline__ float max_number(float m, float v)
 {
     float r;
@@ -896,7 +896,8 @@ void launch_resident_assign(const float *X, int64_t n, const float *C, int64_t n
     if (n <= 0) {
         return;
     }
-    IXA_REQUIRE(resident_assign_serves(X, C, nc, d) && nc >= 1 && n < ((int64_t)1 << 31), kErrInner, "assignment kernel does not serve these operands");
+    IXA_REQUIRE(resident_assign_serves(X, C, nc, d) && nc >= 1 && n < ((int64_t)1 << 31), kErrInner,
+                "assignment kernel does not serve these operands");
     const int qt = 32 * tile_blocks(nc, d);
     const int64_t tiles = (nc + qt - 1) / qt;
     // vectors per pass, and what the scratch holds of them, the widest first: of every tile the best two centroids and its crowd; what
